@@ -22,6 +22,26 @@ if not os.path.exists(LIB_PATH):
 
 lib = ctypes.CDLL(LIB_PATH)
 
+_torch_module = None
+
+
+def torch_module():
+    """The native module over the library (csrc/ap_torch.cpp); torch has to be imported before it is loaded."""
+    global _torch_module
+    if _torch_module is None:
+        import importlib.machinery
+        import importlib.util
+
+        path = os.path.join(_PKG_ROOT, "lib", "_anyprec_torch.so")
+        if not os.path.exists(path):
+            raise ModuleNotFoundError(f"{path} is missing: build it with `python any-precision-llm_amd/build.py`.")
+        loader = importlib.machinery.ExtensionFileLoader("_anyprec_torch", path)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_anyprec_torch", loader))
+        loader.exec_module(module)
+        _torch_module = module
+    return _torch_module
+
+
 _vp, _ci = ctypes.c_void_p, ctypes.c_int
 lib.ap_abi_version.argtypes = []
 lib.ap_abi_version.restype = _ci

@@ -10,7 +10,8 @@ fused dequant -> MFMA GEMM (the reference's ``dequant_kbit`` + ``torch.matmul`` 
 AnyPrecisionLinear.py:60-62, in one launch per ``GEMM_MAX_M`` activation rows).
 
 The ops validate their arguments, allocate the result with torch and hand raw
-device pointers plus torch's current HIP stream to libanyprec_hip.so.  Where
+device pointers plus torch's current HIP stream to libanyprec_hip.so -- the three ops on one linear
+in native code (csrc/ap_torch.cpp), which leaves to Python only to say what is wrong.  Where
 the reference asserts (compiled out in release builds) or exits the process,
 these raise ``ValueError`` / ``RuntimeError``.  Launches go to the *current*
 stream (the reference uses the legacy default stream, main.cu:83,134), so the
@@ -27,6 +28,7 @@ __all__ = ["matmul_kbit", "dequant_kbit", "dequant_kbit_group", "gemm_kbit", "ge
 GEMM_MAX_M = _capi.GEMM_MAX_M
 
 _lib = _capi.lib
+_native = _capi.torch_module()
 
 
 def _check_weight(qweight: torch.Tensor, lut: torch.Tensor, w_bits: int, op: str):
@@ -53,14 +55,29 @@ def _check_weight(qweight: torch.Tensor, lut: torch.Tensor, w_bits: int, op: str
     return N, W * 32
 
 
+def _check_product(in_, qweight, lut, w_bits, op):
+    """Raises what is wrong with the arguments of a product (the batch limit of matmul_kbit aside)."""
+    _, K = _check_weight(qweight, lut, w_bits, op)
+    if in_.dtype != torch.float16:
+        raise ValueError(f"{op}: input must be float16, got {in_.dtype}")
+    if in_.device != qweight.device:
+        raise ValueError(f"{op}: input on {in_.device}, weight on {qweight.device}")
+    if in_.dim() < 1 or in_.shape[-1] != K:
+        raise ValueError(f"{op}: input last dim must be K={K}, got {tuple(in_.shape)}")
+    if in_.numel() < 1:
+        raise ValueError(f"{op}: empty batch M=0")
+    if op == "matmul_kbit" and in_.numel() // K > 8:
+        return
+    if not in_.is_contiguous():
+        raise ValueError(f"{op}: input must be contiguous")
+
+
 def dequant_kbit(qweight: torch.Tensor, lut: torch.Tensor, w_bits: int) -> torch.Tensor:
     """fp16 [N, K] with out[n, k] = lut[n, code[n, k] >> (P - w_bits)]."""
-    N, K = _check_weight(qweight, lut, w_bits, "dequant_kbit")
-    with torch.cuda.device(qweight.device):
-        out = torch.empty((N, K), dtype=torch.float16, device=qweight.device)
-        rc = _lib.ap_dequant_kbit(qweight.data_ptr(), lut.data_ptr(), out.data_ptr(), N, K, w_bits,
-                                  torch.cuda.current_stream().cuda_stream)
-    _capi.check(rc, "dequant_kbit")
+    out = _native.dequant_kbit(qweight, lut, w_bits)
+    if out is None:
+        _check_weight(qweight, lut, w_bits, "dequant_kbit")
+        raise ValueError("dequant_kbit: arguments not supported")
     return out
 
 
@@ -84,23 +101,11 @@ def dequant_kbit_group(qweights, luts, w_bits: int):
 
 def matmul_kbit(in_: torch.Tensor, qweight: torch.Tensor, lut: torch.Tensor, w_bits: int) -> torch.Tensor:
     """fp16 in_.shape[:-1] + [N]; M = in_.numel() // K must be in 1..8 (main.cu:108)."""
-    N, K = _check_weight(qweight, lut, w_bits, "matmul_kbit")
-    if in_.dtype != torch.float16:
-        raise ValueError(f"matmul_kbit: input must be float16, got {in_.dtype}")
-    if in_.device != qweight.device:
-        raise ValueError(f"matmul_kbit: input on {in_.device}, weight on {qweight.device}")
-    if in_.dim() < 1 or in_.shape[-1] != K:
-        raise ValueError(f"matmul_kbit: input last dim must be K={K}, got {tuple(in_.shape)}")
-    M = in_.numel() // K
-    if M < 1 or M > 8:
+    out = _native.matmul_kbit(in_, qweight, lut, w_bits)
+    if out is None:
+        _check_product(in_, qweight, lut, w_bits, "matmul_kbit")
+        M = in_.numel() // in_.shape[-1]
         raise ValueError(f"matmul_kbit: batch M={M} outside 1..8; use dequant_kbit + matmul for larger batches")
-    if not in_.is_contiguous():
-        raise ValueError("matmul_kbit: input must be contiguous")
-    with torch.cuda.device(qweight.device):
-        out = torch.empty(in_.shape[:-1] + (N,), dtype=torch.float16, device=in_.device)
-        rc = _lib.ap_matmul_kbit(in_.data_ptr(), qweight.data_ptr(), lut.data_ptr(), out.data_ptr(), M, N, K,
-                                 w_bits, torch.cuda.current_stream().cuda_stream)
-    _capi.check(rc, "matmul_kbit")
     return out
 
 
@@ -219,21 +224,8 @@ def matmul_kbit_swiglu(in_: torch.Tensor, qweight_gate, lut_gate, qweight_up, lu
 def gemm_kbit(in_: torch.Tensor, qweight: torch.Tensor, lut: torch.Tensor, w_bits: int) -> torch.Tensor:
     """fp16 in_.shape[:-1] + [N] = in_ @ dequant(qweight, lut, w_bits).T without materialising the fp16
     weight; one launch per GEMM_MAX_M rows."""
-    N, K = _check_weight(qweight, lut, w_bits, "gemm_kbit")
-    if in_.dtype != torch.float16:
-        raise ValueError(f"gemm_kbit: input must be float16, got {in_.dtype}")
-    if in_.device != qweight.device:
-        raise ValueError(f"gemm_kbit: input on {in_.device}, weight on {qweight.device}")
-    if in_.dim() < 1 or in_.shape[-1] != K:
-        raise ValueError(f"gemm_kbit: input last dim must be K={K}, got {tuple(in_.shape)}")
-    M = in_.numel() // K
-    if M < 1:
-        raise ValueError("gemm_kbit: empty batch")
-    if not in_.is_contiguous():
-        raise ValueError("gemm_kbit: input must be contiguous")
-    with torch.cuda.device(qweight.device):
-        out = torch.empty(in_.shape[:-1] + (N,), dtype=torch.float16, device=in_.device)
-        rc = _lib.ap_gemm_kbit(in_.data_ptr(), qweight.data_ptr(), lut.data_ptr(), out.data_ptr(), M, N, K,
-                               w_bits, torch.cuda.current_stream().cuda_stream)
-    _capi.check(rc, "gemm_kbit")
+    out = _native.gemm_kbit(in_, qweight, lut, w_bits)
+    if out is None:
+        _check_product(in_, qweight, lut, w_bits, "gemm_kbit")
+        raise ValueError("gemm_kbit: arguments not supported")
     return out

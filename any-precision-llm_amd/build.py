@@ -1,6 +1,6 @@
 """Builds the in-tree native libraries of this package.
 
-    python build.py            # libanyprec_hip.so (hipcc, gfx950) + host-check lib (g++)
+    python build.py            # libanyprec_hip.so (hipcc, gfx950), the torch module over it and the host-check lib (g++)
 
 The HIP library is cross-compiled; no GPU is needed to build it.
 """
@@ -18,6 +18,7 @@ OBJDIR = os.path.join(HERE, "build")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 
 HIP_LIB = os.path.join(LIBDIR, "libanyprec_hip.so")
+TORCH_MODULE = os.path.join(LIBDIR, "_anyprec_torch.so")
 HOSTCHECK_LIB = os.path.join(LIBDIR, "libanyprec_hostcheck.so")
 
 HIPCC_FLAGS = [
@@ -71,6 +72,24 @@ def build_hip(verbose: bool = False, extra_flags=(), jobs: int = 8) -> str:
     return HIP_LIB
 
 
+def build_torch(verbose: bool = False) -> str:
+    """The Python module over libanyprec_hip.so (host code only).  torch's libraries are found by name: whoever imports the
+    module has imported torch before."""
+    import sysconfig
+
+    import torch
+    torch_dir = os.path.dirname(torch.__file__)
+    include = os.path.join(torch_dir, "include")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE, "-isystem", include,
+           "-isystem", os.path.join(include, "torch", "csrc", "api", "include"), "-isystem", "/opt/rocm/include",
+           "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, "ap_torch.cpp"), "-o", TORCH_MODULE,
+           "-L", LIBDIR, "-lanyprec_hip", "-L", os.path.join(torch_dir, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu",
+           "-ltorch_hip", "-ltorch", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    _run(cmd, verbose)
+    return TORCH_MODULE
+
+
 def build_hostcheck(verbose: bool = False) -> str:
     os.makedirs(LIBDIR, exist_ok=True)
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unknown-pragmas", "-I", CSRC,
@@ -83,9 +102,10 @@ def build_hostcheck(verbose: bool = False) -> str:
 
 def build_all(verbose: bool = False) -> None:
     build_hip(verbose)
+    build_torch(verbose)
     build_hostcheck(verbose)
 
 
 if __name__ == "__main__":
     build_all(verbose=True)
-    print("built:", HIP_LIB, HOSTCHECK_LIB)
+    print("built:", HIP_LIB, TORCH_MODULE, HOSTCHECK_LIB)

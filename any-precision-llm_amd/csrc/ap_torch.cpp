@@ -1,0 +1,205 @@
+// Native side of any_precision_ext and AnyPrecisionLinear: the checks, the allocation of the result and the launch of one
+// call, as Python functions over torch tensors.
+//
+// A linear's kernel takes 4 to 15 us at the batch sizes of decoding; the same steps written in Python over ctypes take
+// 11 to 15 us of host time per call, and a stream of such calls runs at the host's pace (28 linears of four decoder layers
+// at one row and 3 bits: 400 us of which the GPU works 167).  Here a call takes about 4 us, most of it HIP's launch.
+//
+// A function returns None for anything it does not serve -- wrong types, shapes, devices, layouts -- and the Python side
+// then takes the way that says what is wrong (or serves the case, where it can).  Errors of the library raise here.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "anyprec_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+PyObject *none() { Py_RETURN_NONE; }
+
+// Set when a C++ exception has been turned into a Python error.
+template <typename F>
+PyObject *guarded(F &&f) {
+    try {
+        return f();
+    } catch (const c10::Error &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
+    } catch (const std::exception &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+    }
+    return nullptr;
+}
+
+PyObject *library_error(int rc, const char *op) {
+    if (rc < 0) PyErr_Format(PyExc_ValueError, "%s: %s (code %d)", op, ap_strerror(rc), rc);
+    else PyErr_Format(PyExc_RuntimeError, "%s: HIP error %d: %s", op, rc, ap_strerror(rc));
+    return nullptr;
+}
+
+bool is_tensor(PyObject *o) { return o != nullptr && THPVariable_Check(o); }
+
+// A bit-width given as an int in 3..8, else 0.
+int bits_of(PyObject *o) {
+    if (!PyLong_Check(o) || PyBool_Check(o)) return 0;
+    const long b = PyLong_AsLong(o);
+    if (b == -1 && PyErr_Occurred()) PyErr_Clear();
+    return b >= 3 && b <= 8 ? (int)b : 0;
+}
+
+struct Weight {
+    const uint32_t *planes;
+    const uint16_t *lut;
+    int N, K;
+    c10::DeviceIndex device;
+};
+
+bool weight_of(const Tensor &q, const Tensor &t, int bits, Weight *w) {
+    if (!q.is_cuda() || q.scalar_type() != at::kInt || q.dim() != 3 || !q.is_contiguous()) return false;
+    if (!t.is_cuda() || t.scalar_type() != at::kHalf || t.dim() != 2 || !t.is_contiguous() || t.device() != q.device()) return false;
+    const int64_t planes = q.size(0), N = q.size(1), W = q.size(2);
+    if (planes < bits || N < 1 || W < 1 || N > INT32_MAX || W > INT32_MAX / 32) return false;
+    if (t.size(0) != N || t.size(1) != (int64_t)1 << bits) return false;
+    w->planes = reinterpret_cast<const uint32_t *>(q.data_ptr());
+    w->lut = reinterpret_cast<const uint16_t *>(t.data_ptr());
+    w->N = (int)N;
+    w->K = (int)(W * 32);
+    w->device = q.device().index();
+    return true;
+}
+
+// Activation rows of x for a linear of K inputs, or 0.
+int64_t rows_of(const Tensor &x, const Weight &w) {
+    if (!x.is_cuda() || x.scalar_type() != at::kHalf || x.dim() < 1 || x.device().index() != w.device) return 0;
+    if (x.size(-1) != w.K) return 0;
+    const int64_t rows = x.numel() / w.K;
+    return rows <= INT32_MAX ? rows : 0;
+}
+
+const uint16_t *half_ptr(const Tensor &t) { return reinterpret_cast<const uint16_t *>(t.data_ptr()); }
+uint16_t *half_out(const Tensor &t) { return reinterpret_cast<uint16_t *>(t.data_ptr()); }
+
+Tensor empty_half(at::IntArrayRef shape, const at::Device &device) {
+    return Tensor(at::detail::empty_cuda(shape, at::kHalf, device, std::nullopt));
+}
+
+// A result of x's leading dimensions and N columns.
+Tensor result_for(const Tensor &x, int64_t N) {
+    c10::SmallVector<int64_t, 6> shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = N;
+    return empty_half(shape, x.device());
+}
+
+// Makes the tensors' device the current one for a call (a no-op where it is) and gives its current stream.
+struct OnDevice {
+    explicit OnDevice(c10::DeviceIndex d) {
+        if (c10::hip::current_device() != d) guard.set_index(d);
+        stream = static_cast<void *>(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(d).stream());
+    }
+    c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard;
+    void *stream;
+};
+
+PyObject *wrap(Tensor t) { return THPVariable_Wrap(std::move(t)); }
+
+// matmul_kbit(x, qweight, lut, w_bits) and gemm_kbit(x, qweight, lut, w_bits)
+PyObject *product(PyObject *const *args, Py_ssize_t n, bool gemm) {
+    if (n != 4 || !is_tensor(args[0]) || !is_tensor(args[1]) || !is_tensor(args[2])) return none();
+    const int bits = bits_of(args[3]);
+    if (bits == 0) return none();
+    return guarded([&]() -> PyObject * {
+        const Tensor &x = THPVariable_Unpack(args[0]);
+        Weight w;
+        if (!weight_of(THPVariable_Unpack(args[1]), THPVariable_Unpack(args[2]), bits, &w)) return none();
+        const int64_t rows = rows_of(x, w);
+        if (rows < 1 || (!gemm && rows > 8) || !x.is_contiguous()) return none();
+        const OnDevice on(w.device);
+        Tensor out = result_for(x, w.N);
+        const int rc = gemm ? ap_gemm_kbit(half_ptr(x), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream)
+                            : ap_matmul_kbit(half_ptr(x), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream);
+        if (rc != AP_OK) return library_error(rc, gemm ? "gemm_kbit" : "matmul_kbit");
+        return wrap(std::move(out));
+    });
+}
+
+PyObject *matmul_kbit(PyObject *, PyObject *const *args, Py_ssize_t n) { return product(args, n, false); }
+PyObject *gemm_kbit(PyObject *, PyObject *const *args, Py_ssize_t n) { return product(args, n, true); }
+
+PyObject *dequant_kbit(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    if (n != 3 || !is_tensor(args[0]) || !is_tensor(args[1])) return none();
+    const int bits = bits_of(args[2]);
+    if (bits == 0) return none();
+    return guarded([&]() -> PyObject * {
+        const Tensor &q = THPVariable_Unpack(args[0]);
+        Weight w;
+        if (!weight_of(q, THPVariable_Unpack(args[1]), bits, &w)) return none();
+        const OnDevice on(w.device);
+        Tensor out = empty_half({w.N, w.K}, q.device());
+        const int rc = ap_dequant_kbit(w.planes, w.lut, half_out(out), w.N, w.K, bits, on.stream);
+        if (rc != AP_OK) return library_error(rc, "dequant_kbit");
+        return wrap(std::move(out));
+    });
+}
+
+// Keys of a module's buffers, made once.
+PyObject *key_qweight, *key_bias, *key_lut[9];
+
+// linear(buffers, x, w_bits): AnyPrecisionLinear.forward on the module's dict of buffers.  Up to 8 rows ap_matmul_kbit, then
+// ap_gemm_kbit where ap_gemm_kbit_pays, else the weight in fp16 and torch's own product (which takes part in autograd).
+PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    if (n != 3 || !PyDict_Check(args[0]) || !is_tensor(args[1])) return none();
+    const int bits = bits_of(args[2]);
+    if (bits == 0) return none();
+    PyObject *q = PyDict_GetItem(args[0], key_qweight), *t = PyDict_GetItem(args[0], key_lut[bits]);
+    PyObject *bias = PyDict_GetItem(args[0], key_bias);
+    if (!is_tensor(q) || !is_tensor(t)) return none();
+    if (bias == Py_None) bias = nullptr;
+    if (bias != nullptr && !is_tensor(bias)) return none();
+    return guarded([&]() -> PyObject * {
+        const Tensor &x = THPVariable_Unpack(args[1]);
+        Weight w;
+        if (!weight_of(THPVariable_Unpack(q), THPVariable_Unpack(t), bits, &w)) return none();
+        const int64_t rows = rows_of(x, w);
+        if (rows < 1) return none();
+        const OnDevice on(w.device);
+        const bool pays = rows <= 8 || ap_gemm_kbit_pays((int)rows, w.N, w.K, bits) == 1;
+        Tensor out;
+        if (pays) {
+            const Tensor dense = x.is_contiguous() ? x : x.contiguous();  // the kernels take dense rows
+            out = result_for(x, w.N);
+            const int rc = rows <= 8 ? ap_matmul_kbit(half_ptr(dense), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream)
+                                     : ap_gemm_kbit(half_ptr(dense), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream);
+            if (rc != AP_OK) return library_error(rc, rows <= 8 ? "matmul_kbit" : "gemm_kbit");
+        } else {
+            const Tensor dense = empty_half({w.N, w.K}, x.device());
+            const int rc = ap_dequant_kbit(w.planes, w.lut, half_out(dense), w.N, w.K, bits, on.stream);
+            if (rc != AP_OK) return library_error(rc, "dequant_kbit");
+            out = at::matmul(x, dense.t());
+        }
+        if (bias != nullptr) out.add_(THPVariable_Unpack(bias));
+        return wrap(std::move(out));
+    });
+}
+
+PyMethodDef methods[] = {
+    {"matmul_kbit", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(matmul_kbit)), METH_FASTCALL, nullptr},
+    {"gemm_kbit", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(gemm_kbit)), METH_FASTCALL, nullptr},
+    {"dequant_kbit", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(dequant_kbit)), METH_FASTCALL, nullptr},
+    {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(linear)), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_anyprec_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__anyprec_torch(void) {
+    key_qweight = PyUnicode_InternFromString("qweight");
+    key_bias = PyUnicode_InternFromString("bias");
+    for (int b = 3; b <= 8; b++) key_lut[b] = PyUnicode_InternFromString(("lut" + std::to_string(b)).c_str());
+    return PyModule_Create(&module);
+}
