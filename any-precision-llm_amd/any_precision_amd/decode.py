@@ -9,8 +9,9 @@ final norm, head, argmax, position increment -- is recorded once per precision a
 per token: no host work between tokens.  With ``fused_ops`` (the default) a layer is 7 launches, all
 of this library: the seven linears in four (q/k/v as one grouped launch; gate and up as one launch that
 also applies SiLU(gate) * up), residual add + RMSNorm twice, rotary + cache append + attention in one kernel.  Without it everything
-but the linears is stock PyTorch ops, as in the reference (19 launches per layer); that path also
-serves the prompt and is what the fused one is tested against.
+but the linears is stock PyTorch ops, as in the reference (19 launches per layer); that is what the fused step is tested
+against.  The prompt takes the same kernels on its rows, with two of its own for rotary + cache write and causal attention
+(9 launches per layer against 21 of stock ops).
 
 Supports Llama-style decoders (RMSNorm, rotary attention with optional grouped KV heads,
 SwiGLU MLP, no biases in norms); anything else raises.
@@ -36,7 +37,7 @@ def _rope(x, cos, sin_signed):
 class GraphDecoder:
     def __init__(self, ap_model, max_len=512, group_launches=True, fused_ops=True):
         """``group_launches``: issue the q/k/v and the gate/up GEMVs of a layer as one launch each.
-        ``fused_ops``: the decode step runs the library's add + RMSNorm, attention and SiLU * up kernels
+        ``fused_ops``: prompt and decode step run the library's add + RMSNorm, attention and SiLU * up kernels
         instead of stock PyTorch ops (head sizes 32, 64, 128, 256 and caches of up to 8192 rows)."""
         self.group_launches = group_launches
         cfg = ap_model.config
@@ -182,6 +183,51 @@ class GraphDecoder:
         add_norm(delta, self.final_norm)
         return torch.mm(self.f_x, self.head.t(), out=self.logits)
 
+    def _prompt_fused(self, ids, precision):
+        """The prompt ids [T] at cache rows 0 .. T-1 through the network -> logits of the last token [1, vocab].  What follows
+        the keys and values of the last layer is computed for the last token alone: nothing else is read of it."""
+        lib, st = _capi.lib, torch.cuda.current_stream(self.dev).cuda_stream
+        H, eps, T = self.cfg.hidden_size, float(self.eps), ids.shape[0]
+        scale = 1.0 / math.sqrt(self.hd)
+        h = self.embed.index_select(0, ids)
+        x = torch.empty_like(h)
+
+        def add_norm(delta, weight):          # h += delta; x = rmsnorm(h) * weight
+            _capi.check(lib.ap_add_rmsnorm(h.data_ptr(), 0 if delta is None else delta.data_ptr(), weight.data_ptr(),
+                                           h.data_ptr(), x.data_ptr(), h.shape[0], H, eps, st), "ap_add_rmsnorm")
+
+        def swiglu(gate, up):                 # silu(gate) * up, over gate
+            _capi.check(lib.ap_silu_mul(gate.data_ptr(), up.data_ptr(), gate.data_ptr(), gate.numel(), st), "ap_silu_mul")
+            return gate
+
+        delta = None
+        for li, layer in enumerate(self.layers):
+            att, mlp = layer.self_attn, layer.mlp
+            add_norm(delta, layer.input_layernorm.weight)
+            if self.group_launches:
+                qkv = forward_group((att.q_proj, att.k_proj, att.v_proj), x, precision, concat=True)
+            else:
+                qkv = torch.cat([m(x, precision=precision) for m in (att.q_proj, att.k_proj, att.v_proj)], dim=-1)
+            cache = (self.kcache[li].data_ptr(), self.vcache[li].data_ptr())
+            shape = (self.nh, self.nkv, self.hd, self.max_len)
+            _capi.check(lib.ap_prompt_rope(qkv.data_ptr(), self.cos32.data_ptr(), self.sin32.data_ptr(), *cache, T, *shape, st),
+                        "ap_prompt_rope")
+            first = T - 1 if li + 1 == len(self.layers) else 0
+            h, x = h[first:], x[first:]
+            ctx = torch.empty((T - first, self.nh * self.hd), dtype=torch.float16, device=self.dev)
+            _capi.check(lib.ap_prompt_attention(qkv.data_ptr(), *cache, ctx.data_ptr(), first, T, *shape, scale, st),
+                        "ap_prompt_attention")
+            add_norm(att.o_proj(ctx, precision=precision), layer.post_attention_layernorm.weight)
+            if not self.group_launches:
+                act = swiglu(mlp.gate_proj(x, precision=precision), mlp.up_proj(x, precision=precision))
+            elif T - first <= 4:
+                act = forward_swiglu(mlp.gate_proj, mlp.up_proj, x, precision)
+            else:
+                act = swiglu(*forward_group((mlp.gate_proj, mlp.up_proj), x, precision))
+            delta = mlp.down_proj(act, precision=precision)
+        add_norm(delta, self.final_norm)
+        return torch.mm(x, self.head.t(), out=self.logits)
+
     def _step(self, precision):
         """One decode step on the static state: consumes self.tok at self.pos, leaves the next token."""
         if self.fused_ops:
@@ -205,6 +251,14 @@ class GraphDecoder:
             raise ValueError(f"prompt length {T} outside 1..{self.max_len - 1}")
         self.stream.wait_stream(torch.cuda.current_stream(self.dev))     # the ids may still be in flight there
         with torch.cuda.stream(self.stream):
+            if self.fused_ops:
+                self._prompt_fused(ids, precision)           # writes self.logits
+                self.emitted.zero_()
+                self.emitted[:T] = ids
+                self.pos.fill_(T - 1)
+                advance(self.logits, self.pos, self.tok, self.emitted)
+                self.stream.synchronize()
+                return
             self.kvcache.zero_()
             pos_idx = torch.arange(T, device=self.dev)
             logits = self._forward(ids, pos_idx, precision)

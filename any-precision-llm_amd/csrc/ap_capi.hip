@@ -14,6 +14,7 @@
 #include "ap_gemvf_launch.hpp"
 #include "ap_gemvp_launch.hpp"
 #include "ap_probe.hpp"
+#include "ap_prompt.hpp"
 
 namespace {
 
@@ -339,6 +340,60 @@ int ap_decode_attention(const uint16_t *qkv, const float *cos_table, const float
         case 64: decode_attention_kernel<64><<<grid, block, 0, st>>>(q, cos_table, sin_table, kc, vc, pos, o, n_heads, n_kv_heads, max_len, scale); break;
         case 128: decode_attention_kernel<128><<<grid, block, 0, st>>>(q, cos_table, sin_table, kc, vc, pos, o, n_heads, n_kv_heads, max_len, scale); break;
         default: decode_attention_kernel<256><<<grid, block, 0, st>>>(q, cos_table, sin_table, kc, vc, pos, o, n_heads, n_kv_heads, max_len, scale); break;
+    }
+    return launch_status();
+}
+
+namespace {
+
+int check_prompt(int T, int nh, int nkv, int hd, int max_len) {
+    if (nh < 1 || nkv < 1 || nh % nkv) return AP_ESHAPE;
+    if (hd != 32 && hd != 64 && hd != 128 && hd != 256) return AP_ESHAPE;
+    if (T < 1 || T > max_len) return AP_ESHAPE;
+    return nh > 65535 || (long long)T * (nh + 2LL * nkv) * (hd / 16) > 0x7fffffffLL * kPromptRopeThreads ? AP_ELIMIT : AP_OK;
+}
+
+}  // namespace
+
+int ap_prompt_rope(uint16_t *qkv, const float *cos_table, const float *sin_table, uint16_t *kcache, uint16_t *vcache, int T,
+                   int n_heads, int n_kv_heads, int head_dim, int max_len, void *stream) {
+    if (!qkv || !cos_table || !sin_table || !kcache || !vcache) return AP_ENULL;
+    const int rc = check_prompt(T, n_heads, n_kv_heads, head_dim, max_len);
+    if (rc != AP_OK) return rc;
+    if (!aligned16(qkv) || !aligned16(kcache) || !aligned16(vcache)) return AP_EALIGN;
+    half_t *x = reinterpret_cast<half_t *>(qkv), *kc = reinterpret_cast<half_t *>(kcache), *vc = reinterpret_cast<half_t *>(vcache);
+    const long long units = (long long)T * (n_heads + 2LL * n_kv_heads) * (head_dim / 16);
+    const dim3 grid((unsigned)((units + kPromptRopeThreads - 1) / kPromptRopeThreads)), block(kPromptRopeThreads);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    drain_stale_error();
+    switch (head_dim) {
+        case 32: prompt_rope_kernel<32><<<grid, block, 0, st>>>(x, cos_table, sin_table, kc, vc, T, n_heads, n_kv_heads, max_len); break;
+        case 64: prompt_rope_kernel<64><<<grid, block, 0, st>>>(x, cos_table, sin_table, kc, vc, T, n_heads, n_kv_heads, max_len); break;
+        case 128: prompt_rope_kernel<128><<<grid, block, 0, st>>>(x, cos_table, sin_table, kc, vc, T, n_heads, n_kv_heads, max_len); break;
+        default: prompt_rope_kernel<256><<<grid, block, 0, st>>>(x, cos_table, sin_table, kc, vc, T, n_heads, n_kv_heads, max_len); break;
+    }
+    return launch_status();
+}
+
+int ap_prompt_attention(const uint16_t *qkv, const uint16_t *kcache, const uint16_t *vcache, uint16_t *out, int first, int T,
+                        int n_heads, int n_kv_heads, int head_dim, int max_len, float scale, void *stream) {
+    if (!qkv || !kcache || !vcache || !out) return AP_ENULL;
+    const int rc = check_prompt(T, n_heads, n_kv_heads, head_dim, max_len);
+    if (rc != AP_OK) return rc;
+    if (first < 0 || first >= T) return AP_ESHAPE;
+    if (!aligned16(qkv) || !aligned16(kcache) || !aligned16(vcache) || !aligned16(out)) return AP_EALIGN;
+    const half_t *x = reinterpret_cast<const half_t *>(qkv), *kc = reinterpret_cast<const half_t *>(kcache), *vc = reinterpret_cast<const half_t *>(vcache);
+    half_t *o = reinterpret_cast<half_t *>(out);
+    const int ldq = (n_heads + 2 * n_kv_heads) * head_dim, group = n_heads / n_kv_heads;
+    const float scale_log2 = scale * 1.44269504088896340736f;  // the kernel's exponentials are powers of two
+    const dim3 grid((unsigned)((T - first + kPromptQueries - 1) / kPromptQueries), (unsigned)n_heads), block(kPromptAttnThreads);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    drain_stale_error();
+    switch (head_dim) {
+        case 32: prompt_attention_kernel<32><<<grid, block, 0, st>>>(x, ldq, kc, vc, o, first, T, n_heads, group, max_len, scale_log2); break;
+        case 64: prompt_attention_kernel<64><<<grid, block, 0, st>>>(x, ldq, kc, vc, o, first, T, n_heads, group, max_len, scale_log2); break;
+        case 128: prompt_attention_kernel<128><<<grid, block, 0, st>>>(x, ldq, kc, vc, o, first, T, n_heads, group, max_len, scale_log2); break;
+        default: prompt_attention_kernel<256><<<grid, block, 0, st>>>(x, ldq, kc, vc, o, first, T, n_heads, group, max_len, scale_log2); break;
     }
     return launch_status();
 }

@@ -1,4 +1,4 @@
-// Native side of any_precision_ext and AnyPrecisionLinear: the checks, the allocation of the result and the launch of one
+// Native side of any_precision_ext, AnyPrecisionLinear and its sets: the checks, the allocation of the result and the launch of one
 // call, as Python functions over torch tensors.
 //
 // A linear's kernel takes 4 to 15 us at the batch sizes of decoding; the same steps written in Python over ctypes take
@@ -186,11 +186,94 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
 }
 
+// linear_group(buffers of 2..4 modules, x, w_bits, concat): forward_group for bias-free linears of one input length.  A list of
+// results, or with concat one tensor of them side by side.  Up to 8 rows ap_matmul_kbit_group, beyond one launch of the tiled
+// GEMM where ap_gemm_kbit_group_pays; None where the modules are better called one by one.
+PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    constexpr int MOST = 4;
+    if (n != 4 || !PyTuple_Check(args[0]) || !is_tensor(args[1])) return none();
+    const int bits = bits_of(args[2]), count = (int)PyTuple_GET_SIZE(args[0]);
+    const bool concat = args[3] == Py_True;
+    if (bits == 0 || count < 2 || count > MOST) return none();
+    PyObject *q[MOST], *t[MOST];
+    for (int g = 0; g < count; g++) {
+        PyObject *buffers = PyTuple_GET_ITEM(args[0], g);
+        if (!PyDict_Check(buffers)) return none();
+        PyObject *bias = PyDict_GetItem(buffers, key_bias);
+        if (bias != nullptr && bias != Py_None) return none();
+        q[g] = PyDict_GetItem(buffers, key_qweight);
+        t[g] = PyDict_GetItem(buffers, key_lut[bits]);
+        if (!is_tensor(q[g]) || !is_tensor(t[g])) return none();
+    }
+    return guarded([&]() -> PyObject * {
+        const Tensor &given = THPVariable_Unpack(args[1]);
+        Weight w[MOST];
+        int N[MOST];
+        int64_t total = 0;
+        const uint32_t *planes[MOST];
+        const uint16_t *luts[MOST];
+        for (int g = 0; g < count; g++) {
+            if (!weight_of(THPVariable_Unpack(q[g]), THPVariable_Unpack(t[g]), bits, &w[g])) return none();
+            if (w[g].K != w[0].K || w[g].device != w[0].device) return none();
+            N[g] = w[g].N;
+            total += N[g];
+            planes[g] = w[g].planes;
+            luts[g] = w[g].lut;
+        }
+        const int64_t rows = rows_of(given, w[0]);
+        const int K = w[0].K;
+        if (rows < 1) return none();
+        const bool gemm = rows > 8;
+        if (gemm && ap_gemm_kbit_group_pays(count, N, (int)rows, K, bits) != 1) return none();
+        const Tensor x = given.is_contiguous() ? given : given.contiguous();
+        const OnDevice on(w[0].device);
+        // side by side in one allocation: one row's results always are dense, and the tiled kernel writes rows that are not
+        const bool joint = concat && (gemm ? K % 128 == 0 : rows == 1);
+        Tensor all, outs[MOST];
+        uint16_t *to[MOST];
+        long long ldo[MOST];
+        if (joint) {
+            all = result_for(x, total);
+            int64_t at = 0;
+            for (int g = 0; g < count; at += N[g], g++) {
+                to[g] = half_out(all) + at;
+                ldo[g] = total;
+            }
+        } else {
+            for (int g = 0; g < count; g++) {
+                outs[g] = result_for(x, N[g]);
+                to[g] = half_out(outs[g]);
+            }
+        }
+        const int rc = gemm ? ap_gemm_kbit_group(half_ptr(x), count, planes, luts, to, N, joint ? ldo : nullptr, (int)rows, K, bits, on.stream)
+                            : ap_matmul_kbit_group(half_ptr(x), count, planes, luts, to, N, (int)rows, K, bits, on.stream);
+        if (rc == AP_ELIMIT) return none();  // beyond the tiled kernel's offsets
+        if (rc != AP_OK) return library_error(rc, gemm ? "gemm_kbit_group" : "matmul_kbit_group");
+        if (joint) return wrap(std::move(all));
+        if (concat) {
+            std::vector<Tensor> parts(outs, outs + count);
+            return wrap(at::cat(parts, -1));
+        }
+        PyObject *list = PyList_New(count);
+        if (list == nullptr) return nullptr;
+        for (int g = 0; g < count; g++) {
+            PyObject *o = wrap(std::move(outs[g]));
+            if (o == nullptr) {
+                Py_DECREF(list);
+                return nullptr;
+            }
+            PyList_SET_ITEM(list, g, o);
+        }
+        return list;
+    });
+}
+
 PyMethodDef methods[] = {
     {"matmul_kbit", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(matmul_kbit)), METH_FASTCALL, nullptr},
     {"gemm_kbit", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(gemm_kbit)), METH_FASTCALL, nullptr},
     {"dequant_kbit", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(dequant_kbit)), METH_FASTCALL, nullptr},
     {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(linear)), METH_FASTCALL, nullptr},
+    {"linear_group", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(linear_group)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_anyprec_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

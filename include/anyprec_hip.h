@@ -34,7 +34,7 @@
 extern "C" {
 #endif
 
-#define AP_ABI_VERSION 8
+#define AP_ABI_VERSION 9
 
 enum {
     AP_OK = 0,
@@ -214,6 +214,19 @@ int ap_decode_advance(const uint16_t *logits, int n, long long *pos, long long *
 int ap_decode_attention(const uint16_t *qkv, const float *cos_table, const float *sin_table, uint16_t *kcache,
                         uint16_t *vcache, const long long *pos, uint16_t *out, int n_heads, int n_kv_heads, int head_dim,
                         int max_len, float scale, void *stream);
+
+/* ---- The rest of a prompt, for the `T` tokens of one sequence (cache rows 0 .. T-1), between its linears.  No counterpart
+ * in the reference (AnyPrecisionForCausalLM.py:88-97 calls the Hugging Face modules).  Shapes and conventions as for
+ * ap_decode_attention; T <= max_len (AP_ESHAPE beyond).
+ *
+ * ap_prompt_rope: qkv [T, (n_heads + 2 n_kv_heads) * head_dim]: the query heads are rotated in place; rows 0 .. T-1 of
+ *   kcache / vcache receive the rotated keys and the values.
+ * ap_prompt_attention: out [T - first, n_heads * head_dim] = causal attention of the tokens first .. T-1 (queries as
+ *   ap_prompt_rope left them) over the cache rows up to each one's own. */
+int ap_prompt_rope(uint16_t *qkv, const float *cos_table, const float *sin_table, uint16_t *kcache, uint16_t *vcache, int T,
+                   int n_heads, int n_kv_heads, int head_dim, int max_len, void *stream);
+int ap_prompt_attention(const uint16_t *qkv, const uint16_t *kcache, const uint16_t *vcache, uint16_t *out, int first, int T,
+                        int n_heads, int n_kv_heads, int head_dim, int max_len, float scale, void *stream);
 
 #ifdef __cplusplus
 }
