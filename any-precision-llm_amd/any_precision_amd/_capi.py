@@ -134,7 +134,7 @@ def gemm_group_pays(M: int, rows, K: int, w_bits: int) -> bool:
         return False
     rc = lib.ap_gemm_kbit_group_pays(n, (ctypes.c_int * n)(*rows), M, K, w_bits)
     if rc < 0:
-        check(rc, "ap_gemm_kbit_group_pays", "ap_prompt_rope", "ap_prompt_attention")
+        check(rc, "ap_gemm_kbit_group_pays")
     return rc == 1
 
 

@@ -210,3 +210,12 @@ def test_route_report_follows_the_rule_and_the_knobs():
         assert _capi.matmul_route(1, 63, 4096, 5) == "dot"                # odd row count: not served
     with pytest.raises(ValueError):
         _capi.matmul_route(9, 64, 4096, 5)
+
+
+def test_what_pays_names_a_wrong_argument():
+    """The queries of the dispatch rules turn the library's code for a wrong bit-width into a ValueError."""
+    from any_precision_amd import _capi
+    with pytest.raises(ValueError, match="w_bits"):
+        _capi.gemm_group_pays(16, [4096, 4096], 4096, 9)
+    with pytest.raises(ValueError, match="w_bits"):
+        _capi.gemm_pays(16, 4096, 4096, 2)
