@@ -132,6 +132,47 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
+// Sums of NV values over the 64 lanes of a wave, folded together: the halves and then the quarters of a wave are exchanged
+// BETWEEN values (v_permlane32_swap, v_permlane16_swap), so that one add serves two and then four of them, and the last
+// four steps run once for four values -- 10 vector instructions for four sums, 9 for two, where wave_sum() takes 10 each
+// and waits for every one of its steps.  A value's sum is added in the same order whatever NV: a batch or a set gives
+// the bits that its members alone give.
+// out[h] holds the sums 4h, 4h + 1, ..: each in every lane of one 16-lane row (two sums left: of one half of the wave, one
+// sum left: of the whole wave).  sum_lane<NV>(h, lane, i): whether `lane` is the first of sum number i.
+template <int NV>
+__device__ __forceinline__ bool sum_lane(int h, int lane, int &i) {
+    const int n = NV - 4 * h, width = n >= 3 ? 16 : (n == 2 ? 32 : 64);
+    i = 4 * h + lane / width;
+    return lane % width == 0 && (n != 3 || lane < 48);
+}
+template <int NV>
+__device__ __forceinline__ void wave_sums(const float (&v)[NV], float (&out)[(NV + 3) / 4]) {
+    auto add = [](uint32_t a, uint32_t b) { return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b); };
+    auto fold32 = [&](float a, float b) {  // rows 0, 1: a's rows 0 + 2, 1 + 3; rows 2, 3: b's
+        const auto h = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+        return add(h[0], h[1]);
+    };
+    auto fold16 = [&](float a, float b) {  // rows 0, 2: a's rows 0 + 1, 2 + 3; rows 1, 3: b's
+        const auto h = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+        return add(h[0], h[1]);
+    };
+#pragma unroll
+    for (int h = 0; 4 * h < NV; h++) {
+        const int n = NV - 4 * h, i = 4 * h;
+        float u;
+        if (n >= 3) {
+            u = fold16(fold32(v[i], v[i + 2]), fold32(v[i + 1], v[n > 3 ? i + 3 : i + 2]));
+        } else {
+            u = fold32(v[i], v[n == 2 ? i + 1 : i]);
+            u = fold16(u, u);
+        }
+        u = dpp_add<0xB1>(u);   // within the 16-lane rows, as in wave_sum()
+        u = dpp_add<0x4E>(u);
+        u = dpp_add<0x141>(u);
+        out[h] = dpp_add<0x140>(u);
+    }
+}
+
 // Copy one row's table of 2^BITS fp16 entries from global memory into this
 // wave's LDS slot.  Split in two so the global load can be issued early.
 template <int BITS>

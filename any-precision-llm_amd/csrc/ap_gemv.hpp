@@ -19,8 +19,15 @@
 //     dequant.cuh:13-30,56-67) of two ADJACENT elements (ap_lookup.hpp): 4^b entries of
 //     two fp16, one 32-bit gather per two weights and no packing.  5..8 bits gather single
 //     fp16 entries and pack two of them per dot2.
-//   * Lane partials are summed with DPP; when S > 1 the segment partials of a row meet in
-//     LDS and are added in a fixed order: results are deterministic.
+//   * Lane partials of all R x M sums are folded together (wave_sums, ap_device.hpp); when S > 1 the segment partials
+//     of a row meet in LDS and are added in a fixed order: results are deterministic.
+// The kernel is bound by instructions and by the launch, not by HBM: with every plane in L2 a gate/up launch of 2 x 11008
+// x 4096 at 3 bits takes 9.6 us against 10.3 from HBM.  Of about 165 vector instructions a wave of that launch issues, 92
+// are transposes, lookups and products.  One sum after the other cost 24 of them and their waits, folded together 13, and
+// the table lane arithmetic 9 instead of 16; from two activation rows on the registers also fall by up to a fifth, which
+// is one more wave per SIMD (us, before -> after: 4096 x 14336 at 3 rows, 4 bits 14.2 -> 12.3; 5120 x 5120 at 4 rows, 8
+// bits 12.9 -> 12.0; 4096 x 11008 at 2 rows, 6 bits 14.7 -> 13.5; 1024 x 4096 at 8 rows, 8 bits 6.3 -> 5.6; one row
+// 0-2 %).
 #pragma once
 #include <type_traits>
 
@@ -224,7 +231,7 @@ void gemv_kbit_kernel(const half_t *__restrict__ x, const GemvMembers mem, int K
     // stores go through a pointer typed as global memory (the argument pointers left the statement above
     // without an address space, and a store through them would be a flat one)
     const global_ptr<half_t> out_g = (global_ptr<half_t>)reinterpret_cast<uint64_t>(out);
-    float tot[R][M];
+    float lane_sum[R * M];
     static_for<R>([&](auto r_c) {
         constexpr int r = decltype(r_c)::value;
         float acc[M][2];
@@ -232,29 +239,31 @@ void gemv_kbit_kernel(const half_t *__restrict__ x, const GemvMembers mem, int K
         for (int m = 0; m < M; m++) acc[m][0] = acc[m][1] = 0.f;
         row_dot<BITS, M, WPL>(q[r], tables[r], X, acc);
 #pragma unroll
-        for (int m = 0; m < M; m++) tot[r][m] = wave_sum(valid ? acc[m][0] + acc[m][1] : 0.f);
+        for (int m = 0; m < M; m++) {
+            float v = acc[m][0] + acc[m][1];
+            // a row's sums are finished before the next row's lookups start, outside of any "if (valid)" region: left to the
+            // optimiser the lookups of all rows are interleaved and take up to 30 registers more (8 bits: scratch memory)
+            asm volatile("" : "+v"(v));
+            lane_sum[r * M + m] = valid ? v : 0.f;
+        }
     });
+    // sum number r M + m
+    constexpr int NS = R * M;
+    float tot[(NS + 3) / 4];
+    wave_sums<NS>(lane_sum, tot);
 
     auto swiglu = [](float gate, float up) { return gate / (1.f + __expf(-gate)) * up; };
-    if (S == 1) {
-        if (lane == kSumLane) {
-            if constexpr (PAIR) {
+    if (S == 1 && !PAIR) {
 #pragma unroll
-                for (int m = 0; m < M; m++) out_g[(size_t)m * N + row0] = (half_t)swiglu(tot[0][m], tot[R - 1][m]);
-            } else {
-#pragma unroll
-                for (int r = 0; r < R; r++)
-#pragma unroll
-                    for (int m = 0; m < M; m++)
-                        if (row0 + r < N) out_g[(size_t)m * N + row0 + r] = (half_t)tot[r][m];
-            }
+        for (int h = 0; h < (NS + 3) / 4; h++) {
+            int i;
+            if (sum_lane<NS>(h, lane, i) && row0 + i / M < N) out_g[(size_t)(i % M) * N + row0 + i / M] = (half_t)tot[h];
         }
     } else {
-        if (lane == kSumLane) {
 #pragma unroll
-            for (int r = 0; r < R; r++)
-#pragma unroll
-                for (int m = 0; m < M; m++) partial[(s * R + r) * M + m] = tot[r][m];
+        for (int h = 0; h < (NS + 3) / 4; h++) {
+            int i;
+            if (sum_lane<NS>(h, lane, i)) partial[s * NS + i] = tot[h];
         }
         __syncthreads();
         const int tid = s * kWave + lane;

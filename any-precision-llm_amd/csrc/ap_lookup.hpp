@@ -20,24 +20,25 @@ struct LookupTable {
     static constexpr int kBytes = kPair ? (4 << (2 * BITS)) : (2 << BITS);
 };
 
-// What a lane needs to know to build its share of a pair table; depends on the lane only.
+// What a lane needs to know to build its share of a pair table (byte offsets into the row's entries); depends on the lane only.
+// With the lane number's bits read as l5 l4 .. l0, f = l5 l3 l1 and s = l4 l2 l0:
+//   3 bits: entry `lane` = (lut[f], lut[s])  (adjacent_pair_split of 4 lane);
+//   4 bits: entries 4 lane .. 4 lane + 3 differ in the lowest bit of either index: they combine the halves of dword
+//           f = (lut[2f], lut[2f+1]) and of dword s.
+// Three masked shifts each, two of them shared: every wave of the GEMV kernels runs this once for two to four rows.
 template <int BITS>
 struct PairLane {
-    uint32_t first, second;  // 3 bits: entry `lane` = (lut[first], lut[second]); 4 bits: dword numbers (below)
+    uint32_t first, second;
 };
 
 template <int BITS>
 __device__ __forceinline__ PairLane<BITS> pair_lane(int lane) {
     PairLane<BITS> r = {0u, 0u};
-    if constexpr (BITS == 3) {
-        adjacent_pair_split<3>((uint32_t)lane << 2, r.first, r.second);
-    } else if constexpr (BITS == 4) {
-        // entries 4*lane .. 4*lane+3 differ in the lowest bit of either index: they combine the halves
-        // of dword `first` = (lut[2a], lut[2a+1]) and of dword `second`
-        uint32_t a, b;
-        adjacent_pair_split<4>((uint32_t)lane << 2, a, b);
-        r.first = a >> 1;
-        r.second = b >> 1;
+    if constexpr (BITS <= 4) {
+        constexpr int SH = BITS == 3 ? 1 : 2;  // log2 of the bytes that f and s count
+        const uint32_t l = (uint32_t)lane << 1, a = l << SH >> 2, b = l << SH >> 3, c = l << SH >> 4;  // lane << SH >> 1, 2, 3
+        r.first = (a & (1u << SH)) | (b & (2u << SH)) | (c & (4u << SH));
+        r.second = (l << SH >> 1 & (1u << SH)) | (a & (2u << SH)) | (b & (4u << SH));
     }
     return r;
 }
@@ -57,11 +58,11 @@ __device__ __forceinline__ TableWords<BITS> lookup_table_fetch(global_ptr<const 
     r.a = r.b = 0u;
     r.c = u32x2{0u, 0u};
     if constexpr (BITS == 3) {
-        r.a = load_at<uint16_t>(lut_row, pl.first * 2u);
-        r.b = load_at<uint16_t>(lut_row, pl.second * 2u);
+        r.a = load_at<uint16_t>(lut_row, pl.first);
+        r.b = load_at<uint16_t>(lut_row, pl.second);
     } else if constexpr (BITS == 4) {
-        r.a = load_at<uint32_t>(lut_row, pl.first * 4u);
-        r.b = load_at<uint32_t>(lut_row, pl.second * 4u);
+        r.a = load_at<uint32_t>(lut_row, pl.first);
+        r.b = load_at<uint32_t>(lut_row, pl.second);
     } else if constexpr (BITS == 8) {   // 512 B: 64 lanes x 8 B
         r.c = load_at<u32x2>(lut_row, (uint32_t)lane * 8u);
     } else if constexpr (BITS == 7) {   // 256 B: 64 lanes x 4 B

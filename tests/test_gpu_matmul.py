@@ -407,3 +407,29 @@ def test_four_rows_per_workgroup_agree_with_the_oracle(ext, oracle):
                                  (4, 28672, 8192, 4, "dot")):
         assert _capi.matmul_geometry(M, N, K, 4)["rows"] == rows and _capi.matmul_route(M, N, K, 4) == route, (M, N, K)
     assert _capi.matmul_route(4, 4096, 14336, 3) == "mfma4" and _capi.matmul_route(3, 5120, 13824, 6) == "dot"
+
+
+@pytest.mark.parametrize("K", [64, 2048, 4128])
+def test_dot_sums_do_not_depend_on_their_number(ext, K):
+    """The wave sums of a workgroup's rows x activation rows are folded together, 1, 2 or 4 at a time with a remainder: each
+    has the bits that it has alone, whatever its number (one wave per row and several; ragged last workgroup)."""
+    from any_precision_amd import _capi
+    N = 13
+    q, luts = layer_to_gpu(make(N, K, seed=K))
+    x, xg = _x(8, K, seed=3)
+    knobs = {"matmul_mfma4": 0, "gemv_fine": 0, "gemv_stream": 0, "matmul_mfma_from": 9, "gemv_rows": 1}
+    before = {k: _capi.get_tuning(k) for k in knobs}
+    try:
+        for k, v in knobs.items():
+            _capi.set_tuning(k, v)
+        for b in (3, 4, 6, 8):
+            alone = torch.cat([ext.matmul_kbit(xg[m:m + 1].contiguous(), q, luts[b], b) for m in range(8)])
+            for rows in (1, 2, 4):
+                _capi.set_tuning("gemv_rows", rows)
+                for M in range(1, 9):
+                    got = ext.matmul_kbit(xg[:M].contiguous(), q, luts[b], b)
+                    assert torch.equal(got.view(torch.int16), alone[:M].view(torch.int16)), (b, rows, M)
+            _capi.set_tuning("gemv_rows", 1)
+    finally:
+        for k, v in before.items():
+            _capi.set_tuning(k, v)
