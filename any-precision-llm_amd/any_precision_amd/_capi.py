@@ -12,7 +12,7 @@ LIB_PATH = os.path.join(_PKG_ROOT, "lib", "libanyprec_hip.so")
 
 AP_OK = 0
 AP_ENULL, AP_EBITS, AP_ESHAPE, AP_EALIGN, AP_EBATCH, AP_ELIMIT, AP_EKNOB = -1, -2, -3, -4, -5, -6, -7
-AP_ABI_VERSION = 9
+AP_ABI_VERSION = 10
 
 if not os.path.exists(LIB_PATH):
     raise ModuleNotFoundError(
@@ -92,6 +92,8 @@ lib.ap_prompt_rope.argtypes = [_vp] * 5 + [_ci] * 5 + [_vp]
 lib.ap_prompt_rope.restype = _ci
 lib.ap_prompt_attention.argtypes = [_vp] * 4 + [_ci] * 6 + [ctypes.c_float, _vp]
 lib.ap_prompt_attention.restype = _ci
+lib.ap_rope_heads.argtypes = [_vp] * 4 + [_ci] * 4 + [_vp]
+lib.ap_rope_heads.restype = _ci
 lib.ap_set_tuning.argtypes = [ctypes.c_char_p, _ci]
 lib.ap_set_tuning.restype = _ci
 lib.ap_get_tuning.argtypes = [ctypes.c_char_p, _pi]
@@ -105,7 +107,7 @@ if lib.ap_abi_version() != AP_ABI_VERSION:
 EXPORTS = ("ap_abi_version", "ap_strerror", "ap_dequant_kbit", "ap_matmul_kbit", "ap_matmul_kbit_group",
            "ap_gemm_kbit", "ap_matmul_kbit_geometry", "ap_set_tuning", "ap_get_tuning", "ap_probe_stream", "ap_probe_empty", "ap_probe_write", "ap_matmul_kbit_route", "ap_matmul_kbit_group_route",
            "ap_add_rmsnorm", "ap_silu_mul", "ap_decode_attention", "ap_matmul_kbit_swiglu", "ap_decode_advance", "ap_gemm_kbit_group", "ap_dequant_kbit_group", "ap_gemm_kbit_pays",
-           "ap_gemm_kbit_group_pays", "ap_prompt_rope", "ap_prompt_attention")
+           "ap_gemm_kbit_group_pays", "ap_prompt_rope", "ap_prompt_attention", "ap_rope_heads")
 GEMM_MAX_M = 128
 GROUP_MAX = 4
 DEQUANT_GROUP_MAX = 8

@@ -1,0 +1,103 @@
+"""The steps between the linears of a Hugging Face Llama model (any_precision/modules/AnyPrecisionForCausalLM.py:88-97 runs the
+modules as they are) through the library's kernels: RMSNorm, SiLU * up and the rotary embedding, one launch each where the
+modules take seven, two and eleven passes over memory.
+
+``attach(model)`` gives the norm, MLP and attention modules of a Llama-architecture model subclasses of their classes;
+parameters, state-dict keys, sub-modules and hooks stay what they are.  Every such forward hands over to the original one
+for whatever it does not serve: gradients, other devices and types, traces, compilation, modes, a key/value cache, an
+attention mask, other attention implementations.
+"""
+from __future__ import annotations
+
+import functools
+
+import torch
+import torch.nn.functional as F
+
+from . import _capi
+
+# keyword arguments of an attention call that do not change what it computes without a cache and a mask
+_IDLE = {"position_ids", "cache_position", "use_cache", "output_attentions", "output_hidden_states", "return_dict"}
+
+
+def _native():
+    return None if torch.compiler.is_compiling() else _capi.torch_module()
+
+
+def _norm_forward(module, original, hidden_states):
+    native = _native()
+    out = None if native is None else native.rmsnorm(hidden_states, module.weight, float(module.variance_epsilon))
+    return original(hidden_states) if out is None else out
+
+
+def _has_hooks(module):
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+
+
+def _mlp_forward(module, original, x):
+    native = _native()
+    act = module.act_fn
+    if native is None or _has_hooks(act) or type(act).__name__ not in ("SiLU", "SiLUActivation"):
+        return original(x)
+    gate, up = module.gate_proj(x), module.up_proj(x)
+    hidden = native.silu_mul(gate, up)
+    return module.down_proj(act(gate) * up if hidden is None else hidden)
+
+
+def _rotated(native, x, cos, sin):
+    """x [B, T, heads * hd] with its rotary embedding, [B, heads, T, hd]."""
+    out = native.rope(x, cos, sin)
+    if out is None:
+        x = x.view(*x.shape[:2], -1, cos.shape[-1])
+        low, high = x.chunk(2, dim=-1)
+        out = x * cos.unsqueeze(2) + torch.cat((-high, low), dim=-1) * sin.unsqueeze(2)
+    return out.transpose(1, 2)
+
+
+def _attention_forward(module, original, hidden_states, position_embeddings=None, attention_mask=None, past_key_values=None,
+                       **kwargs):
+    native = _native()
+    if (native is None or position_embeddings is None or attention_mask is not None or past_key_values is not None
+            or hidden_states.dim() != 3 or module.training or torch.is_grad_enabled()
+            or module.config._attn_implementation != "sdpa" or not getattr(module, "is_causal", True)
+            or kwargs.get("output_attentions") or any(k not in _IDLE and v is not None for k, v in kwargs.items())):
+        return original(hidden_states, position_embeddings=position_embeddings, attention_mask=attention_mask,
+                        past_key_values=past_key_values, **kwargs)
+    cos, sin = position_embeddings
+    B, T = hidden_states.shape[:2]
+    q, k, v = (p(hidden_states) for p in (module.q_proj, module.k_proj, module.v_proj))
+    q, k, v = _rotated(native, q, cos, sin), _rotated(native, k, cos, sin), v.view(B, T, -1, cos.shape[-1]).transpose(1, 2)
+    ctx = F.scaled_dot_product_attention(q, k, v, is_causal=T > 1, scale=module.scaling, enable_gqa=q.shape[1] != k.shape[1])
+    return module.o_proj(ctx.transpose(1, 2).reshape(B, T, -1)), None
+
+
+_FORWARDS = {"LlamaRMSNorm": _norm_forward, "LlamaMLP": _mlp_forward, "LlamaAttention": _attention_forward}
+
+
+@functools.lru_cache(None)
+def _class(name):
+    """The class ``name`` of the Hugging Face Llama model with its forward replaced."""
+    from transformers.models.llama import modeling_llama
+    base, step = getattr(modeling_llama, name), _FORWARDS[name]
+
+    @functools.wraps(base.forward)
+    def forward(self, *args, **kwargs):
+        return step(self, functools.partial(base.forward, self), *args, **kwargs)
+
+    return type(name, (base,), {"forward": forward, "__module__": __name__})
+
+
+def __getattr__(name):      # pickled modules name their class as one of this module
+    if name in _FORWARDS:
+        return _class(name)
+    raise AttributeError(f"module {__name__!r} has no attribute {name!r}")
+
+
+def attach(model):
+    """Gives the modules of a Llama-architecture ``model`` the forwards above."""
+    if getattr(model.config, "model_type", None) != "llama":
+        return
+    for module in model.modules():
+        name = type(module).__name__
+        if name in _FORWARDS and type(module) is _class(name).__base__:
+            module.__class__ = _class(name)

@@ -23,6 +23,7 @@ import os
 import torch
 import torch.nn as nn
 
+from . import between
 from .linear import AnyPrecisionLinear
 
 # module layout of the architectures the reference describes (analyzer/architectures/*.yaml)
@@ -79,6 +80,7 @@ class AnyPrecisionForCausalLM(nn.Module):
 
         self.ap_linears = []
         self._load_quantized_modules()
+        between.attach(self.model)
         self.tie_weights()
         if model_path is not None:
             self._load_checkpoint(model_path)

@@ -375,6 +375,23 @@ int ap_prompt_rope(uint16_t *qkv, const float *cos_table, const float *sin_table
     return launch_status();
 }
 
+int ap_rope_heads(const uint16_t *x, const uint16_t *cos_table, const uint16_t *sin_table, uint16_t *out, int rows, int cos_rows,
+                  int n_heads, int head_dim, void *stream) {
+    if (!x || !cos_table || !sin_table || !out) return AP_ENULL;
+    if (rows < 1 || cos_rows < 1 || n_heads < 1 || head_dim < 16 || head_dim % 16) return AP_ESHAPE;
+    // the kernel numbers its units in 32 bits; a workgroup past the last unit must not wrap around
+    const long long per_row = (long long)n_heads * (head_dim / 16);
+    if (per_row > 0x7fffffffLL || per_row * rows > 0x7fffffffLL) return AP_ELIMIT;
+    const long long units = per_row * rows;
+    if (!aligned16(x) || !aligned16(cos_table) || !aligned16(sin_table) || !aligned16(out)) return AP_EALIGN;
+    drain_stale_error();
+    rope_heads_kernel<<<dim3((unsigned)((units + kPromptRopeThreads - 1) / kPromptRopeThreads)), dim3(kPromptRopeThreads), 0,
+                        static_cast<hipStream_t>(stream)>>>(
+        reinterpret_cast<const half_t *>(x), reinterpret_cast<const half_t *>(cos_table), reinterpret_cast<const half_t *>(sin_table),
+        reinterpret_cast<half_t *>(out), rows, cos_rows, n_heads, head_dim);
+    return launch_status();
+}
+
 int ap_prompt_attention(const uint16_t *qkv, const uint16_t *kcache, const uint16_t *vcache, uint16_t *out, int first, int T,
                         int n_heads, int n_kv_heads, int head_dim, int max_len, float scale, void *stream) {
     if (!qkv || !kcache || !vcache || !out) return AP_ENULL;

@@ -10,9 +10,13 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "anyprec_hip.h"
@@ -268,12 +272,97 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
 }
 
+// What sits between the linears of the Hugging Face Llama modules.  These replace torch ops, which take part in everything torch
+// does with an op: a call that anything but plain execution follows -- gradients, tangents, subclasses, modes, functorch --
+// gets None and runs as torch ops.
+bool plain_half(PyObject *o, const at::Device *device) {
+    if (!is_tensor(o) || !THPVariable_CheckTypeExact(Py_TYPE(o))) return false;
+    const Tensor &t = THPVariable_Unpack(o);
+    if (!t.is_cuda() || t.scalar_type() != at::kHalf || t.layout() != at::kStrided || !t.is_contiguous() || t.numel() == 0) return false;
+    if (device != nullptr && t.device() != *device) return false;
+    if (c10::GradMode::is_enabled() && t.requires_grad()) return false;
+    const auto keys = t.key_set();
+    if (keys.has(c10::DispatchKey::FuncTorchBatched) || keys.has(c10::DispatchKey::FuncTorchGradWrapper) ||
+        keys.has(c10::DispatchKey::Functionalize) || t._fw_grad(0).defined())
+        return false;
+    return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
+}
+
+bool plain_execution() {
+    return !c10::impl::TorchDispatchModeTLS::any_modes_set() && !at::impl::torch_function_mode_enabled() &&
+           !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
+           !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
+}
+
+// rmsnorm(x, weight, eps): x * rsqrt(mean(x^2) + eps) * weight over the last dimension.
+PyObject *rmsnorm(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    if (n != 3 || !PyFloat_Check(args[2]) || !plain_execution()) return none();
+    return guarded([&]() -> PyObject * {
+        if (!plain_half(args[0], nullptr)) return none();
+        const Tensor &x = THPVariable_Unpack(args[0]);
+        const at::Device device = x.device();
+        if (!plain_half(args[1], &device)) return none();
+        const Tensor &weight = THPVariable_Unpack(args[1]);
+        const int64_t H = x.dim() < 1 ? 0 : x.size(-1);
+        if (weight.dim() != 1 || weight.size(0) != H || H < 8 || H % 8 || H > INT32_MAX || x.numel() / H > INT32_MAX) return none();
+        const OnDevice on(device.index());
+        Tensor out = empty_half(x.sizes(), device);
+        // nothing is added, so h_out = h is not written
+        const int rc = ap_add_rmsnorm(half_ptr(x), nullptr, half_ptr(weight), half_out(x), half_out(out), (int)(x.numel() / H), (int)H,
+                                      (float)PyFloat_AS_DOUBLE(args[2]), on.stream);
+        if (rc != AP_OK) return library_error(rc, "rmsnorm");
+        return wrap(std::move(out));
+    });
+}
+
+// silu_mul(gate, up): silu(gate) * up.
+PyObject *silu_mul(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    if (n != 2 || !plain_execution()) return none();
+    return guarded([&]() -> PyObject * {
+        if (!plain_half(args[0], nullptr)) return none();
+        const Tensor &gate = THPVariable_Unpack(args[0]);
+        const at::Device device = gate.device();
+        if (!plain_half(args[1], &device)) return none();
+        const Tensor &up = THPVariable_Unpack(args[1]);
+        if (gate.sizes() != up.sizes() || gate.numel() % 8) return none();
+        const OnDevice on(device.index());
+        Tensor out = empty_half(gate.sizes(), device);
+        const int rc = ap_silu_mul(half_ptr(gate), half_ptr(up), half_out(out), gate.numel(), on.stream);
+        if (rc != AP_OK) return library_error(rc, "silu_mul");
+        return wrap(std::move(out));
+    });
+}
+
+// rope(x [B, T, heads * hd], cos, sin [B or 1, T, hd]): [B, T, heads, hd].
+PyObject *rope(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    if (n != 3 || !plain_execution()) return none();
+    return guarded([&]() -> PyObject * {
+        if (!plain_half(args[0], nullptr)) return none();
+        const Tensor &x = THPVariable_Unpack(args[0]);
+        const at::Device device = x.device();
+        if (!plain_half(args[1], &device) || !plain_half(args[2], &device)) return none();
+        const Tensor &c = THPVariable_Unpack(args[1]), &s = THPVariable_Unpack(args[2]);
+        if (x.dim() != 3 || c.dim() != 3 || c.sizes() != s.sizes()) return none();
+        const int64_t B = x.size(0), T = x.size(1), hd = c.size(2);
+        if (c.size(1) != T || (c.size(0) != B && c.size(0) != 1) || hd % 16 || x.size(2) % hd || x.numel() / 16 > INT32_MAX) return none();
+        const OnDevice on(device.index());
+        Tensor out = empty_half({B, T, x.size(2) / hd, hd}, device);
+        const int rc = ap_rope_heads(half_ptr(x), half_ptr(c), half_ptr(s), half_out(out), (int)(B * T), (int)(c.size(0) * T),
+                                     (int)(x.size(2) / hd), (int)hd, on.stream);
+        if (rc != AP_OK) return library_error(rc, "rope");
+        return wrap(std::move(out));
+    });
+}
+
 PyMethodDef methods[] = {
     {"matmul_kbit", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(matmul_kbit)), METH_FASTCALL, nullptr},
     {"gemm_kbit", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(gemm_kbit)), METH_FASTCALL, nullptr},
     {"dequant_kbit", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(dequant_kbit)), METH_FASTCALL, nullptr},
     {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(linear)), METH_FASTCALL, nullptr},
     {"linear_group", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(linear_group)), METH_FASTCALL, nullptr},
+    {"rmsnorm", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(rmsnorm)), METH_FASTCALL, nullptr},
+    {"silu_mul", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(silu_mul)), METH_FASTCALL, nullptr},
+    {"rope", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(rope)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_anyprec_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

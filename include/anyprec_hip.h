@@ -34,7 +34,7 @@
 extern "C" {
 #endif
 
-#define AP_ABI_VERSION 9
+#define AP_ABI_VERSION 10
 
 enum {
     AP_OK = 0,
@@ -227,6 +227,10 @@ int ap_prompt_rope(uint16_t *qkv, const float *cos_table, const float *sin_table
                    int n_heads, int n_kv_heads, int head_dim, int max_len, void *stream);
 int ap_prompt_attention(const uint16_t *qkv, const uint16_t *kcache, const uint16_t *vcache, uint16_t *out, int first, int T,
                         int n_heads, int n_kv_heads, int head_dim, int max_len, float scale, void *stream);
+/* out [rows, n_heads, head_dim] = rotary embedding of x (same layout) with fp16 tables [cos_rows, head_dim]; row r takes
+ *   table row r % cos_rows.  head_dim a multiple of 16; out may not alias x. */
+int ap_rope_heads(const uint16_t *x, const uint16_t *cos_table, const uint16_t *sin_table, uint16_t *out, int rows, int cos_rows,
+                  int n_heads, int head_dim, void *stream);
 
 #ifdef __cplusplus
 }

@@ -1,0 +1,106 @@
+"""The kernels between the linears of the Hugging Face Llama modules against the modules' own torch ops in float64, and the
+calls that have to stay with the original forwards."""
+import copy
+import pickle
+
+import pytest
+import torch
+
+
+def _config(**kw):
+    from transformers import LlamaConfig
+    return LlamaConfig(**{**dict(hidden_size=64, intermediate_size=96, num_hidden_layers=2, num_attention_heads=4,
+                                 num_key_value_heads=2, vocab_size=128, max_position_embeddings=64), **kw})
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,T,heads,hd", [(1, 1, 1, 16), (2, 3, 5, 48), (3, 33, 4, 64), (1, 130, 32, 128)])
+@pytest.mark.parametrize("tables", ["one", "each"])
+def test_rope_heads(B, T, heads, hd, tables):
+    from any_precision_amd import _capi
+    gen = torch.Generator().manual_seed(T + hd)
+    x = torch.randn((B, T, heads * hd), generator=gen).half()
+    cos, sin = (torch.rand((B if tables == "each" else 1, T, hd), generator=gen).half() for _ in range(2))
+    got = _capi.torch_module().rope(x.cuda(), cos.cuda(), sin.cuda())
+    x = x.double().view(B, T, heads, hd)
+    low, high = x.chunk(2, dim=-1)
+    a, b = x * cos.double().unsqueeze(2), torch.cat((-high, low), dim=-1) * sin.double().unsqueeze(2)
+    # one rounding to fp16 and two in fp32 of each product
+    bound = (a.abs() + b.abs()) * (2.0 ** -11 + 2.0 ** -22) + 2.0 ** -24
+    assert got.shape == x.shape and bool(((got.cpu().double() - (a + b)).abs() <= bound).all())
+
+
+@pytest.mark.gpu
+def test_what_is_not_plain_execution_is_left_to_torch():
+    from any_precision_amd import _capi
+    native = _capi.torch_module()
+    x, w = torch.randn((3, 64), device="cuda").half(), torch.ones((64,), device="cuda").half()
+    assert native.rmsnorm(x, w, 1e-5).shape == x.shape and native.silu_mul(x, x).shape == x.shape
+    wide = torch.randn((3, 128), device="cuda").half()
+    for bad in (x.float(), x.cpu(), wide[:, ::2], wide.view(-1)[1:193].view(3, 64), x[:0], x.clone().requires_grad_(),
+                torch.nn.Parameter(x.clone())):
+        assert native.rmsnorm(bad, w, 1e-5) is None and native.silu_mul(bad, bad) is None
+    assert native.rmsnorm(x, torch.nn.Parameter(w.clone()), 1e-5) is None     # gradients wanted
+    with torch.no_grad():
+        assert native.rmsnorm(x, torch.nn.Parameter(w.clone()), 1e-5) is not None
+    assert native.rmsnorm(x, w[:32], 1e-5) is None
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Counting(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Counting():
+        assert native.rmsnorm(x, w, 1e-5) is None
+    assert torch.vmap(lambda t: torch.zeros(1, device="cuda") if native.silu_mul(t, t) is None else torch.ones(1, device="cuda"))(x).sum() == 0
+    with torch.autograd.forward_ad.dual_level():
+        assert native.silu_mul(torch.autograd.forward_ad.make_dual(x, x), x) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kv_heads", [4, 2])
+def test_model_forward_with_and_without(kv_heads):
+    """The logits of a model with the kernels and with the original forwards, both against float64 activations."""
+    from any_precision_amd import AnyPrecisionForCausalLM, between
+    ap = AnyPrecisionForCausalLM.from_config(_config(num_key_value_heads=kv_heads), seed=3)
+    ids = torch.randint(0, 128, (3, 17), device="cuda")
+    mask = torch.ones_like(ids)
+    mask[0, :4] = 0
+    with torch.inference_mode():
+        got = ap(ids, precision=5, use_cache=False).logits.float()
+        padded = ap(ids, attention_mask=mask, precision=5, use_cache=False).logits
+        cached = ap(ids, precision=5, use_cache=True).logits.float()
+        for m in ap.model.modules():
+            if type(m).__module__ == between.__name__:
+                m.__class__ = type(m).__base__
+        want = ap(ids, precision=5, use_cache=False).logits.float()
+        assert torch.allclose(padded[:, 4:].float(), ap(ids, attention_mask=mask, precision=5, use_cache=False).logits[:, 4:].float(),
+                              atol=2e-2, rtol=2e-2)
+    # two layers of fp16 activations: a few roundings of 2^-11 each
+    for out in (got, cached):
+        assert float((out - want).norm() / want.norm()) < 2.8e-3 * 2 ** 0.5
+
+
+def test_modules_stay_what_they_are():
+    """Names, state-dict keys, copies and pickles on the CPU; the original forward serves CPU tensors."""
+    from transformers.models.llama import modeling_llama
+    from any_precision_amd import between
+    config = _config()
+    config._attn_implementation = "sdpa"
+    plain = modeling_llama.LlamaForCausalLM(config).eval()
+    model = copy.deepcopy(plain)
+    between.attach(model)
+    assert list(model.state_dict()) == list(plain.state_dict())
+    layer = model.model.layers[0]
+    assert isinstance(layer.self_attn, modeling_llama.LlamaAttention) and type(layer.self_attn).__name__ == "LlamaAttention"
+    assert type(layer.mlp) is not modeling_llama.LlamaMLP
+    ids = torch.arange(10).view(2, 5)
+    with torch.no_grad():
+        want = plain(ids, use_cache=False).logits
+        for m in (model, copy.deepcopy(model), pickle.loads(pickle.dumps(model))):
+            assert torch.allclose(m(ids, use_cache=False).logits, want, atol=1e-5)
+            assert type(m.model.norm) is between.LlamaRMSNorm
+    model(ids, use_cache=False).logits.sum().backward()
+    plain(ids, use_cache=False).logits.sum().backward()
+    for (n, a), (_, b) in zip(model.named_parameters(), plain.named_parameters()):
+        assert torch.allclose(a.grad, b.grad, atol=1e-4), n
