@@ -294,9 +294,22 @@ int ap_add_rmsnorm(const uint16_t *h, const uint16_t *delta, const uint16_t *wei
     if (!aligned16(h) || !aligned16(weight) || !aligned16(h_out) || !aligned16(x_out) || (delta && !aligned16(delta)))
         return AP_EALIGN;
     drain_stale_error();
-    add_rmsnorm_kernel<<<dim3(rows), dim3(kNormThreads), 0, static_cast<hipStream_t>(stream)>>>(
-        reinterpret_cast<const half_t *>(h), reinterpret_cast<const half_t *>(delta), reinterpret_cast<const half_t *>(weight),
-        reinterpret_cast<half_t *>(h_out), reinterpret_cast<half_t *>(x_out), H, eps);
+    const half_t *hp = reinterpret_cast<const half_t *>(h), *dp = reinterpret_cast<const half_t *>(delta);
+    const half_t *wp = reinterpret_cast<const half_t *>(weight);
+    half_t *ho = reinterpret_cast<half_t *>(h_out), *xo = reinterpret_cast<half_t *>(x_out);
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    const int units = H / 8;  // a thread each, in whole waves
+    const dim3 grid(rows), block(units < kNormMaxThreads ? (units + kWave - 1) / kWave * kWave : kNormMaxThreads);
+    if (units <= kNormMaxThreads) {
+        if (delta)
+            add_rmsnorm_kernel<1, true><<<grid, block, 0, st>>>(hp, dp, wp, ho, xo, H, eps);
+        else
+            add_rmsnorm_kernel<1, false><<<grid, block, 0, st>>>(hp, dp, wp, ho, xo, H, eps);
+    } else if (delta) {
+        add_rmsnorm_kernel<2, true><<<grid, block, 0, st>>>(hp, dp, wp, ho, xo, H, eps);
+    } else {
+        add_rmsnorm_kernel<2, false><<<grid, block, 0, st>>>(hp, dp, wp, ho, xo, H, eps);
+    }
     return launch_status();
 }
 

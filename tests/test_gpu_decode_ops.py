@@ -207,3 +207,23 @@ def test_advance_is_argmax_and_bookkeeping(n):
         tok.fill_(-1)
         advance(logits, pos, tok, emitted)
         assert int(tok.item()) == want and int(pos.item()) == 15 and int(emitted[15].item()) == -7
+
+
+@pytest.mark.parametrize("H", [8, 16, 504, 512, 520, 2056, 4096, 8184, 8192, 8200, 16384, 16392, 40000])
+@pytest.mark.parametrize("rows", [1, 3])
+@pytest.mark.parametrize("with_delta", [False, True])
+def test_add_rmsnorm_row_lengths(H, rows, with_delta):
+    """Rows around a wave, a workgroup and what a thread holds; sums written elsewhere and over h."""
+    from any_precision_amd.decode_ops import add_rmsnorm
+    gen = torch.Generator().manual_seed(H + rows)
+    h, d, w = (torch.randn(shape, generator=gen).half() for shape in ((rows, H), (rows, H), (H,)))
+    s = (h.float() + d.float()).half() if with_delta else h
+    want = s.double() * (s.double().pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt() * w.double()
+    # one rounding to fp16; the fp32 sum of H squares, its root and two products are off by less than 2^-17
+    bound = want.abs() * (2.0 ** -11 + 2.0 ** -17) + 2.0 ** -24
+    delta = d.cuda() if with_delta else None
+    for alias in (False, True):
+        hc = h.cuda()
+        got_s, got = add_rmsnorm(hc, delta, w.cuda(), 1e-5, h_out=hc if alias else torch.empty_like(hc))
+        assert torch.equal(got_s.cpu(), s)
+        assert bool(((got.cpu().double() - want).abs() <= bound).all())
