@@ -150,24 +150,40 @@ PyObject *dequant_kbit(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
 }
 
-// Keys of a module's buffers, made once.
-PyObject *key_qweight, *key_bias, *key_lut[9];
+// Names in a module's dicts, made once.
+PyObject *key_buffers, *key_qweight, *key_bias, *key_lut[9];
 
-// linear(buffers, x, w_bits): AnyPrecisionLinear.forward on the module's dict of buffers.  Up to 8 rows ap_matmul_kbit, then
+// The tensors of one AnyPrecisionLinear, read from its __dict__ in the order of nn.Module's attribute lookup.
+struct ModuleTensors {
+    PyObject *qweight, *table, *bias;  // bias: null where the module has none
+};
+
+// False where a tensor is not a buffer: a bias may also be a parameter (assigned, loaded with assign=True) or the result of a
+// parametrisation, and then shows in neither dict.
+bool tensors_of(PyObject *module_dict, int bits, ModuleTensors *m) {
+    if (!PyDict_Check(module_dict)) return false;
+    PyObject *buffers = PyDict_GetItem(module_dict, key_buffers);
+    if (buffers == nullptr || !PyDict_Check(buffers)) return false;
+    m->qweight = PyDict_GetItem(buffers, key_qweight);
+    m->table = PyDict_GetItem(buffers, key_lut[bits]);
+    m->bias = PyDict_GetItem(module_dict, key_bias);
+    if (m->bias == nullptr) m->bias = PyDict_GetItem(buffers, key_bias);
+    if (m->bias == nullptr) return false;
+    if (m->bias == Py_None) m->bias = nullptr;
+    return is_tensor(m->qweight) && is_tensor(m->table) && (m->bias == nullptr || is_tensor(m->bias));
+}
+
+// linear(module.__dict__, x, w_bits): AnyPrecisionLinear.forward.  Up to 8 rows ap_matmul_kbit, then
 // ap_gemm_kbit where ap_gemm_kbit_pays, else the weight in fp16 and torch's own product (which takes part in autograd).
 PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
-    if (n != 3 || !PyDict_Check(args[0]) || !is_tensor(args[1])) return none();
+    if (n != 3 || !is_tensor(args[1])) return none();
     const int bits = bits_of(args[2]);
-    if (bits == 0) return none();
-    PyObject *q = PyDict_GetItem(args[0], key_qweight), *t = PyDict_GetItem(args[0], key_lut[bits]);
-    PyObject *bias = PyDict_GetItem(args[0], key_bias);
-    if (!is_tensor(q) || !is_tensor(t)) return none();
-    if (bias == Py_None) bias = nullptr;
-    if (bias != nullptr && !is_tensor(bias)) return none();
+    ModuleTensors m;
+    if (bits == 0 || !tensors_of(args[0], bits, &m)) return none();
     return guarded([&]() -> PyObject * {
         const Tensor &x = THPVariable_Unpack(args[1]);
         Weight w;
-        if (!weight_of(THPVariable_Unpack(q), THPVariable_Unpack(t), bits, &w)) return none();
+        if (!weight_of(THPVariable_Unpack(m.qweight), THPVariable_Unpack(m.table), bits, &w)) return none();
         const int64_t rows = rows_of(x, w);
         if (rows < 1) return none();
         const OnDevice on(w.device);
@@ -185,12 +201,12 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
             if (rc != AP_OK) return library_error(rc, "dequant_kbit");
             out = at::matmul(x, dense.t());
         }
-        if (bias != nullptr) out.add_(THPVariable_Unpack(bias));
+        if (m.bias != nullptr) out.add_(THPVariable_Unpack(m.bias));
         return wrap(std::move(out));
     });
 }
 
-// linear_group(buffers of 2..4 modules, x, w_bits, concat): forward_group for bias-free linears of one input length.  A list of
+// linear_group(__dict__ of 2..4 modules, x, w_bits, concat): forward_group for bias-free linears of one input length.  A list of
 // results, or with concat one tensor of them side by side.  Up to 8 rows ap_matmul_kbit_group, beyond one launch of the tiled
 // GEMM where ap_gemm_kbit_group_pays; None where the modules are better called one by one.
 PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
@@ -199,16 +215,9 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
     const int bits = bits_of(args[2]), count = (int)PyTuple_GET_SIZE(args[0]);
     const bool concat = args[3] == Py_True;
     if (bits == 0 || count < 2 || count > MOST) return none();
-    PyObject *q[MOST], *t[MOST];
-    for (int g = 0; g < count; g++) {
-        PyObject *buffers = PyTuple_GET_ITEM(args[0], g);
-        if (!PyDict_Check(buffers)) return none();
-        PyObject *bias = PyDict_GetItem(buffers, key_bias);
-        if (bias != nullptr && bias != Py_None) return none();
-        q[g] = PyDict_GetItem(buffers, key_qweight);
-        t[g] = PyDict_GetItem(buffers, key_lut[bits]);
-        if (!is_tensor(q[g]) || !is_tensor(t[g])) return none();
-    }
+    ModuleTensors m[MOST];
+    for (int g = 0; g < count; g++)
+        if (!tensors_of(PyTuple_GET_ITEM(args[0], g), bits, &m[g]) || m[g].bias != nullptr) return none();
     return guarded([&]() -> PyObject * {
         const Tensor &given = THPVariable_Unpack(args[1]);
         Weight w[MOST];
@@ -217,7 +226,7 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
         const uint32_t *planes[MOST];
         const uint16_t *luts[MOST];
         for (int g = 0; g < count; g++) {
-            if (!weight_of(THPVariable_Unpack(q[g]), THPVariable_Unpack(t[g]), bits, &w[g])) return none();
+            if (!weight_of(THPVariable_Unpack(m[g].qweight), THPVariable_Unpack(m[g].table), bits, &w[g])) return none();
             if (w[g].K != w[0].K || w[g].device != w[0].device) return none();
             N[g] = w[g].N;
             total += N[g];
@@ -370,6 +379,7 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_anyprec_torch", nullptr, -1, meth
 }  // namespace
 
 PyMODINIT_FUNC PyInit__anyprec_torch(void) {
+    key_buffers = PyUnicode_InternFromString("_buffers");
     key_qweight = PyUnicode_InternFromString("qweight");
     key_bias = PyUnicode_InternFromString("bias");
     for (int b = 3; b <= 8; b++) key_lut[b] = PyUnicode_InternFromString(("lut" + std::to_string(b)).c_str());

@@ -170,3 +170,37 @@ def test_forward_group_beyond_32_rows_is_one_tiled_launch(oracle):
         for L, got in zip(layers, outs):
             _, want = oracle.matmul_kbit(x, L.qweight, L.luts[b], b, return_f64=True)
             assert_close_gemv(got, want, f"forward_group narrow tiles b={b} rows={rows} N={L.N}")
+
+
+@pytest.mark.parametrize("M", [1, 8, 16, 200, 600])
+@pytest.mark.parametrize("kind", ["assigned", "over a buffer", "loaded", "parametrised", "buffer", "none again"])
+def test_a_bias_of_any_kind_is_added(kind, M):
+    """A bias may be a buffer, a parameter (assigned, or loaded with assign=True) or the result of a parametrisation: linears
+    and sets of them give the product plus what ``module.bias`` is.  The rows cover every branch of the dispatch."""
+    from any_precision_amd.linear import forward_group
+    L = make(64, 1024, seed=6)
+    plain, _ = _module(L, bias=False)
+    m, sd = _module(L, bias=kind not in ("assigned", "none again"))
+    value = torch.linspace(-3, 3, L.N).half()
+    if kind == "loaded":
+        m.load_state_dict({**{k: v.cuda() for k, v in sd.items()}, "bias": torch.nn.Parameter(value.cuda())}, assign=True)
+    elif kind == "parametrised":
+        class Doubled(torch.nn.Module):
+            def forward(self, t):
+                return 2 * t
+        m.bias.copy_(value / 2)
+        torch.nn.utils.parametrize.register_parametrization(m, "bias", Doubled())
+    elif kind == "buffer":
+        m.bias.copy_(value)
+    else:
+        m.bias = torch.nn.Parameter(value.cuda())
+        if kind == "none again":
+            m.bias, value = None, torch.zeros_like(value)
+    x = torch.from_numpy(synth.make_x(M, L.K, seed=M)).cuda()
+    product = plain(x, precision=4)
+    want = product + value.cuda()
+    # a set may take another kernel than its member alone: fp32 sums in another order, one unit of fp16 before the bias is
+    # added and one after
+    bound = 2.0 ** -9 * (product.float().abs() + value.cuda().float().abs()) + 2.0 ** -20
+    for got in (m(x, precision=4), forward_group((m, m), x, 4)[1], forward_group((plain, m), x, 4, concat=True)[:, L.N:]):
+        assert bool(((got.float() - want.float()).abs() <= bound).all())
