@@ -44,29 +44,26 @@ def _mlp_forward(module, original, x):
     return module.down_proj(act(gate) * up if hidden is None else hidden)
 
 
-def _rotated(native, x, cos, sin):
-    """x [B, T, heads * hd] with its rotary embedding, [B, heads, T, hd]."""
-    out = native.rope(x, cos, sin)
-    if out is None:
-        x = x.view(*x.shape[:2], -1, cos.shape[-1])
-        low, high = x.chunk(2, dim=-1)
-        out = x * cos.unsqueeze(2) + torch.cat((-high, low), dim=-1) * sin.unsqueeze(2)
-    return out.transpose(1, 2)
-
-
 def _attention_forward(module, original, hidden_states, position_embeddings=None, attention_mask=None, past_key_values=None,
                        **kwargs):
     native = _native()
     if (native is None or position_embeddings is None or attention_mask is not None or past_key_values is not None
-            or hidden_states.dim() != 3 or module.training or torch.is_grad_enabled()
+            or module.training or torch.is_grad_enabled() or hidden_states.dim() != 3
             or module.config._attn_implementation != "sdpa" or not getattr(module, "is_causal", True)
-            or kwargs.get("output_attentions") or any(k not in _IDLE and v is not None for k, v in kwargs.items())):
+            or kwargs.get("output_attentions") or any(k not in _IDLE and v is not None for k, v in kwargs.items())
+            or not native.plain(hidden_states, *position_embeddings)):
         return original(hidden_states, position_embeddings=position_embeddings, attention_mask=attention_mask,
                         past_key_values=past_key_values, **kwargs)
     cos, sin = position_embeddings
     B, T = hidden_states.shape[:2]
     q, k, v = (p(hidden_states) for p in (module.q_proj, module.k_proj, module.v_proj))
-    q, k, v = _rotated(native, q, cos, sin), _rotated(native, k, cos, sin), v.view(B, T, -1, cos.shape[-1]).transpose(1, 2)
+    rotated = native.rope(q, cos, sin), native.rope(k, cos, sin)
+    q, k, v = (t.view(B, T, -1, module.head_dim).transpose(1, 2) for t in (q, k, v))
+    if None in rotated:     # projections that are not this library's
+        from transformers.models.llama.modeling_llama import apply_rotary_pos_emb
+        q, k = apply_rotary_pos_emb(q, k, cos, sin)
+    else:
+        q, k = (t.transpose(1, 2) for t in rotated)
     ctx = F.scaled_dot_product_attention(q, k, v, is_causal=T > 1, scale=module.scaling, enable_gqa=q.shape[1] != k.shape[1])
     return module.o_proj(ctx.transpose(1, 2).reshape(B, T, -1)), None
 

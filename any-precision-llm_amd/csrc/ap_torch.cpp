@@ -303,6 +303,18 @@ bool plain_execution() {
            !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
 }
 
+// plain(tensors): whether the functions below take each of them, all on one device.
+PyObject *plain(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return guarded([&]() -> PyObject * {
+        bool all = n > 0 && plain_execution() && plain_half(args[0], nullptr);
+        for (Py_ssize_t i = 1; all && i < n; i++) {
+            const at::Device device = THPVariable_Unpack(args[0]).device();
+            all = plain_half(args[i], &device);
+        }
+        return PyBool_FromLong(all);
+    });
+}
+
 // rmsnorm(x, weight, eps): x * rsqrt(mean(x^2) + eps) * weight over the last dimension.
 PyObject *rmsnorm(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (n != 3 || !PyFloat_Check(args[2]) || !plain_execution()) return none();
@@ -369,6 +381,7 @@ PyMethodDef methods[] = {
     {"dequant_kbit", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(dequant_kbit)), METH_FASTCALL, nullptr},
     {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(linear)), METH_FASTCALL, nullptr},
     {"linear_group", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(linear_group)), METH_FASTCALL, nullptr},
+    {"plain", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(plain)), METH_FASTCALL, nullptr},
     {"rmsnorm", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(rmsnorm)), METH_FASTCALL, nullptr},
     {"silu_mul", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(silu_mul)), METH_FASTCALL, nullptr},
     {"rope", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(rope)), METH_FASTCALL, nullptr},

@@ -104,3 +104,49 @@ def test_modules_stay_what_they_are():
     plain(ids, use_cache=False).logits.sum().backward()
     for (n, a), (_, b) in zip(model.named_parameters(), plain.named_parameters()):
         assert torch.allclose(a.grad, b.grad, atol=1e-4), n
+
+
+def _attention(attached):
+    from transformers.models.llama import modeling_llama
+    from any_precision_amd import between
+    config = _config()
+    config._attn_implementation = "sdpa"
+    torch.manual_seed(5)
+    model = modeling_llama.LlamaForCausalLM(config).eval()
+    if attached:
+        between.attach(model)
+    return model.model.layers[0].self_attn
+
+
+def test_a_trace_of_the_attention_is_the_modules_own():
+    """Sizes are tensors under a trace; the replaced forward hands a traced call over."""
+    gen = torch.Generator().manual_seed(0)
+    x, cos, sin = torch.randn((2, 7, 64), generator=gen), *(torch.rand((2, 7, 16), generator=gen) for _ in range(2))
+
+    class Alone(torch.nn.Module):
+        def __init__(self, attention):
+            super().__init__()
+            self.attention = attention
+
+        def forward(self, x, cos, sin):
+            return self.attention(x, (cos, sin))[0]
+
+    with torch.no_grad():
+        plain, module = Alone(_attention(False)), Alone(_attention(True))
+        want = plain(x, cos, sin)
+        traced = torch.jit.trace(module, (x, cos, sin))
+        assert torch.equal(traced(x, cos, sin), want) and torch.equal(module(x, cos, sin), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float64])
+def test_attention_on_other_types_and_devices_is_the_modules_own(dtype, monkeypatch):
+    """One decision before the projections: the call as a whole goes to the original forward."""
+    from transformers.models.llama import modeling_llama
+    module = _attention(True).to(dtype)
+    calls = []
+    stock = modeling_llama.LlamaAttention.forward
+    monkeypatch.setattr(modeling_llama.LlamaAttention, "forward", lambda self, *a, **kw: calls.append(1) or stock(self, *a, **kw))
+    cos = torch.rand((1, 7, 16)).to(dtype)
+    with torch.no_grad():
+        module(torch.randn((1, 7, 64)).to(dtype), (cos, cos))
+    assert calls == [1]
