@@ -10,9 +10,12 @@ attention mask, other attention implementations.
 from __future__ import annotations
 
 import functools
+import os
 
 import torch
+import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import _capi
 
@@ -30,14 +33,38 @@ def _norm_forward(module, original, hidden_states):
     return original(hidden_states) if out is None else out
 
 
-def _has_hooks(module):
-    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+def _unchanged(function, package):
+    """Whether ``function`` and everything it wraps is code of ``package``, and not a replacement someone has put in its place."""
+    home = os.path.dirname(package.__file__) + os.sep
+    while function is not None:
+        code = getattr(function, "__code__", None)
+        if code is None or not code.co_filename.startswith(home):
+            return False
+        function = getattr(function, "__wrapped__", None)
+    return True
+
+
+@functools.lru_cache(None)
+def _silu_forwards():
+    """The classes of the activation function that silu_mul computes, with their forwards."""
+    import transformers
+    from transformers import activations
+    found = ((nn.SiLU, torch), (getattr(activations, "SiLUActivation", None), transformers))
+    return {c: c.forward for c, package in found if c is not None and _unchanged(c.forward, package)}
+
+
+def _plain_silu(act):
+    """Whether calling ``act`` is SiLU and nothing else: no replaced forward, no hooks of its own or of all modules."""
+    d = act.__dict__
+    return (type(act).forward is _silu_forwards().get(type(act)) and "forward" not in d and d.get("_compiled_call_impl") is None
+            and not (act._forward_hooks or act._forward_pre_hooks or act._backward_hooks or act._backward_pre_hooks)
+            and not _has_any_global_hook())
 
 
 def _mlp_forward(module, original, x):
     native = _native()
     act = module.act_fn
-    if native is None or _has_hooks(act) or type(act).__name__ not in ("SiLU", "SiLUActivation"):
+    if native is None or not _plain_silu(act) or not native.plain(x):
         return original(x)
     gate, up = module.gate_proj(x), module.up_proj(x)
     hidden = native.silu_mul(gate, up)

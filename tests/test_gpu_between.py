@@ -150,3 +150,80 @@ def test_attention_on_other_types_and_devices_is_the_modules_own(dtype, monkeypa
     with torch.no_grad():
         module(torch.randn((1, 7, 64)).to(dtype), (cos, cos))
     assert calls == [1]
+
+
+class _Serving:
+    """Stands for the native module on the CPU: serves every call, with torch ops."""
+    served = 0
+
+    def plain(self, *tensors):
+        return True
+
+    def silu_mul(self, gate, up):
+        self.served += 1
+        return torch.nn.functional.silu(gate) * up
+
+    def rmsnorm(self, x, weight, eps):
+        self.served += 1
+        return torch.nn.functional.rms_norm(x, weight.shape, weight, eps)
+
+    def rope(self, x, cos, sin):
+        self.served += 1
+        x = x.view(*x.shape[:2], -1, cos.shape[-1])
+        low, high = x.chunk(2, dim=-1)
+        return x * cos.unsqueeze(2) + torch.cat((-high, low), dim=-1) * sin.unsqueeze(2)
+
+
+@pytest.fixture
+def serving(monkeypatch):
+    from any_precision_amd import between
+    stand_in = _Serving()
+    monkeypatch.setattr(between, "_native", lambda: stand_in)
+    return stand_in
+
+
+def _mlp():
+    from transformers.models.llama import modeling_llama
+    from any_precision_amd import between
+    model = modeling_llama.LlamaForCausalLM(_config()).eval()
+    between.attach(model)
+    return model.model.layers[0].mlp
+
+
+@pytest.mark.parametrize("change", ["nothing", "torch's class", "a class of that name", "instance forward", "class forward", "hook",
+                                    "global hook"])
+def test_the_activation_function_is_called_where_it_is_not_plain(serving, monkeypatch, change):
+    mlp = _mlp()
+    calls = []
+    handle = None
+
+    def other(t):
+        calls.append(1)
+        return t * 3
+
+    if change == "torch's class":
+        mlp.act_fn = torch.nn.SiLU()
+    elif change == "a class of that name":
+        mlp.act_fn = type("SiLU", (torch.nn.Module,), {"forward": lambda self, t: other(t)})()
+    elif change == "instance forward":
+        mlp.act_fn.forward = other
+    elif change == "class forward":
+        monkeypatch.setattr(type(mlp.act_fn), "forward", lambda self, t: other(t))
+    elif change == "hook":
+        handle = mlp.act_fn.register_forward_hook(lambda m, args, out: other(args[0]))
+    elif change == "global hook":
+        handle = torch.nn.modules.module.register_module_forward_hook(
+            lambda m, args, out: other(args[0]) if m is mlp.act_fn else None)
+    x = torch.randn((2, 64), generator=torch.Generator().manual_seed(0))
+    try:
+        with torch.no_grad():
+            act = torch.nn.functional.silu if change in ("nothing", "torch's class") else other
+            want = mlp.down_proj(act(mlp.gate_proj(x)) * mlp.up_proj(x))
+            calls.clear()
+            got = mlp(x)
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert torch.allclose(got, want, atol=1e-6)
+    plain = change in ("nothing", "torch's class")
+    assert serving.served == plain and calls == [1] * (not plain)
