@@ -11,10 +11,10 @@ from __future__ import annotations
 
 import functools
 import os
+import sys
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 from torch.nn.modules.module import _has_any_global_hook
 
 from . import _capi
@@ -33,9 +33,10 @@ def _norm_forward(module, original, hidden_states):
     return original(hidden_states) if out is None else out
 
 
+@functools.lru_cache(64)
 def _unchanged(function, package):
     """Whether ``function`` and everything it wraps is code of ``package``, and not a replacement someone has put in its place."""
-    home = os.path.dirname(package.__file__) + os.sep
+    home = os.path.dirname(sys.modules[package].__file__) + os.sep
     while function is not None:
         code = getattr(function, "__code__", None)
         if code is None or not code.co_filename.startswith(home):
@@ -47,9 +48,8 @@ def _unchanged(function, package):
 @functools.lru_cache(None)
 def _silu_forwards():
     """The classes of the activation function that silu_mul computes, with their forwards."""
-    import transformers
     from transformers import activations
-    found = ((nn.SiLU, torch), (getattr(activations, "SiLUActivation", None), transformers))
+    found = ((nn.SiLU, "torch"), (getattr(activations, "SiLUActivation", None), "transformers"))
     return {c: c.forward for c, package in found if c is not None and _unchanged(c.forward, package)}
 
 
@@ -74,7 +74,8 @@ def _mlp_forward(module, original, x):
 def _attention_forward(module, original, hidden_states, position_embeddings=None, attention_mask=None, past_key_values=None,
                        **kwargs):
     native = _native()
-    if (native is None or position_embeddings is None or attention_mask is not None or past_key_values is not None
+    llama = sys.modules["transformers.models.llama.modeling_llama"]       # its rotary embedding and its attention functions
+    if (native is None or not _unchanged(llama.apply_rotary_pos_emb, "transformers") or position_embeddings is None or attention_mask is not None or past_key_values is not None
             or module.training or torch.is_grad_enabled() or hidden_states.dim() != 3
             or module.config._attn_implementation != "sdpa" or not getattr(module, "is_causal", True)
             or kwargs.get("output_attentions") or any(k not in _IDLE and v is not None for k, v in kwargs.items())
@@ -87,12 +88,12 @@ def _attention_forward(module, original, hidden_states, position_embeddings=None
     rotated = native.rope(q, cos, sin), native.rope(k, cos, sin)
     q, k, v = (t.view(B, T, -1, module.head_dim).transpose(1, 2) for t in (q, k, v))
     if None in rotated:     # projections that are not this library's
-        from transformers.models.llama.modeling_llama import apply_rotary_pos_emb
-        q, k = apply_rotary_pos_emb(q, k, cos, sin)
+        q, k = llama.apply_rotary_pos_emb(q, k, cos, sin)
     else:
         q, k = (t.transpose(1, 2) for t in rotated)
-    ctx = F.scaled_dot_product_attention(q, k, v, is_causal=T > 1, scale=module.scaling, enable_gqa=q.shape[1] != k.shape[1])
-    return module.o_proj(ctx.transpose(1, 2).reshape(B, T, -1)), None
+    # the registered function of that name: torch's attention, or what the program has put in its place
+    ctx, weights = llama.ALL_ATTENTION_FUNCTIONS["sdpa"](module, q, k, v, None, dropout=0.0, scaling=module.scaling, **kwargs)
+    return module.o_proj(ctx.reshape(B, T, -1)), weights
 
 
 _FORWARDS = {"LlamaRMSNorm": _norm_forward, "LlamaMLP": _mlp_forward, "LlamaAttention": _attention_forward}
@@ -103,10 +104,13 @@ def _class(name):
     """The class ``name`` of the Hugging Face Llama model with its forward replaced."""
     from transformers.models.llama import modeling_llama
     base, step = getattr(modeling_llama, name), _FORWARDS[name]
+    stock = base.forward if _unchanged(base.forward, "transformers") else None
 
     @functools.wraps(base.forward)
     def forward(self, *args, **kwargs):
-        return step(self, functools.partial(base.forward, self), *args, **kwargs)
+        if base.forward is not stock:       # replaced, before or after the class was made
+            return base.forward(self, *args, **kwargs)
+        return step(self, functools.partial(stock, self), *args, **kwargs)
 
     return type(name, (base,), {"forward": forward, "__module__": __name__})
 

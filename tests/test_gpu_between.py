@@ -1,6 +1,7 @@
 """The kernels between the linears of the Hugging Face Llama modules against the modules' own torch ops in float64, and the
 calls that have to stay with the original forwards."""
 import copy
+import functools
 import pickle
 
 import pytest
@@ -227,3 +228,47 @@ def test_the_activation_function_is_called_where_it_is_not_plain(serving, monkey
     assert torch.allclose(got, want, atol=1e-6)
     plain = change in ("nothing", "torch's class")
     assert serving.served == plain and calls == [1] * (not plain)
+
+
+@pytest.mark.parametrize("change", ["nothing", "LlamaRMSNorm", "LlamaMLP", "LlamaAttention", "rotary", "attention function"])
+@pytest.mark.parametrize("when", ["before", "after"])
+def test_what_a_program_has_replaced_is_called(serving, monkeypatch, change, when):
+    """Forwards replaced on the Hugging Face classes, their rotary embedding and a registered attention function."""
+    from transformers.models.llama import modeling_llama
+    from any_precision_amd import between
+    config = _config()
+    config._attn_implementation = "sdpa"
+    calls = []
+
+    def counted(function):
+        @functools.wraps(function)
+        def call(*args, **kwargs):
+            calls.append(1)
+            return function(*args, **kwargs)
+        return call
+
+    def replace():
+        if change.startswith("Llama"):
+            cls = getattr(modeling_llama, change)
+            monkeypatch.setattr(cls, "forward", counted(cls.forward))
+        elif change == "rotary":
+            monkeypatch.setattr(modeling_llama, "apply_rotary_pos_emb", counted(modeling_llama.apply_rotary_pos_emb))
+        elif change == "attention function":
+            functions = modeling_llama.ALL_ATTENTION_FUNCTIONS
+            monkeypatch.setitem(functions._global_mapping, "sdpa", counted(functions["sdpa"]))
+
+    between._class.cache_clear()        # the classes are made anew
+    try:
+        if when == "before":
+            replace()
+        model = modeling_llama.LlamaForCausalLM(config).eval()
+        between.attach(model)
+        if when == "after":
+            replace()
+        with torch.no_grad():
+            model(torch.arange(10).view(2, 5), use_cache=False)
+    finally:
+        between._class.cache_clear()
+    assert len(calls) == {"nothing": 0, "LlamaRMSNorm": 5}.get(change, 2)
+    # of two layers: five norms, two MLPs, four rotary embeddings
+    assert serving.served == 11 - {"LlamaRMSNorm": 5, "LlamaMLP": 2, "LlamaAttention": 4, "rotary": 4}.get(change, 0)
