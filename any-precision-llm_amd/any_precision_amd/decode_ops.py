@@ -42,7 +42,7 @@ def add_rmsnorm(h, delta, weight, eps, h_out=None, x_out=None):
 
 
 def silu_mul(gate, up, out=None):
-    """``silu(gate) * up`` elementwise."""
+    """``silu(gate) * up`` elementwise; ``out`` may be ``gate`` or ``up`` itself."""
     _f16(gate, "gate"), _f16(up, "up")
     if gate.shape != up.shape:
         raise ValueError("gate and up must have one shape")

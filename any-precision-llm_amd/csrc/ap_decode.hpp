@@ -111,9 +111,9 @@ __global__ __launch_bounds__(kNormMaxThreads) void add_rmsnorm_kernel(const half
     }
 }
 
-// out = gate / (1 + exp(-gate)) * up over n elements (n % 8 == 0).
-__global__ __launch_bounds__(256) void silu_mul_kernel(const half_t *__restrict__ gate, const half_t *__restrict__ up,
-                                                       half_t *__restrict__ out, long long n) {
+// out = gate / (1 + exp(-gate)) * up over n elements (n % 8 == 0).  out may be gate or up: a thread reads its 8 elements before
+// it writes them, and no other thread touches them.
+__global__ __launch_bounds__(256) void silu_mul_kernel(const half_t *gate, const half_t *up, half_t *out, long long n) {
     const long long stride = (long long)gridDim.x * blockDim.x * 8;
     for (long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 8; i < n; i += stride) {
         const half8_t g = *reinterpret_cast<const half8_t *>(gate + i);

@@ -193,7 +193,8 @@ int ap_probe_empty(uint32_t *sink, void *stream);
  *
  * ap_add_rmsnorm: for each of `rows` rows of H elements (H % 8 == 0): s = h + delta (an fp16 add; delta may
  *   be NULL), written to h_out (may alias h); x_out = s * rsqrt(mean(s^2) + eps) * weight[H]  (LlamaRMSNorm).
- * ap_silu_mul: out = gate / (1 + exp(-gate)) * up over n elements (n % 8 == 0)  (the SwiGLU gate).
+ * ap_silu_mul: out = gate / (1 + exp(-gate)) * up over n elements (n % 8 == 0)  (the SwiGLU gate); out may be gate or up
+ *   itself (a partial overlap is not served).
  * ap_decode_attention: rotary embedding, cache append and attention of the token at cache row *pos (a device
  *   scalar, so the launch can sit in a replayed graph):
  *     qkv   [n_heads + 2 n_kv_heads, head_dim]  query, key and value heads of the token, before the rotary embedding

@@ -227,3 +227,14 @@ def test_add_rmsnorm_row_lengths(H, rows, with_delta):
         got_s, got = add_rmsnorm(hc, delta, w.cuda(), 1e-5, h_out=hc if alias else torch.empty_like(hc))
         assert torch.equal(got_s.cpu(), s)
         assert bool(((got.cpu().double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("n", [8, 2056, 4096 * 256 * 8 + 8])      # one unit, a ragged workgroup, more than one round of the grid
+@pytest.mark.parametrize("over", ["gate", "up"])
+def test_silu_mul_in_place(n, over):
+    from any_precision_amd.decode_ops import silu_mul
+    g = torch.Generator(device="cuda").manual_seed(n)
+    gate, up = ((torch.randn((n,), device="cuda", generator=g) * 3).half() for _ in range(2))
+    want = silu_mul(gate, up)
+    out = gate if over == "gate" else up
+    assert silu_mul(gate, up, out=out) is out and torch.equal(out, want)
