@@ -109,6 +109,16 @@ struct OnDevice {
     void *stream;
 };
 
+// Other Python threads run meanwhile: a launch may wait for its queue, an allocation for the device.  Nothing in the scope
+// touches Python, and tensors that come from a module's dicts are held by copies: a thread may replace them meanwhile.
+struct WithoutGil {
+    WithoutGil() : state(PyEval_SaveThread()) {}
+    ~WithoutGil() { PyEval_RestoreThread(state); }
+    WithoutGil(const WithoutGil &) = delete;
+    WithoutGil &operator=(const WithoutGil &) = delete;
+    PyThreadState *state;
+};
+
 PyObject *wrap(Tensor t) { return THPVariable_Wrap(std::move(t)); }
 
 // matmul_kbit(x, qweight, lut, w_bits) and gemm_kbit(x, qweight, lut, w_bits)
@@ -122,10 +132,15 @@ PyObject *product(PyObject *const *args, Py_ssize_t n, bool gemm) {
         if (!weight_of(THPVariable_Unpack(args[1]), THPVariable_Unpack(args[2]), bits, &w)) return none();
         const int64_t rows = rows_of(x, w);
         if (rows < 1 || (!gemm && rows > 8) || !x.is_contiguous()) return none();
-        const OnDevice on(w.device);
-        Tensor out = result_for(x, w.N);
-        const int rc = gemm ? ap_gemm_kbit(half_ptr(x), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream)
-                            : ap_matmul_kbit(half_ptr(x), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream);
+        Tensor out;
+        int rc;
+        {
+            const WithoutGil free;
+            const OnDevice on(w.device);
+            out = result_for(x, w.N);
+            rc = gemm ? ap_gemm_kbit(half_ptr(x), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream)
+                      : ap_matmul_kbit(half_ptr(x), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream);
+        }
         if (rc != AP_OK) return library_error(rc, gemm ? "gemm_kbit" : "matmul_kbit");
         return wrap(std::move(out));
     });
@@ -142,9 +157,14 @@ PyObject *dequant_kbit(PyObject *, PyObject *const *args, Py_ssize_t n) {
         const Tensor &q = THPVariable_Unpack(args[0]);
         Weight w;
         if (!weight_of(q, THPVariable_Unpack(args[1]), bits, &w)) return none();
-        const OnDevice on(w.device);
-        Tensor out = empty_half({w.N, w.K}, q.device());
-        const int rc = ap_dequant_kbit(w.planes, w.lut, half_out(out), w.N, w.K, bits, on.stream);
+        Tensor out;
+        int rc;
+        {
+            const WithoutGil free;
+            const OnDevice on(w.device);
+            out = empty_half({w.N, w.K}, q.device());
+            rc = ap_dequant_kbit(w.planes, w.lut, half_out(out), w.N, w.K, bits, on.stream);
+        }
         if (rc != AP_OK) return library_error(rc, "dequant_kbit");
         return wrap(std::move(out));
     });
@@ -182,26 +202,32 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (bits == 0 || !tensors_of(args[0], bits, &m)) return none();
     return guarded([&]() -> PyObject * {
         const Tensor &x = THPVariable_Unpack(args[1]);
+        const Tensor q = THPVariable_Unpack(m.qweight), t = THPVariable_Unpack(m.table);
+        const Tensor bias = m.bias == nullptr ? Tensor() : THPVariable_Unpack(m.bias);
         Weight w;
-        if (!weight_of(THPVariable_Unpack(m.qweight), THPVariable_Unpack(m.table), bits, &w)) return none();
+        if (!weight_of(q, t, bits, &w)) return none();
         const int64_t rows = rows_of(x, w);
         if (rows < 1) return none();
-        const OnDevice on(w.device);
-        const bool pays = rows <= 8 || ap_gemm_kbit_pays((int)rows, w.N, w.K, bits) == 1;
+        const char *op = rows <= 8 ? "matmul_kbit" : "gemm_kbit";
         Tensor out;
-        if (pays) {
-            const Tensor dense = x.is_contiguous() ? x : x.contiguous();  // the kernels take dense rows
-            out = result_for(x, w.N);
-            const int rc = rows <= 8 ? ap_matmul_kbit(half_ptr(dense), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream)
-                                     : ap_gemm_kbit(half_ptr(dense), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream);
-            if (rc != AP_OK) return library_error(rc, rows <= 8 ? "matmul_kbit" : "gemm_kbit");
-        } else {
-            const Tensor dense = empty_half({w.N, w.K}, x.device());
-            const int rc = ap_dequant_kbit(w.planes, w.lut, half_out(dense), w.N, w.K, bits, on.stream);
-            if (rc != AP_OK) return library_error(rc, "dequant_kbit");
-            out = at::matmul(x, dense.t());
+        int rc;
+        {
+            const WithoutGil free;
+            const OnDevice on(w.device);
+            if (rows <= 8 || ap_gemm_kbit_pays((int)rows, w.N, w.K, bits) == 1) {
+                const Tensor dense = x.is_contiguous() ? x : x.contiguous();  // the kernels take dense rows
+                out = result_for(x, w.N);
+                rc = rows <= 8 ? ap_matmul_kbit(half_ptr(dense), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream)
+                               : ap_gemm_kbit(half_ptr(dense), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream);
+            } else {
+                op = "dequant_kbit";
+                const Tensor dense = empty_half({w.N, w.K}, x.device());
+                rc = ap_dequant_kbit(w.planes, w.lut, half_out(dense), w.N, w.K, bits, on.stream);
+                if (rc == AP_OK) out = at::matmul(x, dense.t());
+            }
+            if (rc == AP_OK && bias.defined()) out.add_(bias);
         }
-        if (m.bias != nullptr) out.add_(THPVariable_Unpack(m.bias));
+        if (rc != AP_OK) return library_error(rc, op);
         return wrap(std::move(out));
     });
 }
@@ -220,13 +246,16 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (!tensors_of(PyTuple_GET_ITEM(args[0], g), bits, &m[g]) || m[g].bias != nullptr) return none();
     return guarded([&]() -> PyObject * {
         const Tensor &given = THPVariable_Unpack(args[1]);
+        Tensor q[MOST], t[MOST];
         Weight w[MOST];
         int N[MOST];
         int64_t total = 0;
         const uint32_t *planes[MOST];
         const uint16_t *luts[MOST];
         for (int g = 0; g < count; g++) {
-            if (!weight_of(THPVariable_Unpack(m[g].qweight), THPVariable_Unpack(m[g].table), bits, &w[g])) return none();
+            q[g] = THPVariable_Unpack(m[g].qweight);
+            t[g] = THPVariable_Unpack(m[g].table);
+            if (!weight_of(q[g], t[g], bits, &w[g])) return none();
             if (w[g].K != w[0].K || w[g].device != w[0].device) return none();
             N[g] = w[g].N;
             total += N[g];
@@ -238,35 +267,36 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (rows < 1) return none();
         const bool gemm = rows > 8;
         if (gemm && ap_gemm_kbit_group_pays(count, N, (int)rows, K, bits) != 1) return none();
-        const Tensor x = given.is_contiguous() ? given : given.contiguous();
-        const OnDevice on(w[0].device);
         // side by side in one allocation: one row's results always are dense, and the tiled kernel writes rows that are not
         const bool joint = concat && (gemm ? K % 128 == 0 : rows == 1);
         Tensor all, outs[MOST];
-        uint16_t *to[MOST];
-        long long ldo[MOST];
-        if (joint) {
-            all = result_for(x, total);
-            int64_t at = 0;
-            for (int g = 0; g < count; at += N[g], g++) {
-                to[g] = half_out(all) + at;
-                ldo[g] = total;
+        int rc;
+        {
+            const WithoutGil free;
+            const OnDevice on(w[0].device);
+            const Tensor x = given.is_contiguous() ? given : given.contiguous();
+            uint16_t *to[MOST];
+            long long ldo[MOST];
+            if (joint) {
+                all = result_for(x, total);
+                int64_t at = 0;
+                for (int g = 0; g < count; at += N[g], g++) {
+                    to[g] = half_out(all) + at;
+                    ldo[g] = total;
+                }
+            } else {
+                for (int g = 0; g < count; g++) {
+                    outs[g] = result_for(x, N[g]);
+                    to[g] = half_out(outs[g]);
+                }
             }
-        } else {
-            for (int g = 0; g < count; g++) {
-                outs[g] = result_for(x, N[g]);
-                to[g] = half_out(outs[g]);
-            }
+            rc = gemm ? ap_gemm_kbit_group(half_ptr(x), count, planes, luts, to, N, joint ? ldo : nullptr, (int)rows, K, bits, on.stream)
+                      : ap_matmul_kbit_group(half_ptr(x), count, planes, luts, to, N, (int)rows, K, bits, on.stream);
+            if (rc == AP_OK && concat && !joint) all = at::cat(std::vector<Tensor>(outs, outs + count), -1);
         }
-        const int rc = gemm ? ap_gemm_kbit_group(half_ptr(x), count, planes, luts, to, N, joint ? ldo : nullptr, (int)rows, K, bits, on.stream)
-                            : ap_matmul_kbit_group(half_ptr(x), count, planes, luts, to, N, (int)rows, K, bits, on.stream);
         if (rc == AP_ELIMIT) return none();  // beyond the tiled kernel's offsets
         if (rc != AP_OK) return library_error(rc, gemm ? "gemm_kbit_group" : "matmul_kbit_group");
-        if (joint) return wrap(std::move(all));
-        if (concat) {
-            std::vector<Tensor> parts(outs, outs + count);
-            return wrap(at::cat(parts, -1));
-        }
+        if (concat) return wrap(std::move(all));
         PyObject *list = PyList_New(count);
         if (list == nullptr) return nullptr;
         for (int g = 0; g < count; g++) {
@@ -324,13 +354,19 @@ PyObject *rmsnorm(PyObject *, PyObject *const *args, Py_ssize_t n) {
         const at::Device device = x.device();
         if (!plain_half(args[1], &device)) return none();
         const Tensor &weight = THPVariable_Unpack(args[1]);
+        const float eps = (float)PyFloat_AS_DOUBLE(args[2]);
         const int64_t H = x.dim() < 1 ? 0 : x.size(-1);
         if (weight.dim() != 1 || weight.size(0) != H || H < 8 || H % 8 || H > INT32_MAX || x.numel() / H > INT32_MAX) return none();
-        const OnDevice on(device.index());
-        Tensor out = empty_half(x.sizes(), device);
-        // nothing is added, so h_out = h is not written
-        const int rc = ap_add_rmsnorm(half_ptr(x), nullptr, half_ptr(weight), half_out(x), half_out(out), (int)(x.numel() / H), (int)H,
-                                      (float)PyFloat_AS_DOUBLE(args[2]), on.stream);
+        Tensor out;
+        int rc;
+        {
+            const WithoutGil free;
+            const OnDevice on(device.index());
+            out = empty_half(x.sizes(), device);
+            // nothing is added, so h_out = h is not written
+            rc = ap_add_rmsnorm(half_ptr(x), nullptr, half_ptr(weight), half_out(x), half_out(out), (int)(x.numel() / H), (int)H, eps,
+                                on.stream);
+        }
         if (rc != AP_OK) return library_error(rc, "rmsnorm");
         return wrap(std::move(out));
     });
@@ -346,9 +382,14 @@ PyObject *silu_mul(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (!plain_half(args[1], &device)) return none();
         const Tensor &up = THPVariable_Unpack(args[1]);
         if (gate.sizes() != up.sizes() || gate.numel() % 8) return none();
-        const OnDevice on(device.index());
-        Tensor out = empty_half(gate.sizes(), device);
-        const int rc = ap_silu_mul(half_ptr(gate), half_ptr(up), half_out(out), gate.numel(), on.stream);
+        Tensor out;
+        int rc;
+        {
+            const WithoutGil free;
+            const OnDevice on(device.index());
+            out = empty_half(gate.sizes(), device);
+            rc = ap_silu_mul(half_ptr(gate), half_ptr(up), half_out(out), gate.numel(), on.stream);
+        }
         if (rc != AP_OK) return library_error(rc, "silu_mul");
         return wrap(std::move(out));
     });
@@ -366,10 +407,15 @@ PyObject *rope(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (x.dim() != 3 || c.dim() != 3 || c.sizes() != s.sizes()) return none();
         const int64_t B = x.size(0), T = x.size(1), hd = c.size(2);
         if (c.size(1) != T || (c.size(0) != B && c.size(0) != 1) || hd % 16 || x.size(2) % hd || x.numel() / 16 > INT32_MAX) return none();
-        const OnDevice on(device.index());
-        Tensor out = empty_half({B, T, x.size(2) / hd, hd}, device);
-        const int rc = ap_rope_heads(half_ptr(x), half_ptr(c), half_ptr(s), half_out(out), (int)(B * T), (int)(c.size(0) * T),
-                                     (int)(x.size(2) / hd), (int)hd, on.stream);
+        Tensor out;
+        int rc;
+        {
+            const WithoutGil free;
+            const OnDevice on(device.index());
+            out = empty_half({B, T, x.size(2) / hd, hd}, device);
+            rc = ap_rope_heads(half_ptr(x), half_ptr(c), half_ptr(s), half_out(out), (int)(B * T), (int)(c.size(0) * T),
+                               (int)(x.size(2) / hd), (int)hd, on.stream);
+        }
         if (rc != AP_OK) return library_error(rc, "rope");
         return wrap(std::move(out));
     });
