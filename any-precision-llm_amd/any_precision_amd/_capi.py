@@ -26,20 +26,34 @@ _torch_module = None
 
 
 def torch_module():
-    """The native module over the library (csrc/ap_torch.cpp); torch has to be imported before it is loaded."""
+    """The native module over the library (csrc/ap_torch.cpp)."""
     global _torch_module
     if _torch_module is None:
-        import importlib.machinery
-        import importlib.util
+        _torch_module = _load_torch_module(os.path.join(_PKG_ROOT, "lib", "_anyprec_torch.so"))
+    return _torch_module
 
-        path = os.path.join(_PKG_ROOT, "lib", "_anyprec_torch.so")
-        if not os.path.exists(path):
-            raise ModuleNotFoundError(f"{path} is missing: build it with `python any-precision-llm_amd/build.py`.")
-        loader = importlib.machinery.ExtensionFileLoader("_anyprec_torch", path)
+
+def _load_torch_module(path):
+    import importlib.machinery
+    import importlib.util
+
+    import torch        # whose libraries the module finds by name
+
+    build = "build it with `python any-precision-llm_amd/build.py`"
+    if not os.path.exists(path):
+        raise ModuleNotFoundError(f"{path} is missing: {build}.")
+    loader = importlib.machinery.ExtensionFileLoader("_anyprec_torch", path)
+    try:
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_anyprec_torch", loader))
         loader.exec_module(module)
-        _torch_module = module
-    return _torch_module
+    except ImportError as e:
+        raise ImportError(f"{path} does not load beside torch {torch.__version__}: {build} here ({e})") from e
+    # it is C++ over torch's own classes, and passes arguments by the header it was built with
+    if module.torch_version != torch.__version__:
+        raise ImportError(f"{path} was built for torch {module.torch_version}, this is {torch.__version__}: {build} here")
+    if module.abi_version != AP_ABI_VERSION:
+        raise ImportError(f"{path} has ABI version {module.abi_version}, this binding needs {AP_ABI_VERSION}: {build} again")
+    return module
 
 
 _vp, _ci = ctypes.c_void_p, ctypes.c_int

@@ -81,7 +81,7 @@ def build_torch(verbose: bool = False) -> str:
     torch_dir = os.path.dirname(torch.__file__)
     include = os.path.join(torch_dir, "include")
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE, "-isystem", include,
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DAP_TORCH_VERSION="{torch.__version__}"', "-I", INCLUDE, "-isystem", include,
            "-isystem", os.path.join(include, "torch", "csrc", "api", "include"), "-isystem", "/opt/rocm/include",
            "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, "ap_torch.cpp"), "-o", TORCH_MODULE,
            "-L", LIBDIR, "-lanyprec_hip", "-L", os.path.join(torch_dir, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu",

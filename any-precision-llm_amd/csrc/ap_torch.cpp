@@ -442,5 +442,11 @@ PyMODINIT_FUNC PyInit__anyprec_torch(void) {
     key_qweight = PyUnicode_InternFromString("qweight");
     key_bias = PyUnicode_InternFromString("bias");
     for (int b = 3; b <= 8; b++) key_lut[b] = PyUnicode_InternFromString(("lut" + std::to_string(b)).c_str());
-    return PyModule_Create(&module);
+    PyObject *m = PyModule_Create(&module);
+    if (m != nullptr && (PyModule_AddIntConstant(m, "abi_version", AP_ABI_VERSION) != 0 ||
+                         PyModule_AddStringConstant(m, "torch_version", AP_TORCH_VERSION) != 0)) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
 }

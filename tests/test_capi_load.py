@@ -219,3 +219,24 @@ def test_what_pays_names_a_wrong_argument():
         _capi.gemm_group_pays(16, [4096, 4096], 4096, 9)
     with pytest.raises(ValueError, match="w_bits"):
         _capi.gemm_pays(16, 4096, 4096, 2)
+
+
+def test_a_native_module_that_does_not_fit_is_named(tmp_path, monkeypatch):
+    """Built for another torch or another header, or no module at all: the import says so and what to do."""
+    import torch
+    from any_precision_amd import _capi
+    path = os.path.join(os.path.dirname(_capi.LIB_PATH), "_anyprec_torch.so")
+    assert _capi._load_torch_module(path).abi_version == _capi.AP_ABI_VERSION
+    broken = tmp_path / "_anyprec_torch.so"
+    with pytest.raises(ModuleNotFoundError, match="missing: build it"):
+        _capi._load_torch_module(str(broken))
+    broken.write_bytes(b"not a library")
+    with pytest.raises(ImportError, match="does not load beside torch .*: build it"):
+        _capi._load_torch_module(str(broken))
+    with monkeypatch.context() as m:
+        m.setattr(_capi, "AP_ABI_VERSION", _capi.AP_ABI_VERSION + 1)
+        with pytest.raises(ImportError, match="ABI version"):
+            _capi._load_torch_module(path)
+    monkeypatch.setattr(torch, "__version__", "0.0.1")
+    with pytest.raises(ImportError, match="built for torch"):
+        _capi._load_torch_module(path)
