@@ -17,14 +17,14 @@ import torch
 import torch.nn as nn
 from torch.nn.modules.module import _has_any_global_hook
 
-from . import _capi
+from .linear import _capi       # None where the library is not built
 
 # keyword arguments of an attention call that do not change what it computes without a cache and a mask
 _IDLE = {"position_ids", "cache_position", "use_cache", "output_attentions", "output_hidden_states", "return_dict"}
 
 
 def _native():
-    return None if torch.compiler.is_compiling() else _capi.torch_module()
+    return None if _capi is None or torch.compiler.is_compiling() else _capi.torch_module()
 
 
 def _norm_forward(module, original, hidden_states):

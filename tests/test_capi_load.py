@@ -4,6 +4,8 @@ import ctypes
 import glob
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -240,3 +242,16 @@ def test_a_native_module_that_does_not_fit_is_named(tmp_path, monkeypatch):
     monkeypatch.setattr(torch, "__version__", "0.0.1")
     with pytest.raises(ImportError, match="built for torch"):
         _capi._load_torch_module(path)
+
+
+def test_what_needs_no_library_imports_without_it():
+    """The module classes import where the library is not built, and say so when one is made."""
+    code = ("import sys\n"
+            "sys.modules['any_precision_ext'] = sys.modules['any_precision_amd._capi'] = None\n"
+            "from any_precision_amd import causal_lm, linear\n"
+            "assert linear._native_linear is None and linear._native_linear_group is None\n"
+            "try:\n    linear.AnyPrecisionLinear(32, 4, [3])\n"
+            "except ModuleNotFoundError as e:\n    print('named:', e)\n")
+    env = dict(os.environ, PYTHONPATH=os.path.join(ROOT, "any-precision-llm_amd"))
+    out = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0 and "named: libanyprec_hip.so is not built" in out.stdout, out.stderr
