@@ -171,14 +171,16 @@ __global__ __launch_bounds__(kPromptAttnThreads) void prompt_attention_kernel(co
             }
             top = fmaxf(top, __shfl_xor(top, 16, kWave));
             top = fmaxf(top, __shfl_xor(top, 32, kWave));
-            const float mn = fmaxf(m, top);  // finite: key 0 is in the first tile
-            const float alpha = exp2f(m - mn);
+            // -inf while every score so far is (keys that overflowed): measured against 0 then, so that such keys weigh nothing
+            // and not NaN once a finite score follows
+            const float mn = fmaxf(m, top), ref = mn == -INFINITY ? 0.f : mn;
+            const float alpha = exp2f(m - ref);
             m = mn;
             half8_t pb;
             float sum = 0.f;
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                const float e = exp2f(p[i] - mn);
+                const float e = exp2f(p[i] - ref);
                 sum += e;
                 pb[i] = (half_t)e;
             }

@@ -63,3 +63,28 @@ def test_prompt_argument_errors():
     assert L.ap_prompt_rope(fake, fake, fake, fake, fake, 4, 2, 2, 48, 16, None) == _capi.AP_ESHAPE
     assert L.ap_prompt_attention(fake, fake, fake, fake, 4, 4, 2, 2, 64, 16, 1.0, None) == _capi.AP_ESHAPE
     assert L.ap_prompt_attention(fake, fake, fake, fake + 8, 0, 4, 2, 2, 64, 16, 1.0, None) == _capi.AP_EALIGN
+
+
+@pytest.mark.parametrize("nh,nkv,hd", SHAPES)
+def test_prompt_attention_with_scores_of_minus_infinity(nh, nkv, hd):
+    """A key whose score is -inf weighs nothing, also where a query meets only such keys in its first tile of 32; a query that
+    sees nothing else has no result (NaN, as softmax has it)."""
+    from any_precision_amd import _capi
+    T, hidden, scale = 100, 40, 0.5
+    gen = torch.Generator().manual_seed(hd)
+    qkv = torch.randn((T, nh + 2 * nkv, hd), generator=gen).half()
+    qkv[:, :nh, 0] = qkv[:, :nh, 0].abs() + 1
+    k, v = (torch.randn((nkv, T, hd), generator=gen).half() for _ in range(2))
+    k[:, :hidden, 0] = float("-inf")
+    x, kc, vc = qkv.cuda(), k.cuda(), v.cuda()
+    out = torch.zeros((T, nh * hd)).half().cuda()
+    _capi.check(_capi.lib.ap_prompt_attention(x.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), 0, T, nh, nkv, hd, T, scale,
+                                              torch.cuda.current_stream().cuda_stream), "ap_prompt_attention")
+    k, v = (t.double().repeat_interleave(nh // nkv, 0) for t in (k, v))
+    scores = torch.einsum("thd,hjd->htj", qkv[:, :nh].double(), k) * scale
+    scores.masked_fill_(torch.arange(T)[None, :] > torch.arange(T)[:, None], float("-inf"))
+    want = torch.einsum("htj,hjd->thd", scores[:, hidden:].softmax(-1), v)
+    got = out.cpu().double().view(T, nh, hd)
+    assert torch.isnan(got[:hidden]).all()
+    # as above: fp16 weights and results over values below about 5
+    assert (got[hidden:] - want).abs().max().item() <= 5 * (2 * 2.0 ** -11) + 1e-3
