@@ -47,6 +47,7 @@ PyObject *library_error(int rc, const char *op) {
 }
 
 bool is_tensor(PyObject *o) { return o != nullptr && THPVariable_Check(o); }
+bool exact_tensor(PyObject *o) { return THPVariable_CheckTypeExact(Py_TYPE(o)); }  // or a parameter, but no other subclass
 
 // A bit-width given as an int in 3..8, else 0.
 int bits_of(PyObject *o) {
@@ -208,13 +209,18 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (!weight_of(q, t, bits, &w)) return none();
         const int64_t rows = rows_of(x, w);
         if (rows < 1) return none();
+        const bool pays = rows <= 8 || ap_gemm_kbit_pays((int)rows, w.N, w.K, bits) == 1;
+        // torch's product and sum as Python calls them, where a subclass or a mode wants to see them
+        const bool torch_op = !pays || bias.defined();
+        if (torch_op && (at::impl::torch_function_mode_enabled() || !exact_tensor(args[1]) || (m.bias != nullptr && !exact_tensor(m.bias))))
+            return none();
         const char *op = rows <= 8 ? "matmul_kbit" : "gemm_kbit";
         Tensor out;
         int rc;
         {
             const WithoutGil free;
             const OnDevice on(w.device);
-            if (rows <= 8 || ap_gemm_kbit_pays((int)rows, w.N, w.K, bits) == 1) {
+            if (pays) {
                 const Tensor dense = x.is_contiguous() ? x : x.contiguous();  // the kernels take dense rows
                 out = result_for(x, w.N);
                 rc = rows <= 8 ? ap_matmul_kbit(half_ptr(dense), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream)
@@ -315,7 +321,7 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
 // does with an op: a call that anything but plain execution follows -- gradients, tangents, subclasses, modes, functorch --
 // gets None and runs as torch ops.
 bool plain_half(PyObject *o, const at::Device *device) {
-    if (!is_tensor(o) || !THPVariable_CheckTypeExact(Py_TYPE(o))) return false;
+    if (!is_tensor(o) || !exact_tensor(o)) return false;
     const Tensor &t = THPVariable_Unpack(o);
     if (!t.is_cuda() || t.scalar_type() != at::kHalf || t.layout() != at::kStrided || !t.is_contiguous() || t.numel() == 0) return false;
     if (device != nullptr && t.device() != *device) return false;

@@ -204,3 +204,32 @@ def test_a_bias_of_any_kind_is_added(kind, M):
     bound = 2.0 ** -9 * (product.float().abs() + value.cuda().float().abs()) + 2.0 ** -20
     for got in (m(x, precision=4), forward_group((m, m), x, 4)[1], forward_group((plain, m), x, 4, concat=True)[:, L.N:]):
         assert bool(((got.float() - want.float()).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M", [4, 600])
+def test_torch_operations_of_a_linear_are_seen_by_subclasses_and_modes(M, bias):
+    """Where the forward takes torch's product (many rows) or adds a bias, a tensor subclass and a torch-function mode see them."""
+    from torch.overrides import TorchFunctionMode
+    L = make(64, 1024, seed=8)
+    m, _ = _module(L, bias=bias)
+    x = torch.from_numpy(synth.make_x(M, L.K, seed=M)).cuda()
+    want = m(x, precision=4)
+
+    class Marked(torch.Tensor):
+        pass
+
+    got = m(x.as_subclass(Marked), precision=4)
+    assert type(got) is (Marked if M == 600 else torch.Tensor) and torch.equal(got.as_subclass(torch.Tensor), want)
+    seen = []
+
+    class Watching(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    with Watching():
+        got = m(x, precision=4)
+    assert torch.equal(got, want) and ("matmul" in seen) == (M == 600) and ("__iadd__" in seen or "add_" in seen) == bias
+    m.bias = m.bias.as_subclass(Marked) if bias else None
+    assert torch.equal(m(x, precision=4).as_subclass(torch.Tensor), want)
