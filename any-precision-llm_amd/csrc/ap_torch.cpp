@@ -328,7 +328,8 @@ bool plain_half(PyObject *o, const at::Device *device) {
     if (c10::GradMode::is_enabled() && t.requires_grad()) return false;
     const auto keys = t.key_set();
     if (keys.has(c10::DispatchKey::FuncTorchBatched) || keys.has(c10::DispatchKey::FuncTorchGradWrapper) ||
-        keys.has(c10::DispatchKey::Functionalize) || t._fw_grad(0).defined())
+        keys.has(c10::DispatchKey::Functionalize) || keys.has(c10::DispatchKey::Negative) || keys.has(c10::DispatchKey::ZeroTensor) ||
+        t._fw_grad(0).defined())
         return false;
     return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
 }

@@ -272,3 +272,17 @@ def test_what_a_program_has_replaced_is_called(serving, monkeypatch, change, whe
     assert len(calls) == {"nothing": 0, "LlamaRMSNorm": 5}.get(change, 2)
     # of two layers: five norms, two MLPs, four rotary embeddings
     assert serving.served == 11 - {"LlamaRMSNorm": 5, "LlamaMLP": 2, "LlamaAttention": 4, "rotary": 4}.get(change, 0)
+
+
+@pytest.mark.gpu
+def test_tensors_whose_memory_is_not_their_value_are_left_to_torch():
+    """A lazily negated view and a zero tensor without memory."""
+    from any_precision_amd import _capi
+    native = _capi.torch_module()
+    x, w = torch.randn((3, 64), device="cuda").half(), torch.ones((64,), device="cuda").half()
+    tables = torch.ones((1, 3, 64), device="cuda").half()
+    zero = torch._efficientzerotensor((3, 64), dtype=torch.float16, device="cuda")
+    for odd in (torch._neg_view(x), zero):
+        assert native.rmsnorm(odd, w, 1e-5) is None and native.silu_mul(odd, x) is None and native.silu_mul(x, odd) is None
+        assert native.rope(odd[None], tables, tables) is None and native.plain(odd) is False
+    assert native.plain(x) is True
