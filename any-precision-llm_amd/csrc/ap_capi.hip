@@ -299,18 +299,24 @@ int ap_add_rmsnorm(const uint16_t *h, const uint16_t *delta, const uint16_t *wei
     half_t *ho = reinterpret_cast<half_t *>(h_out), *xo = reinterpret_cast<half_t *>(x_out);
     const hipStream_t st = static_cast<hipStream_t>(stream);
     const int units = H / 8;  // a thread each, in whole waves
-    const dim3 grid(rows), block(units < kNormMaxThreads ? (units + kWave - 1) / kWave * kWave : kNormMaxThreads);
-    if (units <= kNormMaxThreads) {
-        if (delta)
-            add_rmsnorm_kernel<1, true><<<grid, block, 0, st>>>(hp, dp, wp, ho, xo, H, eps);
+    const int block = units < kNormMaxThreads ? (units + kWave - 1) / kWave * kWave : kNormMaxThreads;
+    const long long most = 0xffffffffLL / block;  // rows of a launch: a grid has fewer than 2^32 threads
+    for (long long row = 0; row < rows; row += most) {
+        const dim3 grid((unsigned)(rows - row < most ? rows - row : most));
+        const long long at = row * H;
+        const half_t *d = dp ? dp + at : nullptr;
+        if (units <= kNormMaxThreads && dp)
+            add_rmsnorm_kernel<1, true><<<grid, dim3(block), 0, st>>>(hp + at, d, wp, ho + at, xo + at, H, eps);
+        else if (units <= kNormMaxThreads)
+            add_rmsnorm_kernel<1, false><<<grid, dim3(block), 0, st>>>(hp + at, d, wp, ho + at, xo + at, H, eps);
+        else if (dp)
+            add_rmsnorm_kernel<2, true><<<grid, dim3(block), 0, st>>>(hp + at, d, wp, ho + at, xo + at, H, eps);
         else
-            add_rmsnorm_kernel<1, false><<<grid, block, 0, st>>>(hp, dp, wp, ho, xo, H, eps);
-    } else if (delta) {
-        add_rmsnorm_kernel<2, true><<<grid, block, 0, st>>>(hp, dp, wp, ho, xo, H, eps);
-    } else {
-        add_rmsnorm_kernel<2, false><<<grid, block, 0, st>>>(hp, dp, wp, ho, xo, H, eps);
+            add_rmsnorm_kernel<2, false><<<grid, dim3(block), 0, st>>>(hp + at, d, wp, ho + at, xo + at, H, eps);
+        const int rc = launch_status();
+        if (rc != AP_OK) return rc;
     }
-    return launch_status();
+    return AP_OK;
 }
 
 int ap_silu_mul(const uint16_t *gate, const uint16_t *up, uint16_t *out, long long n, void *stream) {

@@ -238,3 +238,19 @@ def test_silu_mul_in_place(n, over):
     want = silu_mul(gate, up)
     out = gate if over == "gate" else up
     assert silu_mul(gate, up, out=out) is out and torch.equal(out, want)
+
+
+@pytest.mark.parametrize("with_delta", [False, True])
+def test_add_rmsnorm_of_more_rows_than_a_grid_has_threads_for(with_delta):
+    """2^26 workgroups of 64 threads are 2^32 threads, one more than a grid may have."""
+    from any_precision_amd.decode_ops import add_rmsnorm
+    rows, H = 2 ** 26 + 3, 8
+    h = torch.empty((rows, H), dtype=torch.float16, device="cuda")
+    h.copy_(torch.arange(H, device="cuda") - 2.5)
+    h[-4:] += torch.arange(4, device="cuda")[:, None]        # the last rows differ from the others
+    delta = torch.ones_like(h) if with_delta else None
+    w = torch.linspace(0.5, 1.5, H, device="cuda").half()
+    want = torch.cat([add_rmsnorm(t.clone(), None if delta is None else delta[:4], w, 1e-5)[1] for t in (h[:4], h[-4:])])
+    _, got = add_rmsnorm(h, delta, w, 1e-5, h_out=h)
+    assert torch.equal(torch.cat((got[:4], got[-4:])), want)
+    assert bool((got[4:-4] == want[0]).all()) and bool((h[:-4] == h[0]).all())
