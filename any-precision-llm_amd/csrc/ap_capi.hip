@@ -369,7 +369,8 @@ int check_prompt(int T, int nh, int nkv, int hd, int max_len) {
     if (nh < 1 || nkv < 1 || nh % nkv) return AP_ESHAPE;
     if (hd != 32 && hd != 64 && hd != 128 && hd != 256) return AP_ESHAPE;
     if (T < 1 || T > max_len) return AP_ESHAPE;
-    return nh > 65535 || (long long)T * (nh + 2LL * nkv) * (hd / 16) > 0x7fffffffLL * kPromptRopeThreads ? AP_ELIMIT : AP_OK;
+    // the rotary kernel has a thread per 16 elements; a grid of 2^32 threads would wrap around
+    return nh > 65535 || (long long)T * (nh + 2LL * nkv) * (hd / 16) > 0xffffffffLL - kPromptRopeThreads ? AP_ELIMIT : AP_OK;
 }
 
 }  // namespace

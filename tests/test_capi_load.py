@@ -255,3 +255,13 @@ def test_what_needs_no_library_imports_without_it():
     env = dict(os.environ, PYTHONPATH=os.path.join(ROOT, "any-precision-llm_amd"))
     out = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=120)
     assert out.returncode == 0 and "named: libanyprec_hip.so is not built" in out.stdout, out.stderr
+
+
+def test_a_prompt_of_more_threads_than_a_grid_may_have_is_refused():
+    """2^20 tokens of 258 heads of 256 are 2^32 threads of 16 elements and some; one head less of each kind fits."""
+    from any_precision_amd import _capi
+    call = lambda heads: _capi.lib.ap_prompt_rope(4096, 4096, 4096, 4096, 4096, 2 ** 20, heads, heads, 256, 2 ** 20, None)
+    assert call(86) == _capi.AP_ELIMIT
+    import torch
+    if not (torch.cuda.is_available() or os.path.exists("/dev/kfd")):      # the addresses are not real: nothing may be launched
+        assert call(85) > 0                             # past the checks, and there is no device
