@@ -17,6 +17,7 @@
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "anyprec_hip.h"
@@ -27,17 +28,13 @@ using at::Tensor;
 
 PyObject *none() { Py_RETURN_NONE; }
 
-// Set when a C++ exception has been turned into a Python error.
+// A C++ exception becomes the Python exception that torch's own bindings make of it: a Python exception raised below (a hook's, a
+// mode's) comes out as itself, exhausted memory as torch.OutOfMemoryError.  Warnings become Python warnings.
 template <typename F>
 PyObject *guarded(F &&f) {
-    try {
-        return f();
-    } catch (const c10::Error &e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
-    } catch (const std::exception &e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-    }
-    return nullptr;
+    HANDLE_TH_ERRORS
+    return f();
+    END_HANDLE_TH_ERRORS
 }
 
 PyObject *library_error(int rc, const char *op) {

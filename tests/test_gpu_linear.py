@@ -233,3 +233,49 @@ def test_torch_operations_of_a_linear_are_seen_by_subclasses_and_modes(M, bias):
     assert torch.equal(got, want) and ("matmul" in seen) == (M == 600) and ("__iadd__" in seen or "add_" in seen) == bias
     m.bias = m.bias.as_subclass(Marked) if bias else None
     assert torch.equal(m(x, precision=4).as_subclass(torch.Tensor), want)
+
+
+class _Raised(Exception):
+    pass
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_exceptions_below_a_linear_come_out_as_themselves(bias):
+    """A saved-tensor hook's and a dispatch mode's exception, and exhausted memory, keep their types; a non-reentrant checkpoint
+    (which ends its second forward by raising in a hook) gives the gradient."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from torch.utils.checkpoint import checkpoint
+    from any_precision_amd.linear import AnyPrecisionLinear, forward_group
+    L = make(64, 1024, seed=6)
+    m, _ = _module(L, bias=bias)
+    x = torch.from_numpy(synth.make_x(600, L.K, seed=1)).cuda()          # enough rows for torch's product
+
+    def raising(*_):
+        raise _Raised
+
+    with pytest.raises(_Raised), torch.autograd.graph.saved_tensors_hooks(raising, lambda t: t):
+        m(x.clone().requires_grad_(), precision=4)
+
+    class Raising(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            raise _Raised
+
+    with pytest.raises(_Raised), Raising():
+        m(x, precision=4)
+    grads = []
+    for kept in (True, False):
+        leaf = x.clone().requires_grad_()
+        step = lambda t: m(torch.sin(t), precision=4)
+        (step(leaf) if kept else checkpoint(step, leaf, use_reentrant=False)).float().square().sum().backward()
+        grads.append(leaf.grad)
+    assert torch.equal(*grads)
+    wide = [AnyPrecisionLinear(1024, 65536, [3], bias=bias, device="cuda", dtype=torch.float16) for _ in range(2)]
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 2 ** 23) / torch.cuda.mem_get_info()[1])
+    try:
+        for call in (lambda: wide[0](x), lambda: forward_group(wide, x), lambda: wide[0](x[:200])):
+            with pytest.raises(torch.OutOfMemoryError):
+                call()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
