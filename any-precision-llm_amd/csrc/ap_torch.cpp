@@ -235,7 +235,7 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
 }
 
-// linear_group(__dict__ of 2..4 modules, x, w_bits, concat): forward_group for bias-free linears of one input length.  A list of
+// linear_group(__dict__ of 2..4 modules, x, w_bits, concat as a bool): forward_group for bias-free linears of one input length.  A list of
 // results, or with concat one tensor of them side by side.  Up to 8 rows ap_matmul_kbit_group, beyond one launch of the tiled
 // GEMM where ap_gemm_kbit_group_pays; None where the modules are better called one by one.
 PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {

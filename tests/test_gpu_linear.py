@@ -279,3 +279,15 @@ def test_exceptions_below_a_linear_come_out_as_themselves(bias):
                 call()
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+@pytest.mark.parametrize("rows", [1, 4, 40])
+@pytest.mark.parametrize("concat", [1, "yes", np.True_, 0, None, np.False_])
+def test_concat_is_taken_for_what_it_is_as_a_truth_value(rows, concat):
+    from any_precision_amd.linear import forward_group
+    L = make(64, 1024, seed=6)
+    m, _ = _module(L, bias=False)
+    x = torch.from_numpy(synth.make_x(rows, L.K, seed=rows)).cuda()
+    want = forward_group((m, m), x, 4, concat=bool(concat))
+    got = forward_group((m, m), x, 4, concat=concat)
+    assert type(got) is type(want) and torch.equal(torch.cat(tuple(got)), torch.cat(tuple(want)))
