@@ -207,6 +207,30 @@ int launch_status() {
 
 }  // namespace
 
+namespace {
+
+// Units of 8 elements that a thread of the norm kernel holds.  Few rows: one (a row is a chain of latencies, more threads do
+// not lengthen it).  From 1024 rows on the chip is full of rows, and large workgroups leave wave slots empty while one of
+// them waits at its barrier: four, for rows beyond 3072 elements (shorter ones are as fast either way).  us without a delta,
+// one unit against four: 2048 rows of 5120 8.2 / 7.2, 16384 rows 67.5 / 57.6; 1024 rows of 8192 with a delta 11.2 / 9.9;
+// 512 rows of 5120 3.3 / 3.5.  Longer than 8192, two against four: 16384 rows of 11008 145 / 126; few rows are as fast
+// with two.
+int norm_units_per_thread(int rows, int units) {
+    if (rows >= 1024 && units > 384) return 4;
+    return units <= kNormMaxThreads ? 1 : 2;
+}
+
+template <int HELD>
+void launch_norm(dim3 grid, int block, hipStream_t st, const half_t *h, const half_t *delta, const half_t *weight, half_t *h_out,
+                 half_t *x_out, int H, float eps) {
+    if (delta)
+        add_rmsnorm_kernel<HELD, true><<<grid, dim3(block), 0, st>>>(h, delta, weight, h_out, x_out, H, eps);
+    else
+        add_rmsnorm_kernel<HELD, false><<<grid, dim3(block), 0, st>>>(h, delta, weight, h_out, x_out, H, eps);
+}
+
+}  // namespace
+
 extern "C" {
 
 int ap_abi_version(void) { return AP_ABI_VERSION; }
@@ -298,21 +322,21 @@ int ap_add_rmsnorm(const uint16_t *h, const uint16_t *delta, const uint16_t *wei
     const half_t *wp = reinterpret_cast<const half_t *>(weight);
     half_t *ho = reinterpret_cast<half_t *>(h_out), *xo = reinterpret_cast<half_t *>(x_out);
     const hipStream_t st = static_cast<hipStream_t>(stream);
-    const int units = H / 8;  // a thread each, in whole waves
-    const int block = units < kNormMaxThreads ? (units + kWave - 1) / kWave * kWave : kNormMaxThreads;
+    const int units = H / 8;
+    const int held = norm_units_per_thread(rows, units);
+    const int waves = (units + held * kWave - 1) / (held * kWave);
+    const int block = waves * kWave < kNormMaxThreads ? waves * kWave : kNormMaxThreads;
     const long long most = 0xffffffffLL / block;  // rows of a launch: a grid has fewer than 2^32 threads
     for (long long row = 0; row < rows; row += most) {
         const dim3 grid((unsigned)(rows - row < most ? rows - row : most));
         const long long at = row * H;
         const half_t *d = dp ? dp + at : nullptr;
-        if (units <= kNormMaxThreads && dp)
-            add_rmsnorm_kernel<1, true><<<grid, dim3(block), 0, st>>>(hp + at, d, wp, ho + at, xo + at, H, eps);
-        else if (units <= kNormMaxThreads)
-            add_rmsnorm_kernel<1, false><<<grid, dim3(block), 0, st>>>(hp + at, d, wp, ho + at, xo + at, H, eps);
-        else if (dp)
-            add_rmsnorm_kernel<2, true><<<grid, dim3(block), 0, st>>>(hp + at, d, wp, ho + at, xo + at, H, eps);
+        if (held == 1)
+            launch_norm<1>(grid, block, st, hp + at, d, wp, ho + at, xo + at, H, eps);
+        else if (held == 2)
+            launch_norm<2>(grid, block, st, hp + at, d, wp, ho + at, xo + at, H, eps);
         else
-            add_rmsnorm_kernel<2, false><<<grid, dim3(block), 0, st>>>(hp + at, d, wp, ho + at, xo + at, H, eps);
+            launch_norm<4>(grid, block, st, hp + at, d, wp, ho + at, xo + at, H, eps);
         const int rc = launch_status();
         if (rc != AP_OK) return rc;
     }

@@ -27,8 +27,7 @@ __device__ __forceinline__ float wave_max(float v) {
 //     x_out = s * rsqrt(mean(s^2) + eps) * weight.
 // h_out may alias h.  A thread has HELD units of 8 elements in registers between the two passes, all of them (and their
 // deltas and weights) requested before the first is used, without a branch on the way: a unit past the row's end loads the
-// row's last one and counts for nothing.  HELD = 1 takes rows of up to 8192 elements with a thread per unit; what is past
-// HELD units of longer rows is re-read.
+// row's last one and counts for nothing.  What is past HELD units of longer rows is re-read.
 // Bound by its chain at a decoder's one row (scalar arguments, one trip to memory for what the linear before has written from
 // every XCD, the reduction, the store); with 256 threads and the units one after the other that were two to four trips.
 // 48 tokens with 32 layers of 4096 (65 launches a token): 68.8 -> 66.2 ms, 0.85 us a launch.

@@ -214,6 +214,18 @@ def test_advance_is_argmax_and_bookkeeping(n):
 @pytest.mark.parametrize("with_delta", [False, True])
 def test_add_rmsnorm_row_lengths(H, rows, with_delta):
     """Rows around a wave, a workgroup and what a thread holds; sums written elsewhere and over h."""
+    _check_add_rmsnorm(H, rows, with_delta)
+
+
+@pytest.mark.parametrize("H", [3072, 3080, 4096, 4104, 6136, 8192, 32768, 32776])
+@pytest.mark.parametrize("with_delta", [False, True])
+def test_add_rmsnorm_of_many_rows(H, with_delta):
+    """From 1024 rows on a thread holds four units of rows beyond 3072 elements: whole and ragged waves, and what is re-read."""
+    for rows in (1023, 1024):
+        _check_add_rmsnorm(H, rows, with_delta)
+
+
+def _check_add_rmsnorm(H, rows, with_delta):
     from any_precision_amd.decode_ops import add_rmsnorm
     gen = torch.Generator().manual_seed(H + rows)
     h, d, w = (torch.randn(shape, generator=gen).half() for shape in ((rows, H), (rows, H), (H,)))
