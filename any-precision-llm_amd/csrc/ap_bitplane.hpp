@@ -136,13 +136,28 @@ AP_HD void planes_to_adjacent_pairs(const uint32_t (&q)[BITS], uint32_t (&apair)
     for (int i = 0; i < 4; i++) apair[i] = r[3 - i];
 }
 
-// The two table indices a byte of planes_to_adjacent_pairs stands for (host and device; the kernels use
-// it to build their pair tables): first = index of element 2i, second = index of element 2i+1.
+// The two table indices a byte of planes_to_adjacent_pairs stands for: first = index of element 2i, second = index of
+// element 2i+1.  What pair_lane_offsets() is checked against on the host.
 template <int BITS>
 AP_HD void adjacent_pair_split(uint32_t byte, uint32_t &first, uint32_t &second) {
     const uint32_t v = BITS == 3 ? byte >> 2 : byte;
     first = ((v >> 1) & 1u) | ((v >> 2) & 2u) | ((v >> 3) & 4u) | ((v >> 4) & 8u);
     second = (v & 1u) | ((v >> 1) & 2u) | ((v >> 2) & 4u) | ((v >> 3) & 8u);
+}
+
+// What lane `lane` of a wave reads of a row's table to build its share of the pair table, as byte offsets.  With the lane
+// number's bits read as l5 l4 .. l0, f = l5 l3 l1 and s = l4 l2 l0:
+//   3 bits: entry `lane` = (lut[f], lut[s])  (adjacent_pair_split of 4 lane);
+//   4 bits: entries 4 lane .. 4 lane + 3 differ in the lowest bit of either index: they combine the halves of dword
+//           f = (lut[2f], lut[2f+1]) and of dword s.
+// Three masked shifts each, two of them shared: every wave of the GEMV kernels runs this once for two to four rows.
+template <int BITS>
+AP_HD void pair_lane_offsets(uint32_t lane, uint32_t &first, uint32_t &second) {
+    static_assert(BITS == 3 || BITS == 4, "");
+    constexpr int SH = BITS == 3 ? 1 : 2;  // log2 of the bytes that f and s count
+    const uint32_t l = lane << 1, a = l << SH >> 2, b = l << SH >> 3, c = l << SH >> 4;  // lane << SH >> 1, 2, 3
+    first = (a & (1u << SH)) | (b & (2u << SH)) | (c & (4u << SH));
+    second = (l << SH >> 1 & (1u << SH)) | (a & (2u << SH)) | (b & (4u << SH));
 }
 
 }  // namespace ap

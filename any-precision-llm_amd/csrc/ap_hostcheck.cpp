@@ -44,6 +44,13 @@ int aph_adjacent_pair_split(int bits, uint32_t byte, uint32_t *first, uint32_t *
     return 0;
 }
 
+int aph_pair_lane_offsets(int bits, uint32_t lane, uint32_t *first, uint32_t *second) {
+    if (bits == 3) ap::pair_lane_offsets<3>(lane, *first, *second);
+    else if (bits == 4) ap::pair_lane_offsets<4>(lane, *first, *second);
+    else return -1;
+    return 0;
+}
+
 int aph_chunk_words(int w, int K) { return ap::chunk_words(w, K); }
 int aph_group_base(int w, int j, int K) { return ap::group_base(w, j, K); }
 

@@ -20,12 +20,7 @@ struct LookupTable {
     static constexpr int kBytes = kPair ? (4 << (2 * BITS)) : (2 << BITS);
 };
 
-// What a lane needs to know to build its share of a pair table (byte offsets into the row's entries); depends on the lane only.
-// With the lane number's bits read as l5 l4 .. l0, f = l5 l3 l1 and s = l4 l2 l0:
-//   3 bits: entry `lane` = (lut[f], lut[s])  (adjacent_pair_split of 4 lane);
-//   4 bits: entries 4 lane .. 4 lane + 3 differ in the lowest bit of either index: they combine the halves of dword
-//           f = (lut[2f], lut[2f+1]) and of dword s.
-// Three masked shifts each, two of them shared: every wave of the GEMV kernels runs this once for two to four rows.
+// What a lane needs to know to build its share of a pair table (pair_lane_offsets); depends on the lane only.
 template <int BITS>
 struct PairLane {
     uint32_t first, second;
@@ -34,12 +29,7 @@ struct PairLane {
 template <int BITS>
 __device__ __forceinline__ PairLane<BITS> pair_lane(int lane) {
     PairLane<BITS> r = {0u, 0u};
-    if constexpr (BITS <= 4) {
-        constexpr int SH = BITS == 3 ? 1 : 2;  // log2 of the bytes that f and s count
-        const uint32_t l = (uint32_t)lane << 1, a = l << SH >> 2, b = l << SH >> 3, c = l << SH >> 4;  // lane << SH >> 1, 2, 3
-        r.first = (a & (1u << SH)) | (b & (2u << SH)) | (c & (4u << SH));
-        r.second = (l << SH >> 1 & (1u << SH)) | (a & (2u << SH)) | (b & (4u << SH));
-    }
+    if constexpr (BITS <= 4) pair_lane_offsets<BITS>((uint32_t)lane, r.first, r.second);
     return r;
 }
 

@@ -62,6 +62,22 @@ def test_adjacent_pair_indices(hostcheck, oracle, bits):
                 assert second.value == (int(want[2 * i + 1]) >> (8 * b)) & 0xFF, (i, b)
 
 
+@pytest.mark.parametrize("bits", [3, 4])
+def test_pair_table_lane_offsets(hostcheck, bits):
+    """Lane by lane: the entries that the kernels build from what they read are those that the pair bytes name."""
+    a, b, first, second = (ctypes.c_uint32() for _ in range(4))
+    for lane in range(64):
+        assert hostcheck.aph_pair_lane_offsets(bits, lane, ctypes.byref(a), ctypes.byref(b)) == 0
+        for half in range(1 if bits == 3 else 4):       # 4 bits: the halves of two dwords combine to four entries
+            byte = 4 * lane + half
+            assert hostcheck.aph_adjacent_pair_split(bits, byte, ctypes.byref(first), ctypes.byref(second)) == 0
+            if bits == 3:
+                assert (a.value, b.value) == (2 * first.value, 2 * second.value)
+            else:
+                assert a.value % 4 == 0 and b.value % 4 == 0
+                assert (a.value + 2 * (half >> 1), b.value + 2 * (half & 1)) == (2 * first.value, 2 * second.value)
+
+
 @pytest.mark.parametrize("K", [32, 64, 992, 1024, 1056, 4096, 11008, 14336])
 def test_group_base_enumerates_every_element_once(hostcheck, K):
     W = K // 32
