@@ -60,26 +60,50 @@ def test_what_is_not_plain_execution_is_left_to_torch():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kv_heads", [4, 2])
-def test_model_forward_with_and_without(kv_heads):
-    """The logits of a model with the kernels and with the original forwards, both against float64 activations."""
-    from any_precision_amd import AnyPrecisionForCausalLM, between
-    ap = AnyPrecisionForCausalLM.from_config(_config(num_key_value_heads=kv_heads), seed=3)
+def test_model_forward_with_and_without(kv_heads, monkeypatch):
+    """The logits of a model with the kernels and with the original forwards, both against the dense weights in float64; and
+    that the kernels served the calls."""
+    from transformers.models.llama import modeling_llama
+    from any_precision_amd import AnyPrecisionForCausalLM, _capi, between
+    config = _config(num_key_value_heads=kv_heads)
+    ap = AnyPrecisionForCausalLM.from_config(config, seed=3)
+    exact = modeling_llama.LlamaForCausalLM(config).double().eval()
+    exact.load_state_dict({k: v.double() for k, v in ap.dense_state_dict(5).items()})
     ids = torch.randint(0, 128, (3, 17), device="cuda")
     mask = torch.ones_like(ids)
     mask[0, :4] = 0
+    native, served = _capi.torch_module(), []
+
+    class Counting:
+        def __getattr__(self, name):
+            def call(*args):
+                out = getattr(native, name)(*args)
+                if name != "plain" and out is not None:
+                    served.append(name)
+                return out
+            return call
+
+    monkeypatch.setattr(between, "_native", Counting)
     with torch.inference_mode():
-        got = ap(ids, precision=5, use_cache=False).logits.float()
+        want = exact(ids.cpu(), use_cache=False).logits
+        outs = [ap(ids, precision=5, use_cache=False).logits]
+        assert sorted(served) == ["rmsnorm"] * 5 + ["rope"] * 4 + ["silu_mul"] * 2          # two layers
         padded = ap(ids, attention_mask=mask, precision=5, use_cache=False).logits
-        cached = ap(ids, precision=5, use_cache=True).logits.float()
-        for m in ap.model.modules():
-            if type(m).__module__ == between.__name__:
-                m.__class__ = type(m).__base__
-        want = ap(ids, precision=5, use_cache=False).logits.float()
+        served.clear()
+        outs.append(ap(ids, precision=5, use_cache=True).logits)
+        assert sorted(served) == ["rmsnorm"] * 5 + ["silu_mul"] * 2                         # a cache: the module's own attention
+        replaced = [m for m in ap.model.modules() if type(m).__module__ == between.__name__]
+        assert len(replaced) == 9                                                           # five norms, two MLPs, two attentions
+        for m in replaced:
+            m.__class__ = type(m).__base__
+        served.clear()
+        outs.append(ap(ids, precision=5, use_cache=False).logits)
+        assert not served
         assert torch.allclose(padded[:, 4:].float(), ap(ids, attention_mask=mask, precision=5, use_cache=False).logits[:, 4:].float(),
                               atol=2e-2, rtol=2e-2)
     # two layers of fp16 activations: a few roundings of 2^-11 each
-    for out in (got, cached):
-        assert float((out - want).norm() / want.norm()) < 2.8e-3 * 2 ** 0.5
+    for out in outs:
+        assert float((out.cpu().double() - want).norm() / want.norm()) < 2.8e-3 * 2 ** 0.5
 
 
 def test_modules_stay_what_they_are():
