@@ -273,7 +273,11 @@ def test_exceptions_below_a_linear_come_out_as_themselves(bias):
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 2 ** 23) / torch.cuda.mem_get_info()[1])
+    held = []
     try:
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:                 # what is free inside the allocator's segments, in blocks of the smallest result
+                held.append(torch.empty((200, 65536), dtype=torch.float16, device="cuda"))
         for call in (lambda: wide[0](x), lambda: forward_group(wide, x), lambda: wide[0](x[:200])):
             with pytest.raises(torch.OutOfMemoryError):
                 call()
