@@ -3,7 +3,7 @@
 //
 // A linear's kernel takes 4 to 15 us at the batch sizes of decoding; the same steps written in Python over ctypes take
 // 11 to 15 us of host time per call, and a stream of such calls runs at the host's pace (28 linears of four decoder layers
-// at one row and 3 bits: 400 us of which the GPU works 167).  Here a call takes about 4 us, most of it HIP's launch.
+// at one row and 3 bits: 400 us of which the GPU works 167).  Here a call takes about 5 us, most of it HIP's launch.
 //
 // A function returns None for anything it does not serve -- wrong types, shapes, devices, layouts -- and the Python side
 // then takes the way that says what is wrong (or serves the case, where it can).  Errors of the library raise here.
@@ -272,6 +272,7 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (gemm && ap_gemm_kbit_group_pays(count, N, (int)rows, K, bits) != 1) return none();
         // side by side in one allocation: one row's results always are dense, and the tiled kernel writes rows that are not
         const bool joint = concat && (gemm ? K % 128 == 0 : rows == 1);
+        if (concat && !joint && at::impl::torch_function_mode_enabled()) return none();  // the mode sees torch.cat
         Tensor all, outs[MOST];
         int rc;
         {

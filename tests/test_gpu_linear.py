@@ -295,3 +295,24 @@ def test_concat_is_taken_for_what_it_is_as_a_truth_value(rows, concat):
     want = forward_group((m, m), x, 4, concat=bool(concat))
     got = forward_group((m, m), x, 4, concat=concat)
     assert type(got) is type(want) and torch.equal(torch.cat(tuple(got)), torch.cat(tuple(want)))
+
+
+@pytest.mark.parametrize("rows,K", [(1, 1024), (4, 1024), (40, 1056), (600, 1024)])
+def test_a_mode_sees_the_results_of_a_set_joined(rows, K):
+    """Where the results of forward_group are joined by torch, a torch-function mode sees it."""
+    from torch.overrides import TorchFunctionMode
+    from any_precision_amd.linear import forward_group
+    L = make(64, K, seed=6)
+    m, _ = _module(L, bias=False)
+    x = torch.from_numpy(synth.make_x(rows, K, seed=rows)).cuda()
+    want = forward_group((m, m), x, 4, concat=True)
+    seen = []
+
+    class Watching(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    with Watching():
+        got = forward_group((m, m), x, 4, concat=True)
+    assert torch.equal(got, want) and ("cat" in seen) == (rows > 1)
