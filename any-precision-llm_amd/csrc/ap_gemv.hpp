@@ -22,12 +22,12 @@
 //   * Lane partials of all R x M sums are folded together (wave_sums, ap_device.hpp); when S > 1 the segment partials
 //     of a row meet in LDS and are added in a fixed order: results are deterministic.
 // The kernel is bound by instructions and by the launch, not by HBM: with every plane in L2 a gate/up launch of 2 x 11008
-// x 4096 at 3 bits takes 9.6 us against 10.3 from HBM.  Of about 165 vector instructions a wave of that launch issues, 92
-// are transposes, lookups and products.  One sum after the other cost 24 of them and their waits, folded together 13, and
-// the table lane arithmetic 9 instead of 16; from two activation rows on the registers also fall by up to a fifth, which
-// is one more wave per SIMD (us, before -> after: 4096 x 14336 at 3 rows, 4 bits 14.2 -> 12.3; 5120 x 5120 at 4 rows, 8
-// bits 12.9 -> 12.0; 4096 x 11008 at 2 rows, 6 bits 14.7 -> 13.5; 1024 x 4096 at 8 rows, 8 bits 6.3 -> 5.6; one row
-// 0-2 %).
+// x 4096 at 3 bits takes 9.6 us against 10.3 from HBM.  A wave of that launch issues 168 vector instructions, 92 of them
+// transposes, lookups and products; with one sum after the other and longer table lane arithmetic they were 181.5.  The more
+// sums a wave has, the more the folding saves (vector instructions a wave, registers and us in the kernel trace, before ->
+// after: 4096 x 14336 at 3 rows, 4 bits 552 -> 462, 44 -> 40, 15.1 -> 13.3; 5120 x 5120 at 4 rows, 8 bits 921 -> 803,
+// 60 -> 56, 14.8 -> 14.1; 4096 x 11008 at 2 rows, 6 bits 665 -> 606, 40 -> 36, 16.8 -> 16.1; 1024 x 4096 at 8 rows, 8 bits
+// 752 -> 635, 84 both, 6.7 -> 6.1; 4096 x 4096 at one row, 3 bits the same).
 #pragma once
 #include <type_traits>
 
