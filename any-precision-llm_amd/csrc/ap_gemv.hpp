@@ -25,9 +25,9 @@
 // x 4096 at 3 bits takes 9.6 us against 10.3 from HBM.  A wave of that launch issues 168 vector instructions, 92 of them
 // transposes, lookups and products; with one sum after the other and longer table lane arithmetic they were 181.5.  The more
 // sums a wave has, the more the folding saves (vector instructions a wave, registers and us in the kernel trace, before ->
-// after: 4096 x 14336 at 3 rows, 4 bits 552 -> 462, 44 -> 40, 15.1 -> 13.3; 5120 x 5120 at 4 rows, 8 bits 921 -> 803,
-// 60 -> 56, 14.8 -> 14.1; 4096 x 11008 at 2 rows, 6 bits 665 -> 606, 40 -> 36, 16.8 -> 16.1; 1024 x 4096 at 8 rows, 8 bits
-// 752 -> 635, 84 both, 6.7 -> 6.1; 4096 x 4096 at one row, 3 bits the same).
+// after: 4096 x 14336 at 3 rows, 4 bits 552 -> 462, 88 -> 80, 15.1 -> 13.3; 5120 x 5120 at 4 rows, 8 bits 921 -> 803,
+// 116 -> 112, 14.8 -> 14.1; 4096 x 11008 at 2 rows, 6 bits 665 -> 606, 74 -> 69, 16.8 -> 16.1; 1024 x 4096 at 8 rows, 8 bits
+// 752 -> 635, 166 -> 167, 6.7 -> 6.1; 4096 x 4096 at one row, 3 bits the same).
 #pragma once
 #include <type_traits>
 
@@ -51,9 +51,20 @@ __device__ __forceinline__ uint32_t word_of(const typename WordVec<WPL>::type &v
     if constexpr (WPL == 1) return v; else return v[i];
 }
 
+// Whether all lookups of a word are asked to come before its first product.  Left to the scheduler they are issued a pair at
+// a time from three activation rows on, each pair's products waiting for it, and the first of them for all activations: one
+// LDS round trip after the other.  Together they also pass the time until the activations are there.  us without -> with:
+// 1024 x 4096 at 3 rows, 5 bits 4.66 -> 4.28; 2048 x 2048 at 6 rows, 6 bits 4.95 -> 4.42; over thirteen shapes of 64 to
+// 14336 rows 2-13 % at 3 to 8 rows.  One or two rows are scheduled well as they are; the sixteen registers that the lookups
+// take spill at three and four rows of 8 bits, cost one of three waves per SIMD at eight rows (5120 x 5120 at 8 bits 18.7 ->
+// 20.2), and are needed otherwise in workgroups of more than four waves (1024 x 14336 at 6 rows, 3 bits 7.9 -> 9.5).
+constexpr bool gemv_lookups_first(int bits, int m, int threads) {
+    return threads <= 256 && m >= (bits == 8 ? 5 : 3) && m <= 7;
+}
+
 // One row x one lane: rebuild the indices of this lane's WPL words, gather from
 // `table` (an LDS array at a compile-time address) and accumulate the M dot products.
-template <int BITS, int M, int WPL>
+template <int BITS, int M, int WPL, bool FIRST>
 __device__ __forceinline__ void row_dot(const typename WordVec<WPL>::type (&q)[BITS],
                                         const uint8_t (&table)[LookupTable<BITS>::kBytes],
                                         const uint32_t (&X)[M][WPL][4][4], float (&acc)[M][2]) {
@@ -62,32 +73,43 @@ __device__ __forceinline__ void row_dot(const typename WordVec<WPL>::type (&q)[B
         uint32_t qq[BITS];
 #pragma unroll
         for (int p = 0; p < BITS; p++) qq[p] = word_of<WPL>(q[p], wi);
+        uint32_t w[16];  // w[4 i + c]: elements 2 i and 2 i + 1 of byte c
+        auto product = [&](auto i_c, auto c_c) {
+            constexpr int i = decltype(i_c)::value, c = decltype(c_c)::value;
+#pragma unroll
+            for (int m = 0; m < M; m++) acc[m][c & 1] = dot2(w[4 * i + c], X[m][wi][3 - c][i], acc[m][c & 1]);
+        };
+        auto all = [&](auto &&lookup) {
+            static_for<4>([&](auto i_c) {
+                static_for<4>([&](auto c_c) {
+                    w[4 * decltype(i_c)::value + decltype(c_c)::value] = lookup(i_c, c_c);
+                    if constexpr (!FIRST) product(i_c, c_c);
+                });
+            });
+            if constexpr (FIRST) {
+                asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(w[4]), "+v"(w[5]), "+v"(w[6]), "+v"(w[7]),
+                                  "+v"(w[8]), "+v"(w[9]), "+v"(w[10]), "+v"(w[11]), "+v"(w[12]), "+v"(w[13]), "+v"(w[14]),
+                                  "+v"(w[15]));
+                static_for<4>([&](auto i_c) { static_for<4>([&](auto c_c) { product(i_c, c_c); }); });
+            }
+        };
         if constexpr (LookupTable<BITS>::kPair) {
             uint32_t apair[4];
             // byte = entry number (4 bits) or the entry's byte offset (3 bits); a table entry is 4 bytes
             planes_to_adjacent_pairs<BITS>(qq, apair);
-            auto gather_pair = [&](auto i_c, auto c_c) {
+            all([&](auto i_c, auto c_c) -> uint32_t {
                 constexpr int i = decltype(i_c)::value, c = decltype(c_c)::value;
-                const uint32_t off = byte_offset<c, BITS == 4 ? 2 : 0>(apair[i]);
-                const uint32_t w2 = *reinterpret_cast<const uint32_t *>(&table[off]);
-#pragma unroll
-                for (int m = 0; m < M; m++) acc[m][c & 1] = dot2(w2, X[m][wi][3 - c][i], acc[m][c & 1]);
-            };
-            static_for<4>([&](auto i_c) { static_for<4>([&](auto c_c) { gather_pair(i_c, c_c); }); });
+                return *reinterpret_cast<const uint32_t *>(&table[byte_offset<c, BITS == 4 ? 2 : 0>(apair[i])]);
+            });
         } else {
             uint32_t idx[8];
             planes_to_indices<BITS>(qq, idx);
-            auto gather_two = [&](auto i_c, auto c_c) {
+            all([&](auto i_c, auto c_c) -> uint32_t {
                 constexpr int i = decltype(i_c)::value, c = decltype(c_c)::value;
-                const uint32_t o0 = byte_offset<c, 1>(idx[2 * i]);
-                const uint32_t o1 = byte_offset<c, 1>(idx[2 * i + 1]);
-                const uint32_t lo = *reinterpret_cast<const uint16_t *>(&table[o0]);
-                const uint32_t hi = *reinterpret_cast<const uint16_t *>(&table[o1]);
-                const uint32_t w2 = lo | (hi << 16);
-#pragma unroll
-                for (int m = 0; m < M; m++) acc[m][c & 1] = dot2(w2, X[m][wi][3 - c][i], acc[m][c & 1]);
-            };
-            static_for<4>([&](auto i_c) { static_for<4>([&](auto c_c) { gather_two(i_c, c_c); }); });
+                const uint32_t lo = *reinterpret_cast<const uint16_t *>(&table[byte_offset<c, 1>(idx[2 * i])]);
+                const uint32_t hi = *reinterpret_cast<const uint16_t *>(&table[byte_offset<c, 1>(idx[2 * i + 1])]);
+                return lo | (hi << 16);
+            });
         }
     }
 }
@@ -231,13 +253,14 @@ void gemv_kbit_kernel(const half_t *__restrict__ x, const GemvMembers mem, int K
     // stores go through a pointer typed as global memory (the argument pointers left the statement above
     // without an address space, and a store through them would be a flat one)
     const global_ptr<half_t> out_g = (global_ptr<half_t>)reinterpret_cast<uint64_t>(out);
-    float lane_sum[R * M];
+    constexpr int NS = R * M;
+    float lane_sum[NS];
     static_for<R>([&](auto r_c) {
         constexpr int r = decltype(r_c)::value;
         float acc[M][2];
 #pragma unroll
         for (int m = 0; m < M; m++) acc[m][0] = acc[m][1] = 0.f;
-        row_dot<BITS, M, WPL>(q[r], tables[r], X, acc);
+        row_dot<BITS, M, WPL, gemv_lookups_first(BITS, M, THREADS)>(q[r], tables[r], X, acc);
 #pragma unroll
         for (int m = 0; m < M; m++) {
             float v = acc[m][0] + acc[m][1];
@@ -248,7 +271,6 @@ void gemv_kbit_kernel(const half_t *__restrict__ x, const GemvMembers mem, int K
         }
     });
     // sum number r M + m
-    constexpr int NS = R * M;
     float tot[(NS + 3) / 4];
     wave_sums<NS>(lane_sum, tot);
 

@@ -433,3 +433,23 @@ def test_dot_sums_do_not_depend_on_their_number(ext, K):
     finally:
         for k, v in before.items():
             _capi.set_tuning(k, v)
+
+
+@pytest.mark.parametrize("K", [64, 2048, 4096, 8192, 10272, 17440])
+def test_dot_kernel_at_every_number_of_rows_and_waves(ext, oracle, K):
+    """One wave per row to nine: lookups before the products or among them, sums folded or finished one by one -- within the
+    oracle's bar, and every activation row with the bits that it has alone."""
+    from any_precision_amd import _capi
+    N = 13
+    L = make(N, K, seed=K + 1)
+    q, luts = layer_to_gpu(L)
+    x, xg = _x(8, K, seed=5)
+    with _capi.tuning(matmul_mfma4=0, gemv_fine=0, gemv_stream=0, matmul_mfma_from=9, gemv_rows=2):
+        for b in range(3, 9):
+            _, want = oracle.matmul_kbit(x, L.qweight, L.luts[b], b, return_f64=True)
+            alone = torch.cat([ext.matmul_kbit(xg[m:m + 1].contiguous(), q, luts[b], b) for m in range(8)])
+            for M in range(1, 9):
+                assert _capi.matmul_route(M, N, K, b) == "dot"
+                got = ext.matmul_kbit(xg[:M].contiguous(), q, luts[b], b)
+                assert_close_gemv(got, want[:M], f"N={N} K={K} b={b} M={M}")
+                assert torch.equal(got.view(torch.int16), alone[:M].view(torch.int16)), (b, M)
