@@ -254,6 +254,11 @@ void gemv_kbit_kernel(const half_t *__restrict__ x, const GemvMembers mem, int K
     // without an address space, and a store through them would be a flat one)
     const global_ptr<half_t> out_g = (global_ptr<half_t>)reinterpret_cast<uint64_t>(out);
     constexpr int NS = R * M;
+    // Seven and eight activation rows in a workgroup of more than eight waves (at most 128 registers a lane, which the
+    // activations fill): every sum is finished and stored at once; held for the folding they more than double what goes to
+    // scratch memory (us folded -> at once: 512 x 17408 at 7 rows, 5 bits 30.3 -> 13.9; 2048 x 20480 at 8 rows, 8 bits 180 -> 70).
+    // The order within a sum is the same.
+    constexpr bool FOLD = M <= 6 || THREADS <= 512;
     float lane_sum[NS];
     static_for<R>([&](auto r_c) {
         constexpr int r = decltype(r_c)::value;
@@ -264,18 +269,25 @@ void gemv_kbit_kernel(const half_t *__restrict__ x, const GemvMembers mem, int K
 #pragma unroll
         for (int m = 0; m < M; m++) {
             float v = acc[m][0] + acc[m][1];
-            // a row's sums are finished before the next row's lookups start, outside of any "if (valid)" region: left to the
-            // optimiser the lookups of all rows are interleaved and take up to 30 registers more (8 bits: scratch memory)
-            asm volatile("" : "+v"(v));
-            lane_sum[r * M + m] = valid ? v : 0.f;
+            if constexpr (FOLD) {
+                // a row's sums are finished before the next row's lookups start, outside of any "if (valid)" region: left to the
+                // optimiser the lookups of all rows are interleaved and take up to 30 registers more (8 bits: scratch memory)
+                asm volatile("" : "+v"(v));
+                lane_sum[r * M + m] = valid ? v : 0.f;
+            } else {
+                const float one[1] = {valid ? v : 0.f};
+                float sum[1];
+                wave_sums<1>(one, sum);
+                if (lane == 0) partial[s * NS + r * M + m] = sum[0];
+            }
         }
     });
     // sum number r M + m
     float tot[(NS + 3) / 4];
-    wave_sums<NS>(lane_sum, tot);
+    if constexpr (FOLD) wave_sums<NS>(lane_sum, tot);
 
     auto swiglu = [](float gate, float up) { return gate / (1.f + __expf(-gate)) * up; };
-    if (S == 1 && !PAIR) {
+    if (FOLD && S == 1 && !PAIR) {
 #pragma unroll
         for (int h = 0; h < (NS + 3) / 4; h++) {
             int i;
@@ -283,7 +295,7 @@ void gemv_kbit_kernel(const half_t *__restrict__ x, const GemvMembers mem, int K
         }
     } else {
 #pragma unroll
-        for (int h = 0; h < (NS + 3) / 4; h++) {
+        for (int h = 0; FOLD && h < (NS + 3) / 4; h++) {
             int i;
             if (sum_lane<NS>(h, lane, i)) partial[s * NS + i] = tot[h];
         }
