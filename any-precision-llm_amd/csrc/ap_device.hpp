@@ -145,12 +145,6 @@ __device__ __forceinline__ bool sum_lane(int h, int lane, int &i) {
     i = 4 * h + lane / width;
     return lane % width == 0 && (n != 3 || lane < 48);
 }
-// Sum number i (a compile-time number once unrolled) of out, in every lane.
-template <int NV>
-__device__ __forceinline__ float sum_everywhere(const float (&out)[(NV + 3) / 4], int i) {
-    const int n = NV - i / 4 * 4, width = n >= 3 ? 16 : (n == 2 ? 32 : 64);
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, out[i / 4]), i % 4 * width));
-}
 template <int NV>
 __device__ __forceinline__ void wave_sums(const float (&v)[NV], float (&out)[(NV + 3) / 4]) {
     auto add = [](uint32_t a, uint32_t b) { return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b); };

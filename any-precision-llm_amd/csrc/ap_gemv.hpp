@@ -293,10 +293,6 @@ void gemv_kbit_kernel(const half_t *__restrict__ x, const GemvMembers mem, int K
             int i;
             if (sum_lane<NS>(h, lane, i) && row0 + i / M < N) out_g[(size_t)(i % M) * N + row0 + i / M] = (half_t)tot[h];
         }
-    } else if (FOLD && S == 1 && PAIR && M == 1) {
-        // without the trip through LDS: 5504 x 2048 at 5 bits 5.79 -> 5.67 us, 512 x 512 at 4 bits 2.71 -> 2.65; with more rows
-        // LDS is as fast or faster
-        if (lane == 0) out_g[row0] = (half_t)swiglu(sum_everywhere<NS>(tot, 0), sum_everywhere<NS>(tot, R - 1));
     } else {
 #pragma unroll
         for (int h = 0; FOLD && h < (NS + 3) / 4; h++) {
