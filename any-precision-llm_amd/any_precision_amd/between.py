@@ -33,10 +33,14 @@ def _norm_forward(module, original, hidden_states):
     return original(hidden_states) if out is None else out
 
 
-@functools.lru_cache(64)
+@functools.lru_cache(None)
+def _home(package):
+    return os.path.dirname(sys.modules[package].__file__) + os.sep
+
+
 def _unchanged(function, package):
     """Whether ``function`` and everything it wraps is code of ``package``, and not a replacement someone has put in its place."""
-    home = os.path.dirname(sys.modules[package].__file__) + os.sep
+    home = _home(package)
     while function is not None:
         code = getattr(function, "__code__", None)
         if code is None or not code.co_filename.startswith(home):
@@ -75,7 +79,8 @@ def _attention_forward(module, original, hidden_states, position_embeddings=None
                        **kwargs):
     native = _native()
     llama = sys.modules["transformers.models.llama.modeling_llama"]       # its rotary embedding and its attention functions
-    if (native is None or not _unchanged(llama.apply_rotary_pos_emb, "transformers") or position_embeddings is None or attention_mask is not None or past_key_values is not None
+    if (native is None or position_embeddings is None or attention_mask is not None or past_key_values is not None
+            or not _unchanged(llama.apply_rotary_pos_emb, "transformers")
             or module.training or torch.is_grad_enabled() or hidden_states.dim() != 3
             or module.config._attn_implementation != "sdpa" or not getattr(module, "is_causal", True)
             or kwargs.get("output_attentions") or any(k not in _IDLE and v is not None for k, v in kwargs.items())

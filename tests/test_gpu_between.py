@@ -298,6 +298,28 @@ def test_what_a_program_has_replaced_is_called(serving, monkeypatch, change, whe
     assert serving.served == 11 - {"LlamaRMSNorm": 5, "LlamaMLP": 2, "LlamaAttention": 4, "rotary": 4}.get(change, 0)
 
 
+def test_a_rotary_embedding_replaced_by_any_callable_is_called(serving, monkeypatch):
+    """Also one that has no hash and no code of its own."""
+    from transformers.models.llama import modeling_llama
+    stock, calls = modeling_llama.apply_rotary_pos_emb, []
+
+    class Replacement:
+        __hash__ = None
+
+        def __call__(self, *args, **kwargs):
+            calls.append(1)
+            return stock(*args, **kwargs)
+
+    module = _attention(True)
+    x, cos = torch.randn((1, 7, 64)), torch.rand((1, 7, 16))
+    with torch.no_grad():
+        module(x, (cos, cos))
+        assert serving.served == 2 and calls == []
+        monkeypatch.setattr(modeling_llama, "apply_rotary_pos_emb", Replacement())
+        module(x, (cos, cos))
+    assert serving.served == 2 and calls == [1]
+
+
 @pytest.mark.gpu
 def test_tensors_whose_memory_is_not_their_value_are_left_to_torch():
     """A lazily negated view and a zero tensor without memory."""
