@@ -67,6 +67,48 @@ AP_HD void swap_blocks(uint32_t &a, uint32_t &b) {
     b = nb;
 }
 
+// The three butterfly stages of planes_to_indices, for callers that spread them over other work.  Row i of r feeds bit i of
+// the output byte; rows [SHIFT, SHIFT + BITS) are live before stage 1, and a stage makes the rows it pairs live together.
+template <int BITS, int SHIFT>
+AP_HD constexpr bool index_row_live(int i, int stage) {
+    if (stage == 0) return i >= SHIFT && i < SHIFT + BITS;
+    const int d = stage == 1 ? 4 : 2;  // stage 1 pairs rows i and i + 4, stage 2 rows i and i + 2
+    return index_row_live<BITS, SHIFT>(i & ~d, stage - 1) || index_row_live<BITS, SHIFT>(i | d, stage - 1);
+}
+template <int BITS, int SHIFT, int S, uint32_t LO, int A, int STAGE>
+AP_HD void swap_index_rows(uint32_t (&r)[8]) {
+    swap_blocks<S, LO, !index_row_live<BITS, SHIFT>(A, STAGE), !index_row_live<BITS, SHIFT>(A + S, STAGE)>(r[A], r[A + S]);
+}
+template <int BITS, int SHIFT = 0>
+AP_HD void indices_stage1(const uint32_t (&q)[BITS], uint32_t (&r)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const bool live = i >= SHIFT && i < SHIFT + BITS;
+        r[i] = live ? q[live ? BITS - 1 - (i - SHIFT) : 0] : 0u;
+    }
+    swap_index_rows<BITS, SHIFT, 4, 0x0F0F0F0Fu, 0, 0>(r);
+    swap_index_rows<BITS, SHIFT, 4, 0x0F0F0F0Fu, 1, 0>(r);
+    swap_index_rows<BITS, SHIFT, 4, 0x0F0F0F0Fu, 2, 0>(r);
+    swap_index_rows<BITS, SHIFT, 4, 0x0F0F0F0Fu, 3, 0>(r);
+}
+template <int BITS, int SHIFT = 0>
+AP_HD void indices_stage2(uint32_t (&r)[8]) {
+    swap_index_rows<BITS, SHIFT, 2, 0x33333333u, 0, 1>(r);
+    swap_index_rows<BITS, SHIFT, 2, 0x33333333u, 1, 1>(r);
+    swap_index_rows<BITS, SHIFT, 2, 0x33333333u, 4, 1>(r);
+    swap_index_rows<BITS, SHIFT, 2, 0x33333333u, 5, 1>(r);
+}
+template <int BITS, int SHIFT = 0>
+AP_HD void indices_stage3(uint32_t (&r)[8], uint32_t (&idx)[8]) {
+    swap_index_rows<BITS, SHIFT, 1, 0x55555555u, 0, 2>(r);
+    swap_index_rows<BITS, SHIFT, 1, 0x55555555u, 2, 2>(r);
+    swap_index_rows<BITS, SHIFT, 1, 0x55555555u, 4, 2>(r);
+    swap_index_rows<BITS, SHIFT, 1, 0x55555555u, 6, 2>(r);
+    // r[u] byte b bit i = row i bit (8 b + u); element e sits at u = 7 - e.
+#pragma unroll
+    for (int e = 0; e < 8; e++) idx[e] = r[7 - e];
+}
+
 // q[p], p = 0..BITS-1: the word of plane p (plane 0 most significant) for 32
 // elements.  idx[e], e = 0..7: byte b of idx[e] is the BITS-bit index of the
 // element stored at bit 8 b + (7 - e) of the plane words, shifted left by
@@ -76,34 +118,10 @@ AP_HD void swap_blocks(uint32_t &a, uint32_t &b) {
 template <int BITS, int SHIFT = 0>
 AP_HD void planes_to_indices(const uint32_t (&q)[BITS], uint32_t (&idx)[8]) {
     static_assert(BITS >= 1 && BITS + SHIFT <= 8, "index must fit a byte");
-    // row i feeds bit i of the output byte: plane BITS-1-(i-SHIFT), zero outside
-    constexpr int LOW = SHIFT, HIGH = SHIFT + BITS;   // rows [LOW, HIGH) are live
-#define AP_LIVE(i) ((i) >= LOW && (i) < HIGH)
     uint32_t r[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) r[i] = AP_LIVE(i) ? q[AP_LIVE(i) ? BITS - 1 - (i - SHIFT) : 0] : 0u;
-    // stage 1: 4-bit blocks between rows i and i+4
-    swap_blocks<4, 0x0F0F0F0Fu, !AP_LIVE(0), !AP_LIVE(4)>(r[0], r[4]);
-    swap_blocks<4, 0x0F0F0F0Fu, !AP_LIVE(1), !AP_LIVE(5)>(r[1], r[5]);
-    swap_blocks<4, 0x0F0F0F0Fu, !AP_LIVE(2), !AP_LIVE(6)>(r[2], r[6]);
-    swap_blocks<4, 0x0F0F0F0Fu, !AP_LIVE(3), !AP_LIVE(7)>(r[3], r[7]);
-    // after stage 1 rows i and i+4 are live iff either was
-#define AP_LIVE1(i) (AP_LIVE((i) & 3) || AP_LIVE(((i) & 3) + 4))
-    swap_blocks<2, 0x33333333u, !AP_LIVE1(0), !AP_LIVE1(2)>(r[0], r[2]);
-    swap_blocks<2, 0x33333333u, !AP_LIVE1(1), !AP_LIVE1(3)>(r[1], r[3]);
-    swap_blocks<2, 0x33333333u, !AP_LIVE1(4), !AP_LIVE1(6)>(r[4], r[6]);
-    swap_blocks<2, 0x33333333u, !AP_LIVE1(5), !AP_LIVE1(7)>(r[5], r[7]);
-#define AP_LIVE2(i) (AP_LIVE1((i) & 5) || AP_LIVE1(((i) & 5) + 2))
-    swap_blocks<1, 0x55555555u, !AP_LIVE2(0), !AP_LIVE2(1)>(r[0], r[1]);
-    swap_blocks<1, 0x55555555u, !AP_LIVE2(2), !AP_LIVE2(3)>(r[2], r[3]);
-    swap_blocks<1, 0x55555555u, !AP_LIVE2(4), !AP_LIVE2(5)>(r[4], r[5]);
-    swap_blocks<1, 0x55555555u, !AP_LIVE2(6), !AP_LIVE2(7)>(r[6], r[7]);
-#undef AP_LIVE2
-#undef AP_LIVE1
-#undef AP_LIVE
-    // r[u] byte b bit i = row i bit (8 b + u); element e sits at u = 7 - e.
-#pragma unroll
-    for (int e = 0; e < 8; e++) idx[e] = r[7 - e];
+    indices_stage1<BITS, SHIFT>(q, r);
+    indices_stage2<BITS, SHIFT>(r);
+    indices_stage3<BITS, SHIFT>(r, idx);
 }
 
 // Adjacent-pair form for BITS = 3, 4: apair[i], i = 0..3; byte b of apair[i] addresses the table entry

@@ -1,12 +1,14 @@
 // C ABI of libanyprec_hip: argument checks, launch geometry, dispatch.
 // The declarations and their reference counterparts are in include/anyprec_hip.h.
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <string.h>
 
 #include "anyprec_hip.h"
 #include "ap_decode.hpp"
 #include "ap_dequant.hpp"
 #include "ap_gemm_launch.hpp"
+#include "ap_gemmb_launch.hpp"
 #include "ap_gemmt_launch.hpp"
 #include "ap_gemmw_launch.hpp"
 #include "ap_gemv4_launch.hpp"
@@ -46,6 +48,8 @@ enum {
     kGemmTile,          // > 0: blocks of 16 activation rows in its tile: 1, 2, 4 or 8
     kGemmTileSplit,     // > 0: groups of four waves per workgroup of the 64-row tile, each on its share of K: 1 or 2
     kGemmLookahead,     // K-split fused GEMM, lookups one word ahead of the matrix instructions: 0 never, 1 where it pays, 2 wherever the variant exists
+    kGemmBlock,         // block-tile fused GEMM (ap_gemm_kbit): 0 never, 1 where it pays, 2 wherever it fits
+    kGemmBlockTile,     // > 0: its tile, 100 x blocks of 32 activation rows + 10 x waves over the weight rows + groups over K
     kKnobCount
 };
 Knob g_knobs[kKnobCount] = {
@@ -55,6 +59,7 @@ Knob g_knobs[kKnobCount] = {
     {"gemv_fine", 1},
     {"gemm_walk", 1},             {"gemm_walk_wgs", 1},  {"gemm_tiled", 1},   {"gemm_tile", 0},
     {"gemm_tile_split", 0},       {"gemm_lookahead", 1},
+    {"gemm_block", 1},            {"gemm_block_tile", 0},
 };
 inline int knob(int k) { return __atomic_load_n(&g_knobs[k].value, __ATOMIC_RELAXED); }
 
@@ -601,6 +606,105 @@ bool gemmt_pays(int M, int N, int K, int w_bits) {
     return M > (w_bits <= 4 ? 32 : (w_bits == 5 ? 48 : (w_bits == 6 ? 64 : 80)));
 }
 
+// The tiles of the block-tile fused GEMM (ap_gemmb.hpp): blocks of 32 activation rows, waves over the weight rows, groups over K.
+constexpr struct { int mb, wn, wk; } kGemmbTiles[] = {{8, 4, 1}, {3, 4, 2}, {3, 2, 4}, {4, 4, 2}, {4, 2, 4}, {2, 4, 2}, {2, 2, 4}, {2, 1, 8}, {1, 2, 4}};
+constexpr int kGemmbTileCount = sizeof(kGemmbTiles) / sizeof(kGemmbTiles[0]);
+
+// What a launch with a tile takes, in us: a + r (p + h (s + f u)), where r = rounds of tiles over the CUs, h = the half-steps of
+// 256 elements that a group walks and u = the share of the CUs that has a tile (up to 1: the more there are, the slower each runs).
+// {a, p, s, f} per bit-width and tile of the list above, least squares over 15 linear shapes (1024 x 4096 .. 22016 x 4096, 4096 x
+// 14336, 8192 x 8192; rows of 2048 .. 14336 elements, one of no multiple of 128) x 14 numbers of activation rows (16 .. 2048), planes
+// from HBM, 2500 launches a bit-width.  The tile it picks is within 0.2 % of the fastest on average, 17 % at worst.  (0 0 0 0: the
+// tables of that tile and bit-width do not fit the LDS.)
+constexpr float kGemmbCost[6][kGemmbTileCount][4] = {
+    {{-1.66f, 7.89f, 2.38f, 1.05f}, {1.60f, 4.50f, 2.36f, 0.75f}, {3.25f, 2.18f, 2.96f, 1.20f},
+     {2.23f, 4.38f, 2.62f, 1.21f}, {2.82f, 2.88f, 3.45f, 1.55f}, {2.14f, 3.39f, 2.07f, 0.52f},
+     {3.74f, 2.18f, 2.31f, 0.71f}, {4.04f, 1.94f, 3.18f, 1.24f}, {6.14f, -0.05f, 1.84f, 0.13f}},
+    {{-1.29f, 7.96f, 2.80f, 1.02f}, {1.55f, 4.78f, 3.22f, 0.66f}, {3.64f, 2.49f, 3.18f, 1.23f},
+     {2.73f, 4.27f, 3.44f, 1.17f}, {3.41f, 3.51f, 4.17f, 1.44f}, {2.38f, 3.55f, 2.93f, 0.47f},
+     {4.01f, 1.61f, 2.82f, 0.86f}, {4.03f, 2.75f, 3.95f, 1.12f}, {3.72f, 2.54f, 2.03f, 0.42f}},
+    {{-0.04f, 5.99f, 2.89f, 1.04f}, {1.49f, 4.55f, 3.50f, 0.60f}, {4.15f, 2.74f, 4.13f, 1.08f},
+     {2.92f, 3.47f, 3.74f, 1.12f}, {3.69f, 3.24f, 4.51f, 1.51f}, {2.87f, 2.79f, 3.21f, 0.44f},
+     {4.12f, 2.53f, 3.48f, 0.71f}, {4.30f, 3.07f, 4.21f, 1.25f}, {4.00f, 2.55f, 3.00f, 0.35f}},
+    {{-1.07f, 8.12f, 2.89f, 1.03f}, {2.28f, 5.15f, 3.58f, 0.64f}, {4.90f, 2.97f, 4.20f, 1.21f},
+     {3.68f, 3.93f, 3.80f, 1.14f}, {4.25f, 3.63f, 4.59f, 1.64f}, {3.18f, 3.92f, 3.32f, 0.41f},
+     {4.92f, 2.95f, 3.51f, 0.85f}, {4.56f, 3.48f, 4.39f, 1.28f}, {4.36f, 3.30f, 3.15f, 0.39f}},
+    {{-0.65f, 8.29f, 2.99f, 1.09f}, {2.46f, 5.73f, 3.81f, 0.58f}, {5.65f, 2.79f, 4.44f, 1.32f},
+     {4.36f, 3.88f, 4.09f, 1.12f}, {5.35f, 3.14f, 4.82f, 1.75f}, {3.45f, 4.25f, 3.60f, 0.34f},
+     {5.68f, 2.86f, 3.79f, 0.96f}, {4.72f, 3.82f, 4.62f, 1.40f}, {5.12f, 3.43f, 3.33f, 0.47f}},
+    {{6.00f, 0.63f, 3.58f, 1.19f}, {3.20f, 6.33f, 4.16f, 0.62f}, {5.87f, 3.34f, 4.82f, 1.39f},
+     {5.87f, 2.96f, 4.73f, 1.10f}, {0.f, 0.f, 0.f, 0.f}, {4.65f, 4.48f, 3.97f, 0.30f},
+     {6.34f, 2.30f, 4.49f, 1.18f}, {0.f, 0.f, 0.f, 0.f}, {5.38f, 4.42f, 3.61f, 0.54f}},
+};
+
+// The fastest tile for linears that share x; false if the kernel does not serve the shape.
+bool gemmb_geometry(int M, const int *N, int count, int K, int w_bits, GemmbGeometry *geo) {
+    if (K < 256 || (long long)M * K * 2 > 0xffffffffLL || count > kGemmbMaxGroup) return false;
+    for (int g = 0; g < count; g++)
+        if ((long long)N[g] * (K >> 5) * 4 > 0xffffffffLL) return false;
+    const int forced = knob(kGemmBlockTile);
+    const double cus = cu_count();
+    double best = 0;
+    geo->mb = 0;
+    for (int t = 0; t < kGemmbTileCount; t++) {
+        const auto &tile = kGemmbTiles[t];
+        const float *c = kGemmbCost[w_bits - 3][t];
+        if (c[2] == 0.f || (forced > 0 && forced != 100 * tile.mb + 10 * tile.wn + tile.wk)) continue;
+        long long n = 0;
+        for (int g = 0; g < count; g++) n += (N[g] + kGemmbRows * tile.wn - 1) / (kGemmbRows * tile.wn);
+        const long long m = (M + 32LL * tile.mb - 1) / (32 * tile.mb);
+        if ((n + 7) / 8 * 8 * m > 0x7fffffffLL) continue;
+        const double rounds = ceil((double)(n * m) / cus), fill = fmin(1.0, (double)(n * m) / cus);
+        const int halves = (K + 255) / 256, h = (halves + tile.wk - 1) / tile.wk;
+        const double us = c[0] + rounds * (c[1] + h * (c[2] + c[3] * fill));
+        if (geo->mb == 0 || us < best) {
+            best = us;
+            *geo = {tile.mb, tile.wn, tile.wk, (int)n, (int)m};
+        }
+    }
+    return geo->mb != 0;
+}
+
+// Where the block-tile kernel beats the other fused forms (same sweep; us there and here).  Beyond 256 activation rows on every linear of
+// 1024 rows or more (14336 x 4096, 512 rows: 90 / 62 at 3 bits, 114 / 70 at 5); from 129 rows on linears of 2048 rows or
+// more (11008 x 4096, 192 rows, 5 bits: 56 / 38), and from 65 of 4096 or more (4096 x 11008, 128 rows, 5 bits: 50 / 39); narrower
+// ones at 5 to 7 bits (1024 x 4096, 128 rows, 5 bits: 20 / 16; at 3 bits 12 / 13), at 8 bits from 2048 rows on.  At 33..64
+// rows on linears of 5120 rows or more (6144 x 4096, 48 rows, 5 bits: 27 / 17), on narrower ones where the 16-row tiles of the tiled kernel
+// wait for their lookups: 5 to 7 bits beyond 48 rows, or on rows of more than 4096 elements; 8 bits on both (4096 x 4096,
+// 48 rows: 18 / 23).  Rows of no multiple of 128 elements, which the tiled kernel does not take: on linears of less than
+// 5120 rows up to 4 bits from 33 activation rows on, else from 65 (4096 x 11040, 128 rows: 98 / 35 at 3 bits, 104 / 60 at 8).  Sets of
+// more than 20000 rows from 17 (22016 x 4096 at 32 rows: 31 / 23, 65 / 49).
+bool gemmb_pays(int M, long long N, int K, int b) {
+    if (N < 1024 || M <= 16 || K < 256) return false;
+    if ((long long)M * K * 2 > 0xffffffffLL || N * (K >> 5) * 4 > 0xffffffffLL) return false;  // its 32-bit offsets
+    if (M <= 32) return N >= 20000;
+    if (M <= 64) {
+        if (N >= 5120) return true;
+        if ((K & 127) != 0) return b <= 4;
+        return b >= 5 && K >= 4096 && (b == 8 ? M > 48 && K > 4096 : M > 48 || K > 4096);
+    }
+    const bool middle = b >= 5 && b <= 7;
+    if (M <= 128) return N >= 4096 || middle || (b == 8 && N >= 2048);
+    return M > 256 || N >= 2048 || middle;
+}
+
+// Where it also beats dequant_kbit + a library GEMM, beyond what fused_gemm_pays says of the other forms (same sweep; pair / block, us): up to
+// 256 rows wherever it is the best fused form (14336 x 4096, 256 rows, 8 bits: 84 / 55); up to 512 at 3 to 7 bits (14336 x 4096: 85 / 62 at
+// 3 bits, 89 / 70 at 5; 4096 x 14336: 117 / 86 at 5) except at 7 bits on sets of 16384 rows or more beyond 384, at 8 bits on linears
+// of 4096..16383 rows (14336 x 4096: 93 / 80; 2048 x 5504 37 / 53) or of at most 4096 elements a row; up to 1024 at 3 bits (4096 x 11008:
+// 131 / 97; 22016 x 4096 201 / 188), at 4 to 6 bits on linears of less than 10240 rows (4096 x 4096, 5 bits: 50 / 45; 14336 x 4096 121 / 143),
+// at 7 bits of 4096 rows or more with rows of 4096 elements or more among those, not at 8 (4096 x 11008, 1024 rows: 134 / 139);
+// up to 2048 at 3 bits on linears of at most 4096 rows (4096 x 11008: 189 / 171).
+bool gemmb_beats_pair(int M, long long N, int K, int b) {
+    if (!gemmb_pays(M, N, K, b)) return false;
+    if (M <= 256) return b <= 7 || N >= 2048;
+    if (M <= 512) return b <= 7 ? !(b == 7 && N >= 16384 && M > 384) : N < 16384 && (N >= 4096 || (N >= 2048 && K <= 4096));
+    if (M > 1024) return b == 3 && N <= 4096 && M <= 2048;
+    if (b == 3) return true;
+    if (N >= 10240) return false;
+    return b <= 6 || (b == 7 && N >= 4096 && K >= 4096);
+}
+
 // Launch of the fused dequant -> MFMA kernel (arguments already checked).
 int run_gemm(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, uint16_t *out, int M, int N, int K,
              int w_bits, hipStream_t st) {
@@ -948,7 +1052,8 @@ int plan_matmul(int M, const int *N, int count, int K, int w_bits, uint16_t *con
     return AP_OK;
 }
 
-// Whether the fused GEMM (ap_gemm_kbit) beats dequant_kbit + a library GEMM for `M` activation rows.  Measured on the
+// Whether the K-split and tiled fused GEMMs beat dequant_kbit + a library GEMM for `M` activation rows (gemmb_beats_pair has the
+// block-tile kernel, which serves more).  Measured on the
 // linear shapes of the Llama-2-7B / Llama-3-8B / 13B / 70B layers at 96..512 activation rows, every bit-width
 // (fused / pair, us):
 //  - always up to 32 activation rows (1.3-4x at 16);
@@ -1068,6 +1173,38 @@ int run_gemmt(const GemmtGeometry &geo, const uint16_t *x, int count, const uint
     return launch_status();
 }
 
+// Whether ap_gemm_kbit takes the block-tile kernel (N: rows of all linears of the launch).  The knobs of the tiled kernel come first: a
+// caller that forces or forbids it means this one too.
+bool takes_gemmb(int M, long long N, int K, int w_bits) {
+    const int mode = knob(kGemmBlock);
+    return mode >= 2 || (mode > 0 && knob(kGemmTiled) == 1 && gemmb_pays(M, N, K, w_bits));
+}
+
+// One launch of the block-tile kernel over `count` linears (arguments already checked; geo from gemmb_geometry over all of them).
+int run_gemmb(const GemmbGeometry &geo, const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut,
+              uint16_t *const *out, const int *N, const long long *ldo, int M, int K, int w_bits, hipStream_t st) {
+    GemmbMembers mem = {};
+    mem.count = count;
+    for (int g = 0; g < count; g++) {
+        mem.qweight[g] = qweight[g];
+        mem.lut[g] = lut[g];
+        mem.out[g] = out[g];
+        mem.N[g] = N[g];
+        mem.ldo[g] = ldo ? ldo[g] : N[g];
+        mem.tile0[g + 1] = mem.tile0[g] + (N[g] + 32 * geo.wn - 1) / (32 * geo.wn);
+    }
+    bool ok;
+    switch (w_bits) {
+        case 3: ok = launch_gemmb<3>(geo, x, mem, M, K, st); break;
+        case 4: ok = launch_gemmb<4>(geo, x, mem, M, K, st); break;
+        case 5: ok = launch_gemmb<5>(geo, x, mem, M, K, st); break;
+        case 6: ok = launch_gemmb<6>(geo, x, mem, M, K, st); break;
+        case 7: ok = launch_gemmb<7>(geo, x, mem, M, K, st); break;
+        default: ok = launch_gemmb<8>(geo, x, mem, M, K, st); break;
+    }
+    return ok ? launch_status() : AP_ELIMIT;
+}
+
 int ap_gemm_kbit(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, uint16_t *out, int M, int N, int K,
                  int w_bits, void *stream) {
     if (!x || !qweight || !lut || !out) return AP_ENULL;
@@ -1077,6 +1214,9 @@ int ap_gemm_kbit(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut
     if (!aligned16(x) || !aligned16(qweight) || !aligned16(lut)) return AP_EALIGN;
     drain_stale_error();
     {
+        GemmbGeometry bgeo;
+        if (takes_gemmb(M, N, K, w_bits) && gemmb_geometry(M, &N, 1, K, w_bits, &bgeo))
+            return run_gemmb(bgeo, x, 1, &qweight, &lut, &out, &N, nullptr, M, K, w_bits, static_cast<hipStream_t>(stream));
         GemmtGeometry tgeo;
         const int mode = knob(kGemmTiled);
         if (mode > 0 && gemmt_geometry(M, (N + 63) / 64, K, w_bits, &tgeo) && (mode >= 2 || gemmt_pays(M, N, K, w_bits)))
@@ -1098,7 +1238,7 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
     if (!x || !qweight || !lut || !out || !N) return AP_ENULL;
     if (count < 1 || count > kGemmtMaxGroup) return AP_ELIMIT;
     if (M < 1) return AP_EBATCH;
-    long long tiles = 0, rows = 0;  // tiles of all members; rows of the largest
+    long long tiles = 0, rows = 0, total = 0;  // tiles of all members; rows of the largest and of all
     bool strided = false;
     for (int g = 0; g < count; g++) {
         if (!qweight[g] || !lut[g] || !out[g]) return AP_ENULL;
@@ -1109,6 +1249,7 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
         strided = strided || (ldo && ldo[g] != N[g]);
         tiles += (N[g] + 63) / 64;
         rows = N[g] > rows ? N[g] : rows;
+        total += N[g];
     }
     if (!aligned16(x)) return AP_EALIGN;
     drain_stale_error();
@@ -1124,6 +1265,11 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
     // (7B q/k/v at 16 rows: 16-24 us against 23-26 at 3-5 bits; 13B: 20-40 against 36-68; 70B: 21-48 against 39-64); wide
     // members (gate/up) are within 10 % either way one by one.
     const bool pays = M > 32 || (M > 8 && rows <= 8192 && K >= 1024);
+    // The block-tile kernel takes the set by the rule for one linear of all its rows.  (Rows of no multiple of 128 elements are
+    // served dense only.)
+    GemmbGeometry bgeo;
+    if ((count > 1 || strided) && (!strided || (K & 127) == 0) && takes_gemmb(M, total, K, w_bits) && gemmb_geometry(M, N, count, K, w_bits, &bgeo))
+        return run_gemmb(bgeo, x, count, qweight, lut, out, N, ldo, M, K, w_bits, static_cast<hipStream_t>(stream));
     if (fits && (strided || (count > 1 && mode > 0 && (mode >= 2 || pays))))
         return run_gemmt(tgeo, x, count, qweight, lut, out, N, ldo, M, K, w_bits, static_cast<hipStream_t>(stream));
     // only the tiled kernel writes rows that are not dense: rows it cannot walk at all are a shape error, a size or a
@@ -1210,6 +1356,19 @@ int ap_gemm_kbit_group_pays(int count, const int *N, int M, int K, int w_bits) {
     }
     if (M < 1) return AP_EBATCH;
     return fused_set_pays(M, N, count, K, w_bits) ? 1 : 0;
+}
+
+int ap_gemm_kbit_taken(int M, int N, int K, int w_bits) {
+    const int rc = ap_gemm_kbit_pays(M, N, K, w_bits);
+    return rc != 0 ? rc : (takes_gemmb(M, N, K, w_bits) && gemmb_beats_pair(M, N, K, w_bits) ? 1 : 0);
+}
+
+int ap_gemm_kbit_group_taken(int count, const int *N, int M, int K, int w_bits) {
+    const int rc = ap_gemm_kbit_group_pays(count, N, M, K, w_bits);
+    if (rc != 0) return rc;
+    long long sum = 0;
+    for (int g = 0; g < count; g++) sum += N[g];
+    return M > 32 && M <= 512 && sum >= 4096 && takes_gemmb(M, sum, K, w_bits) && gemmb_beats_pair(M, sum, K, w_bits) ? 1 : 0;
 }
 
 int ap_matmul_kbit_route(int M, int N, int K, int w_bits, int *route) {

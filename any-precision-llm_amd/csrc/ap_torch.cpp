@@ -168,6 +168,28 @@ PyObject *dequant_kbit(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
 }
 
+// Some functions of this module replace torch ops, which take part in everything torch does with an op: a call that anything but plain execution follows -- gradients, tangents, subclasses, modes, functorch --
+// gets None and runs as torch ops.
+bool plain_half(PyObject *o, const at::Device *device) {
+    if (!is_tensor(o) || !exact_tensor(o)) return false;
+    const Tensor &t = THPVariable_Unpack(o);
+    if (!t.is_cuda() || t.scalar_type() != at::kHalf || t.layout() != at::kStrided || !t.is_contiguous() || t.numel() == 0) return false;
+    if (device != nullptr && t.device() != *device) return false;
+    if (c10::GradMode::is_enabled() && t.requires_grad()) return false;
+    const auto keys = t.key_set();
+    if (keys.has(c10::DispatchKey::FuncTorchBatched) || keys.has(c10::DispatchKey::FuncTorchGradWrapper) ||
+        keys.has(c10::DispatchKey::Functionalize) || keys.has(c10::DispatchKey::Negative) || keys.has(c10::DispatchKey::ZeroTensor) ||
+        t._fw_grad(0).defined())
+        return false;
+    return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
+}
+
+bool plain_execution() {
+    return !c10::impl::TorchDispatchModeTLS::any_modes_set() && !at::impl::torch_function_mode_enabled() &&
+           !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
+           !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
+}
+
 // Names in a module's dicts, made once.
 PyObject *key_buffers, *key_qweight, *key_bias, *key_lut[9];
 
@@ -192,7 +214,8 @@ bool tensors_of(PyObject *module_dict, int bits, ModuleTensors *m) {
 }
 
 // linear(module.__dict__, x, w_bits): AnyPrecisionLinear.forward.  Up to 8 rows ap_matmul_kbit, then
-// ap_gemm_kbit where ap_gemm_kbit_pays, else the weight in fp16 and torch's own product (which takes part in autograd).
+// ap_gemm_kbit where ap_gemm_kbit_pays, or ap_gemm_kbit_taken and nothing but plain execution follows the call; else the weight in fp16 and
+// torch's own product (which takes part in autograd).
 PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (n != 3 || !is_tensor(args[1])) return none();
     const int bits = bits_of(args[2]);
@@ -206,7 +229,8 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (!weight_of(q, t, bits, &w)) return none();
         const int64_t rows = rows_of(x, w);
         if (rows < 1) return none();
-        const bool pays = rows <= 8 || ap_gemm_kbit_pays((int)rows, w.N, w.K, bits) == 1;
+        const bool pays = rows <= 8 || ap_gemm_kbit_pays((int)rows, w.N, w.K, bits) == 1 ||
+                          (ap_gemm_kbit_taken((int)rows, w.N, w.K, bits) == 1 && plain_execution() && plain_half(args[1], nullptr));
         // torch's product and sum as Python calls them, where a subclass or a mode wants to see them
         const bool torch_op = !pays || bias.defined();
         if (torch_op && (at::impl::torch_function_mode_enabled() || !exact_tensor(args[1]) || (m.bias != nullptr && !exact_tensor(m.bias))))
@@ -269,7 +293,9 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
         const int K = w[0].K;
         if (rows < 1) return none();
         const bool gemm = rows > 8;
-        if (gemm && ap_gemm_kbit_group_pays(count, N, (int)rows, K, bits) != 1) return none();
+        if (gemm && ap_gemm_kbit_group_pays(count, N, (int)rows, K, bits) != 1 &&
+            !(ap_gemm_kbit_group_taken(count, N, (int)rows, K, bits) == 1 && plain_execution() && plain_half(args[1], nullptr)))
+            return none();
         // side by side in one allocation: one row's results always are dense, and the tiled kernel writes rows that are not
         const bool joint = concat && (gemm ? K % 128 == 0 : rows == 1);
         if (concat && !joint && at::impl::torch_function_mode_enabled()) return none();  // the mode sees torch.cat
@@ -313,29 +339,6 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
         }
         return list;
     });
-}
-
-// What sits between the linears of the Hugging Face Llama modules.  These replace torch ops, which take part in everything torch
-// does with an op: a call that anything but plain execution follows -- gradients, tangents, subclasses, modes, functorch --
-// gets None and runs as torch ops.
-bool plain_half(PyObject *o, const at::Device *device) {
-    if (!is_tensor(o) || !exact_tensor(o)) return false;
-    const Tensor &t = THPVariable_Unpack(o);
-    if (!t.is_cuda() || t.scalar_type() != at::kHalf || t.layout() != at::kStrided || !t.is_contiguous() || t.numel() == 0) return false;
-    if (device != nullptr && t.device() != *device) return false;
-    if (c10::GradMode::is_enabled() && t.requires_grad()) return false;
-    const auto keys = t.key_set();
-    if (keys.has(c10::DispatchKey::FuncTorchBatched) || keys.has(c10::DispatchKey::FuncTorchGradWrapper) ||
-        keys.has(c10::DispatchKey::Functionalize) || keys.has(c10::DispatchKey::Negative) || keys.has(c10::DispatchKey::ZeroTensor) ||
-        t._fw_grad(0).defined())
-        return false;
-    return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
-}
-
-bool plain_execution() {
-    return !c10::impl::TorchDispatchModeTLS::any_modes_set() && !at::impl::torch_function_mode_enabled() &&
-           !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
-           !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
 }
 
 // plain(tensors): whether the functions below take each of them, all on one device.

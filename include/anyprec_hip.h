@@ -34,7 +34,7 @@
 extern "C" {
 #endif
 
-#define AP_ABI_VERSION 10
+#define AP_ABI_VERSION 11
 
 enum {
     AP_OK = 0,
@@ -131,6 +131,13 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
  * keeping thresholds of its own.  Negative argument errors as for ap_gemm_kbit. */
 int ap_gemm_kbit_pays(int M, int N, int K, int w_bits);
 int ap_gemm_kbit_group_pays(int count, const int *N, int M, int K, int w_bits);
+
+/* What AnyPrecisionLinear asks: 1 also where only the block-tile kernel that ap_gemm_kbit (ap_gemm_kbit_group) launches from 17
+ * activation rows on beats ap_dequant_kbit + a library fp16 GEMM.  The pair takes part in automatic differentiation and the fused
+ * GEMM does not: ap_gemm_kbit_pays says where the host module has always taken the fused form, these where it may for a plain
+ * forward.  Argument errors as above. */
+int ap_gemm_kbit_taken(int M, int N, int K, int w_bits);
+int ap_gemm_kbit_group_taken(int count, const int *N, int M, int K, int w_bits);
 
 /* Human-readable text for a return code of the functions above. */
 const char *ap_strerror(int code);

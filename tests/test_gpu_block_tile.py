@@ -1,0 +1,150 @@
+"""The block-tile fused GEMM (ap_gemm_kbit from 17 activation rows on): every tile against the oracle at the edges of its range."""
+import pytest
+import torch
+
+from _util import assert_bit_exact, assert_close_gemv, layer_to_gpu, make
+
+pytestmark = pytest.mark.gpu
+TILES = (841, 342, 324, 442, 424, 242, 224, 218, 124)
+NOT_BUILT = {(8, 424), (8, 218)}      # their tables do not fit the LDS
+
+
+@pytest.fixture(scope="module")
+def ext():
+    import any_precision_ext
+    return any_precision_ext
+
+
+def _x(M, K, seed):
+    from any_precision_amd import synth
+    x = synth.make_x(M, K, seed=seed)
+    return x, torch.from_numpy(x).cuda()
+
+
+def _tiles(b):
+    return [t for t in TILES if (b, t) not in NOT_BUILT]
+
+
+# K: one half-step of 256 elements; a part of one behind it (288, 992, 2720); fewer half-steps than groups; a different number per
+# group (1280, 11008).  N: no multiple of any tile, of 4, of 8.
+@pytest.mark.parametrize("N,K", ((131, 256), (64, 288), (77, 992), (128, 1280), (200, 2720), (96, 4096), (33, 11008)))
+def test_every_tile_agrees_with_the_oracle(ext, oracle, N, K):
+    from any_precision_amd import _capi
+    L = make(N, K, seed=N + K)
+    q, luts = layer_to_gpu(L)
+    for b in range(3, 9):
+        for M in (1, 32, 65, 257):
+            x, xg = _x(M, K, seed=M)
+            _, want = oracle.matmul_kbit(x, L.qweight, L.luts[b], b, return_f64=True)
+            for tile in _tiles(b):
+                print(f"block tile N={N} K={K} b={b} M={M} tile={tile}", flush=True)
+                with _capi.tuning(gemm_block=2, gemm_block_tile=tile):
+                    got = ext.gemm_kbit(xg, q, luts[b], b)
+                assert_close_gemv(got, want, f"N={N} K={K} b={b} M={M} tile={tile}")
+
+
+def test_one_hot_rows_give_the_weights_exactly(ext, oracle):
+    from any_precision_amd import _capi
+    N, K = 70, 2080 + 512
+    L = make(N, K, seed=5)
+    q, luts = layer_to_gpu(L)
+    ks = list(range(0, K, 37)) + [255, 256, 1023, 1024, 2047, 2048, K - 1, K - 32, K - 33]
+    x = torch.zeros((len(ks), K), dtype=torch.float16, device="cuda")
+    x[torch.arange(len(ks)), torch.tensor(ks)] = 1.0
+    for b in range(3, 9):
+        w = oracle.dequant_kbit(L.qweight, L.luts[b], b)
+        for tile in _tiles(b):
+            with _capi.tuning(gemm_block=2, gemm_block_tile=tile):
+                got = ext.gemm_kbit(x, q, luts[b], b)
+            assert_bit_exact(got.t().contiguous(), w[:, ks], f"one-hot b={b} tile={tile}")
+
+
+@pytest.mark.parametrize("K", (1024, 1056))
+def test_what_is_not_a_number_stays_in_its_row(ext, K):
+    """NaN and infinities in one activation row, an infinite table entry that no weight of the row uses."""
+    from any_precision_amd import _capi
+    N, M = 40, 70
+    for b in (3, 4, 5, 8):
+        q, luts = layer_to_gpu(make(N, K, seed=b))
+        x = torch.randn((M, K), device="cuda").half()
+        x[5, 3], x[M - 1, K - 1] = float("nan"), float("inf")
+        table = luts[b].clone()
+        # row 7 uses one code only (all planes 0): the others are infinite
+        q[:, 7] = 0
+        table[7, 1:] = float("inf")
+        w = ext.dequant_kbit(q, table, b)
+        for tile in _tiles(b):
+            with _capi.tuning(gemm_block=2, gemm_block_tile=tile):
+                got = ext.gemm_kbit(x, q, table, b)
+            clean = [m for m in range(M) if m not in (5, M - 1)]
+            assert torch.isfinite(got[clean]).all(), (K, b, tile)
+            want = x[clean].float() @ w.float().t()
+            assert (got[clean].float() - want).norm() <= 1e-3 * want.norm()      # fp16 results of fp32 sums
+            assert torch.isnan(got[5]).all() and not torch.isfinite(got[M - 1]).any()
+
+
+def test_sets_and_strided_results(ext):
+    """Linears that share x in one launch, dense and side by side, bit for bit what each alone gives; replayed from a graph."""
+    from any_precision_amd import _capi
+    Ns, K, M = (200, 64, 72, 129), 1280, 100
+    for b in (3, 4, 6, 8):
+        gpu = [layer_to_gpu(make(N, K, seed=N)) for N in Ns]
+        qs, ts = [q for q, _ in gpu], [luts[b] for _, luts in gpu]
+        x = torch.randn((M, K), device="cuda").half()
+        for tile in _tiles(b):
+            with _capi.tuning(gemm_block=2, gemm_block_tile=tile):
+                singles = [ext.gemm_kbit(x, q, t, b) for q, t in zip(qs, ts)]
+                outs = ext.gemm_kbit_group(x, qs, ts, b)
+                joint = ext.gemm_kbit_group(x, qs, ts, b, concat=True)
+                torch.cuda.synchronize()
+                g = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(g):
+                    replayed = ext.gemm_kbit_group(x, qs, ts, b, concat=True)
+            assert all(torch.equal(s, o) for s, o in zip(singles, outs)), (b, tile)
+            assert torch.equal(joint, torch.cat(singles, dim=-1)), (b, tile)
+            for _ in range(3):
+                replayed.zero_()
+                torch.cuda.synchronize()
+                g.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(replayed, joint), (b, tile)
+
+
+def test_linear_takes_it_for_plain_forwards_and_stays_differentiable(ext):
+    """At 600 rows and 5 bits a 1024-row linear goes through the block-tile kernel; where gradients, tangents or batching follow the
+    call it goes through torch's product as before."""
+    from any_precision_amd import AnyPrecisionLinear, _capi
+    N, K, M, b = 1024, 512, 600, 5
+    assert not _capi.gemm_pays(M, N, K, b) and _capi.lib.ap_gemm_kbit_taken(M, N, K, b) == 1
+    lin = AnyPrecisionLinear(K, N, list(range(3, 9)), bias=False, device="cuda", dtype=torch.float16)
+    q, luts = layer_to_gpu(make(N, K, seed=1))
+    lin.qweight.copy_(q)
+    for i, t in luts.items():
+        lin._buffers[f"lut{i}"].copy_(t)
+    x = torch.randn((M, K), device="cuda").half()
+    w = ext.dequant_kbit(q, luts[b], b)
+    y = lin(x, precision=b)
+    assert torch.equal(y, ext.gemm_kbit(x, q, luts[b], b))
+    leaf = x.clone().requires_grad_()
+    out = lin(leaf, precision=b)
+    out.backward(torch.ones_like(out))
+    want = w.float().sum(0)
+    assert (leaf.grad.float() - want).norm() <= 1e-2 * want.norm() * M ** 0.5
+    with torch.no_grad():
+        assert torch.equal(lin(leaf, precision=b), y)
+    tangent = torch.func.jvp(lambda a: lin(a, precision=b), (x,), (x,))[1]
+    assert (tangent.float() - y.float()).norm() <= 1e-2 * y.float().norm()
+    batched = torch.func.vmap(lambda a: lin(a, precision=b))(x.view(1, M, K))
+    assert (batched.float().view(M, N) - y.float()).norm() <= 1e-2 * y.float().norm()
+
+
+def test_the_rule_keeps_to_its_range():
+    """No GPU is asked: where ap_gemm_kbit_taken says yes beyond ap_gemm_kbit_pays."""
+    from any_precision_amd import _capi
+    taken = _capi.lib.ap_gemm_kbit_taken
+    assert taken(512, 14336, 4096, 5) == 1 and taken(1024, 14336, 4096, 5) == 0 and taken(1024, 4096, 14336, 5) == 1
+    assert taken(2048, 4096, 4096, 3) == 1 and taken(2049, 4096, 4096, 3) == 0 and taken(512, 512, 4096, 5) == 0
+    assert taken(256, 4096, 224, 5) == _capi.lib.ap_gemm_kbit_pays(256, 4096, 224, 5)     # shorter than a half-step
+    assert taken(512, 4096, 4100, 5) == _capi.AP_ESHAPE and taken(0, 4096, 4096, 5) == _capi.AP_EBATCH
+    with _capi.tuning(gemm_block=0):
+        assert taken(512, 14336, 4096, 5) == 0
