@@ -705,9 +705,10 @@ bool gemmb_beats_pair(int M, long long N, int K, int b) {
     return b <= 6 || (b == 7 && N >= 4096 && K >= 4096);
 }
 
-// Launch of the fused dequant -> MFMA kernel (arguments already checked).
-int run_gemm(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, uint16_t *out, int M, int N, int K,
-             int w_bits, hipStream_t st) {
+// Launch of the fused dequant -> MFMA kernel (arguments already checked).  *added: whether the launch has added `bias` (of N, or null) to its
+// results; what is left as it is -- the row-walking kernel, several launches -- is the caller's to add.
+int run_gemm(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, const uint16_t *bias, uint16_t *out, int M, int N, int K,
+             int w_bits, hipStream_t st, bool *added) {
     // the kernels address the activations, and a row inside a plane, with 32-bit byte offsets
     if ((long long)M * K * 2 > 0xffffffffLL || (long long)N * (K >> 5) * 4 > 0xffffffffLL) return AP_ELIMIT;
     {
@@ -756,8 +757,8 @@ int run_gemm(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, ui
         // the two-block variant exists for up to 32 activation rows: more go in chunks of 32 (the
         // planes are re-read per chunk, which still costs less than one launch of the one-block variant)
         for (int m0 = 0; m0 < M; m0 += 32) {
-            const int r = run_gemm(x + (size_t)m0 * K, qweight, lut, out + (size_t)m0 * N, M - m0 < 32 ? M - m0 : 32, N, K,
-                                   w_bits, st);
+            const int r = run_gemm(x + (size_t)m0 * K, qweight, lut, nullptr, out + (size_t)m0 * N, M - m0 < 32 ? M - m0 : 32, N, K,
+                                   w_bits, st, added);
             if (r != AP_OK) return r;
         }
         return AP_OK;
@@ -778,13 +779,14 @@ int run_gemm(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, ui
     const bool la_fits = geo.rb == 1 && geo.mb <= 2 && (W & 3) == 0;
     const bool la_pays = geo.grid <= cu_count() && !(w_bits == 8 && geo.mb == 1 && steps <= ks);
     geo.lookahead = la_fits && (la_mode >= 2 || (la_mode == 1 && la_pays)) ? 1 : 0;
+    *added = bias != nullptr;
     switch (w_bits) {
-        case 3: launch_gemm<3>(geo, x, qweight, lut, out, M, N, K, st); break;
-        case 4: launch_gemm<4>(geo, x, qweight, lut, out, M, N, K, st); break;
-        case 5: launch_gemm<5>(geo, x, qweight, lut, out, M, N, K, st); break;
-        case 6: launch_gemm<6>(geo, x, qweight, lut, out, M, N, K, st); break;
-        case 7: launch_gemm<7>(geo, x, qweight, lut, out, M, N, K, st); break;
-        default: launch_gemm<8>(geo, x, qweight, lut, out, M, N, K, st); break;
+        case 3: launch_gemm<3>(geo, x, qweight, lut, bias, out, M, N, K, st); break;
+        case 4: launch_gemm<4>(geo, x, qweight, lut, bias, out, M, N, K, st); break;
+        case 5: launch_gemm<5>(geo, x, qweight, lut, bias, out, M, N, K, st); break;
+        case 6: launch_gemm<6>(geo, x, qweight, lut, bias, out, M, N, K, st); break;
+        case 7: launch_gemm<7>(geo, x, qweight, lut, bias, out, M, N, K, st); break;
+        default: launch_gemm<8>(geo, x, qweight, lut, bias, out, M, N, K, st); break;
     }
     return launch_status();
 }
@@ -1111,6 +1113,9 @@ bool fused_set_pays(int M, const int *N, int count, int K, int b) {
 
 extern "C" {
 
+static int matmul_set(const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut, const uint16_t *bias,
+                      uint16_t *const *out, const int *N, int M, int K, int w_bits, void *stream, bool *added);
+
 int ap_matmul_kbit_swiglu(const uint16_t *x, const uint32_t *qweight_gate, const uint16_t *lut_gate,
                           const uint32_t *qweight_up, const uint16_t *lut_up, uint16_t *out, int M, int N, int K, int w_bits,
                           void *stream) {
@@ -1182,8 +1187,9 @@ bool takes_gemmb(int M, long long N, int K, int w_bits) {
 
 // One launch of the block-tile kernel over `count` linears (arguments already checked; geo from gemmb_geometry over all of them).
 int run_gemmb(const GemmbGeometry &geo, const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut,
-              uint16_t *const *out, const int *N, const long long *ldo, int M, int K, int w_bits, hipStream_t st) {
+              const uint16_t *bias, uint16_t *const *out, const int *N, const long long *ldo, int M, int K, int w_bits, hipStream_t st) {
     GemmbMembers mem = {};
+    mem.bias = bias;
     mem.count = count;
     for (int g = 0; g < count; g++) {
         mem.qweight[g] = qweight[g];
@@ -1205,8 +1211,8 @@ int run_gemmb(const GemmbGeometry &geo, const uint16_t *x, int count, const uint
     return ok ? launch_status() : AP_ELIMIT;
 }
 
-int ap_gemm_kbit(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, uint16_t *out, int M, int N, int K,
-                 int w_bits, void *stream) {
+static int gemm_one(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, const uint16_t *bias, uint16_t *out, int M, int N, int K,
+                    int w_bits, void *stream, bool *added) {
     if (!x || !qweight || !lut || !out) return AP_ENULL;
     const int rc = check_common(N, K, w_bits);
     if (rc != AP_OK) return rc;
@@ -1215,8 +1221,10 @@ int ap_gemm_kbit(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut
     drain_stale_error();
     {
         GemmbGeometry bgeo;
-        if (takes_gemmb(M, N, K, w_bits) && gemmb_geometry(M, &N, 1, K, w_bits, &bgeo))
-            return run_gemmb(bgeo, x, 1, &qweight, &lut, &out, &N, nullptr, M, K, w_bits, static_cast<hipStream_t>(stream));
+        if (takes_gemmb(M, N, K, w_bits) && gemmb_geometry(M, &N, 1, K, w_bits, &bgeo)) {
+            *added = bias != nullptr;
+            return run_gemmb(bgeo, x, 1, &qweight, &lut, bias, &out, &N, nullptr, M, K, w_bits, static_cast<hipStream_t>(stream));
+        }
         GemmtGeometry tgeo;
         const int mode = knob(kGemmTiled);
         if (mode > 0 && gemmt_geometry(M, (N + 63) / 64, K, w_bits, &tgeo) && (mode >= 2 || gemmt_pays(M, N, K, w_bits)))
@@ -1226,11 +1234,27 @@ int ap_gemm_kbit(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut
     // are re-read per chunk; row offsets of 128 rows keep x and out 16-byte aligned for every K and N that passed)
     for (int m0 = 0; m0 < M; m0 += kGemmMaxM) {
         const int rows = M - m0 < kGemmMaxM ? M - m0 : kGemmMaxM;
-        const int r = run_gemm(x + (size_t)m0 * K, qweight, lut, out + (size_t)m0 * N, rows, N, K, w_bits,
-                               static_cast<hipStream_t>(stream));
+        const int r = run_gemm(x + (size_t)m0 * K, qweight, lut, M <= kGemmMaxM ? bias : nullptr, out + (size_t)m0 * N, rows, N, K, w_bits,
+                               static_cast<hipStream_t>(stream), added);
         if (r != AP_OK) return r;
     }
     return AP_OK;
+}
+
+int ap_gemm_kbit(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, uint16_t *out, int M, int N, int K,
+                 int w_bits, void *stream) {
+    bool added = false;
+    return gemm_one(x, qweight, lut, nullptr, out, M, N, K, w_bits, stream, &added);
+}
+
+int ap_linear_bias(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, const uint16_t *bias, uint16_t *out, int M, int N, int K,
+                   int w_bits, void *stream, int *added) {
+    if (!bias || !added) return AP_ENULL;
+    bool with = false;
+    const int rc = M <= 8 ? matmul_set(x, 1, &qweight, &lut, bias, &out, &N, M, K, w_bits, stream, &with)
+                          : gemm_one(x, qweight, lut, bias, out, M, N, K, w_bits, stream, &with);
+    *added = with ? 1 : 0;
+    return rc;
 }
 
 int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut,
@@ -1269,7 +1293,7 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
     // served dense only.)
     GemmbGeometry bgeo;
     if ((count > 1 || strided) && (!strided || (K & 127) == 0) && takes_gemmb(M, total, K, w_bits) && gemmb_geometry(M, N, count, K, w_bits, &bgeo))
-        return run_gemmb(bgeo, x, count, qweight, lut, out, N, ldo, M, K, w_bits, static_cast<hipStream_t>(stream));
+        return run_gemmb(bgeo, x, count, qweight, lut, nullptr, out, N, ldo, M, K, w_bits, static_cast<hipStream_t>(stream));
     if (fits && (strided || (count > 1 && mode > 0 && (mode >= 2 || pays))))
         return run_gemmt(tgeo, x, count, qweight, lut, out, N, ldo, M, K, w_bits, static_cast<hipStream_t>(stream));
     // only the tiled kernel writes rows that are not dense: rows it cannot walk at all are a shape error, a size or a
@@ -1289,6 +1313,13 @@ int ap_matmul_kbit(const uint16_t *x, const uint32_t *qweight, const uint16_t *l
 
 int ap_matmul_kbit_group(const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut,
                          uint16_t *const *out, const int *N, int M, int K, int w_bits, void *stream) {
+    bool added = false;
+    return matmul_set(x, count, qweight, lut, nullptr, out, N, M, K, w_bits, stream, &added);
+}
+
+// bias: of the only linear (count = 1), or null.  *added: whether the launch has added it.
+static int matmul_set(const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut, const uint16_t *bias,
+                      uint16_t *const *out, const int *N, int M, int K, int w_bits, void *stream, bool *added) {
     if (!x || !qweight || !lut || !out || !N) return AP_ENULL;
     if (count < 1 || count > kGemvMaxGroup) return AP_ELIMIT;
     for (int g = 0; g < count; g++)
@@ -1317,6 +1348,8 @@ int ap_matmul_kbit_group(const uint16_t *x, int count, const uint32_t *const *qw
         return AP_OK;
     }
     if (one_launch) {  // the whole set in one launch
+        mem.bias = bias;
+        *added = bias != nullptr;
         switch (w_bits) {
             case 3: launch_gemv<3>(M, geo, x, mem, K, st); break;
             case 4: launch_gemv<4>(M, geo, x, mem, K, st); break;
@@ -1333,7 +1366,7 @@ int ap_matmul_kbit_group(const uint16_t *x, int count, const uint32_t *const *qw
             case AP_ROUTE_STREAM: r = run_gemvp(x, qweight[g], lut[g], out[g], M, N[g], K, w_bits, st); break;
             case AP_ROUTE_FINE: r = run_gemvf(x, qweight[g], lut[g], out[g], M, N[g], K, w_bits, st); break;
             case AP_ROUTE_MFMA4: r = run_gemv4(x, qweight[g], lut[g], out[g], M, N[g], K, w_bits, st); break;
-            default: r = run_gemm(x, qweight[g], lut[g], out[g], M, N[g], K, w_bits, st); break;
+            default: r = run_gemm(x, qweight[g], lut[g], bias, out[g], M, N[g], K, w_bits, st, added); break;
         }
         if (r != AP_OK) return r;
     }

@@ -580,6 +580,7 @@ __global__ __launch_bounds__(WN *WK *kWave) void gemmb_kbit_kernel(const half_t 
             for (int i = 0; i < PART; i += 4) finish4(own * PART + i, sum[i / 4]);
         });
     }
+    const global_ptr<const half_t> bias = (global_ptr<const half_t>)reinterpret_cast<uint64_t>(mem.bias);
     const bool wide = (ldo & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
 #pragma unroll
     for (int pass = 0; pass < PASSES; pass++) {
@@ -597,8 +598,11 @@ __global__ __launch_bounds__(WN *WK *kWave) void gemmb_kbit_kernel(const half_t 
             const int at = i * (WN * WK * kWave) + wave * kWave + lane, r = at / UNITS, u = at % UNITS;
             if (at >= PM * UNITS) break;
             const int m = m0 + pass * PM + r, n = nb + 8 * u;
-            const half8_t v = *reinterpret_cast<const half8_t *>(tile + (r * UNITS + (u ^ (r & (UNITS - 1)))) * 16);
+            half8_t v = *reinterpret_cast<const half8_t *>(tile + (r * UNITS + (u ^ (r & (UNITS - 1)))) * 16);
             if (m >= M) continue;
+            if (bias != nullptr)  // as on the finished result
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[e] = (half_t)((float)v[e] + (float)bias[min(n + e, N - 1)]);
             half_t *o = out + (size_t)m * ldo + n;
             if (wide && n + 7 < N) {
                 *reinterpret_cast<half8_t *>(o) = v;

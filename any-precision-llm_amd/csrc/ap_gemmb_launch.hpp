@@ -28,6 +28,7 @@ struct GemmbMembers {
     int tile0[kGemmbMaxGroup + 1];
     int count;
     long long ldo[kGemmbMaxGroup];
+    const uint16_t *bias;  // of member 0, the only one then; null: none
 };
 
 // Launches gemmb_kbit_kernel<BITS, geo.mb, geo.wn, geo.wk> on `stream`; false if there is no such kernel.

@@ -19,6 +19,7 @@ struct GemvMembers {
     int n[kGemvMaxGroup];       // rows
     int wg_end[kGemvMaxGroup];  // first workgroup past the member
     int count;
+    const uint16_t *bias;       // of member 0, the only one then; null: none
 };
 
 struct GemvGeometry {

@@ -236,23 +236,29 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (torch_op && (at::impl::torch_function_mode_enabled() || !exact_tensor(args[1]) || (m.bias != nullptr && !exact_tensor(m.bias))))
             return none();
         const char *op = rows <= 8 ? "matmul_kbit" : "gemm_kbit";
+        // a bias that is N plain numbers, with nothing that follows the sum as an operation of its own, goes along in the launch
+        const at::Device device = x.device();
+        const bool fused_bias = pays && bias.defined() && bias.dim() == 1 && bias.size(0) == w.N && plain_execution() && plain_half(m.bias, &device);
         Tensor out;
-        int rc;
+        int rc, added = 0;
         {
             const WithoutGil free;
             const OnDevice on(w.device);
             if (pays) {
                 const Tensor dense = x.is_contiguous() ? x : x.contiguous();  // the kernels take dense rows
                 out = result_for(x, w.N);
-                rc = rows <= 8 ? ap_matmul_kbit(half_ptr(dense), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream)
-                               : ap_gemm_kbit(half_ptr(dense), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream);
+                if (fused_bias)
+                    rc = ap_linear_bias(half_ptr(dense), w.planes, w.lut, half_ptr(bias), half_out(out), (int)rows, w.N, w.K, bits, on.stream, &added);
+                else
+                    rc = rows <= 8 ? ap_matmul_kbit(half_ptr(dense), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream)
+                                   : ap_gemm_kbit(half_ptr(dense), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream);
             } else {
                 op = "dequant_kbit";
                 const Tensor dense = empty_half({w.N, w.K}, x.device());
                 rc = ap_dequant_kbit(w.planes, w.lut, half_out(dense), w.N, w.K, bits, on.stream);
                 if (rc == AP_OK) out = at::matmul(x, dense.t());
             }
-            if (rc == AP_OK && bias.defined()) out.add_(bias);
+            if (rc == AP_OK && bias.defined() && !added) out.add_(bias);
         }
         if (rc != AP_OK) return library_error(rc, op);
         return wrap(std::move(out));

@@ -123,6 +123,12 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
                        const uint16_t *const *lut, uint16_t *const *out, const int *N,
                        const long long *ldo, int M, int K, int w_bits, void *stream);
 
+/* A linear with a bias (fp16 [N]): ap_matmul_kbit up to 8 activation rows, ap_gemm_kbit beyond, the bias added to the fp16 results in
+ * the same launch where the kernel that serves the call can (*added = 1); else the results are left without it (*added = 0) and adding
+ * it is the caller's.  Same value either way: fp16(fp16(sum) + bias). */
+int ap_linear_bias(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, const uint16_t *bias, uint16_t *out,
+                   int M, int N, int K, int w_bits, void *stream, int *added);
+
 /* Where the fused GEMM is the faster way to compute x . dequant(W)^T, from this library's measurements on
  * MI355X: ap_gemm_kbit_pays returns 1 if ap_gemm_kbit beats ap_dequant_kbit + a library fp16 GEMM for M
  * activation rows on an [N, K] linear at w_bits, 0 if the pair wins (the reference always takes the pair

@@ -316,3 +316,28 @@ def test_a_mode_sees_the_results_of_a_set_joined(rows, K):
     with Watching():
         got = forward_group((m, m), x, 4, concat=True)
     assert torch.equal(got, want) and ("cat" in seen) == (rows > 1)
+
+
+@pytest.mark.parametrize("N,K", ((1999, 2720), (7, 32), (64, 4096), (1024, 4096), (4096, 11008), (33, 40000)))
+def test_a_bias_in_the_launch_is_the_bias_added_afterwards(N, K):
+    """Every kernel that takes the bias along, and those that leave it: bit for bit the sum of the bias-free result and the bias."""
+    from any_precision_amd import AnyPrecisionLinear, _capi
+    lin = AnyPrecisionLinear(K, N, [3, 5, 8], bias=True, device="cuda", dtype=torch.float16)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    lin.qweight.copy_(torch.randint(-2**31, 2**31, lin.qweight.shape, dtype=torch.int32, device="cuda", generator=g))
+    for b in (3, 5, 8):
+        lin._buffers[f"lut{b}"].copy_(torch.randn((N, 1 << b), device="cuda", generator=g) * 0.02)
+    bias = (torch.randn(N, device="cuda", generator=g) * 4).half()
+    bias[0], bias[N - 1] = float("inf"), 60000.0
+    lin.bias.copy_(bias)
+    for M in (1, 2, 3, 5, 8, 9, 16, 31, 40, 100, 200):
+        x = torch.randn((M, K), device="cuda", generator=g).half()
+        for b in (3, 5, 8):
+            print(f"bias N={N} K={K} M={M} b={b}", flush=True)
+            got = lin(x, precision=b)
+            lin.bias = None
+            want = lin(x, precision=b)
+            del lin.bias
+            lin.register_buffer("bias", bias.clone())
+            assert torch.equal(got, want + bias), (N, K, M, b)
+    assert _capi.lib.ap_linear_bias(None, None, None, None, None, 1, 8, 32, 3, None, None) == _capi.AP_ENULL
