@@ -614,27 +614,27 @@ constexpr int kGemmbTileCount = sizeof(kGemmbTiles) / sizeof(kGemmbTiles[0]);
 // 256 elements that a group walks and u = the share of the CUs that has a tile (up to 1: the more there are, the slower each runs).
 // {a, p, s, f} per bit-width and tile of the list above, least squares over 15 linear shapes (1024 x 4096 .. 22016 x 4096, 4096 x
 // 14336, 8192 x 8192; rows of 2048 .. 14336 elements, one of no multiple of 128) x 14 numbers of activation rows (16 .. 2048), planes
-// from HBM, 2500 launches a bit-width.  The tile it picks is within 0.2 % of the fastest on average, 17 % at worst.  (0 0 0 0: the
+// from HBM, 2500 launches a bit-width.  The tile it picks is within 0.1 % of the fastest on average, 8 % at worst.  (0 0 0 0: the
 // tables of that tile and bit-width do not fit the LDS.)
 constexpr float kGemmbCost[6][kGemmbTileCount][4] = {
-    {{-1.66f, 7.89f, 2.38f, 1.05f}, {1.60f, 4.50f, 2.36f, 0.75f}, {3.25f, 2.18f, 2.96f, 1.20f},
-     {2.23f, 4.38f, 2.62f, 1.21f}, {2.82f, 2.88f, 3.45f, 1.55f}, {2.14f, 3.39f, 2.07f, 0.52f},
-     {3.74f, 2.18f, 2.31f, 0.71f}, {4.04f, 1.94f, 3.18f, 1.24f}, {6.14f, -0.05f, 1.84f, 0.13f}},
-    {{-1.29f, 7.96f, 2.80f, 1.02f}, {1.55f, 4.78f, 3.22f, 0.66f}, {3.64f, 2.49f, 3.18f, 1.23f},
-     {2.73f, 4.27f, 3.44f, 1.17f}, {3.41f, 3.51f, 4.17f, 1.44f}, {2.38f, 3.55f, 2.93f, 0.47f},
-     {4.01f, 1.61f, 2.82f, 0.86f}, {4.03f, 2.75f, 3.95f, 1.12f}, {3.72f, 2.54f, 2.03f, 0.42f}},
-    {{-0.04f, 5.99f, 2.89f, 1.04f}, {1.49f, 4.55f, 3.50f, 0.60f}, {4.15f, 2.74f, 4.13f, 1.08f},
-     {2.92f, 3.47f, 3.74f, 1.12f}, {3.69f, 3.24f, 4.51f, 1.51f}, {2.87f, 2.79f, 3.21f, 0.44f},
-     {4.12f, 2.53f, 3.48f, 0.71f}, {4.30f, 3.07f, 4.21f, 1.25f}, {4.00f, 2.55f, 3.00f, 0.35f}},
-    {{-1.07f, 8.12f, 2.89f, 1.03f}, {2.28f, 5.15f, 3.58f, 0.64f}, {4.90f, 2.97f, 4.20f, 1.21f},
-     {3.68f, 3.93f, 3.80f, 1.14f}, {4.25f, 3.63f, 4.59f, 1.64f}, {3.18f, 3.92f, 3.32f, 0.41f},
-     {4.92f, 2.95f, 3.51f, 0.85f}, {4.56f, 3.48f, 4.39f, 1.28f}, {4.36f, 3.30f, 3.15f, 0.39f}},
-    {{-0.65f, 8.29f, 2.99f, 1.09f}, {2.46f, 5.73f, 3.81f, 0.58f}, {5.65f, 2.79f, 4.44f, 1.32f},
-     {4.36f, 3.88f, 4.09f, 1.12f}, {5.35f, 3.14f, 4.82f, 1.75f}, {3.45f, 4.25f, 3.60f, 0.34f},
-     {5.68f, 2.86f, 3.79f, 0.96f}, {4.72f, 3.82f, 4.62f, 1.40f}, {5.12f, 3.43f, 3.33f, 0.47f}},
-    {{6.00f, 0.63f, 3.58f, 1.19f}, {3.20f, 6.33f, 4.16f, 0.62f}, {5.87f, 3.34f, 4.82f, 1.39f},
-     {5.87f, 2.96f, 4.73f, 1.10f}, {0.f, 0.f, 0.f, 0.f}, {4.65f, 4.48f, 3.97f, 0.30f},
-     {6.34f, 2.30f, 4.49f, 1.18f}, {0.f, 0.f, 0.f, 0.f}, {5.38f, 4.42f, 3.61f, 0.54f}},
+    {{-3.41f, 10.35f, 2.23f, 0.87f}, {2.11f, 4.07f, 2.10f, 0.77f}, {3.46f, 1.32f, 2.89f, 1.19f},
+     {2.58f, 3.77f, 2.39f, 1.17f}, {3.36f, 1.70f, 3.35f, 1.53f}, {3.64f, 2.01f, 1.83f, 0.53f},
+     {4.06f, 1.87f, 2.03f, 0.76f}, {3.65f, 1.34f, 3.40f, 1.18f}, {6.07f, -0.02f, 1.63f, 0.17f}},
+    {{-3.58f, 10.22f, 2.70f, 0.83f}, {1.72f, 4.56f, 2.89f, 0.70f}, {3.62f, 1.76f, 3.08f, 1.29f},
+     {2.88f, 3.68f, 3.10f, 1.18f}, {3.91f, 2.23f, 3.78f, 1.53f}, {3.76f, 2.25f, 2.66f, 0.47f},
+     {4.04f, 0.99f, 2.73f, 0.95f}, {3.65f, 1.90f, 3.88f, 1.20f}, {3.56f, 2.71f, 1.80f, 0.44f}},
+    {{-2.41f, 8.42f, 2.83f, 0.88f}, {1.46f, 4.13f, 3.20f, 0.63f}, {4.34f, 2.08f, 3.74f, 1.14f},
+     {3.34f, 2.47f, 3.40f, 1.19f}, {4.34f, 2.02f, 4.11f, 1.61f}, {3.75f, 1.78f, 2.95f, 0.40f},
+     {4.23f, 2.21f, 3.14f, 0.72f}, {3.74f, 2.09f, 4.12f, 1.40f}, {4.14f, 2.27f, 2.74f, 0.35f}},
+    {{-1.84f, 8.82f, 2.83f, 0.92f}, {2.02f, 4.76f, 3.28f, 0.68f}, {5.07f, 2.43f, 3.77f, 1.29f},
+     {3.77f, 3.17f, 3.48f, 1.23f}, {5.22f, 2.17f, 4.08f, 1.85f}, {4.21f, 2.49f, 3.02f, 0.46f},
+     {4.85f, 2.72f, 3.15f, 0.88f}, {3.69f, 2.87f, 4.24f, 1.42f}, {4.21f, 3.33f, 2.85f, 0.43f}},
+    {{-0.95f, 7.99f, 2.89f, 0.97f}, {2.08f, 5.41f, 3.56f, 0.63f}, {5.64f, 2.55f, 3.97f, 1.42f},
+     {4.12f, 3.31f, 3.78f, 1.21f}, {5.82f, 2.22f, 4.30f, 1.96f}, {4.44f, 2.90f, 3.32f, 0.41f},
+     {5.49f, 2.83f, 3.41f, 0.99f}, {3.80f, 3.02f, 4.61f, 1.49f}, {4.73f, 3.42f, 3.09f, 0.50f}},
+    {{2.23f, 5.05f, 3.22f, 1.05f}, {3.22f, 6.08f, 3.76f, 0.70f}, {6.07f, 3.13f, 4.21f, 1.56f},
+     {5.35f, 3.27f, 4.19f, 1.23f}, {0.f, 0.f, 0.f, 0.f}, {4.99f, 3.99f, 3.53f, 0.43f},
+     {5.99f, 2.62f, 3.93f, 1.21f}, {0.f, 0.f, 0.f, 0.f}, {4.97f, 4.48f, 3.26f, 0.58f}},
 };
 
 // The fastest tile for linears that share x; false if the kernel does not serve the shape.

@@ -65,6 +65,7 @@ struct GemmbLoads {
     static constexpr int kOctets = 2 * kSync;                    // octets that they are spread over: half of what a meeting lies ahead
     static constexpr int kPieces = (kSync * kDirect + kOctets - 1) / kOctets;
     static constexpr int kLast = (kSync * kDirect - 1) / kPieces;  // octets from the first to the last of them
+    static_assert(kPieces < 16, "");
     static constexpr int kPlanes = 14 - 2 * BITS;                // the last two words of the planes before are done with by octet 30
     // Loads that were requested after the last of the direct loads that this meeting (before octet 4 s + 3) waits for.  Loads
     // complete in order: waiting until no more than these are outstanding means that the direct loads have landed.  Plane loads
@@ -211,6 +212,9 @@ __global__ __launch_bounds__(WN *WK *kWave) void gemmb_kbit_kernel(const half_t 
 #pragma unroll
         for (int i = 0; i < ND; i++) {
             if (i < first || i >= last) continue;
+            // scalar base + 32-bit lane offset in the load itself: extended to 64 bits ahead of the loop, as the optimiser would have it, the
+            // offsets take twice the registers and every load a 64-bit vector add
+            asm volatile("" : "+v"(xoff[i]));
             const char *src = (const char *)(base + xoff[i]);
             if constexpr (CHECK) src = w0 + xunit[i] < W ? src : reinterpret_cast<const char *>(kGemmbZeros) + 16 * (lane & 7);
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src, (__attribute__((address_space(3))) void *)&xt[kh][8 * (wn + WN * i)][0], 16, 0, 0);
@@ -293,19 +297,6 @@ __global__ __launch_bounds__(WN *WK *kWave) void gemmb_kbit_kernel(const half_t 
         });
     };
 
-    // Workgroups walk K side by side, so that without more every stage would come to each XCD's L2 as a miss to the cache behind it,
-    // 2000 cycles: the workgroups of an XCD (round robin over eight) touch the lines of x together first, as far as L2 has room.
-    constexpr int NT = 2;
-    uint32_t touched[NT] = {};
-    const uint32_t x_bytes = (uint32_t)M * (uint32_t)K * 2u;
-    const bool touch = x_bytes <= 2u << 20;
-    if (touch)
-#pragma unroll
-        for (int i = 0; i < NT; i++) {
-            const uint32_t at = ((((uint32_t)i * ((gridDim.x + 7u) >> 3) + (blockIdx.x >> 3)) * (uint32_t)(WN * WK) + (uint32_t)wave) * 64u + (uint32_t)lane) * 128u;
-            touched[i] = *(global_ptr<const uint32_t>)(xg + min(at, x_bytes - 4u));
-        }
-
     // the planes were requested first: their index arithmetic while the tables and the activations are on their way
     __builtin_amdgcn_sched_barrier(0);
     {
@@ -375,8 +366,6 @@ __global__ __launch_bounds__(WN *WK *kWave) void gemmb_kbit_kernel(const half_t 
     }
     __builtin_amdgcn_s_waitcnt(0x0070);
     __syncthreads();
-#pragma unroll
-    for (int i = 0; i < NT; i++) asm volatile("" ::"v"(touched[i]));  // (nothing but to have them loaded)
 
     typedef __attribute__((address_space(3))) uint16_t lds_u16_t;
     typedef __attribute__((address_space(3))) uint32_t lds_u32_t;
@@ -422,8 +411,10 @@ __global__ __launch_bounds__(WN *WK *kWave) void gemmb_kbit_kernel(const half_t 
         return __builtin_bit_cast(half8_t, bw);
     };
     // One half-step: four stages (byte group j of its 8 words) of four octets (word wi of a lane's quad).
-    auto run_half = [&](auto check_c, auto half_c, int hs) {
-        constexpr bool CHECK = decltype(check_c)::value;
+    // NEXT: a half-step follows, so that planes are requested and indices made for it.  (The counts of loads in flight depend on it: without a
+    // use for them the compiler drops the plane loads.)
+    auto run_half = [&](auto check_c, auto next_c, auto half_c, int hs) {
+        constexpr bool CHECK = decltype(check_c)::value, NEXT = decltype(next_c)::value;
         constexpr int half = decltype(half_c)::value;
         bool live[4];
 #pragma unroll
@@ -434,10 +425,16 @@ __global__ __launch_bounds__(WN *WK *kWave) void gemmb_kbit_kernel(const half_t 
             if constexpr (wi == 3 && (j + 1) % SYNC == 0) {
                 // Every read of these stages has been requested.  When they are done in every wave the buffers can be refilled;
                 // and the next stages have landed (GemmbLoads::outstanding).
-                constexpr int keep = Loads::outstanding(4 * half + j, !CHECK);
+                constexpr int keep = Loads::outstanding(4 * half + j, NEXT);
                 static_assert(keep < 64, "");
                 __builtin_amdgcn_s_waitcnt(0x0070 | (keep & 15) | ((keep >> 4) << 14));
                 __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (NEXT && half == 1 && t == 0) {
+                // The planes of the next step are used from here on; what was requested after them, in the octet before, stays
+                // outstanding.  (Without this the compiler waits for every load: it does not count across direct loads.)
+                __builtin_amdgcn_s_waitcnt(0x0f70 | (Loads::kPieces & 15));
                 __builtin_amdgcn_sched_barrier(0);
             }
             const half8_t w = finish_b(check_c, raw[cur], live[wi]);
@@ -461,7 +458,7 @@ __global__ __launch_bounds__(WN *WK *kWave) void gemmb_kbit_kernel(const half_t 
                         if constexpr (i < SYNC && decltype(p_c)::value * MB / Loads::kPieces == m)
                             stage_dma(check_c, hs + st / 4, st % 4, std::integral_constant<int, st % NBUF>{}, load % ND, load % ND + 1);
                     });
-                if constexpr (!CHECK) {
+                if constexpr (NEXT) {
                     static_for<4>([&](auto part_c) {
                         if constexpr (decltype(part_c)::value * MB / 4 == m)
                             convert(std::integral_constant<int, half ^ 1>{}, std::integral_constant<int, j>{}, std::integral_constant<int, wi>{}, part_c);
@@ -486,11 +483,14 @@ __global__ __launch_bounds__(WN *WK *kWave) void gemmb_kbit_kernel(const half_t 
         for (int i = 0; i < 4 / Loads::kSync; i++) __builtin_amdgcn_s_barrier();
     };
     first_reads();
-    for (int hs = hs0; hs < hs_end; hs++) {
-        run_half(std::false_type{}, std::integral_constant<int, 0>{}, hs);
-        if (++hs >= hs_end) break;
-        run_half(std::false_type{}, std::integral_constant<int, 1>{}, hs);
+    // (an odd half-step runs a copy of its own: left through the middle, the loop has an edge on which plane loads are pending, and the
+    // compiler waits for every load at its head)
+    int hs = hs0;
+    for (; hs + 1 < hs_end; hs += 2) {
+        run_half(std::false_type{}, std::true_type{}, std::integral_constant<int, 0>{}, hs);
+        run_half(std::false_type{}, std::true_type{}, std::integral_constant<int, 1>{}, hs + 1);
     }
+    if (hs < hs_end) run_half(std::false_type{}, std::false_type{}, std::integral_constant<int, 0>{}, hs);
     if (own < most) idle_half();
     if (W & 7) {
         __builtin_amdgcn_s_waitcnt(0x0070);
@@ -507,7 +507,7 @@ __global__ __launch_bounds__(WN *WK *kWave) void gemmb_kbit_kernel(const half_t 
         __syncthreads();
         if (kh == 0) {
             first_reads();
-            run_half(std::true_type{}, std::integral_constant<int, 0>{}, H_full);
+            run_half(std::true_type{}, std::false_type{}, std::integral_constant<int, 0>{}, H_full);
         } else {
             idle_half();
         }
