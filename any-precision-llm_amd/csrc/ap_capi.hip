@@ -672,12 +672,16 @@ bool gemmb_geometry(int M, const int *N, int count, int K, int w_bits, GemmbGeom
 // rows on linears of 5120 rows or more (6144 x 4096, 48 rows, 5 bits: 27 / 17), on narrower ones where the 16-row tiles of the tiled kernel
 // wait for their lookups: 5 to 7 bits beyond 48 rows, or on rows of more than 4096 elements; 8 bits on both (4096 x 4096,
 // 48 rows: 18 / 23).  Rows of no multiple of 128 elements, which the tiled kernel does not take: on linears of less than
-// 5120 rows up to 4 bits from 33 activation rows on, else from 65 (4096 x 11040, 128 rows: 98 / 35 at 3 bits, 104 / 60 at 8).  Sets of
-// more than 20000 rows from 17 (22016 x 4096 at 32 rows: 31 / 23, 65 / 49).
+// 5120 rows up to 4 bits from 33 activation rows on, else from 65 (4096 x 11040, 128 rows: 98 / 35 at 3 bits, 104 / 60 at 8).  From 17
+// rows on linears and sets of 10240 rows or more (22016 x 4096, 24 rows, 4 bits: 41 / 30; 12288 x 4096: 17.9 / 15.9; 10240 x 8192, 5 bits:
+// 52 / 32; 14336 x 4096 at 6 bits a tie, 26.9 / 26.6; 8192 x 8192 up to 6 bits and 4096 x 11008 lose, 29.4 / 30.8 and 24 / 25), of 20000 on
+// shorter rows; from 9 where these have 8192 elements or more (10240 x 8192, 16 rows: 28 / 22, 43 / 32, 61 / 42; 28672 x 8192: 50 / 40 and
+// 124 / 96, at 4 bits 54 / 55 at 9 rows); 4096 elements are not enough there (22016 x 4096, 4 bits: 25 / 30).
 bool gemmb_pays(int M, long long N, int K, int b) {
-    if (N < 1024 || M <= 16 || K < 256) return false;
+    if (N < 1024 || M <= 8 || K < 256) return false;
     if ((long long)M * K * 2 > 0xffffffffLL || N * (K >> 5) * 4 > 0xffffffffLL) return false;  // its 32-bit offsets
-    if (M <= 32) return N >= 20000;
+    if (M <= 16) return N >= 10240 && K >= 8192 && (K & 127) == 0 && (b != 4 || N < 20000);
+    if (M <= 32) return N >= (K >= 4096 ? 10240 : 20000);
     if (M <= 64) {
         if (N >= 5120) return true;
         if ((K & 127) != 0) return b <= 4;
@@ -1185,6 +1189,19 @@ bool takes_gemmb(int M, long long N, int K, int w_bits) {
     return mode >= 2 || (mode > 0 && knob(kGemmTiled) == 1 && gemmb_pays(M, N, K, w_bits));
 }
 
+// The same for one launch over a set of `total` rows, `largest` in one member.  At 9..16 rows members of more than 8192 rows (gate/up), which
+// would otherwise run one by one in the K-split kernel, take it where they have 20000 together and none more than two thirds of them
+// (9 rows / 16 rows, us one by one and here: 2 x 14336 x 4096 at 3 bits 27 / 25, 27 / 25, at 5 48 / 40, 47 / 40, at 8 63 / 58, 65 / 57;
+// 2 x 13824 x 5120 at 6 bits 57 / 53, 58 / 53) -- not at 4 bits on rows of less than 5120 elements (34 / 33, 32 / 33), at 5 and 6 bits below
+// 24000 rows only from 13 rows on (2 x 11008 x 4096, 5 bits: 34 / 36, 39 / 35), nor on rows of no multiple of 128 elements (62 / 67, 65 / 66).
+// The tiled kernel keeps sets of small members at 3 bits there (8192 + 2 x 1024 x 8192: 21.3 / 22.1).
+bool takes_gemmb_set(int M, long long total, long long largest, int K, int w_bits) {
+    if (M > 16 || largest <= 8192) return !(M <= 16 && w_bits == 3 && knob(kGemmBlock) == 1) && takes_gemmb(M, total, K, w_bits);
+    if (takes_gemmb(M, total, K, w_bits)) return true;
+    return knob(kGemmBlock) > 0 && knob(kGemmTiled) == 1 && M > 8 && K >= (w_bits == 4 ? 5120 : 4096) && (K & 127) == 0 &&
+           total >= (w_bits == 5 || w_bits == 6 ? (M > 12 ? 20000 : 24000) : 20000) && 3 * largest <= 2 * total;
+}
+
 // One launch of the block-tile kernel over `count` linears (arguments already checked; geo from gemmb_geometry over all of them).
 int run_gemmb(const GemmbGeometry &geo, const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut,
               const uint16_t *bias, uint16_t *const *out, const int *N, const long long *ldo, int M, int K, int w_bits, hipStream_t st) {
@@ -1292,7 +1309,7 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
     // The block-tile kernel takes the set by the rule for one linear of all its rows.  (Rows of no multiple of 128 elements are
     // served dense only.)
     GemmbGeometry bgeo;
-    if ((count > 1 || strided) && (!strided || (K & 127) == 0) && takes_gemmb(M, total, K, w_bits) && gemmb_geometry(M, N, count, K, w_bits, &bgeo))
+    if ((count > 1 || strided) && (!strided || (K & 127) == 0) && takes_gemmb_set(M, total, rows, K, w_bits) && gemmb_geometry(M, N, count, K, w_bits, &bgeo))
         return run_gemmb(bgeo, x, count, qweight, lut, nullptr, out, N, ldo, M, K, w_bits, static_cast<hipStream_t>(stream));
     if (fits && (strided || (count > 1 && mode > 0 && (mode >= 2 || pays))))
         return run_gemmt(tgeo, x, count, qweight, lut, out, N, ldo, M, K, w_bits, static_cast<hipStream_t>(stream));
@@ -1399,8 +1416,13 @@ int ap_gemm_kbit_taken(int M, int N, int K, int w_bits) {
 int ap_gemm_kbit_group_taken(int count, const int *N, int M, int K, int w_bits) {
     const int rc = ap_gemm_kbit_group_pays(count, N, M, K, w_bits);
     if (rc != 0) return rc;
-    long long sum = 0;
-    for (int g = 0; g < count; g++) sum += N[g];
+    long long sum = 0, largest = 0;
+    for (int g = 0; g < count; g++) {
+        sum += N[g];
+        largest = N[g] > largest ? N[g] : largest;
+    }
+    // up to 32 rows gate and up in one launch instead of two (2 x 11008 x 4096, 32 rows: 30 / 22 at 3 bits, 45 / 35 at 5, 64 / 47 at 8)
+    if (M > 8 && M <= 32) return count > 1 && K >= 4096 && sum >= 20000 && 3 * largest <= 2 * sum && takes_gemmb_set(M, sum, largest, K, w_bits) ? 1 : 0;
     return M > 32 && M <= 512 && sum >= 4096 && takes_gemmb(M, sum, K, w_bits) && gemmb_beats_pair(M, sum, K, w_bits) ? 1 : 0;
 }
 

@@ -15,9 +15,10 @@
 //     instructions of either wave of the SIMD fit in 24.  Every slot holds its share of the lookups of the next octet, of the index
 //     arithmetic of the NEXT half-step, of the loads, an activation read, fenced.  Bursts of any of them stood before: the index
 //     arithmetic at the start of a half-step, loads by all waves behind the barrier, planes at once (4096 x 4096, 128 rows, 128 x 128
-//     tile, 5 bits: 45 us so, 43 with reads interleaved only, 38 with the loads spread and half the barriers, 36 fenced).
-// What bounds it now (same tile, 5 bits, of 36 us): matrix cores alone 14, with the vector instructions 15.5, with the LDS reads 24,
-// and 7 for launch, tables, first loads and the sums at the end.
+//     tile, 5 bits: 45 us so, 43 with reads interleaved only, 38 with the loads spread and half the barriers, 36 fenced,
+//     33 with waits that leave the stages ahead outstanding).
+// What bounds it now (same tile, 5 bits): matrix cores alone 14 us, with the vector instructions 15.5, with the LDS reads 24, and 7 for
+// launch, tables, first loads and the sums at the end.
 // Measured (us, planes from HBM; before = the better of tiled kernel and dequantise + library product), rows / 3 / 5 / 8 bits:
 //   4096 x 11008, 128: 32 -> 31, 52 -> 39, 71 -> 52;   512: 82 -> 61, 98 -> 70, 103 -> 98
 //   14336 x 4096, 192: 41 -> 31, 58 -> 41, 76 -> 50;   512: 85 -> 62, 89 -> 70, 93 -> 80 (0.97 / 0.86 / 0.75 PFLOP/s)

@@ -1,4 +1,4 @@
-"""The block-tile fused GEMM (ap_gemm_kbit from 17 activation rows on): every tile against the oracle at the edges of its range."""
+"""The block-tile fused GEMM (ap_gemm_kbit from 9 activation rows on): every tile against the oracle at the edges of its range."""
 import pytest
 import torch
 
@@ -148,3 +148,43 @@ def test_the_rule_keeps_to_its_range():
     assert taken(512, 4096, 4100, 5) == _capi.AP_ESHAPE and taken(0, 4096, 4096, 5) == _capi.AP_EBATCH
     with _capi.tuning(gemm_block=0):
         assert taken(512, 14336, 4096, 5) == 0
+
+
+# (members, K, rows, bits): gate and up in one launch from 9 rows on, and where the rule leaves them one by one
+@pytest.mark.parametrize("Ns,K,M,b,taken", (
+    ((10016, 10000), 4096, 9, 3, 1), ((10016, 10000), 4096, 16, 8, 1), ((10016, 10000), 4096, 13, 5, 1), ((10016, 10000), 4096, 12, 5, 0),
+    ((10016, 10000), 4096, 16, 4, 0), ((10016, 10000), 5120, 11, 4, 1), ((10016, 10000), 4096, 32, 4, 1), ((10016, 9983), 4096, 32, 3, 0),
+    ((14000, 6016), 4096, 16, 3, 0), ((10016, 10000), 4128, 9, 3, 0), ((10016, 10000), 4128, 17, 3, 1)))
+def test_wide_sets_of_few_rows(ext, Ns, K, M, b, taken):
+    """Against the fp32 product of the exact weights: one rounding to fp16 and K additions in fp32 on either side."""
+    import ctypes
+    from any_precision_amd import _capi
+    assert _capi.lib.ap_gemm_kbit_group_taken(len(Ns), (ctypes.c_int * len(Ns))(*Ns), M, K, b) == taken
+    g = torch.Generator(device="cuda").manual_seed(K + M + b)
+    qs = [torch.randint(-2**31, 2**31, (b, n, K // 32), dtype=torch.int32, device="cuda", generator=g) for n in Ns]
+    ts = [(torch.randn((n, 1 << b), device="cuda", generator=g) * 0.02).half() for n in Ns]
+    x = torch.randn((M, K), device="cuda", generator=g).half()
+    got = ext.gemm_kbit_group(x, qs, ts, b)
+    with _capi.tuning(gemm_block=2 if taken else 0):
+        same = ext.gemm_kbit_group(x, qs, ts, b)
+    for q, t, y, z in zip(qs, ts, got, same):
+        w = ext.dequant_kbit(q, t, b).float()
+        bound = 2.0 ** -24 * 2 * K * (x.float().abs() @ w.abs().t()) + 2.0 ** -11 * (x.float() @ w.t()).abs() + 2.0 ** -24
+        assert ((y.float() - x.float() @ w.t()).abs() <= bound).all(), (Ns, K, M, b)
+        if taken:
+            assert torch.equal(y, z), (Ns, K, M, b)
+
+
+def test_long_wide_linears_of_few_rows(ext):
+    """9..16 activation rows on 10240 rows of 8192 elements, and 17 on 10240 of 4096: the block-tile kernel."""
+    from any_precision_amd import _capi
+    for N, K, M in ((10240, 8192, 9), (10240, 8192, 16), (10240, 4096, 17)):
+        for b in range(3, 9):
+            q = torch.randint(-2**31, 2**31, (b, N, K // 32), dtype=torch.int32, device="cuda")
+            t = (torch.randn((N, 1 << b), device="cuda") * 0.02).half()
+            x = torch.randn((M, K), device="cuda").half()
+            y = ext.gemm_kbit(x, q, t, b)
+            with _capi.tuning(gemm_block=2):
+                assert torch.equal(ext.gemm_kbit(x, q, t, b), y), (N, K, M, b)
+            want = x.float() @ ext.dequant_kbit(q, t, b).float().t()
+            assert (y.float() - want).norm() <= 1e-3 * want.norm(), (N, K, M, b)
