@@ -98,13 +98,14 @@ int ap_matmul_kbit_swiglu(const uint16_t *x, const uint32_t *qweight_gate, const
 /* Fused dequant -> MFMA GEMM, M >= 1: out[M,N] = x[M,K] . dequant(qweight, lut)^T
  * without materialising the fp16 weight.  No single counterpart in the reference: it is the
  * M > 8 branch of AnyPrecisionLinear.forward (AnyPrecisionLinear.py:60-62: dequant_kbit,
- * main.cu:60-91, then torch.matmul) fused.  Two kernels: up to 128 activation rows a K-split
+ * main.cu:60-91, then torch.matmul) fused.  Three kernels: up to 128 activation rows a K-split
  * kernel with the weights of 16 rows in registers (more than 32 rows may run as launches of 32
  * each); from 81 rows on, and from 9..65 rows on where it measured faster, a tiled kernel whose
  * workgroups own 64 weight rows x 16..128 activation rows (the narrower the fewer tiles the grid
  * has) for the whole of K, ONE launch for any M (it needs K % 128 == 0; other row lengths go through the K-split kernel in chunks of 128 rows,
- * in order, on the same stream).  Correct for every M; faster than dequant + a library GEMM up to
- * about 256 rows at 3 bits and 64..128 rows at more bits -- beyond that use that pair.
+ * in order, on the same stream); from 9 rows on on wide linears, and nearly everywhere from 65, a block-tile kernel that rebuilds
+ * a weight once per tile of up to 256 activation rows, ONE launch for any M and K >= 256.  Correct for every M; faster than dequant +
+ * a library GEMM up to 256..2048 rows (ap_gemm_kbit_taken) -- beyond that use that pair.
  * fp32 accumulation, fp16 result. */
 int ap_gemm_kbit(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut,
                  uint16_t *out, int M, int N, int K, int w_bits, void *stream);
