@@ -114,7 +114,8 @@ int ap_gemm_kbit(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut
  * layer on a batch of rows): out[g][M, N[g]] = x[M,K] . dequant(qweight[g], lut[g])^T.  Where the tiled
  * kernel serves the set (K % 128 == 0) and pays -- more than 32 rows, or more than 8 where no member
  * has more than 8192 rows -- ONE launch whose tiles of 64 weight rows run through the members -- three 4096 x 4096 projections at 128 rows fill
- * the chip that one of them leaves half idle; otherwise one ap_gemm_kbit per member, in order.
+ * the chip that one of them leaves half idle; ONE launch of the block-tile kernel where that is faster for the rows of all members
+ * together (gate/up from 9 rows on, K >= 256); otherwise one ap_gemm_kbit per member, in order.
  * ldo (may be NULL: dense results) gives the distance in elements between consecutive rows of each
  * out[g], so that the results can be written side by side into one [M, sum N] array (out[g] = its
  * column offset, ldo[g] = sum N); results that are not dense need the tiled kernel: AP_ESHAPE if
