@@ -11,6 +11,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -190,6 +191,9 @@ bool plain_execution() {
            !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
 }
 
+// Whether torch's product of fp16 operands gives fp16 results: under autocast it gives autocast's type.
+bool product_is_half() { return !at::autocast::is_autocast_enabled(at::kCUDA) || at::autocast::get_autocast_dtype(at::kCUDA) == at::kHalf; }
+
 // Names in a module's dicts, made once.
 PyObject *key_buffers, *key_qweight, *key_bias, *key_lut[9];
 
@@ -215,7 +219,7 @@ bool tensors_of(PyObject *module_dict, int bits, ModuleTensors *m) {
 
 // linear(module.__dict__, x, w_bits): AnyPrecisionLinear.forward.  Up to 8 rows ap_matmul_kbit, then
 // ap_gemm_kbit where ap_gemm_kbit_pays, or ap_gemm_kbit_taken and nothing but plain execution follows the call; else the weight in fp16 and
-// torch's own product (which takes part in autograd).
+// torch's own product (which takes part in autograd and autocast).
 PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (n != 3 || !is_tensor(args[1])) return none();
     const int bits = bits_of(args[2]);
@@ -230,7 +234,7 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
         const int64_t rows = rows_of(x, w);
         if (rows < 1) return none();
         const bool pays = rows <= 8 || ap_gemm_kbit_pays((int)rows, w.N, w.K, bits) == 1 ||
-                          (ap_gemm_kbit_taken((int)rows, w.N, w.K, bits) == 1 && plain_execution() && plain_half(args[1], nullptr));
+                          (ap_gemm_kbit_taken((int)rows, w.N, w.K, bits) == 1 && plain_execution() && product_is_half() && plain_half(args[1], nullptr));
         // torch's product and sum as Python calls them, where a subclass or a mode wants to see them
         const bool torch_op = !pays || bias.defined();
         if (torch_op && (at::impl::torch_function_mode_enabled() || !exact_tensor(args[1]) || (m.bias != nullptr && !exact_tensor(m.bias))))
@@ -300,7 +304,7 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (rows < 1) return none();
         const bool gemm = rows > 8;
         if (gemm && ap_gemm_kbit_group_pays(count, N, (int)rows, K, bits) != 1 &&
-            !(ap_gemm_kbit_group_taken(count, N, (int)rows, K, bits) == 1 && plain_execution() && plain_half(args[1], nullptr)))
+            !(ap_gemm_kbit_group_taken(count, N, (int)rows, K, bits) == 1 && plain_execution() && product_is_half() && plain_half(args[1], nullptr)))
             return none();
         // side by side in one allocation: one row's results always are dense, and the tiled kernel writes rows that are not
         const bool joint = concat && (gemm ? K % 128 == 0 : rows == 1);

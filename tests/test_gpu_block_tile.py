@@ -138,6 +138,38 @@ def test_linear_takes_it_for_plain_forwards_and_stays_differentiable(ext):
     assert (batched.float().view(M, N) - y.float()).norm() <= 1e-2 * y.float().norm()
 
 
+def test_autocast_decides_the_type_of_the_product(ext):
+    """A linear and a set where only the plain route is the kernel: under autocast the results are those of torch's product, of its type."""
+    import ctypes
+    from any_precision_amd import AnyPrecisionLinear, _capi
+    from any_precision_amd.linear import forward_group
+    K, M, b, Ns = 512, 512, 5, (2048, 2080)
+    mods = []
+    for N in Ns:
+        mods.append(AnyPrecisionLinear(K, N, list(range(3, 9)), bias=False, device="cuda", dtype=torch.float16))
+        q, luts = layer_to_gpu(make(N, K, seed=N))
+        mods[-1].qweight.copy_(q)
+        mods[-1]._buffers[f"lut{b}"].copy_(luts[b])
+        assert not _capi.gemm_pays(M, N, K, b) and _capi.lib.ap_gemm_kbit_taken(M, N, K, b) == 1
+    assert not _capi.gemm_group_pays(M, list(Ns), K, b)
+    assert _capi.lib.ap_gemm_kbit_group_taken(len(Ns), (ctypes.c_int * len(Ns))(*Ns), M, K, b) == 1
+    x = torch.randn((M, K), device="cuda").half()
+    dense = [ext.dequant_kbit(m.qweight, m._buffers[f"lut{b}"], b) for m in mods]
+    plain = [ext.gemm_kbit(x, m.qweight, m._buffers[f"lut{b}"], b) for m in mods]
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        want = [torch.matmul(x, w.t()) for w in dense]
+        got, joint = [m(x, precision=b) for m in mods], forward_group(mods, x, b, concat=True)
+        sets = forward_group(mods, x, b)
+        with torch.autocast("cuda", enabled=False):
+            inner = [m(x, precision=b) for m in mods]
+    assert all(y.dtype == torch.bfloat16 and torch.equal(y, z) for y, z in zip(got, want))
+    assert all(y.dtype == torch.bfloat16 and torch.equal(y, z) for y, z in zip(sets, want))
+    assert joint.dtype == torch.bfloat16 and torch.equal(joint, torch.cat(want, dim=-1))
+    with torch.autocast("cuda", dtype=torch.float16):
+        half = [m(x, precision=b) for m in mods]
+    assert all(torch.equal(y, p) and torch.equal(z, p) for y, z, p in zip(half, inner, plain))
+
+
 def test_the_rule_keeps_to_its_range():
     """No GPU is asked: where ap_gemm_kbit_taken says yes beyond ap_gemm_kbit_pays."""
     from any_precision_amd import _capi
