@@ -1365,15 +1365,14 @@ static int matmul_set(const uint16_t *x, int count, const uint32_t *const *qweig
         return AP_OK;
     }
     if (one_launch) {  // the whole set in one launch
-        mem.bias = bias;
         *added = bias != nullptr;
         switch (w_bits) {
-            case 3: launch_gemv<3>(M, geo, x, mem, K, st); break;
-            case 4: launch_gemv<4>(M, geo, x, mem, K, st); break;
-            case 5: launch_gemv<5>(M, geo, x, mem, K, st); break;
-            case 6: launch_gemv<6>(M, geo, x, mem, K, st); break;
-            case 7: launch_gemv<7>(M, geo, x, mem, K, st); break;
-            default: launch_gemv<8>(M, geo, x, mem, K, st); break;
+            case 3: launch_gemv<3>(M, geo, x, mem, bias, K, st); break;
+            case 4: launch_gemv<4>(M, geo, x, mem, bias, K, st); break;
+            case 5: launch_gemv<5>(M, geo, x, mem, bias, K, st); break;
+            case 6: launch_gemv<6>(M, geo, x, mem, bias, K, st); break;
+            case 7: launch_gemv<7>(M, geo, x, mem, bias, K, st); break;
+            default: launch_gemv<8>(M, geo, x, mem, bias, K, st); break;
         }
         return launch_status();
     }

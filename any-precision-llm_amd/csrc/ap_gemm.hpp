@@ -62,10 +62,11 @@ __device__ __forceinline__ void transpose_rows4(uint32_t (&r)[4]) {
 // which divides the L2 traffic of the activations by RB -- at the price of 1/RB as many
 // workgroups, so only linears with many rows use RB = 2.  Grid: ceil(N / (16 RB)) workgroups of (64, KS).
 // LOOKAHEAD: see the step below.
-template <int BITS, int MB, bool VEC4, int MP, int RB, bool LOOKAHEAD = false>
+// BIAS: `bias` (one of each row) is added to the results; launches without one run kernels that know nothing of it.
+template <int BITS, int MB, bool VEC4, int MP, int RB, bool LOOKAHEAD, bool BIAS>
 __global__ __launch_bounds__(kGemmMaxSplit *kWave) void gemm_kbit_kernel(
     const half_t *__restrict__ x, const uint32_t *__restrict__ qweight, const half_t *__restrict__ lut,
-    const half_t *__restrict__ bias, half_t *__restrict__ out, int M, int N, int K, int KS, uint32_t ks_magic) {
+    half_t *__restrict__ out, int M, int N, int K, int KS, uint32_t ks_magic, const half_t *__restrict__ bias) {
     constexpr int NC = 1 << BITS;
     constexpr int WPS = VEC4 ? 4 : 1;             // words per lane and step
     constexpr int ROWS = kGemmRows * RB;    // weight rows per workgroup
@@ -85,7 +86,8 @@ __global__ __launch_bounds__(kGemmMaxSplit *kWave) void gemm_kbit_kernel(
 
     // every argument in scalar registers by one clause of scalar loads and one wait (the compiler alone loads
     // an argument where it is first used: a dependent round trip to the scalar cache each)
-    asm volatile("" : "+s"(x), "+s"(qweight), "+s"(lut), "+s"(bias), "+s"(out), "+s"(M), "+s"(N), "+s"(K), "+s"(KS), "+s"(ks_magic));
+    asm volatile("" : "+s"(x), "+s"(qweight), "+s"(lut), "+s"(out), "+s"(M), "+s"(N), "+s"(K), "+s"(KS), "+s"(ks_magic));
+    if constexpr (BIAS) asm volatile("" : "+s"(bias));
     const int lane = threadIdx.x;
     const int ks = __builtin_amdgcn_readfirstlane(threadIdx.y);  // KS = blockDim.y, passed as an argument
     const int col = lane & 15, grp = lane >> 4;
@@ -397,10 +399,11 @@ __global__ __launch_bounds__(kGemmMaxSplit *kWave) void gemm_kbit_kernel(
         float sum = 0.f;
         for (int kk = 0; kk < KS; kk++) sum += reinterpret_cast<const float *>(&xs[kk][0])[t * kWave + lane];
         const int m = mb * 16 + 4 * grp + v, n = n0 + rb * kGemmRows + col;
-        if (m >= M || n >= N) continue;
-        half_t y = (half_t)sum;
-        if (bias != nullptr) y = (half_t)((float)y + (float)((global_ptr<const half_t>)reinterpret_cast<uint64_t>(bias))[n]);  // as on the finished result
-        out_g[(size_t)m * N + n] = y;
+        if (m < M && n < N) {
+            half_t y = (half_t)sum;
+            if constexpr (BIAS) y = (half_t)((float)y + (float)((global_ptr<const half_t>)reinterpret_cast<uint64_t>(bias))[n]);  // as on the finished result
+            out_g[(size_t)m * N + n] = y;
+        }
     }
 }
 

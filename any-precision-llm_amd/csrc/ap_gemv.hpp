@@ -144,10 +144,11 @@ constexpr int gemv_waves_per_simd(int bits, int m, int wpl, int r) {
     return waves > 8 ? 8 : waves;
 }
 
-template <int BITS, int M, int WPL, int R, int THREADS, bool PAIR = false>
+template <int BITS, int M, int WPL, int R, int THREADS, bool PAIR = false, typename Members = GemvMembers>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(gemv_waves_per_simd(BITS, M, WPL, R))))
-void gemv_kbit_kernel(const half_t *__restrict__ x, const GemvMembers mem, int K, int S) {
+void gemv_kbit_kernel(const half_t *__restrict__ x, const Members mem, int K, int S) {
     static_assert(!PAIR || R == 2, "a pair is two rows");
+    constexpr bool BIAS = std::is_same<Members, GemvBiasMembers>::value;
     constexpr int NC = 1 << BITS;
     constexpr int MAXS = THREADS / kWave;
     typedef typename WordVec<WPL>::type wvec_t;
@@ -165,18 +166,21 @@ void gemv_kbit_kernel(const half_t *__restrict__ x, const GemvMembers mem, int K
     const uint32_t *q0 = mem.qweight[0], *q1 = mem.qweight[PAIR ? 1 : 0];
     const uint16_t *lut0 = mem.lut[0], *lut1 = mem.lut[PAIR ? 1 : 0];
     uint16_t *out0 = mem.out[0];
-    const uint16_t *bias0 = mem.bias;
+    const uint16_t *bias0 = nullptr;
+    if constexpr (BIAS) bias0 = mem.bias;
     int n0 = mem.n[0], end0 = mem.wg_end[0], end1 = mem.wg_end[1], end2 = mem.wg_end[2], count = mem.count;
     if constexpr (PAIR)
         asm volatile("" : "+s"(q0), "+s"(q1), "+s"(lut0), "+s"(lut1), "+s"(out0), "+s"(n0), "+s"(K), "+s"(S), "+s"(x));
+    else if constexpr (BIAS)
+        asm volatile("" : "+s"(q0), "+s"(lut0), "+s"(out0), "+s"(n0), "+s"(K), "+s"(S), "+s"(x), "+s"(bias0));
     else
         asm volatile("" : "+s"(q0), "+s"(lut0), "+s"(out0), "+s"(n0), "+s"(end0), "+s"(end1), "+s"(end2), "+s"(count),
-                          "+s"(K), "+s"(S), "+s"(x), "+s"(bias0));
+                          "+s"(K), "+s"(S), "+s"(x));
     const uint32_t *__restrict__ qweight = q0;
     const half_t *__restrict__ lut = reinterpret_cast<const half_t *>(lut0);
     half_t *__restrict__ out = reinterpret_cast<half_t *>(out0);
     int N = n0, wg0 = 0;
-    if constexpr (!PAIR) {
+    if constexpr (!PAIR && !BIAS) {
         if (count > 1) {
             // a launch of several linears (a scalar branch; plain calls skip it): which member the workgroup
             // belongs to, then that member's fields by index -- one more clause of scalar loads, cheaper than
@@ -290,11 +294,10 @@ void gemv_kbit_kernel(const half_t *__restrict__ x, const GemvMembers mem, int K
     // What is stored: the sum as fp16, plus the bias of its row in fp16 arithmetic, as the operation on the finished result has it.  A
     // bias as an operation of its own costs a launch and half as much again of the host's time (1999 x 2720, 3 rows, 6 bits: 10.9 us a
     // call, 7.0 with it here).
-    const global_ptr<const half_t> bias = (global_ptr<const half_t>)reinterpret_cast<uint64_t>(bias0);
     auto finished = [&](float v, int n) {
-        half_t y = (half_t)v;
-        if (!PAIR && bias0 != nullptr) y = (half_t)((float)y + (float)bias[n]);
-        return y;
+        const half_t y = (half_t)v;
+        if constexpr (BIAS) return (half_t)((float)y + (float)((global_ptr<const half_t>)reinterpret_cast<uint64_t>(bias0))[n]);
+        else return y;
     };
     auto swiglu = [](float gate, float up) { return gate / (1.f + __expf(-gate)) * up; };
     if (FOLD && S == 1 && !PAIR) {

@@ -19,7 +19,12 @@ struct GemvMembers {
     int n[kGemvMaxGroup];       // rows
     int wg_end[kGemvMaxGroup];  // first workgroup past the member
     int count;
-    const uint16_t *bias;       // of member 0, the only one then; null: none
+};
+
+// One linear with a bias that is added to its results.  A type of its own, and so kernels of their own: launches without a bias, nearly all of
+// them, take no argument, no test and no instruction for it.
+struct GemvBiasMembers : GemvMembers {
+    const uint16_t *bias;
 };
 
 struct GemvGeometry {
@@ -29,9 +34,9 @@ struct GemvGeometry {
     int grid;  // workgroups (of all members together)
 };
 
-// Launches gemv_kbit_kernel<BITS, M, geo.wpl, geo.R, *> on `stream`.  1 <= M <= 8.
+// Launches gemv_kbit_kernel<BITS, M, geo.wpl, geo.R, *> on `stream`.  1 <= M <= 8.  bias: null, or of member 0, the only one then.
 template <int BITS>
-void launch_gemv(int M, const GemvGeometry &geo, const uint16_t *x, const GemvMembers &members, int K,
+void launch_gemv(int M, const GemvGeometry &geo, const uint16_t *x, const GemvMembers &members, const uint16_t *bias, int K,
                  hipStream_t stream);
 
 // Launches gemv_kbit_kernel<BITS, M, 1, 2, *, true>: members 0 and 1 of `members` are two linears of n[0] rows
@@ -47,11 +52,11 @@ extern template void launch_gemv_pair<6>(int, const GemvGeometry &, const uint16
 extern template void launch_gemv_pair<7>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, int, hipStream_t);
 extern template void launch_gemv_pair<8>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, int, hipStream_t);
 
-extern template void launch_gemv<3>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, int, hipStream_t);
-extern template void launch_gemv<4>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, int, hipStream_t);
-extern template void launch_gemv<5>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, int, hipStream_t);
-extern template void launch_gemv<6>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, int, hipStream_t);
-extern template void launch_gemv<7>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, int, hipStream_t);
-extern template void launch_gemv<8>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, int, hipStream_t);
+extern template void launch_gemv<3>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, const uint16_t *, int, hipStream_t);
+extern template void launch_gemv<4>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, const uint16_t *, int, hipStream_t);
+extern template void launch_gemv<5>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, const uint16_t *, int, hipStream_t);
+extern template void launch_gemv<6>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, const uint16_t *, int, hipStream_t);
+extern template void launch_gemv<7>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, const uint16_t *, int, hipStream_t);
+extern template void launch_gemv<8>(int, const GemvGeometry &, const uint16_t *, const GemvMembers &, const uint16_t *, int, hipStream_t);
 
 }  // namespace ap
