@@ -546,15 +546,13 @@ __global__ __launch_bounds__(WN *WK *kWave) void gemmb_kbit_kernel(const half_t 
             half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
     };
     constexpr int REGS = 16 * MB, PART = REGS / WK;  // accumulators of a wave; group g finishes PART of them
-    static_assert(PART % 4 == 0 && WN * (WK - 1) <= NBUF * WK, "");
+    // what is parked stays in the first two buffers: with four the finished tile goes to the third, with no barrier between
+    static_assert(PART % 4 == 0 && WN * (WK - 1) <= 2 * WK, "");
     if constexpr (WK > 1) {
         // what a wave of group `from` leaves for the wave of group `to` over the same weight rows: PART accumulators
         auto parked = [&](int to, int from) {
             const int block = (wn * WK + to) * (WK - 1) + (from < to ? from : from - 1), buf = block / (WK * WK);
-            float4_t *base = reinterpret_cast<float4_t *>(&xt0[0][0][0]);
-            if (buf == 1) base = reinterpret_cast<float4_t *>(&xt1[0][0][0]);
-            if (NBUF == 4 && buf == 2) base = reinterpret_cast<float4_t *>(&xt2[0][0][0]);
-            if (NBUF == 4 && buf == 3) base = reinterpret_cast<float4_t *>(&xt3[0][0][0]);
+            float4_t *base = reinterpret_cast<float4_t *>(buf == 0 ? &xt0[0][0][0] : &xt1[0][0][0]);
             return base + block % (WK * WK) * (PART / 4 * kWave) + lane;
         };
         static_for<WK>([&](auto to_c) {
