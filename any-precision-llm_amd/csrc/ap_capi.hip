@@ -610,41 +610,53 @@ bool gemmt_pays(int M, int N, int K, int w_bits) {
 constexpr struct { int mb, wn, wk; } kGemmbTiles[] = {{8, 4, 1}, {3, 4, 2}, {3, 2, 4}, {4, 4, 2}, {4, 2, 4}, {2, 4, 2}, {2, 2, 4}, {2, 1, 8}, {1, 2, 4}};
 constexpr int kGemmbTileCount = sizeof(kGemmbTiles) / sizeof(kGemmbTiles[0]);
 
-// What a launch with a tile takes, in us: a + r (p + h (s + f u)), where r = rounds of tiles over the CUs, h = the half-steps of
-// 256 elements that a group walks and u = the share of the CUs that has a tile (up to 1: the more there are, the slower each runs).
-// {a, p, s, f} per bit-width and tile of the list above, least squares over 15 linear shapes (1024 x 4096 .. 22016 x 4096, 4096 x
-// 14336, 8192 x 8192; rows of 2048 .. 14336 elements, one of no multiple of 128) x 14 numbers of activation rows (16 .. 2048), planes
-// from HBM, 2500 launches a bit-width.  The tile it picks is within 0.1 % of the fastest on average, 8 % at worst.  (0 0 0 0: the
-// tables of that tile and bit-width do not fit the LDS.)
-constexpr float kGemmbCost[6][kGemmbTileCount][4] = {
-    {{-3.41f, 10.35f, 2.23f, 0.87f}, {2.11f, 4.07f, 2.10f, 0.77f}, {3.46f, 1.32f, 2.89f, 1.19f},
-     {2.58f, 3.77f, 2.39f, 1.17f}, {3.36f, 1.70f, 3.35f, 1.53f}, {3.64f, 2.01f, 1.83f, 0.53f},
-     {4.06f, 1.87f, 2.03f, 0.76f}, {3.65f, 1.34f, 3.40f, 1.18f}, {6.07f, -0.02f, 1.63f, 0.17f}},
-    {{-3.58f, 10.22f, 2.70f, 0.83f}, {1.72f, 4.56f, 2.89f, 0.70f}, {3.62f, 1.76f, 3.08f, 1.29f},
-     {2.88f, 3.68f, 3.10f, 1.18f}, {3.91f, 2.23f, 3.78f, 1.53f}, {3.76f, 2.25f, 2.66f, 0.47f},
-     {4.04f, 0.99f, 2.73f, 0.95f}, {3.65f, 1.90f, 3.88f, 1.20f}, {3.56f, 2.71f, 1.80f, 0.44f}},
-    {{-2.41f, 8.42f, 2.83f, 0.88f}, {1.46f, 4.13f, 3.20f, 0.63f}, {4.34f, 2.08f, 3.74f, 1.14f},
-     {3.34f, 2.47f, 3.40f, 1.19f}, {4.34f, 2.02f, 4.11f, 1.61f}, {3.75f, 1.78f, 2.95f, 0.40f},
-     {4.23f, 2.21f, 3.14f, 0.72f}, {3.74f, 2.09f, 4.12f, 1.40f}, {4.14f, 2.27f, 2.74f, 0.35f}},
-    {{-1.84f, 8.82f, 2.83f, 0.92f}, {2.02f, 4.76f, 3.28f, 0.68f}, {5.07f, 2.43f, 3.77f, 1.29f},
-     {3.77f, 3.17f, 3.48f, 1.23f}, {5.22f, 2.17f, 4.08f, 1.85f}, {4.21f, 2.49f, 3.02f, 0.46f},
-     {4.85f, 2.72f, 3.15f, 0.88f}, {3.69f, 2.87f, 4.24f, 1.42f}, {4.21f, 3.33f, 2.85f, 0.43f}},
-    {{-0.95f, 7.99f, 2.89f, 0.97f}, {2.08f, 5.41f, 3.56f, 0.63f}, {5.64f, 2.55f, 3.97f, 1.42f},
-     {4.12f, 3.31f, 3.78f, 1.21f}, {5.82f, 2.22f, 4.30f, 1.96f}, {4.44f, 2.90f, 3.32f, 0.41f},
-     {5.49f, 2.83f, 3.41f, 0.99f}, {3.80f, 3.02f, 4.61f, 1.49f}, {4.73f, 3.42f, 3.09f, 0.50f}},
-    {{2.23f, 5.05f, 3.22f, 1.05f}, {3.22f, 6.08f, 3.76f, 0.70f}, {6.07f, 3.13f, 4.21f, 1.56f},
-     {5.35f, 3.27f, 4.19f, 1.23f}, {0.f, 0.f, 0.f, 0.f}, {4.99f, 3.99f, 3.53f, 0.43f},
-     {5.99f, 2.62f, 3.93f, 1.21f}, {0.f, 0.f, 0.f, 0.f}, {4.97f, 4.48f, 3.26f, 0.58f}},
+// Rounds of tiles over the CUs: workgroups go to the 8 XCDs in turn, and both tiled kernels number their tiles so that those of one block of
+// weight rows run on one XCD.  So the XCDs with one block more decide: 20 blocks are 3 on four XCDs and 2 on the others (2560 x 2560 at
+// 1395 rows, 128 x 128 tiles: 220 tiles are 33 for 32 CUs, two rounds, 43 us where one round of 192 would be 24).
+inline long long tile_rounds(long long tiles_n, long long tiles_m) {
+    const long long cus = cu_count() < 8 ? 1 : cu_count() / 8;  // of an XCD
+    return ((tiles_n + 7) / 8 * tiles_m + cus - 1) / cus;
+}
+
+// What a launch of the block-tile kernel takes with each tile, in us: a + r (p + h (s + f u) + t + o), where r = rounds of tiles, h = the
+// half-steps of 256 elements that the busiest group walks, u = the share of the CUs that has a tile (up to 1: the more there are, the slower
+// each runs), t = the part of a half-step at the end of rows of no multiple of 256 elements (nothing of it overlaps), o = results that leave
+// in 2-byte stores, of linears whose rows are no multiple of 8.  {a, p, s, f, t, o} per bit-width and tile of the list above, non-negative least
+// squares over 23500 calls: linears of 512..24000 rows of 256..14336 elements, half of them of generic sizes, at 17..2048 activation rows, each
+// with every tile.  The estimate is 8 % off on average.  The tile it picks is within 0.3 % of the fastest on average and 8 % in 99 of 100 calls.
+// With rounds over all CUs at once and no t and o, fitted on 15 linears of whole half-steps (the first form of this table), it was 5.5 %
+// and 46 % in 5 of 100.  (0 0 0 0 0 0: the tables of that tile and bit-width do not fit the LDS.)
+constexpr float kGemmbCost[6][kGemmbTileCount][6] = {
+    {{0.46f, 7.90f, 2.21f, 0.95f, 5.83f, 1.64f}, {2.67f, 2.61f, 2.10f, 0.86f, 3.81f, 1.55f}, {3.22f, 1.04f, 2.73f, 1.33f, 3.22f, 0.77f},
+     {2.63f, 3.09f, 2.43f, 1.12f, 4.17f, 1.79f}, {3.30f, 1.10f, 3.26f, 1.57f, 3.72f, 0.92f}, {2.77f, 2.02f, 1.84f, 0.50f, 3.48f, 1.32f},
+     {3.15f, 1.56f, 2.10f, 0.71f, 2.82f, 0.62f}, {3.56f, 0.33f, 3.21f, 1.30f, 2.88f, 0.41f}, {4.40f, 0.43f, 1.69f, 0.f, 1.65f, 0.21f}},
+    {{0.01f, 8.51f, 2.64f, 0.85f, 6.97f, 1.50f}, {2.59f, 2.95f, 2.86f, 0.78f, 4.89f, 1.55f}, {3.52f, 1.08f, 2.92f, 1.43f, 3.51f, 0.68f},
+     {2.69f, 3.23f, 3.14f, 1.08f, 5.37f, 1.74f}, {3.68f, 1.45f, 3.78f, 1.45f, 4.63f, 0.80f}, {2.78f, 2.30f, 2.68f, 0.39f, 4.57f, 1.19f},
+     {3.39f, 1.07f, 2.57f, 1.00f, 3.00f, 0.53f}, {3.72f, 0.89f, 3.65f, 1.29f, 3.51f, 0.14f}, {3.15f, 1.84f, 1.80f, 0.43f, 2.47f, 0.19f}},
+    {{1.03f, 7.78f, 2.67f, 0.93f, 7.30f, 1.57f}, {2.74f, 2.97f, 2.94f, 0.84f, 5.40f, 1.62f}, {3.40f, 1.48f, 3.57f, 1.20f, 4.24f, 0.70f},
+     {2.80f, 3.44f, 3.17f, 1.16f, 5.85f, 1.82f}, {3.60f, 1.53f, 3.94f, 1.55f, 4.76f, 0.82f}, {2.73f, 2.52f, 2.75f, 0.42f, 5.01f, 1.33f},
+     {3.31f, 1.98f, 2.97f, 0.67f, 3.84f, 0.54f}, {3.65f, 0.75f, 3.92f, 1.33f, 3.64f, 0.33f}, {3.45f, 1.62f, 2.58f, 0.35f, 3.36f, 0.17f}},
+    {{0.49f, 8.69f, 2.71f, 0.96f, 7.85f, 1.85f}, {2.78f, 3.15f, 3.11f, 0.90f, 5.97f, 1.84f}, {3.54f, 1.43f, 3.80f, 1.30f, 4.59f, 0.80f},
+     {2.83f, 3.63f, 3.32f, 1.20f, 6.43f, 2.08f}, {3.77f, 1.43f, 4.16f, 1.66f, 5.16f, 0.97f}, {2.98f, 2.53f, 2.90f, 0.50f, 5.55f, 1.51f},
+     {3.47f, 1.91f, 3.16f, 0.81f, 4.17f, 0.57f}, {3.81f, 0.58f, 4.18f, 1.49f, 4.03f, 0.27f}, {3.26f, 1.85f, 2.81f, 0.47f, 3.67f, 0.25f}},
+    {{1.43f, 8.53f, 2.70f, 1.14f, 8.39f, 1.83f}, {3.01f, 3.35f, 3.27f, 0.98f, 6.64f, 1.65f}, {3.70f, 1.49f, 3.94f, 1.45f, 4.83f, 0.70f},
+     {3.28f, 3.62f, 3.48f, 1.36f, 7.12f, 1.85f}, {4.11f, 1.37f, 4.26f, 1.89f, 5.37f, 0.89f}, {3.17f, 2.78f, 3.07f, 0.57f, 6.23f, 1.25f},
+     {3.58f, 1.99f, 3.35f, 0.90f, 4.43f, 0.49f}, {3.81f, 0.63f, 4.41f, 1.58f, 3.89f, 0.45f}, {3.32f, 1.94f, 2.98f, 0.57f, 3.93f, 0.16f}},
+    {{1.22f, 9.61f, 2.96f, 1.18f, 8.69f, 2.00f}, {3.09f, 4.40f, 3.48f, 1.09f, 7.11f, 1.82f}, {3.89f, 1.92f, 4.16f, 1.65f, 5.15f, 0.56f},
+     {3.39f, 4.47f, 3.85f, 1.43f, 7.57f, 2.07f}, {0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, {3.19f, 3.95f, 3.24f, 0.65f, 6.80f, 1.42f},
+     {3.71f, 1.88f, 3.86f, 1.15f, 4.70f, 0.44f}, {0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, {3.45f, 2.50f, 3.12f, 0.71f, 4.26f, 0.08f}},
 };
 
 // The fastest tile for linears that share x; false if the kernel does not serve the shape.
 bool gemmb_geometry(int M, const int *N, int count, int K, int w_bits, GemmbGeometry *geo) {
     if (K < 256 || (long long)M * K * 2 > 0xffffffffLL || count > kGemmbMaxGroup) return false;
-    for (int g = 0; g < count; g++)
+    bool odd = false;
+    for (int g = 0; g < count; g++) {
         if ((long long)N[g] * (K >> 5) * 4 > 0xffffffffLL) return false;
+        odd = odd || (N[g] & 7) != 0;
+    }
     const int forced = knob(kGemmBlockTile);
     const double cus = cu_count();
-    double best = 0;
     geo->mb = 0;
     for (int t = 0; t < kGemmbTileCount; t++) {
         const auto &tile = kGemmbTiles[t];
@@ -654,13 +666,10 @@ bool gemmb_geometry(int M, const int *N, int count, int K, int w_bits, GemmbGeom
         for (int g = 0; g < count; g++) n += (N[g] + kGemmbRows * tile.wn - 1) / (kGemmbRows * tile.wn);
         const long long m = (M + 32LL * tile.mb - 1) / (32 * tile.mb);
         if ((n + 7) / 8 * 8 * m > 0x7fffffffLL) continue;
-        const double rounds = ceil((double)(n * m) / cus), fill = fmin(1.0, (double)(n * m) / cus);
-        const int halves = (K + 255) / 256, h = (halves + tile.wk - 1) / tile.wk;
-        const double us = c[0] + rounds * (c[1] + h * (c[2] + c[3] * fill));
-        if (geo->mb == 0 || us < best) {
-            best = us;
-            *geo = {tile.mb, tile.wn, tile.wk, (int)n, (int)m};
-        }
+        const int h = (K / 256 + tile.wk - 1) / tile.wk;
+        const double fill = fmin(1.0, (double)(n * m) / cus);
+        const double us = c[0] + tile_rounds(n, m) * (c[1] + h * (c[2] + c[3] * fill) + ((K & 255) ? c[4] : 0.f) + (odd ? c[5] : 0.f));
+        if (geo->mb == 0 || us < geo->us) *geo = {tile.mb, tile.wn, tile.wk, (int)n, (int)m, us};
     }
     return geo->mb != 0;
 }

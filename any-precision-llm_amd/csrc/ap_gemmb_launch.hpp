@@ -14,6 +14,7 @@ struct GemmbGeometry {
     int wk;      // groups of wn waves, each on its share of K
     int grid_n;  // tiles of 32 wn weight rows over all members
     int grid_m;  // ceil(M / (32 mb))
+    double us;   // what the launch is estimated to take
 };
 
 constexpr int kGemmbMaxGroup = 4;  // linears one launch can serve (they share x, K, M and w_bits)

@@ -182,6 +182,22 @@ def test_the_rule_keeps_to_its_range():
         assert taken(512, 14336, 4096, 5) == 0
 
 
+def test_tiles_are_counted_on_the_xcd_that_has_most(ext):
+    """2560 rows are 20 blocks of 128: three on four of the XCDs, two on the others.  At 1527 rows 12 x 20 tiles of 128 x 128 are two rounds
+    of the former; 6 x 20 of 256 x 128 are one.  The two add up K in different orders, so the results tell which ran."""
+    from any_precision_amd import _capi
+    N, K, M, b = 2560, 2560, 1527, 6
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q = torch.randint(-2**31, 2**31, (b, N, K // 32), dtype=torch.int32, device="cuda", generator=g)
+    t = (torch.randn((N, 1 << b), device="cuda", generator=g) * 0.02).half()
+    x = torch.randn((M, K), device="cuda", generator=g).half()
+    got = {}
+    for tile in (0, 442, 841):
+        with _capi.tuning(gemm_block=2, gemm_block_tile=tile):
+            got[tile] = ext.gemm_kbit(x, q, t, b)
+    assert torch.equal(got[0], got[841]) and not torch.equal(got[0], got[442])
+
+
 # (members, K, rows, bits): gate and up in one launch from 9 rows on, and where the rule leaves them one by one
 @pytest.mark.parametrize("Ns,K,M,b,taken", (
     ((10016, 10000), 4096, 9, 3, 1), ((10016, 10000), 4096, 16, 8, 1), ((10016, 10000), 4096, 13, 5, 1), ((10016, 10000), 4096, 12, 5, 0),
