@@ -606,6 +606,9 @@ bool gemmt_pays(int M, int N, int K, int w_bits) {
     return M > (w_bits <= 4 ? 32 : (w_bits == 5 ? 48 : (w_bits == 6 ? 64 : 80)));
 }
 
+// Where one launch of the tiled kernel over a set (largest: rows of its largest member) beats its members one by one (ap_gemm_kbit_group).
+inline bool gemmt_set_pays(int M, long long largest, int K) { return M > 32 || (M > 8 && largest <= 8192 && K >= 1024); }
+
 // The tiles of the block-tile fused GEMM (ap_gemmb.hpp): blocks of 32 activation rows, waves over the weight rows, groups over K.
 constexpr struct { int mb, wn, wk; } kGemmbTiles[] = {{8, 4, 1}, {3, 4, 2}, {3, 2, 4}, {4, 4, 2}, {4, 2, 4}, {2, 4, 2}, {2, 2, 4}, {2, 1, 8}, {1, 2, 4}};
 constexpr int kGemmbTileCount = sizeof(kGemmbTiles) / sizeof(kGemmbTiles[0]);
@@ -674,9 +677,25 @@ bool gemmb_geometry(int M, const int *N, int count, int K, int w_bits, GemmbGeom
     return geo->mb != 0;
 }
 
-// Where the block-tile kernel beats the other fused forms (same sweep; us there and here).  Beyond 256 activation rows on every linear of
+// The same for the tiled kernel: a + r (p + h s), h = steps of 512 elements.  {a, p, s} per bit-width and form of its tile (gemmt_geometry):
+// 16, 32 and 64 activation rows with two groups of waves, 64 and 128 with one.  Least squares over 34000 calls, as above; 6 % off on average.
+constexpr float kGemmtCost[6][5][3] = {
+    {{4.98f, 0.f, 1.00f}, {3.45f, 2.69f, 1.23f}, {2.93f, 3.33f, 1.72f}, {5.50f, 0.f, 1.61f}, {4.16f, 1.87f, 2.58f}},
+    {{2.12f, 2.98f, 1.22f}, {3.56f, 2.73f, 1.45f}, {3.56f, 2.88f, 1.95f}, {4.86f, 0.f, 2.67f}, {6.04f, 0.85f, 3.26f}},
+    {{2.51f, 2.78f, 1.77f}, {3.95f, 2.63f, 2.04f}, {3.22f, 3.25f, 2.57f}, {5.24f, 0.f, 2.67f}, {6.82f, 0.29f, 3.46f}},
+    {{2.62f, 3.21f, 1.91f}, {3.72f, 3.03f, 2.24f}, {4.86f, 2.42f, 2.76f}, {5.24f, 0.f, 2.92f}, {6.69f, 0.43f, 3.65f}},
+    {{2.47f, 3.65f, 2.10f}, {4.13f, 3.32f, 2.44f}, {5.21f, 2.72f, 2.97f}, {5.81f, 0.f, 3.74f}, {7.60f, 0.33f, 4.25f}},
+    {{2.70f, 3.51f, 2.53f}, {4.97f, 2.57f, 2.83f}, {5.92f, 2.72f, 3.32f}, {6.29f, 0.f, 4.09f}, {3.17f, 4.49f, 4.91f}},
+};
+double gemmt_us(const GemmtGeometry &geo, int K, int w_bits) {
+    const int form = geo.mbw == 1 ? 0 : (geo.mbw == 2 ? 1 : (geo.mbw == 8 ? 4 : (geo.kh == 2 ? 2 : 3)));
+    const float *c = kGemmtCost[w_bits - 3][form];
+    return c[0] + tile_rounds(geo.grid_n, geo.grid_m) * (c[1] + (K + 511) / 512 * c[2]);
+}
+
+// Where the block-tile kernel beats the other fused forms (us there and here).  Beyond 256 activation rows on every linear of
 // 1024 rows or more (14336 x 4096, 512 rows: 90 / 62 at 3 bits, 114 / 70 at 5); from 129 rows on linears of 2048 rows or
-// more (11008 x 4096, 192 rows, 5 bits: 56 / 38), and from 65 of 4096 or more (4096 x 11008, 128 rows, 5 bits: 50 / 39); narrower
+// more (11008 x 4096, 192 rows, 5 bits: 56 / 38), and from 65 of 4096 or more (4096 x 11008, 128 rows, 5 bits: 50 / 38); narrower
 // ones at 5 to 7 bits (1024 x 4096, 128 rows, 5 bits: 20 / 16; at 3 bits 12 / 13), at 8 bits from 2048 rows on.  At 33..64
 // rows on linears of 5120 rows or more (6144 x 4096, 48 rows, 5 bits: 27 / 17), on narrower ones where the 16-row tiles of the tiled kernel
 // wait for their lookups: 5 to 7 bits beyond 48 rows, or on rows of more than 4096 elements; 8 bits on both (4096 x 4096,
@@ -686,6 +705,9 @@ bool gemmb_geometry(int M, const int *N, int count, int K, int w_bits, GemmbGeom
 // 52 / 32; 14336 x 4096 at 6 bits a tie, 26.9 / 26.6; 8192 x 8192 up to 6 bits and 4096 x 11008 lose, 29.4 / 30.8 and 24 / 25), of 20000 on
 // shorter rows; from 9 where these have 8192 elements or more (10240 x 8192, 16 rows: 28 / 22, 43 / 32, 61 / 42; 28672 x 8192: 50 / 40 and
 // 124 / 96, at 4 bits 54 / 55 at 9 rows); 4096 elements are not enough there (22016 x 4096, 4 bits: 25 / 30).
+// Within that range each other form keeps what it does faster (takes_gemmb): the lines above were drawn on rows of 2048 elements and more, and
+// by them alone 10 % of the calls at other sizes lost, up to 2.7 times (7.1 / 10.6 us on 1181 x 544, 98 rows, 5 bits; 6.8 / 9.2 on 5696 x
+// 384, 107 rows, 4 bits; 21 / 28 on 2560 x 2560, 705 rows, 3 bits).
 bool gemmb_pays(int M, long long N, int K, int b) {
     if (N < 1024 || M <= 8 || K < 256) return false;
     if ((long long)M * K * 2 > 0xffffffffLL || N * (K >> 5) * 4 > 0xffffffffLL) return false;  // its 32-bit offsets
@@ -699,6 +721,19 @@ bool gemmb_pays(int M, long long N, int K, int b) {
     const bool middle = b >= 5 && b <= 7;
     if (M <= 128) return N >= 4096 || middle || (b == 8 && N >= 2048);
     return M > 256 || N >= 2048 || middle;
+}
+
+// Against the K-split kernel, whose time has no simple form: on short rows it wins, the more so the fewer weight rows and activation rows
+// there are and the more bits (the block tile's tables and its first loads are not paid back).  us K-split / block tile at the edges: 1181 x 544,
+// 98 rows, 5 bits 7.1 / 10.6; 4096 x 480, 64 rows, 3 bits 4.9 / 7.2; 1999 x 2720, 64 rows, 4 bits 10.3 / 11.9, 128 rows, 6 bits 19.6 / 19.4; beyond
+// 128 activation rows the K-split kernel reads the planes again for every 128, and wins on rows of less than 512 elements only.
+bool gemmb_beats_split(int M, long long N, int K, int b) {
+    if ((K & 127) == 0) return (K & 255) == 0 || K >= 640;
+    if (M > 256) return true;
+    if (M > 128) return K >= 512 || N >= 5120;
+    if (M > 64) return K >= (N >= 10240 || b <= 4 ? 512 : (N >= 5120 ? 768 : (N >= 2048 ? 2048 : 3072)));
+    if (M > 32) return K >= (N >= 10240 ? (b <= 4 ? 512 : 1024) : (N >= 5120 ? (b <= 4 ? 1536 : 3072) : 4096));
+    return K >= 512;
 }
 
 // Where it also beats dequant_kbit + a library GEMM, beyond what fused_gemm_pays says of the other forms (same sweep; pair / block, us): up to
@@ -1191,24 +1226,46 @@ int run_gemmt(const GemmtGeometry &geo, const uint16_t *x, int count, const uint
     return launch_status();
 }
 
-// Whether ap_gemm_kbit takes the block-tile kernel (N: rows of all linears of the launch).  The knobs of the tiled kernel come first: a
-// caller that forces or forbids it means this one too.
-bool takes_gemmb(int M, long long N, int K, int w_bits) {
+// Whether ap_gemm_kbit takes the block-tile kernel, and with which tile.  The knobs of the tiled kernel come first: a caller that forces or
+// forbids it means this one too.
+bool takes_gemmb(int M, int N, int K, int w_bits, GemmbGeometry *geo) {
     const int mode = knob(kGemmBlock);
-    return mode >= 2 || (mode > 0 && knob(kGemmTiled) == 1 && gemmb_pays(M, N, K, w_bits));
+    if (mode >= 2) return gemmb_geometry(M, &N, 1, K, w_bits, geo);
+    if (mode <= 0 || knob(kGemmTiled) != 1 || !gemmb_pays(M, N, K, w_bits) || !gemmb_geometry(M, &N, 1, K, w_bits, geo)) return false;
+    GemmtGeometry tiled;
+    if (gemmt_pays(M, N, K, w_bits) && gemmt_geometry(M, (N + 63) / 64, K, w_bits, &tiled)) return geo->us <= gemmt_us(tiled, K, w_bits);
+    return gemmb_beats_split(M, N, K, w_bits);
 }
 
-// The same for one launch over a set of `total` rows, `largest` in one member.  At 9..16 rows members of more than 8192 rows (gate/up), which
+// The same for one launch over a set (what ap_gemm_kbit_group does, and from 9 to 32 rows what ap_gemm_kbit_group_taken says).  The range is that
+// of one linear of all its rows.  At 9..16 rows members of more than 8192 rows (gate/up), which
 // would otherwise run one by one in the K-split kernel, take it where they have 20000 together and none more than two thirds of them
 // (9 rows / 16 rows, us one by one and here: 2 x 14336 x 4096 at 3 bits 27 / 25, 27 / 25, at 5 48 / 40, 47 / 40, at 8 63 / 58, 65 / 57;
 // 2 x 13824 x 5120 at 6 bits 57 / 53, 58 / 53) -- not at 4 bits on rows of less than 5120 elements (34 / 33, 32 / 33), at 5 and 6 bits below
 // 24000 rows only from 13 rows on (2 x 11008 x 4096, 5 bits: 34 / 36, 39 / 35), nor on rows of no multiple of 128 elements (62 / 67, 65 / 66).
 // The tiled kernel keeps sets of small members at 3 bits there (8192 + 2 x 1024 x 8192: 21.3 / 22.1).
-bool takes_gemmb_set(int M, long long total, long long largest, int K, int w_bits) {
-    if (M > 16 || largest <= 8192) return !(M <= 16 && w_bits == 3 && knob(kGemmBlock) == 1) && takes_gemmb(M, total, K, w_bits);
-    if (takes_gemmb(M, total, K, w_bits)) return true;
-    return knob(kGemmBlock) > 0 && knob(kGemmTiled) == 1 && M > 8 && K >= (w_bits == 4 ? 5120 : 4096) && (K & 127) == 0 &&
+bool gemmb_pays_set(int M, long long total, long long largest, int K, int w_bits) {
+    if (M <= 16 && w_bits == 3 && largest <= 8192) return false;
+    if (gemmb_pays(M, total, K, w_bits)) return true;
+    return M > 8 && M <= 16 && largest > 8192 && K >= (w_bits == 4 ? 5120 : 4096) && (K & 127) == 0 &&
            total >= (w_bits == 5 || w_bits == 6 ? (M > 12 ? 20000 : 24000) : 20000) && 3 * largest <= 2 * total;
+}
+bool takes_gemmb_set(int M, const int *N, int count, int K, int w_bits, GemmbGeometry *geo) {
+    const int mode = knob(kGemmBlock);
+    if (mode >= 2) return gemmb_geometry(M, N, count, K, w_bits, geo);
+    long long total = 0, tiles = 0;
+    int largest = 0;
+    for (int g = 0; g < count; g++) {
+        total += N[g];
+        tiles += (N[g] + 63) / 64;
+        largest = N[g] > largest ? N[g] : largest;
+    }
+    if (mode <= 0 || knob(kGemmTiled) != 1 || !gemmb_pays_set(M, total, largest, K, w_bits) || !gemmb_geometry(M, N, count, K, w_bits, geo)) return false;
+    GemmtGeometry tiled;
+    if (gemmt_set_pays(M, largest, K) && gemmt_geometry(M, tiles, K, w_bits, &tiled)) return geo->us <= gemmt_us(tiled, K, w_bits);
+    // One by one otherwise: the sum of their launches is less only on short rows of no multiple of 128 elements at few activation rows (us one
+    // by one / here: 2 x 5120 x 288, 38 rows, 6 bits 10.3 / 13.4; 2 x 12800 x 320, 63 rows, 3 bits 21.4 / 11.0; 2 x 11168 x 256, 18 rows, 7 bits 20.4 / 12.6).
+    return (K & 127) == 0 || K >= 512 || M > 64 || w_bits <= 4;
 }
 
 // One launch of the block-tile kernel over `count` linears (arguments already checked; geo from gemmb_geometry over all of them).
@@ -1247,7 +1304,7 @@ static int gemm_one(const uint16_t *x, const uint32_t *qweight, const uint16_t *
     drain_stale_error();
     {
         GemmbGeometry bgeo;
-        if (takes_gemmb(M, N, K, w_bits) && gemmb_geometry(M, &N, 1, K, w_bits, &bgeo)) {
+        if (takes_gemmb(M, N, K, w_bits, &bgeo)) {
             *added = bias != nullptr;
             return run_gemmb(bgeo, x, 1, &qweight, &lut, bias, &out, &N, nullptr, M, K, w_bits, static_cast<hipStream_t>(stream));
         }
@@ -1288,7 +1345,7 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
     if (!x || !qweight || !lut || !out || !N) return AP_ENULL;
     if (count < 1 || count > kGemmtMaxGroup) return AP_ELIMIT;
     if (M < 1) return AP_EBATCH;
-    long long tiles = 0, rows = 0, total = 0;  // tiles of all members; rows of the largest and of all
+    long long tiles = 0, rows = 0;  // tiles of all members; rows of the largest
     bool strided = false;
     for (int g = 0; g < count; g++) {
         if (!qweight[g] || !lut[g] || !out[g]) return AP_ENULL;
@@ -1299,7 +1356,6 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
         strided = strided || (ldo && ldo[g] != N[g]);
         tiles += (N[g] + 63) / 64;
         rows = N[g] > rows ? N[g] : rows;
-        total += N[g];
     }
     if (!aligned16(x)) return AP_EALIGN;
     drain_stale_error();
@@ -1314,11 +1370,10 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
     // At 9..32 rows, sets whose members have at most 8192 rows (q/k/v) take it too, in tiles of 16 or 32 activation rows
     // (7B q/k/v at 16 rows: 16-24 us against 23-26 at 3-5 bits; 13B: 20-40 against 36-68; 70B: 21-48 against 39-64); wide
     // members (gate/up) are within 10 % either way one by one.
-    const bool pays = M > 32 || (M > 8 && rows <= 8192 && K >= 1024);
-    // The block-tile kernel takes the set by the rule for one linear of all its rows.  (Rows of no multiple of 128 elements are
-    // served dense only.)
+    const bool pays = gemmt_set_pays(M, rows, K);
+    // (Rows of no multiple of 128 elements are served dense only.)
     GemmbGeometry bgeo;
-    if ((count > 1 || strided) && (!strided || (K & 127) == 0) && takes_gemmb_set(M, total, rows, K, w_bits) && gemmb_geometry(M, N, count, K, w_bits, &bgeo))
+    if ((count > 1 || strided) && (!strided || (K & 127) == 0) && takes_gemmb_set(M, N, count, K, w_bits, &bgeo))
         return run_gemmb(bgeo, x, count, qweight, lut, nullptr, out, N, ldo, M, K, w_bits, static_cast<hipStream_t>(stream));
     if (fits && (strided || (count > 1 && mode > 0 && (mode >= 2 || pays))))
         return run_gemmt(tgeo, x, count, qweight, lut, out, N, ldo, M, K, w_bits, static_cast<hipStream_t>(stream));
@@ -1418,7 +1473,9 @@ int ap_gemm_kbit_group_pays(int count, const int *N, int M, int K, int w_bits) {
 
 int ap_gemm_kbit_taken(int M, int N, int K, int w_bits) {
     const int rc = ap_gemm_kbit_pays(M, N, K, w_bits);
-    return rc != 0 ? rc : (takes_gemmb(M, N, K, w_bits) && gemmb_beats_pair(M, N, K, w_bits) ? 1 : 0);
+    if (rc != 0 || knob(kGemmBlock) <= 0 || (knob(kGemmBlock) == 1 && knob(kGemmTiled) != 1) || !gemmb_beats_pair(M, N, K, w_bits)) return rc;
+    GemmbGeometry block;  // by the block-tile kernel, or by what ap_gemm_kbit takes for it where that is faster still
+    return gemmb_geometry(M, &N, 1, K, w_bits, &block) ? 1 : 0;
 }
 
 int ap_gemm_kbit_group_taken(int count, const int *N, int M, int K, int w_bits) {
@@ -1429,9 +1486,10 @@ int ap_gemm_kbit_group_taken(int count, const int *N, int M, int K, int w_bits) 
         sum += N[g];
         largest = N[g] > largest ? N[g] : largest;
     }
+    GemmbGeometry geo;
     // up to 32 rows gate and up in one launch instead of two (2 x 11008 x 4096, 32 rows: 30 / 22 at 3 bits, 45 / 35 at 5, 64 / 47 at 8)
-    if (M > 8 && M <= 32) return count > 1 && K >= 4096 && sum >= 20000 && 3 * largest <= 2 * sum && takes_gemmb_set(M, sum, largest, K, w_bits) ? 1 : 0;
-    return M > 32 && M <= 512 && sum >= 4096 && takes_gemmb(M, sum, K, w_bits) && gemmb_beats_pair(M, sum, K, w_bits) ? 1 : 0;
+    if (M > 8 && M <= 32) return count > 1 && K >= 4096 && sum >= 20000 && 3 * largest <= 2 * sum && takes_gemmb_set(M, N, count, K, w_bits, &geo) ? 1 : 0;
+    return M > 32 && M <= 512 && sum >= 4096 && gemmb_beats_pair(M, sum, K, w_bits) && takes_gemmb_set(M, N, count, K, w_bits, &geo) ? 1 : 0;
 }
 
 int ap_matmul_kbit_route(int M, int N, int K, int w_bits, int *route) {

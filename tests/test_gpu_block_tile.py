@@ -198,6 +198,29 @@ def test_tiles_are_counted_on_the_xcd_that_has_most(ext):
     assert torch.equal(got[0], got[841]) and not torch.equal(got[0], got[442])
 
 
+# (N, K, rows, bits): one shape of each line that keeps a call with the kernels before this one, and one just across it.  Short rows: the
+# tiled kernel, and the K-split kernel on rows of no multiple of 128 elements; 2560 x 2560: tiles that do not go evenly over the XCDs.
+@pytest.mark.parametrize("N,K,M,b,block", (
+    (5696, 384, 107, 4, False), (3520, 256, 208, 6, False), (3520, 1280, 208, 6, True), (2560, 2560, 1395, 3, False), (2560, 2560, 512, 3, True),
+    (1181, 544, 98, 5, False), (1184, 3232, 98, 5, True), (4096, 480, 64, 3, False), (4096, 4128, 64, 3, True), (6000, 1120, 40, 4, False),
+    (6000, 1760, 40, 4, True), (6000, 2720, 40, 6, False), (12000, 992, 40, 6, False), (12000, 1056, 40, 6, True), (3000, 480, 200, 5, False),
+    (3000, 544, 200, 5, True), (6912, 384, 46, 6, False), (6912, 256, 46, 6, True), (2000, 288, 300, 5, True)))
+def test_who_serves_a_call(ext, N, K, M, b, block):
+    """Bit for bit the kernel that the rule names: the order of the additions tells the others' results from its own."""
+    from any_precision_amd import _capi
+    g = torch.Generator(device="cuda").manual_seed(N + K + M)
+    q = torch.randint(-2**31, 2**31, (b, N, K // 32), dtype=torch.int32, device="cuda", generator=g)
+    t = (torch.randn((N, 1 << b), device="cuda", generator=g) * 0.02).half()
+    x = torch.randn((M, K), device="cuda", generator=g).half()
+    got = ext.gemm_kbit(x, q, t, b)
+    with _capi.tuning(gemm_block=0):
+        others = ext.gemm_kbit(x, q, t, b)
+    with _capi.tuning(gemm_block=2):
+        own = ext.gemm_kbit(x, q, t, b)
+    assert not torch.equal(own, others)
+    assert torch.equal(got, own if block else others)
+
+
 # (members, K, rows, bits): gate and up in one launch from 9 rows on, and where the rule leaves them one by one
 @pytest.mark.parametrize("Ns,K,M,b,taken", (
     ((10016, 10000), 4096, 9, 3, 1), ((10016, 10000), 4096, 16, 8, 1), ((10016, 10000), 4096, 13, 5, 1), ((10016, 10000), 4096, 12, 5, 0),
