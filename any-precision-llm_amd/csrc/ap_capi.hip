@@ -693,6 +693,13 @@ double gemmt_us(const GemmtGeometry &geo, int K, int w_bits) {
     return c[0] + tile_rounds(geo.grid_n, geo.grid_m) * (c[1] + (K + 511) / 512 * c[2]);
 }
 
+// And for dequant_kbit + a library GEMM: the two launches, the weight written and read, the product, what the library takes per 1000
+// activation rows, and rounds of 256 x 256 tiles.  11 % off on average (the library's own choice of kernels).
+double pair_us(double M, double N, double K, int w_bits) {
+    const double tiles = ceil(N / 256) * ceil(M / 256);
+    return 11.6 + (0.89 + 0.007 * w_bits) * 1e-6 * N * K + 1.31e-9 * M * N * K + 3.5e-3 * M + 1.43e-3 * K * ceil(tiles / cu_count());
+}
+
 // Where the block-tile kernel beats the other fused forms (us there and here).  Beyond 256 activation rows on every linear of
 // 1024 rows or more (14336 x 4096, 512 rows: 90 / 62 at 3 bits, 114 / 70 at 5); from 129 rows on linears of 2048 rows or
 // more (11008 x 4096, 192 rows, 5 bits: 56 / 38), and from 65 of 4096 or more (4096 x 11008, 128 rows, 5 bits: 50 / 38); narrower
@@ -736,13 +743,14 @@ bool gemmb_beats_split(int M, long long N, int K, int b) {
     return K >= 512;
 }
 
-// Where it also beats dequant_kbit + a library GEMM, beyond what fused_gemm_pays says of the other forms (same sweep; pair / block, us): up to
+// Where it also beats dequant_kbit + a library GEMM, beyond what fused_gemm_pays says of the other forms (pair / block, us): up to
 // 256 rows wherever it is the best fused form (14336 x 4096, 256 rows, 8 bits: 84 / 55); up to 512 at 3 to 7 bits (14336 x 4096: 85 / 62 at
 // 3 bits, 89 / 70 at 5; 4096 x 14336: 117 / 86 at 5) except at 7 bits on sets of 16384 rows or more beyond 384, at 8 bits on linears
 // of 4096..16383 rows (14336 x 4096: 93 / 80; 2048 x 5504 37 / 53) or of at most 4096 elements a row; up to 1024 at 3 bits (4096 x 11008:
 // 131 / 97; 22016 x 4096 201 / 188), at 4 to 6 bits on linears of less than 10240 rows (4096 x 4096, 5 bits: 50 / 45; 14336 x 4096 121 / 143),
-// at 7 bits of 4096 rows or more with rows of 4096 elements or more among those, not at 8 (4096 x 11008, 1024 rows: 134 / 139);
-// up to 2048 at 3 bits on linears of at most 4096 rows (4096 x 11008: 189 / 171).
+// at 7 bits of 4096 rows or more with rows of 4096 elements or more among those, not at 8 bits;
+// up to 2048 at 3 bits on linears of at most 4096 rows (4096 x 11008: 189 / 171).  And there only where pair_us is not less (10 % of the
+// calls at other sizes than these were slower than the pair, up to 1.9 times).
 bool gemmb_beats_pair(int M, long long N, int K, int b) {
     if (!gemmb_pays(M, N, K, b)) return false;
     if (M <= 256) return b <= 7 || N >= 2048;
@@ -1474,22 +1482,28 @@ int ap_gemm_kbit_group_pays(int count, const int *N, int M, int K, int w_bits) {
 int ap_gemm_kbit_taken(int M, int N, int K, int w_bits) {
     const int rc = ap_gemm_kbit_pays(M, N, K, w_bits);
     if (rc != 0 || knob(kGemmBlock) <= 0 || (knob(kGemmBlock) == 1 && knob(kGemmTiled) != 1) || !gemmb_beats_pair(M, N, K, w_bits)) return rc;
-    GemmbGeometry block;  // by the block-tile kernel, or by what ap_gemm_kbit takes for it where that is faster still
-    return gemmb_geometry(M, &N, 1, K, w_bits, &block) ? 1 : 0;
+    // by the block-tile kernel, or by what ap_gemm_kbit takes for it where that is faster still
+    GemmbGeometry block;
+    GemmtGeometry tiled;
+    const double pair = pair_us(M, N, K, w_bits);
+    return (gemmb_geometry(M, &N, 1, K, w_bits, &block) && block.us <= pair) ||
+           (gemmt_pays(M, N, K, w_bits) && gemmt_geometry(M, (N + 63) / 64, K, w_bits, &tiled) && gemmt_us(tiled, K, w_bits) <= pair);
 }
 
 int ap_gemm_kbit_group_taken(int count, const int *N, int M, int K, int w_bits) {
     const int rc = ap_gemm_kbit_group_pays(count, N, M, K, w_bits);
     if (rc != 0) return rc;
     long long sum = 0, largest = 0;
+    double pairs = 0;  // one by one
     for (int g = 0; g < count; g++) {
         sum += N[g];
         largest = N[g] > largest ? N[g] : largest;
+        pairs += pair_us(M, N[g], K, w_bits);
     }
     GemmbGeometry geo;
     // up to 32 rows gate and up in one launch instead of two (2 x 11008 x 4096, 32 rows: 30 / 22 at 3 bits, 45 / 35 at 5, 64 / 47 at 8)
     if (M > 8 && M <= 32) return count > 1 && K >= 4096 && sum >= 20000 && 3 * largest <= 2 * sum && takes_gemmb_set(M, N, count, K, w_bits, &geo) ? 1 : 0;
-    return M > 32 && M <= 512 && sum >= 4096 && gemmb_beats_pair(M, sum, K, w_bits) && takes_gemmb_set(M, N, count, K, w_bits, &geo) ? 1 : 0;
+    return M > 32 && M <= 512 && sum >= 4096 && gemmb_beats_pair(M, sum, K, w_bits) && takes_gemmb_set(M, N, count, K, w_bits, &geo) && geo.us <= pairs ? 1 : 0;
 }
 
 int ap_matmul_kbit_route(int M, int N, int K, int w_bits, int *route) {

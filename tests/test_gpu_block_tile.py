@@ -177,6 +177,9 @@ def test_the_rule_keeps_to_its_range():
     assert taken(512, 14336, 4096, 5) == 1 and taken(1024, 14336, 4096, 5) == 0 and taken(1024, 4096, 14336, 5) == 1
     assert taken(2048, 4096, 4096, 3) == 1 and taken(2049, 4096, 4096, 3) == 0 and taken(512, 512, 4096, 5) == 0
     assert taken(256, 4096, 224, 5) == _capi.lib.ap_gemm_kbit_pays(256, 4096, 224, 5)     # shorter than a half-step
+    # inside the range, where the pair is faster (us pair / block tile: 31 / 49, 60 / 93, 47 / 62, 149 / 185)
+    for M, N, K, b in ((507, 2652, 2368, 8), (584, 6473, 4224, 5), (281, 10304, 2368, 8), (898, 8784, 7168, 6)):
+        assert taken(M, N, K, b) == 0, (M, N, K, b)
     assert taken(512, 4096, 4100, 5) == _capi.AP_ESHAPE and taken(0, 4096, 4096, 5) == _capi.AP_EBATCH
     with _capi.tuning(gemm_block=0):
         assert taken(512, 14336, 4096, 5) == 0
