@@ -1493,17 +1493,17 @@ int ap_gemm_kbit_taken(int M, int N, int K, int w_bits) {
 int ap_gemm_kbit_group_taken(int count, const int *N, int M, int K, int w_bits) {
     const int rc = ap_gemm_kbit_group_pays(count, N, M, K, w_bits);
     if (rc != 0) return rc;
-    long long sum = 0, largest = 0;
+    long long sum = 0;
     double pairs = 0;  // one by one
     for (int g = 0; g < count; g++) {
         sum += N[g];
-        largest = N[g] > largest ? N[g] : largest;
         pairs += pair_us(M, N[g], K, w_bits);
     }
     GemmbGeometry geo;
-    // up to 32 rows gate and up in one launch instead of two (2 x 11008 x 4096, 32 rows: 30 / 22 at 3 bits, 45 / 35 at 5, 64 / 47 at 8)
-    if (M > 8 && M <= 32) return count > 1 && K >= 4096 && sum >= 20000 && 3 * largest <= 2 * sum && takes_gemmb_set(M, N, count, K, w_bits, &geo) ? 1 : 0;
-    return M > 32 && M <= 512 && sum >= 4096 && gemmb_beats_pair(M, sum, K, w_bits) && takes_gemmb_set(M, N, count, K, w_bits, &geo) && geo.us <= pairs ? 1 : 0;
+    if ((M <= 32 ? count < 2 || M <= 8 : M > 512 || !gemmb_beats_pair(M, sum, K, w_bits)) || sum < 4096 || !takes_gemmb_set(M, N, count, K, w_bits, &geo)) return 0;
+    // Up to 32 rows one launch of the set is what ap_gemm_kbit_group makes, and faster than its members one by one (2 x 11008 x 4096, 32 rows:
+    // 30 / 22 at 3 bits, 45 / 35 at 5, 64 / 47 at 8; sets of 10240..20000 rows of 4096 elements or more 10-45 %).
+    return M <= 32 || geo.us <= pairs ? 1 : 0;
 }
 
 int ap_matmul_kbit_route(int M, int N, int K, int w_bits, int *route) {

@@ -140,8 +140,9 @@ int ap_linear_bias(const uint16_t *x, const uint32_t *qweight, const uint16_t *l
 int ap_gemm_kbit_pays(int M, int N, int K, int w_bits);
 int ap_gemm_kbit_group_pays(int count, const int *N, int M, int K, int w_bits);
 
-/* What AnyPrecisionLinear asks: 1 also where only the block-tile kernel that ap_gemm_kbit (ap_gemm_kbit_group) launches from 17
- * activation rows on beats ap_dequant_kbit + a library fp16 GEMM.  The pair takes part in automatic differentiation and the fused
+/* What AnyPrecisionLinear asks: 1 also where only the block-tile kernel that ap_gemm_kbit (ap_gemm_kbit_group) launches from 9
+ * activation rows on beats ap_dequant_kbit + a library fp16 GEMM; for a set of 9..32 rows, 1 wherever ap_gemm_kbit_group serves it by
+ * one launch of that kernel.  The pair takes part in automatic differentiation and the fused
  * GEMM does not: ap_gemm_kbit_pays says where the host module has always taken the fused form, these where it may for a plain
  * forward.  Argument errors as above. */
 int ap_gemm_kbit_taken(int M, int N, int K, int w_bits);
