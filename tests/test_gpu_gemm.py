@@ -204,8 +204,9 @@ def test_row_walking_kernel_agrees_with_the_oracle(ext, oracle):
 
 
 def test_row_walking_kernel_on_a_wide_linear_by_default(ext, oracle):
-    """14336 x 4096 at 8 bits and at 17..32 rows takes the walking kernel by the default rule; a slice of its
-    outputs against the oracle on the same rows."""
+    """14336 x 4096 at 8 bits and up to 16 rows takes the walking kernel by the default rule, at 17..32 rows by its own rule where the
+    block-tile kernel, which serves them by default, is off; a slice of the outputs of either against the oracle on the same rows."""
+    from any_precision_amd import _capi
     N, K = 14336, 4096
     L = make(N, K, seed=9)
     q, luts = layer_to_gpu(L)
@@ -216,6 +217,12 @@ def test_row_walking_kernel_on_a_wide_linear_by_default(ext, oracle):
         got = ext.gemm_kbit(xg, q, luts[b], b)
         _, want = oracle.matmul_kbit(x, L.qweight[:, rows], L.luts[b][rows], b, return_f64=True)
         assert_close_gemv(got[:, torch.from_numpy(rows).cuda()], want, f"N={N} K={K} b={b} M={M}")
+        with _capi.tuning(gemm_block=0, gemm_tiled=0):
+            by_rule = ext.gemm_kbit(xg, q, luts[b], b)
+        assert_close_gemv(by_rule[:, torch.from_numpy(rows).cuda()], want, f"block tile off N={N} K={K} b={b} M={M}")
+        with _capi.tuning(gemm_walk=2, gemm_block=0, gemm_tiled=0):
+            walked = ext.gemm_kbit(xg, q, luts[b], b)
+        assert torch.equal(by_rule, walked) and (M > 16 or torch.equal(got, walked)), (b, M)
 
 
 def test_tiled_kernel_agrees_with_the_oracle(ext, oracle):

@@ -29,6 +29,7 @@ def torch_indices(qweight, b):
 @pytest.mark.parametrize("N,K", [(28672, 8192), (8192, 28672)])
 def test_llama70b_mlp_shapes(N, K):
     import any_precision_ext as ext
+    from any_precision_amd import _capi
     gen = torch.Generator(device="cuda")
     gen.manual_seed(N)
     q = torch.randint(-2**31, 2**31 - 1, (8, N, K // 32), dtype=torch.int32, device="cuda", generator=gen)
@@ -39,22 +40,27 @@ def test_llama70b_mlp_shapes(N, K):
         got_w = ext.dequant_kbit(q, lut, b)
         assert torch.equal(got_w, want_w), f"dequant N={N} K={K} b={b}"
         del got_w
-        # 200 and 520 rows: the tiled GEMM (tiles of 64 x 128 rows here, four and five of them along the activation rows)
+        # 200 and 520 rows: the block-tile GEMM, and the tiled GEMM (tiles of 64 x 128 rows here, two and five of them along the
+        # activation rows)
         for M, fn in ((1, ext.matmul_kbit), (4, ext.matmul_kbit), (8, ext.matmul_kbit), (32, ext.gemm_kbit), (200, ext.gemm_kbit),
                       (520, ext.gemm_kbit)):
             x = torch.randn((M, K), device="cuda", generator=gen).half()
             want = x.double() @ want_w.double().T
-            got = fn(x, q, lut, b).double()
-            assert (got - want).norm() <= REL_TOL * want.norm(), f"{fn.__name__} M={M} b={b}"
-            assert (got - want).abs().max() <= REL_TOL * want.abs().max(), f"{fn.__name__} M={M} b={b}"
+            for knobs in (({}, {"gemm_block": 0, "gemm_tiled": 2}) if M > 32 else ({},)):
+                with _capi.tuning(**knobs):
+                    got = fn(x, q, lut, b).double()
+                assert (got - want).norm() <= REL_TOL * want.norm(), f"{fn.__name__} M={M} b={b} {knobs}"
+                assert (got - want).abs().max() <= REL_TOL * want.abs().max(), f"{fn.__name__} M={M} b={b} {knobs}"
         del want_w
 
 
 def test_llama3_8b_mlp_shape_under_the_default_routing():
     """14336 x 4096 at M = 1..8 under the default routing: the dot-product kernel (1, 2 and part of
     3), the 4x4x4 matrix-core kernel with one (3, 4) and two (5..8) groups of activation rows; then the
-    fused GEMM at 16, 32 and 48 rows (K-split kernel up to 32, tiled kernel beyond) and at 100 and 300."""
+    fused GEMM at 16, 32, 48, 100 and 300 rows, by default (block-tile kernel beyond 16) and with the block-tile kernel off (K-split and
+    row-walking kernels up to 32, tiled kernel beyond)."""
     import any_precision_ext as ext
+    from any_precision_amd import _capi
     N, K = 14336, 4096
     gen = torch.Generator(device="cuda")
     gen.manual_seed(5)
@@ -69,15 +75,15 @@ def test_llama3_8b_mlp_shape_under_the_default_routing():
             got = ext.matmul_kbit(x, q, lut, b).double()
             assert (got - want).norm() <= REL_TOL * want.norm(), f"M={M} b={b}"
             assert (got - want).abs().max() <= REL_TOL * want.abs().max(), f"M={M} b={b}"
-        # the fused GEMM under its default routing: two weight-row blocks per workgroup at up to 5 / 6
-        # bits, chunks of 32 activation rows above 32
         for M in (16, 32, 48, 100, 300):
             print(f"llama3 mlp gemm b={b} M={M}", flush=True)
             x = torch.randn((M, K), device="cuda", generator=gen).half()
             want = x.double() @ want_w.T
-            got = ext.gemm_kbit(x, q, lut, b).double()
-            assert (got - want).norm() <= REL_TOL * want.norm(), f"gemm M={M} b={b}"
-            assert (got - want).abs().max() <= REL_TOL * want.abs().max(), f"gemm M={M} b={b}"
+            for block in (1, 0):
+                with _capi.tuning(gemm_block=block):
+                    got = ext.gemm_kbit(x, q, lut, b).double()
+                assert (got - want).norm() <= REL_TOL * want.norm(), f"gemm M={M} b={b} block={block}"
+                assert (got - want).abs().max() <= REL_TOL * want.abs().max(), f"gemm M={M} b={b} block={block}"
         del want_w
 
 

@@ -341,3 +341,29 @@ def test_a_bias_in_the_launch_is_the_bias_added_afterwards(N, K):
             lin.register_buffer("bias", bias.clone())
             assert torch.equal(got, want + bias), (N, K, M, b)
     assert _capi.lib.ap_linear_bias(None, None, None, None, None, 1, 8, 32, 3, None, None) == _capi.AP_ENULL
+
+
+# (N, K, rows, bits, knobs, added): the dot-product, K-split and block-tile kernels take the bias along; the row-streaming, fine, 4x4x4,
+# row-walking and tiled kernels and launches in chunks leave it to the caller
+@pytest.mark.parametrize("N,K,M,b,knobs,added", (
+    (1999, 2720, 3, 6, {}, 1), (1024, 4096, 1, 4, {}, 1), (512, 2048, 8, 5, {"matmul_mfma4": 0, "matmul_mfma_from": 9}, 1),
+    (1024, 4096, 16, 4, {"gemm_block": 0, "gemm_tiled": 0, "gemm_walk": 0}, 1), (1024, 4096, 8, 4, {"matmul_mfma4": 0, "matmul_mfma_from": 4}, 1),
+    (4096, 4096, 128, 5, {"gemm_block": 2}, 1), (1999, 2720, 300, 6, {"gemm_block": 2}, 1),
+    (14336, 4096, 8, 8, {"matmul_mfma4": 2}, 0), (4096, 4096, 2, 8, {"gemv_stream": 2}, 0), (1024, 4096, 4, 4, {"gemv_fine": 2}, 0),
+    (14336, 4096, 16, 8, {"gemm_block": 0, "gemm_tiled": 0, "gemm_walk": 2}, 0),
+    (4096, 4096, 128, 5, {"gemm_block": 0, "gemm_tiled": 2}, 0), (1024, 2720, 200, 5, {"gemm_block": 0}, 0)))
+def test_which_kernels_take_the_bias_along(N, K, M, b, knobs, added):
+    import ctypes
+    import any_precision_ext as ext
+    from any_precision_amd import _capi
+    g = torch.Generator(device="cuda").manual_seed(N + M)
+    q = torch.randint(-2**31, 2**31, (b, N, K // 32), dtype=torch.int32, device="cuda", generator=g)
+    t = (torch.randn((N, 1 << b), device="cuda", generator=g) * 0.02).half()
+    x, bias = torch.randn((M, K), device="cuda", generator=g).half(), (torch.randn(N, device="cuda", generator=g) * 4).half()
+    out, flag = torch.empty((M, N), dtype=torch.float16, device="cuda"), ctypes.c_int(-1)
+    with _capi.tuning(**knobs):
+        rc = _capi.lib.ap_linear_bias(x.data_ptr(), q.data_ptr(), t.data_ptr(), bias.data_ptr(), out.data_ptr(), M, N, K, b,
+                                      torch.cuda.current_stream().cuda_stream, ctypes.byref(flag))
+        want = (ext.matmul_kbit if M <= 8 else ext.gemm_kbit)(x, q, t, b)
+    assert rc == 0 and flag.value == added
+    assert torch.equal(out, want + bias if added else want)

@@ -2,9 +2,10 @@
 
 Two routes compute ``x @ dequant(qweight, lut, b).T`` (the reference's branch for more than 8 rows,
 any_precision/modules/AnyPrecisionLinear.py:60-62): the module's forward (``dequant_kbit`` + library GEMM at this
-size) and ``gemm_kbit`` (the fused tiled kernel, here with tiles of 128 activation rows and 128 tiles along the
-rows, the order of tiles that grids of more than 8 row tiles take).  Both are checked against the oracle on a
-slice (128 weight rows x 256 sampled activation rows) and against each other over the whole [16384, N] result.
+size) and ``gemm_kbit``: the fused block-tile kernel, which serves this size, and the tiled kernel with tiles of 128 activation
+rows, 128 of them along the rows (the order of tiles that grids of more than 8 row tiles take, in either kernel).  All are
+checked against the oracle on a slice (128 weight rows x 256 sampled activation rows) and against the module over the
+whole [16384, N] result.
 Tolerance: 1e-2 relative, normwise and against the largest magnitude (fp32 accumulate, fp16 out).
 """
 import numpy as np
@@ -21,7 +22,7 @@ PREFILL_ROWS = 32 * 512
 @pytest.mark.parametrize("N,K", [(4096, 4096), (11008, 4096), (4096, 11008)])
 def test_prefill_16384_rows_module_and_fused_gemm(N, K, oracle):
     import any_precision_ext as ext
-    from any_precision_amd import AnyPrecisionLinear, synth
+    from any_precision_amd import AnyPrecisionLinear, _capi, synth
     from any_precision_amd.packing import pack_codes
 
     rng = np.random.default_rng(N + K)
@@ -51,25 +52,28 @@ def test_prefill_16384_rows_module_and_fused_gemm(N, K, oracle):
         lin._buffers[f"lut{b}"] = table
         y_mod = lin(x, precision=b)
         assert y_mod.shape == (32, 512, N) and y_mod.dtype == torch.float16
-        y_fused = ext.gemm_kbit(x, q, table, b)
-        assert y_fused.shape == (32, 512, N)
-        torch.cuda.synchronize()
-
         sel = torch.from_numpy(pick).cuda()
-        for name, y in (("module", y_mod), ("gemm_kbit", y_fused)):
-            got = y.view(PREFILL_ROWS, N)[sel][:, rows]
-            assert_close_gemv(got, want, f"{name} N={N} K={K} b={b} vs oracle")
-        # the two routes over the whole result (chunks of rows keep the fp32 temporaries small)
-        a, c = y_mod.view(PREFILL_ROWS, N), y_fused.view(PREFILL_ROWS, N)
-        num = den = 0.0
-        worst = top = 0.0
-        for m0 in range(0, PREFILL_ROWS, 2048):
-            fa, fc = a[m0:m0 + 2048].float(), c[m0:m0 + 2048].float()
-            assert torch.isfinite(fa).all() and torch.isfinite(fc).all()
-            num += float((fa - fc).double().pow(2).sum())
-            den += float(fa.double().pow(2).sum())
-            worst = max(worst, float((fa - fc).abs().max()))
-            top = max(top, float(fa.abs().max()))
-        assert num ** 0.5 <= REL_TOL * den ** 0.5, f"module vs gemm_kbit N={N} K={K} b={b}: {num ** 0.5 / den ** 0.5:.3e}"
-        assert worst <= REL_TOL * top, f"module vs gemm_kbit N={N} K={K} b={b}: max abs {worst:.3e} of {top:.3e}"
-        del y_mod, y_fused, lin, table
+        assert_close_gemv(y_mod.view(PREFILL_ROWS, N)[sel][:, rows], want, f"module N={N} K={K} b={b} vs oracle")
+        for name, knobs in (("gemm_kbit", {"gemm_block": 2}), ("tiled", {"gemm_block": 0, "gemm_tiled": 2, "gemm_tile": 8})):
+            with _capi.tuning(**knobs):
+                y_fused = ext.gemm_kbit(x, q, table, b)
+            assert y_fused.shape == (32, 512, N)
+            torch.cuda.synchronize()
+            assert_close_gemv(y_fused.view(PREFILL_ROWS, N)[sel][:, rows], want, f"{name} N={N} K={K} b={b} vs oracle")
+            # the two routes over the whole result (chunks of rows keep the fp32 temporaries small)
+            a, c = y_mod.view(PREFILL_ROWS, N), y_fused.view(PREFILL_ROWS, N)
+            num = den = 0.0
+            worst = top = 0.0
+            for m0 in range(0, PREFILL_ROWS, 2048):
+                fa, fc = a[m0:m0 + 2048].float(), c[m0:m0 + 2048].float()
+                assert torch.isfinite(fa).all() and torch.isfinite(fc).all()
+                num += float((fa - fc).double().pow(2).sum())
+                den += float(fa.double().pow(2).sum())
+                worst = max(worst, float((fa - fc).abs().max()))
+                top = max(top, float(fa.abs().max()))
+            assert num ** 0.5 <= REL_TOL * den ** 0.5, f"module vs {name} N={N} K={K} b={b}: {num ** 0.5 / den ** 0.5:.3e}"
+            assert worst <= REL_TOL * top, f"module vs {name} N={N} K={K} b={b}: max abs {worst:.3e} of {top:.3e}"
+            if name == "gemm_kbit":
+                assert torch.equal(y_fused, ext.gemm_kbit(x, q, table, b)), f"not the block-tile kernel by default: N={N} K={K} b={b}"
+            del y_fused
+        del y_mod, lin, table
