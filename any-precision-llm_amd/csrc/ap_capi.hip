@@ -600,6 +600,7 @@ bool gemmt_geometry(int M, long long tiles_n, int K, int w_bits, GemmtGeometry *
 // 18-36 us against 28-41), from 17 at 3 bits (8192 x 8192 at 32 rows: 19.7 against 21.9); the rest (up to 4096 rows)
 // from 33 rows on at 3 and 4 bits (4096 x 4096 at 64 rows: 13-15 us against 19), from 49 at 5 bits (4096 x 11008 at 64
 // rows: 45 against 50), 65 at 6, 81 at 7 and 8 (4096 x 11008 at 96 rows, 8 bits: 68 against 75).
+// (This ranks the tiled kernel against the K-split one.  Most of the linears named here go to the block-tile kernel by now, takes_gemmb.)
 bool gemmt_pays(int M, int N, int K, int w_bits) {
     if ((N >= 8192 && K <= 4096) || N > 10240) return M > 16 || (M > 8 && N <= 16384 && (w_bits <= 4 || K > 4096));
     if (N >= 5120 && K > 4096) return M > 32 || (M > 16 && w_bits == 3);
@@ -776,6 +777,9 @@ int run_gemm(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, co
         // activation rows at low bit-widths: their short waves hide the lookup latency better).
         // With two steps per wave it needs twice the rows (28672 x 8192: 5-21 %; on 13824 x 5120 the two-block
         // one-shot kernel is up to 20 % faster).
+        // (By default the block-tile kernel comes first beyond 16 rows except on rows of less than 4096 elements of linears below 20000 rows,
+        // and at 9..16 rows of 8192 elements or more: what reaches this rule there is short rows, 4 bits on 20000 rows or more, and calls
+        // with that kernel off.)
         const bool pays = gemmw_geometry(M, N, K, w_bits, &wgeo) && N >= 40 * wgeo.spw * cu_count() &&
                           (wgeo.spw == 1 ? (M > 16 || w_bits == 8) : (M > 8 || (M >= 5 && w_bits <= 4)));
         if (mode > 0 && (mode >= 2 ? gemmw_geometry(M, N, K, w_bits, &wgeo) : pays)) {
@@ -1126,7 +1130,9 @@ int plan_matmul(int M, const int *N, int count, int K, int w_bits, uint16_t *con
 //  - other row lengths (the K-split kernel only): up to 64 on linears of fewer than 8192 rows, and on larger ones at up
 //    to 5 bits -- except, on rows of more than 4096 elements, from 6 bits on linears of 5120 rows or more and from 5
 //    bits on linears of at most 2048 rows; up to 128 on linears of 4096..8191 rows of at most 4096 elements.
-// Beyond, one table lookup per weight and tile of activation rows costs more than materialising the weight once.
+// Beyond, one table lookup per weight and tile of these kernels' activation rows costs more than materialising the weight once.
+// The figures are those of the K-split and tiled kernels.  The rule stays as it is drawn on them, also where the block-tile kernel serves the
+// call by now (14336 x 4096, 256 rows, 8 bits: fused 55, pair 84): it says where calls that autograd or autocast follows are fused.
 bool fused_gemm_pays(int M, int N, int K, int b) {
     if (M <= 32) return true;
     if ((K & 127) == 0 && M <= 512) {
@@ -1152,6 +1158,7 @@ bool fused_gemm_pays(int M, int N, int K, int b) {
 // dequant + GEMM pairs; gate/up at 8 bits: 96 against 115 for the pairs), up to 256 at up to 6 bits (gate/up at 5 bits:
 // 105 against 145) and, at 7 and 8 bits, where every member has fewer than 8192 rows (q/k/v at 8 bits: 94 against 114;
 // gate/up: 145 against 149); up to 512 at 3 bits where no member has more than 8192 rows, as each member alone would.
+// (Figures of the tiled kernel's one launch; the block-tile kernel makes most of these launches by now, takes_gemmb_set.)
 bool fused_set_pays(int M, const int *N, int count, int K, int b) {
     long long sum = 0;
     int hi = 0;
