@@ -739,7 +739,7 @@ bool gemmb_beats_split(int M, long long N, int K, int b) {
     if ((K & 127) == 0) return (K & 255) == 0 || K >= 640;
     if (M > 256) return true;
     if (M > 128) return K >= 512 || N >= 5120;
-    if (M > 64) return K >= (N >= 10240 || b <= 4 ? 512 : (N >= 5120 ? 768 : (N >= 2048 ? 2048 : 3072)));
+    if (M > 64) return K >= (N >= 10240 || b <= 4 ? 512 : (N >= 5120 ? 768 : (M > 96 ? 1536 : 4096)));
     if (M > 32) return K >= (N >= 10240 ? (b <= 4 ? 512 : 1024) : (N >= 5120 ? (b <= 4 ? 1536 : 3072) : 4096));
     return K >= 512;
 }

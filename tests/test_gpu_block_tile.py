@@ -177,7 +177,7 @@ def test_the_rule_keeps_to_its_range():
     assert taken(512, 14336, 4096, 5) == 1 and taken(1024, 14336, 4096, 5) == 0 and taken(1024, 4096, 14336, 5) == 1
     assert taken(2048, 4096, 4096, 3) == 1 and taken(2049, 4096, 4096, 3) == 0 and taken(512, 512, 4096, 5) == 0
     assert taken(256, 4096, 224, 5) == _capi.lib.ap_gemm_kbit_pays(256, 4096, 224, 5)     # shorter than a half-step
-    # inside the range, where the pair is faster (us pair / block tile: 31 / 49, 60 / 93, 47 / 62, 149 / 185)
+    # inside the range, where the pair is faster (us pair / block tile: 31 / 33, 60 / 73, 47 / 56, 152 / 198)
     for M, N, K, b in ((507, 2652, 2368, 8), (584, 6473, 4224, 5), (281, 10304, 2368, 8), (898, 8784, 7168, 6)):
         assert taken(M, N, K, b) == 0, (M, N, K, b)
     assert taken(512, 4096, 4100, 5) == _capi.AP_ESHAPE and taken(0, 4096, 4096, 5) == _capi.AP_EBATCH
@@ -205,7 +205,7 @@ def test_tiles_are_counted_on_the_xcd_that_has_most(ext):
 # tiled kernel, and the K-split kernel on rows of no multiple of 128 elements; 2560 x 2560: tiles that do not go evenly over the XCDs.
 @pytest.mark.parametrize("N,K,M,b,block", (
     (5696, 384, 107, 4, False), (3520, 256, 208, 6, False), (3520, 1280, 208, 6, True), (2560, 2560, 1395, 3, False), (2560, 2560, 512, 3, True),
-    (1181, 544, 98, 5, False), (1184, 3232, 98, 5, True), (4096, 480, 64, 3, False), (4096, 4128, 64, 3, True), (6000, 1120, 40, 4, False),
+    (1181, 544, 98, 5, False), (1184, 3232, 98, 5, True), (1999, 2720, 128, 6, True), (1999, 2720, 80, 6, False), (4096, 480, 64, 3, False), (4096, 4128, 64, 3, True), (6000, 1120, 40, 4, False),
     (6000, 1760, 40, 4, True), (6000, 2720, 40, 6, False), (12000, 992, 40, 6, False), (12000, 1056, 40, 6, True), (3000, 480, 200, 5, False),
     (3000, 544, 200, 5, True), (6912, 384, 46, 6, False), (6912, 256, 46, 6, True), (2000, 288, 300, 5, True)))
 def test_who_serves_a_call(ext, N, K, M, b, block):
