@@ -568,6 +568,7 @@ bool gemmt_geometry(int M, long long tiles_n, int K, int w_bits, GemmtGeometry *
         // bits against 52 / 56 / 73 with one group of waves per 64-row tile); at 4 bits, whose two-half form has the
         // pair table, from 1.5 tiles per CU (up to there two rounds of that form: 44 us against 47); at 3 bits from 3
         // tiles per CU (one group of waves per 64-row tile is as fast up to there).
+        // (What reaches these tiles by default: rows of up to about 1024 elements, and linears of less than 1024 rows -- takes_gemmb.)
         const long long cus = cu_count();
         if (w_bits == 3 ? small >= 3 * cus : (w_bits == 4 ? 2 * small > 3 * cus : small > cus)) mbw = 8;
     }
@@ -616,7 +617,7 @@ constexpr int kGemmbTileCount = sizeof(kGemmbTiles) / sizeof(kGemmbTiles[0]);
 
 // Rounds of tiles over the CUs: workgroups go to the 8 XCDs in turn, and both tiled kernels number their tiles so that those of one block of
 // weight rows run on one XCD.  So the XCDs with one block more decide: 20 blocks are 3 on four XCDs and 2 on the others (2560 x 2560 at
-// 1395 rows, 128 x 128 tiles: 220 tiles are 33 for 32 CUs, two rounds, 43 us where one round of 192 would be 24).
+// 1395 rows, 128 x 128 tiles: 220 tiles are 33 for 32 CUs, two rounds, 43 us at 3 bits; one round of 180 tiles, 1026 rows, is 22).
 inline long long tile_rounds(long long tiles_n, long long tiles_m) {
     const long long cus = cu_count() < 8 ? 1 : cu_count() / 8;  // of an XCD
     return ((tiles_n + 7) / 8 * tiles_m + cus - 1) / cus;
@@ -702,20 +703,20 @@ double pair_us(double M, double N, double K, int w_bits) {
 }
 
 // Where the block-tile kernel beats the other fused forms (us there and here).  Beyond 256 activation rows on every linear of
-// 1024 rows or more (14336 x 4096, 512 rows: 90 / 62 at 3 bits, 114 / 70 at 5); from 129 rows on linears of 2048 rows or
-// more (11008 x 4096, 192 rows, 5 bits: 56 / 38), and from 65 of 4096 or more (4096 x 11008, 128 rows, 5 bits: 50 / 38); narrower
-// ones at 5 to 7 bits (1024 x 4096, 128 rows, 5 bits: 20 / 16; at 3 bits 12 / 13), at 8 bits from 2048 rows on.  At 33..64
-// rows on linears of 5120 rows or more (6144 x 4096, 48 rows, 5 bits: 27 / 17), on narrower ones where the 16-row tiles of the tiled kernel
+// 1024 rows or more (14336 x 4096, 512 rows: 93 / 62 at 3 bits, 118 / 71 at 5); from 129 rows on linears of 2048 rows or
+// more (11008 x 4096, 192 rows, 5 bits: 58 / 36), and from 65 of 4096 or more (4096 x 11008, 128 rows, 5 bits: 50 / 36); narrower
+// ones at 5 to 7 bits (1024 x 4096, 128 rows, 5 bits: 17.6 / 14.5; at 3 bits 12.2 / 11.8), at 8 bits from 2048 rows on.  At 33..64
+// rows on linears of 5120 rows or more (6144 x 4096, 48 rows, 5 bits: 27 / 16), on narrower ones where the 16-row tiles of the tiled kernel
 // wait for their lookups: 5 to 7 bits beyond 48 rows, or on rows of more than 4096 elements; 8 bits on both (4096 x 4096,
-// 48 rows: 18 / 23).  Rows of no multiple of 128 elements, which the tiled kernel does not take: on linears of less than
-// 5120 rows up to 4 bits from 33 activation rows on, else from 65 (4096 x 11040, 128 rows: 98 / 35 at 3 bits, 104 / 60 at 8).  From 17
-// rows on linears and sets of 10240 rows or more (22016 x 4096, 24 rows, 4 bits: 41 / 30; 12288 x 4096: 17.9 / 15.9; 10240 x 8192, 5 bits:
-// 52 / 32; 14336 x 4096 at 6 bits a tie, 26.9 / 26.6; 8192 x 8192 up to 6 bits and 4096 x 11008 lose, 29.4 / 30.8 and 24 / 25), of 20000 on
-// shorter rows; from 9 where these have 8192 elements or more (10240 x 8192, 16 rows: 28 / 22, 43 / 32, 61 / 42; 28672 x 8192: 50 / 40 and
-// 124 / 96, at 4 bits 54 / 55 at 9 rows); 4096 elements are not enough there (22016 x 4096, 4 bits: 25 / 30).
+// 48 rows: 18 / 22).  Rows of no multiple of 128 elements, which the tiled kernel does not take: on linears of less than
+// 5120 rows up to 4 bits from 33 activation rows on, else from 65 (4096 x 11040, 128 rows: 69 / 32 at 3 bits, 88 / 57 at 8).  From 17
+// rows on linears and sets of 10240 rows or more (24 rows: 22016 x 4096, 4 bits 42 / 30; 12288 x 4096, 4 bits 17.9 / 15.5; 10240 x 8192, 5 bits
+// 53 / 32; 14336 x 4096, 6 bits a tie, 27.1 / 26.3; 8192 x 8192 and 4096 x 11008, 5 bits lose, 29.3 / 30.4 and 27 / 30), of 20000 on
+// shorter rows; from 9 where these have 8192 elements or more (10240 x 8192, 16 rows: 28 / 22, 43 / 31, 60 / 43; 28672 x 8192: 49 / 40 and
+// 124 / 95, at 4 bits 53 / 55 at 9 rows); 4096 elements are not enough there (22016 x 4096, 16 rows, 4 bits: 25 / 30).
 // Within that range each other form keeps what it does faster (takes_gemmb): the lines above were drawn on rows of 2048 elements and more, and
-// by them alone 10 % of the calls at other sizes lost, up to 2.7 times (7.1 / 10.6 us on 1181 x 544, 98 rows, 5 bits; 6.8 / 9.2 on 5696 x
-// 384, 107 rows, 4 bits; 21 / 28 on 2560 x 2560, 705 rows, 3 bits).
+// by them alone 10 % of the calls at other sizes lost, up to 2.7 times (7.1 / 10.4 us on 1181 x 544, 98 rows, 5 bits; 7.2 / 9.2 on 5696 x
+// 384, 107 rows, 4 bits).
 bool gemmb_pays(int M, long long N, int K, int b) {
     if (N < 1024 || M <= 8 || K < 256) return false;
     if ((long long)M * K * 2 > 0xffffffffLL || N * (K >> 5) * 4 > 0xffffffffLL) return false;  // its 32-bit offsets
@@ -732,9 +733,9 @@ bool gemmb_pays(int M, long long N, int K, int b) {
 }
 
 // Against the K-split kernel, whose time has no simple form: on short rows it wins, the more so the fewer weight rows and activation rows
-// there are and the more bits (the block tile's tables and its first loads are not paid back).  us K-split / block tile at the edges: 1181 x 544,
-// 98 rows, 5 bits 7.1 / 10.6; 4096 x 480, 64 rows, 3 bits 4.9 / 7.2; 1999 x 2720, 64 rows, 4 bits 10.3 / 11.9, 128 rows, 6 bits 19.6 / 19.4; beyond
-// 128 activation rows the K-split kernel reads the planes again for every 128, and wins on rows of less than 512 elements only.
+// there are and the more bits (the block tile's tables and its first loads are not paid back).  us K-split / block tile: 1181 x 544, 98 rows,
+// 5 bits 7.1 / 10.4; 4096 x 480, 64 rows, 3 bits 5.4 / 7.6; 1999 x 2720 at 64 rows, 4 bits 11.8 / 12.6, at 128 rows, 6 bits 20.0 / 17.5; beyond
+// 128 activation rows the K-split kernel reads the planes again for every 128, and wins on narrow linears of less than 512 elements a row only.
 bool gemmb_beats_split(int M, long long N, int K, int b) {
     if ((K & 127) == 0) return (K & 255) == 0 || K >= 640;
     if (M > 256) return true;
@@ -745,13 +746,13 @@ bool gemmb_beats_split(int M, long long N, int K, int b) {
 }
 
 // Where it also beats dequant_kbit + a library GEMM, beyond what fused_gemm_pays says of the other forms (pair / block, us): up to
-// 256 rows wherever it is the best fused form (14336 x 4096, 256 rows, 8 bits: 84 / 55); up to 512 at 3 to 7 bits (14336 x 4096: 85 / 62 at
-// 3 bits, 89 / 70 at 5; 4096 x 14336: 117 / 86 at 5) except at 7 bits on sets of 16384 rows or more beyond 384, at 8 bits on linears
-// of 4096..16383 rows (14336 x 4096: 93 / 80; 2048 x 5504 37 / 53) or of at most 4096 elements a row; up to 1024 at 3 bits (4096 x 11008:
-// 131 / 97; 22016 x 4096 201 / 188), at 4 to 6 bits on linears of less than 10240 rows (4096 x 4096, 5 bits: 50 / 45; 14336 x 4096 121 / 143),
+// 256 rows wherever it is the best fused form (14336 x 4096, 256 rows, 8 bits: 84 / 53); up to 512 at 3 to 7 bits (14336 x 4096: 86 / 62 at
+// 3 bits, 88 / 71 at 5; 4096 x 14336: 118 / 83 at 5) except at 7 bits on sets of 16384 rows or more beyond 384, at 8 bits on linears
+// of 4096..16383 rows (14336 x 4096: 92 / 78; 2048 x 5504 37 / 36) or of at most 4096 elements a row; up to 1024 at 3 bits (4096 x 11008:
+// 128 / 90; 22016 x 4096 204 / 193), at 4 to 6 bits on linears of less than 10240 rows (4096 x 4096, 5 bits: 51 / 45; 14336 x 4096 117 / 141),
 // at 7 bits of 4096 rows or more with rows of 4096 elements or more among those, not at 8 bits;
-// up to 2048 at 3 bits on linears of at most 4096 rows (4096 x 11008: 189 / 171).  And there only where pair_us is not less (10 % of the
-// calls at other sizes than these were slower than the pair, up to 1.9 times).
+// up to 2048 at 3 bits on linears of at most 4096 rows (4096 x 11008: 190 / 164).  And there only where pair_us is not less: at sizes between
+// these the pair was faster in 10 % of the calls, up to 1.9 times (6473 x 4224, 584 rows, 5 bits: 60 / 73; 8784 x 7168, 898 rows, 6 bits: 152 / 198).
 bool gemmb_beats_pair(int M, long long N, int K, int b) {
     if (!gemmb_pays(M, N, K, b)) return false;
     if (M <= 256) return b <= 7 || N >= 2048;
@@ -1132,7 +1133,7 @@ int plan_matmul(int M, const int *N, int count, int K, int w_bits, uint16_t *con
 //    bits on linears of at most 2048 rows; up to 128 on linears of 4096..8191 rows of at most 4096 elements.
 // Beyond, one table lookup per weight and tile of these kernels' activation rows costs more than materialising the weight once.
 // The figures are those of the K-split and tiled kernels.  The rule stays as it is drawn on them, also where the block-tile kernel serves the
-// call by now (14336 x 4096, 256 rows, 8 bits: fused 55, pair 84): it says where calls that autograd or autocast follows are fused.
+// call by now (14336 x 4096, 256 rows, 8 bits: fused 53, pair 84): it says where calls that autograd or autocast follows are fused.
 bool fused_gemm_pays(int M, int N, int K, int b) {
     if (M <= 32) return true;
     if ((K & 127) == 0 && M <= 512) {
@@ -1255,10 +1256,10 @@ bool takes_gemmb(int M, int N, int K, int w_bits, GemmbGeometry *geo) {
 // The same for one launch over a set (what ap_gemm_kbit_group does, and from 9 to 32 rows what ap_gemm_kbit_group_taken says).  The range is that
 // of one linear of all its rows.  At 9..16 rows members of more than 8192 rows (gate/up), which
 // would otherwise run one by one in the K-split kernel, take it where they have 20000 together and none more than two thirds of them
-// (9 rows / 16 rows, us one by one and here: 2 x 14336 x 4096 at 3 bits 27 / 25, 27 / 25, at 5 48 / 40, 47 / 40, at 8 63 / 58, 65 / 57;
-// 2 x 13824 x 5120 at 6 bits 57 / 53, 58 / 53) -- not at 4 bits on rows of less than 5120 elements (34 / 33, 32 / 33), at 5 and 6 bits below
-// 24000 rows only from 13 rows on (2 x 11008 x 4096, 5 bits: 34 / 36, 39 / 35), nor on rows of no multiple of 128 elements (62 / 67, 65 / 66).
-// The tiled kernel keeps sets of small members at 3 bits there (8192 + 2 x 1024 x 8192: 21.3 / 22.1).
+// (9 rows / 16 rows, us one by one and here: 2 x 14336 x 4096 at 3 bits 26 / 25, 26 / 25, at 5 47 / 43, 46 / 42, at 8 61 / 56, 63 / 55;
+// 2 x 13824 x 5120 at 6 bits 57 / 52, 58 / 52) -- not at 4 bits on rows of less than 5120 elements (2 x 14336 x 4096: 32 / 31, 32 / 31), at 5 and 6
+// bits below 24000 rows only from 13 rows on (2 x 11008 x 4096, 5 bits: 33 / 35, 38 / 35), nor on rows of no multiple of 128 elements (12000 +
+// 10000 x 4128, 6 bits: 46 / 51, 50 / 52).  The tiled kernel keeps sets of small members at 3 bits there (8192 + 2 x 1024 x 8192: 21.4 / 22.3).
 bool gemmb_pays_set(int M, long long total, long long largest, int K, int w_bits) {
     if (M <= 16 && w_bits == 3 && largest <= 8192) return false;
     if (gemmb_pays(M, total, K, w_bits)) return true;
@@ -1279,7 +1280,7 @@ bool takes_gemmb_set(int M, const int *N, int count, int K, int w_bits, GemmbGeo
     GemmtGeometry tiled;
     if (gemmt_set_pays(M, largest, K) && gemmt_geometry(M, tiles, K, w_bits, &tiled)) return geo->us <= gemmt_us(tiled, K, w_bits);
     // One by one otherwise: the sum of their launches is less only on short rows of no multiple of 128 elements at few activation rows (us one
-    // by one / here: 2 x 5120 x 288, 38 rows, 6 bits 10.3 / 13.4; 2 x 12800 x 320, 63 rows, 3 bits 21.4 / 11.0; 2 x 11168 x 256, 18 rows, 7 bits 20.4 / 12.6).
+    // by one / here: 2 x 5120 x 288, 38 rows, 6 bits 10.0 / 11.4; 2 x 12800 x 320, 63 rows, 3 bits 21 / 10; 2 x 11168 x 256, 18 rows, 7 bits 20 / 9).
     return (K & 127) == 0 || K >= 512 || M > 64 || w_bits <= 4;
 }
 
@@ -1509,7 +1510,7 @@ int ap_gemm_kbit_group_taken(int count, const int *N, int M, int K, int w_bits) 
     GemmbGeometry geo;
     if ((M <= 32 ? count < 2 || M <= 8 : M > 512 || !gemmb_beats_pair(M, sum, K, w_bits)) || sum < 4096 || !takes_gemmb_set(M, N, count, K, w_bits, &geo)) return 0;
     // Up to 32 rows one launch of the set is what ap_gemm_kbit_group makes, and faster than its members one by one (2 x 11008 x 4096, 32 rows:
-    // 30 / 22 at 3 bits, 45 / 35 at 5, 64 / 47 at 8; sets of 10240..20000 rows of 4096 elements or more 10-45 %).
+    // 30 / 22 at 3 bits, 45 / 35 at 5, 63 / 47 at 8; sets of 10240..20000 rows of 4096 elements or more 8-45 %).
     return M <= 32 || geo.us <= pairs ? 1 : 0;
 }
 

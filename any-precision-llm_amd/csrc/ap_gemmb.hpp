@@ -17,11 +17,11 @@
 //     arithmetic at the start of a half-step, loads by all waves behind the barrier, planes at once (4096 x 4096, 128 rows, 128 x 128
 //     tile, 5 bits: 45 us so, 43 with reads interleaved only, 38 with the loads spread and half the barriers, 36 fenced,
 //     33 with waits that leave the stages ahead outstanding).
-// What bounds it now (same tile, 5 bits): matrix cores alone 14 us, with the vector instructions 15.5, with the LDS reads 24, and 7 for
-// launch, tables, first loads and the sums at the end.
+// What bounds it (same tile, 5 bits, taken on the form of 36 us): matrix cores alone 14 us, with the vector instructions 15.5, with the LDS reads 24, and 7
+// for launch, tables, first loads and the sums at the end.
 // Measured (us, planes from HBM; before = the better of tiled kernel and dequantise + library product), rows / 3 / 5 / 8 bits:
-//   4096 x 11008, 128: 32 -> 31, 52 -> 39, 71 -> 52;   512: 82 -> 61, 98 -> 70, 103 -> 98
-//   14336 x 4096, 192: 41 -> 31, 58 -> 41, 76 -> 50;   512: 85 -> 62, 89 -> 70, 93 -> 80 (0.97 / 0.86 / 0.75 PFLOP/s)
+//   4096 x 11008, 128: 34 -> 26, 53 -> 37, 71 -> 49;   512: 81 -> 57, 99 -> 67, 102 -> 91
+//   14336 x 4096, 192: 41 -> 29, 58 -> 38, 77 -> 49;   512: 88 -> 62, 88 -> 71, 92 -> 79 (0.98 / 0.85 / 0.77 PFLOP/s)
 #pragma once
 #include <type_traits>
 
