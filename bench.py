@@ -838,7 +838,7 @@ def routing_audit(args, torch, _capi, synth):
                 if us["default"] > 1.05 * us[best]:
                     losses.append(dict(case, excess=round(us["default"] / us[best] - 1, 3)))
         # the fused GEMM of ap_gemm_kbit on the same weights: one or two row blocks per workgroup, the row-walking kernel,
-        # the tiled kernel
+        # the tiled kernel, the block-tile kernel
         for b in bits:
             for M in ((16, 32, 48, 64, 96, 128) if args.audit_gemm else ()):
                 x = torch.randn((M, K), device="cuda", generator=gen).to(torch.float16)
@@ -855,7 +855,8 @@ def routing_audit(args, torch, _capi, synth):
                 us = {"default": _graph_us(torch, side, gemm, reps)}
                 for name, knobs in (("one_block", {"gemm_tiled": 0, "gemm_walk": 0, "gemm_rb2": 0}),
                                     ("two_blocks", {"gemm_tiled": 0, "gemm_walk": 0, "gemm_rb2": 2}),
-                                    ("walking", {"gemm_tiled": 0, "gemm_walk": 2}), ("tiled", {"gemm_tiled": 2})):
+                                    ("walking", {"gemm_tiled": 0, "gemm_walk": 2}), ("tiled", {"gemm_tiled": 2}),
+                                    ("block_tile", {"gemm_block": 2})):
                     if name == "tiled" and K % 128:
                         continue
                     with _capi.tuning(**knobs):
@@ -918,7 +919,7 @@ def routing_audit(args, torch, _capi, synth):
                     if us["default"] > 1.05 * us[best]:
                         losses.append(dict(case, excess=round(us["default"] / us[best] - 1, 3)))
             # the same sets through ap_gemm_kbit_group at 16, 32, 48 and 128 rows: the default against one launch of the
-            # tiled kernel and against a launch per member
+            # tiled kernel, one of the block-tile kernel and against a launch per member
             for b in (bits if args.audit_gemm else ()):
                 for M in (16, 32, 48, 128):
                     x = torch.randn((M, K), device="cuda", generator=gen).to(torch.float16)
@@ -946,6 +947,8 @@ def routing_audit(args, torch, _capi, synth):
                     if K % 128 == 0:
                         with _capi.tuning(gemm_tiled=2):
                             us["one_tiled_launch"] = _graph_us(torch, side, gemm_set, reps)
+                    with _capi.tuning(gemm_block=2):
+                        us["one_block_tile_launch"] = _graph_us(torch, side, gemm_set, reps)
                     us["default"] = min(us["default"], _graph_us(torch, side, gemm_set, reps))
                     best = min((k for k in us if k != "default"), key=lambda k: us[k])
                     case = {"entry": "ap_gemm_kbit_group", "N": list(Ns), "K": K, "w_bits": b, "M": M,
