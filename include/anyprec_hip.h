@@ -103,8 +103,8 @@ int ap_matmul_kbit_swiglu(const uint16_t *x, const uint32_t *qweight_gate, const
  * each); from 81 rows on, and from 9..65 rows on where it measured faster, a tiled kernel whose
  * workgroups own 64 weight rows x 16..128 activation rows (the narrower the fewer tiles the grid
  * has) for the whole of K, ONE launch for any M (it needs K % 128 == 0; other row lengths go through the K-split kernel in chunks of 128 rows,
- * in order, on the same stream); from 9 rows on on wide linears, and nearly everywhere from 65, a block-tile kernel that rebuilds
- * a weight once per tile of up to 256 activation rows, ONE launch for any M and K >= 256.  Correct for every M; faster than dequant +
+ * in order, on the same stream); from 9 rows on on wide linears, and from 65 nearly everywhere on rows of
+ * 1024 elements or more, a block-tile kernel that rebuilds a weight once per tile of up to 256 activation rows, ONE launch for any M and K >= 256.  Correct for every M; faster than dequant +
  * a library GEMM up to 256..2048 rows (ap_gemm_kbit_taken) -- beyond that use that pair.
  * fp32 accumulation, fp16 result. */
 int ap_gemm_kbit(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut,
