@@ -12,7 +12,7 @@ LIB_PATH = os.path.join(_PKG_ROOT, "lib", "libanyprec_hip.so")
 
 AP_OK = 0
 AP_ENULL, AP_EBITS, AP_ESHAPE, AP_EALIGN, AP_EBATCH, AP_ELIMIT, AP_EKNOB = -1, -2, -3, -4, -5, -6, -7
-AP_ABI_VERSION = 11
+AP_ABI_VERSION = 12
 
 if not os.path.exists(LIB_PATH):
     raise ModuleNotFoundError(
@@ -75,6 +75,8 @@ lib.ap_gemm_kbit_pays.argtypes = [_ci, _ci, _ci, _ci]
 lib.ap_gemm_kbit_pays.restype = _ci
 lib.ap_linear_bias.argtypes = [_vp, _vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp, _pi]
 lib.ap_linear_bias.restype = _ci
+lib.ap_linear.argtypes = [_vp, _vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp, _pi]
+lib.ap_linear.restype = _ci
 lib.ap_gemm_kbit_taken.argtypes = [_ci, _ci, _ci, _ci]
 lib.ap_gemm_kbit_taken.restype = _ci
 lib.ap_gemm_kbit_group_taken.argtypes = [_ci, _pi, _ci, _ci, _ci]
@@ -83,9 +85,13 @@ lib.ap_gemm_kbit_group_pays.argtypes = [_ci, _pi, _ci, _ci, _ci]
 lib.ap_gemm_kbit_group_pays.restype = _ci
 lib.ap_matmul_kbit_group.argtypes = [_vp, _ci, _pvp, _pvp, _pvp, _pi, _ci, _ci, _ci, _vp]
 lib.ap_matmul_kbit_group.restype = _ci
+lib.ap_linear_staged.argtypes = [_ci, _pi, _ci, _ci, _ci]
+lib.ap_linear_staged.restype = _ci
 _pll = ctypes.POINTER(ctypes.c_longlong)
 lib.ap_gemm_kbit_group.argtypes = [_vp, _ci, _pvp, _pvp, _pvp, _pi, _pll, _ci, _ci, _ci, _vp]
 lib.ap_gemm_kbit_group.restype = _ci
+lib.ap_linear_group.argtypes = lib.ap_gemm_kbit_group.argtypes
+lib.ap_linear_group.restype = _ci
 lib.ap_matmul_kbit_geometry.argtypes = [_ci, _ci, _ci, _ci, _pi, _pi, _pi, _pi]
 lib.ap_matmul_kbit_geometry.restype = _ci
 lib.ap_probe_stream.argtypes = [_vp, ctypes.c_longlong, _vp, ctypes.c_longlong, _vp, _ci, _vp]
@@ -127,7 +133,7 @@ if lib.ap_abi_version() != AP_ABI_VERSION:
 EXPORTS = ("ap_abi_version", "ap_strerror", "ap_dequant_kbit", "ap_matmul_kbit", "ap_matmul_kbit_group",
            "ap_gemm_kbit", "ap_matmul_kbit_geometry", "ap_set_tuning", "ap_get_tuning", "ap_probe_stream", "ap_probe_empty", "ap_probe_write", "ap_matmul_kbit_route", "ap_matmul_kbit_group_route",
            "ap_add_rmsnorm", "ap_silu_mul", "ap_decode_attention", "ap_matmul_kbit_swiglu", "ap_decode_advance", "ap_gemm_kbit_group", "ap_dequant_kbit_group", "ap_gemm_kbit_pays",
-           "ap_gemm_kbit_group_pays", "ap_gemm_kbit_taken", "ap_gemm_kbit_group_taken", "ap_linear_bias", "ap_prompt_rope", "ap_prompt_attention", "ap_rope_heads")
+           "ap_gemm_kbit_group_pays", "ap_gemm_kbit_taken", "ap_gemm_kbit_group_taken", "ap_linear_bias", "ap_linear", "ap_linear_group", "ap_linear_staged", "ap_prompt_rope", "ap_prompt_attention", "ap_rope_heads")
 GEMM_MAX_M = 128
 GROUP_MAX = 4
 DEQUANT_GROUP_MAX = 8

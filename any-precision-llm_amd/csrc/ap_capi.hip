@@ -9,6 +9,7 @@
 #include "ap_dequant.hpp"
 #include "ap_gemm_launch.hpp"
 #include "ap_gemmb_launch.hpp"
+#include "ap_gemms_launch.hpp"
 #include "ap_gemmt_launch.hpp"
 #include "ap_gemmw_launch.hpp"
 #include "ap_gemv4_launch.hpp"
@@ -50,6 +51,7 @@ enum {
     kGemmLookahead,     // K-split fused GEMM, lookups one word ahead of the matrix instructions: 0 never, 1 where it pays, 2 wherever the variant exists
     kGemmBlock,         // block-tile fused GEMM (ap_gemm_kbit): 0 never, 1 where it pays, 2 wherever it fits
     kGemmBlockTile,     // > 0: its tile, 100 x blocks of 32 activation rows + 10 x waves over the weight rows + groups over K
+    kGemmStaged,        // staged K-split fused GEMM (up to 32 rows): 0 never, 1 where it pays, 2 wherever it fits
     kKnobCount
 };
 Knob g_knobs[kKnobCount] = {
@@ -59,7 +61,7 @@ Knob g_knobs[kKnobCount] = {
     {"gemv_fine", 1},
     {"gemm_walk", 1},             {"gemm_walk_wgs", 1},  {"gemm_tiled", 1},   {"gemm_tile", 0},
     {"gemm_tile_split", 0},       {"gemm_lookahead", 1},
-    {"gemm_block", 1},            {"gemm_block_tile", 0},
+    {"gemm_block", 1},            {"gemm_block_tile", 0}, {"gemm_staged", 1},
 };
 inline int knob(int k) { return __atomic_load_n(&g_knobs[k].value, __ATOMIC_RELAXED); }
 
@@ -763,6 +765,61 @@ bool gemmb_beats_pair(int M, long long N, int K, int b) {
     return b <= 6 || (b == 7 && N >= 4096 && K >= 4096);
 }
 
+// The staged K-split kernel serves rows of a multiple of 128 elements and up to 32 activation rows, with 32-bit offsets.
+bool gemms_fits(int M, const int *N, int count, int K) {
+    if (M < 1 || M > kGemmsMaxM || (K & 127) != 0 || count > kGemmsMaxGroup || (long long)M * K * 2 > 0xffffffffLL) return false;
+    long long blocks = 0;
+    for (int g = 0; g < count; g++) {
+        if ((long long)N[g] * (K >> 5) * 4 > 0xffffffffLL) return false;
+        blocks += (N[g] + kGemmsRows - 1) / kGemmsRows;
+    }
+    return blocks <= 0x7fffffffLL;
+}
+
+
+// What a launch of the staged kernel takes at 9..16 and at 17..32 activation rows, in us: a + h s + g (p + h q) + w c, where h = the steps of 512
+// elements of the busiest wave, g = workgroups of a CU (at least 1) and w = steps x workgroups a wave slot of all CUs has.  {a, s, p, q, c} per
+// bit-width, non-negative least squares over 4200 calls: linears and sets of 256..30000 rows of 512..16384 elements; 6 % off on average.
+constexpr float kGemmsCost[6][2][5] = {
+    {{2.19f, 0.49f, 1.37f, 0.45f, 0.49f}, {2.25f, 0.73f, 1.34f, 0.76f, 0.75f}},
+    {{2.58f, 0.45f, 1.12f, 0.62f, 0.69f}, {2.38f, 0.55f, 1.25f, 1.13f, 0.79f}},
+    {{2.89f, 0.40f, 0.82f, 1.10f, 0.70f}, {2.47f, 0.80f, 1.32f, 1.20f, 0.92f}},
+    {{2.68f, 0.66f, 0.99f, 1.00f, 0.92f}, {2.64f, 0.96f, 1.16f, 1.19f, 1.26f}},
+    {{2.91f, 0.60f, 0.79f, 1.34f, 0.96f}, {2.85f, 0.77f, 0.96f, 1.72f, 1.22f}},
+    {{3.03f, 0.57f, 0.67f, 1.52f, 1.08f}, {2.61f, 0.93f, 1.22f, 1.66f, 1.52f}}
+};
+double gemms_us(int M, long long blocks, int K, int w_bits) {
+    const float *c = kGemmsCost[w_bits - 3][M > 16 ? 1 : 0];
+    const int T = (K + 511) / 512, h = (T + kGemmsWaves - 1) / kGemmsWaves;
+    const double cus = cu_count(), load = fmax(1.0, blocks / cus);
+    return c[0] + h * c[1] + load * (c[2] + h * c[3]) + blocks * T / (cus * kGemmsWaves) * c[4];
+}
+
+// One launch of the staged kernel over `count` linears (arguments already checked; takes_gemms).
+int run_gemms(const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut, const uint16_t *bias, uint16_t *const *out,
+              const int *N, const long long *ldo, int M, int K, int w_bits, hipStream_t st) {
+    GemmsMembers mem = {};
+    mem.bias = bias;
+    mem.count = count;
+    for (int g = 0; g < count; g++) {
+        mem.qweight[g] = qweight[g];
+        mem.lut[g] = lut[g];
+        mem.out[g] = out[g];
+        mem.N[g] = N[g];
+        mem.ldo[g] = ldo ? ldo[g] : N[g];
+        mem.block0[g + 1] = mem.block0[g] + (N[g] + kGemmsRows - 1) / kGemmsRows;
+    }
+    switch (w_bits) {
+        case 3: launch_gemms<3>(x, mem, M, K, st); break;
+        case 4: launch_gemms<4>(x, mem, M, K, st); break;
+        case 5: launch_gemms<5>(x, mem, M, K, st); break;
+        case 6: launch_gemms<6>(x, mem, M, K, st); break;
+        case 7: launch_gemms<7>(x, mem, M, K, st); break;
+        default: launch_gemms<8>(x, mem, M, K, st); break;
+    }
+    return launch_status();
+}
+
 // Launch of the fused dequant -> MFMA kernel (arguments already checked).  *added: whether the launch has added `bias` (of N, or null) to its
 // results; what is left as it is -- the row-walking kernel, several launches -- is the caller's to add.
 int run_gemm(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, const uint16_t *bias, uint16_t *out, int M, int N, int K,
@@ -1284,6 +1341,72 @@ bool takes_gemmb_set(int M, const int *N, int count, int K, int w_bits, GemmbGeo
     return (K & 127) == 0 || K >= 512 || M > 64 || w_bits <= 4;
 }
 
+// Where the staged kernel beats the others (`total` rows of all members; count > 1: one launch of the set against what serves it else).  Drawn on
+// 3060 linears and 1140 sets (sizes as in gemms_us; us before / staged):
+//  - from 9 rows on nearly everywhere -- it has the K-split kernel's workgroups without its re-read of the activations in runs of 64 bytes and its
+//    bank conflicts (4096 x 11008 at 16 rows: 17.6 / 11.0 at 3 bits, 27.3 / 21.0 at 8; 1024 x 4096, 3 bits 7.3 / 5.6; at 32 rows, 3 bits 22 / 15) --
+//    but short rows, where the tables are not paid back, and beyond 8192 rows, where the kernels that share a tile of activations between 64 weight
+//    rows or more may be faster: there the estimates decide (14336 x 4096 at 3 bits: 12.9 / 14.4 at 16 rows; 14.7 / 18.8 at 32), and rows that
+//    only the K-split kernel serves otherwise are the staged kernel's from 1280 elements on (17408 x 1152, 28 rows, 6 bits 21.4 / 17.9; 16752 x 1536,
+//    4 bits 23.0 / 15.1).  Sets of up to 8192 rows always: the others take their members one by one (3 x 4096 x 4096 at 16 rows, 3 bits 15.5 / 10.4);
+//  - at 5..8 rows beyond 2048 rows (4096 x 4096 at 8 rows 6.5 / 5.4 at 3 bits, 10.3 / 9.2 at 8; 4096 x 14336, 5 bits 22.5 / 14.5; 11008 x 4096,
+//    3 bits 13.1 / 9.4), fewer only where the rows are long (1600 x 11392, 7 rows, 3 bits 12.1 / 9.9): on few workgroups the dot-product kernel's short
+//    waves win (1024 x 4096 at 8 rows, 5 bits 5.7 / 6.3);
+//  - at 3 and 4 rows on long rows, at few bits (4096 x 14336 at 4 rows, 4 bits 15.6 / 11.3; 8 bits 22 / 19.5 but 16432 x 6784, 6 bits 32 / 35), sets at
+//    few bits (2 x 11008 x 4096, 4 rows, 3 bits 18 / 14); not at 2 (0.9-1.4 times as long).
+bool gemms_pays(int M, const int *N, int count, int K, int b) {
+    long long total = 0, blocks = 0, tiles = 0;
+    int largest = 0;
+    for (int g = 0; g < count; g++) {
+        total += N[g];
+        blocks += (N[g] + kGemmsRows - 1) / kGemmsRows;
+        tiles += (N[g] + 63) / 64;
+        largest = N[g] > largest ? N[g] : largest;
+    }
+    if (M < 3) return false;
+    if (M == 3) {
+        if (count > 1) return b == 3 && total > 8192;
+        return K > 8192 ? (b <= 4 ? total > 2048 : b <= 6 && total > 2560 && total <= 4096) : b <= 4 && total > 8192 && K > 4096;
+    }
+    if (M == 4) {
+        if (total <= 2048 || K < 4096) return false;
+        if (count > 1) return total > 8192 ? b <= 5 || (b == 6 && total > 12288) : b == 3;
+        if (K > 8192) return b <= 6 || (total > 3072 && total <= 4096);
+        return K > 4096 ? total > 4096 && (b <= 4 || (b <= 6 && total > 8192 && total <= 16384)) : b <= 4 && total > 8192;
+    }
+    if (M <= 8) {
+        if (count > 1 && M == 5 && b >= 5) return false;
+        if (total > 2048) return K > 1024 || (b <= 4 && total <= 4096);
+        return count == 1 && total > 1024 && M >= 7 && ((K > 8192 && b <= 6) || (K > 4096 && b <= 4));
+    }
+    if (total <= 8192) return count > 1 ? K > 1024 || total <= 4096 || M <= 16 : K > 1024 || (total <= 4096 && (b <= 4 || M > 16));
+    if (K <= 1024) return false;
+    GemmbGeometry block;
+    GemmtGeometry tiled;
+    if (K > 1536 && (M <= 16 ? b >= 5 : b >= 7 && count == 1)) return true;
+    if (count > 1 ? takes_gemmb_set(M, N, count, K, b, &block) : takes_gemmb(M, N[0], K, b, &block))
+        return gemms_us(M, blocks, K, b) <= block.us;
+    if ((count > 1 ? gemmt_set_pays(M, largest, K) : gemmt_pays(M, N[0], K, b)) && gemmt_geometry(M, tiles, K, b, &tiled))
+        return gemms_us(M, blocks, K, b) <= gemmt_us(tiled, K, b);
+    return b >= 5 || (K > 1152 && (total <= 12288 || K > 1536));
+}
+
+// Whether the staged kernel takes a linear or a set in one launch: by its rule in ap_linear and ap_linear_group (`linear`).  ap_gemm_kbit and
+// ap_matmul_kbit keep to the kernels that they have always named, whose sums a caller may hold to each other bit for bit.  A caller that forces or
+// forbids another kernel means this one too.
+bool takes_gemms(int M, const int *N, int count, int K, int w_bits, bool linear) {
+    const int mode = knob(kGemmStaged);
+    if (mode <= 0 || !gemms_fits(M, N, count, K)) return false;
+    if (mode >= 2) return true;
+    if (!linear) return false;
+    static const int others[] = {kGemmSplit, kGemmRb2, kGemmWalk, kGemmTiled, kGemmTile, kGemmTileSplit, kGemmLookahead, kGemmBlock, kGemmBlockTile,
+                                 kMatmulMfmaFrom, kMatmulMfma4, kGemvStream, kGemvFine, kGemvRows, kGemvWpl, kGemvTargetWaves, kGemv4Groups};
+    static const int defaults[] = {0, 1, 1, 1, 0, 0, 1, 1, 0, 5, 1, 1, 1, 0, 0, 16384, 0};
+    for (int i = 0; i < (int)(sizeof others / sizeof others[0]); i++)
+        if (knob(others[i]) != defaults[i]) return false;
+    return gemms_pays(M, N, count, K, w_bits);
+}
+
 // One launch of the block-tile kernel over `count` linears (arguments already checked; geo from gemmb_geometry over all of them).
 int run_gemmb(const GemmbGeometry &geo, const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut,
               const uint16_t *bias, uint16_t *const *out, const int *N, const long long *ldo, int M, int K, int w_bits, hipStream_t st) {
@@ -1311,13 +1434,17 @@ int run_gemmb(const GemmbGeometry &geo, const uint16_t *x, int count, const uint
 }
 
 static int gemm_one(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, const uint16_t *bias, uint16_t *out, int M, int N, int K,
-                    int w_bits, void *stream, bool *added) {
+                    int w_bits, void *stream, bool *added, bool linear = false) {
     if (!x || !qweight || !lut || !out) return AP_ENULL;
     const int rc = check_common(N, K, w_bits);
     if (rc != AP_OK) return rc;
     if (M < 1) return AP_EBATCH;
     if (!aligned16(x) || !aligned16(qweight) || !aligned16(lut)) return AP_EALIGN;
     drain_stale_error();
+    if (takes_gemms(M, &N, 1, K, w_bits, linear)) {
+        *added = bias != nullptr;
+        return run_gemms(x, 1, &qweight, &lut, bias, &out, &N, nullptr, M, K, w_bits, static_cast<hipStream_t>(stream));
+    }
     {
         GemmbGeometry bgeo;
         if (takes_gemmb(M, N, K, w_bits, &bgeo)) {
@@ -1356,8 +1483,19 @@ int ap_linear_bias(const uint16_t *x, const uint32_t *qweight, const uint16_t *l
     return rc;
 }
 
-int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut,
-                       uint16_t *const *out, const int *N, const long long *ldo, int M, int K, int w_bits, void *stream) {
+int ap_linear(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, const uint16_t *bias, uint16_t *out, int M, int N, int K, int w_bits,
+              void *stream, int *added) {
+    if (!added) return AP_ENULL;
+    bool with = false;
+    const int rc = M <= 8 && !(check_common(N, K, w_bits) == AP_OK && takes_gemms(M, &N, 1, K, w_bits, true))
+                       ? matmul_set(x, 1, &qweight, &lut, bias, &out, &N, M, K, w_bits, stream, &with)
+                       : gemm_one(x, qweight, lut, bias, out, M, N, K, w_bits, stream, &with, true);
+    *added = with ? 1 : 0;
+    return rc;
+}
+
+static int gemm_set(const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut, uint16_t *const *out, const int *N,
+                    const long long *ldo, int M, int K, int w_bits, void *stream, bool linear) {
     if (!x || !qweight || !lut || !out || !N) return AP_ENULL;
     if (count < 1 || count > kGemmtMaxGroup) return AP_ELIMIT;
     if (M < 1) return AP_EBATCH;
@@ -1388,6 +1526,8 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
     // members (gate/up) are within 10 % either way one by one.
     const bool pays = gemmt_set_pays(M, rows, K);
     // (Rows of no multiple of 128 elements are served dense only.)
+    if ((count > 1 || strided) && takes_gemms(M, N, count, K, w_bits, linear))
+        return run_gemms(x, count, qweight, lut, nullptr, out, N, ldo, M, K, w_bits, static_cast<hipStream_t>(stream));
     GemmbGeometry bgeo;
     if ((count > 1 || strided) && (!strided || (K & 127) == 0) && takes_gemmb_set(M, N, count, K, w_bits, &bgeo))
         return run_gemmb(bgeo, x, count, qweight, lut, nullptr, out, N, ldo, M, K, w_bits, static_cast<hipStream_t>(stream));
@@ -1397,10 +1537,21 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
     // forced tile beyond its geometry a limit (the caller may still ask for dense results)
     if (strided) return (K & 127) != 0 ? AP_ESHAPE : AP_ELIMIT;
     for (int g = 0; g < count; g++) {
-        const int r = ap_gemm_kbit(x, qweight[g], lut[g], out[g], M, N[g], K, w_bits, stream);
+        bool added = false;
+        const int r = gemm_one(x, qweight[g], lut[g], nullptr, out[g], M, N[g], K, w_bits, stream, &added, linear);
         if (r != AP_OK) return r;
     }
     return AP_OK;
+}
+
+int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut,
+                       uint16_t *const *out, const int *N, const long long *ldo, int M, int K, int w_bits, void *stream) {
+    return gemm_set(x, count, qweight, lut, out, N, ldo, M, K, w_bits, stream, false);
+}
+
+int ap_linear_group(const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut, uint16_t *const *out, const int *N,
+                    const long long *ldo, int M, int K, int w_bits, void *stream) {
+    return gemm_set(x, count, qweight, lut, out, N, ldo, M, K, w_bits, stream, true);
 }
 
 int ap_matmul_kbit(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, uint16_t *out, int M, int N,
@@ -1467,6 +1618,17 @@ static int matmul_set(const uint16_t *x, int count, const uint32_t *const *qweig
         if (r != AP_OK) return r;
     }
     return AP_OK;
+}
+
+int ap_linear_staged(int count, const int *N, int M, int K, int w_bits) {
+    if (!N) return AP_ENULL;
+    if (count < 1 || count > kGemmsMaxGroup) return AP_ELIMIT;
+    for (int g = 0; g < count; g++) {
+        const int rc = check_common(N[g], K, w_bits);
+        if (rc != AP_OK) return rc;
+    }
+    if (M < 1) return AP_EBATCH;
+    return takes_gemms(M, N, count, K, w_bits, true) ? 1 : 0;
 }
 
 int ap_gemm_kbit_pays(int M, int N, int K, int w_bits) {

@@ -107,6 +107,18 @@ __device__ __forceinline__ void store_at_nt(global_ptr<T> base, uint32_t byte, c
     __builtin_nontemporal_store(v, (global_ptr<V>)((global_ptr<char>)base + byte));
 }
 
+// 16 bytes a lane straight into LDS: from byte lane_offset + offset (the second wave-uniform) of the `bytes` at `base` to dst + 16 lane.
+// A buffer instruction and not global_load_lds: that one is of the FLAT family to the compiler, which then takes every wait of the
+// kernel, for LDS and for memory, for all that is outstanding (its counts of the two no longer say which of them a FLAT access holds), and
+// with it an operand requested ahead is waited for with the one that is needed.
+__device__ __forceinline__ void load_to_lds(uint64_t base, uint32_t bytes, __attribute__((address_space(3))) void *dst, uint32_t lane_offset,
+                                            uint32_t offset) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (the host pass has no such type)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)bytes, 0x00020000), dst, 16, lane_offset,
+                                             offset, 0, 0);
+#endif
+}
+
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {
     const int moved = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true);

@@ -217,8 +217,8 @@ bool tensors_of(PyObject *module_dict, int bits, ModuleTensors *m) {
     return is_tensor(m->qweight) && is_tensor(m->table) && (m->bias == nullptr || is_tensor(m->bias));
 }
 
-// linear(module.__dict__, x, w_bits): AnyPrecisionLinear.forward.  Up to 8 rows ap_matmul_kbit, then
-// ap_gemm_kbit where ap_gemm_kbit_pays, or ap_gemm_kbit_taken and nothing but plain execution follows the call; else the weight in fp16 and
+// linear(module.__dict__, x, w_bits): AnyPrecisionLinear.forward.  ap_linear up to 8 rows, and beyond
+// where ap_gemm_kbit_pays, or ap_gemm_kbit_taken and nothing but plain execution follows the call; else the weight in fp16 and
 // torch's own product (which takes part in autograd and autocast).
 PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (n != 3 || !is_tensor(args[1])) return none();
@@ -251,11 +251,8 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
             if (pays) {
                 const Tensor dense = x.is_contiguous() ? x : x.contiguous();  // the kernels take dense rows
                 out = result_for(x, w.N);
-                if (fused_bias)
-                    rc = ap_linear_bias(half_ptr(dense), w.planes, w.lut, half_ptr(bias), half_out(out), (int)rows, w.N, w.K, bits, on.stream, &added);
-                else
-                    rc = rows <= 8 ? ap_matmul_kbit(half_ptr(dense), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream)
-                                   : ap_gemm_kbit(half_ptr(dense), w.planes, w.lut, half_out(out), (int)rows, w.N, w.K, bits, on.stream);
+                rc = ap_linear(half_ptr(dense), w.planes, w.lut, fused_bias ? half_ptr(bias) : nullptr, half_out(out), (int)rows, w.N, w.K, bits,
+                               on.stream, &added);
             } else {
                 op = "dequant_kbit";
                 const Tensor dense = empty_half({w.N, w.K}, x.device());
@@ -270,8 +267,8 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
 }
 
 // linear_group(__dict__ of 2..4 modules, x, w_bits, concat as a bool): forward_group for bias-free linears of one input length.  A list of
-// results, or with concat one tensor of them side by side.  Up to 8 rows ap_matmul_kbit_group, beyond one launch of the tiled
-// GEMM where ap_gemm_kbit_group_pays; None where the modules are better called one by one.
+// results, or with concat one tensor of them side by side.  ap_linear_group where ap_linear_staged or, beyond 8 rows, where
+// ap_gemm_kbit_group_pays or _taken; up to 8 rows ap_matmul_kbit_group else; None where the modules are better called one by one.
 PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
     constexpr int MOST = 4;
     if (n != 4 || !PyTuple_Check(args[0]) || !is_tensor(args[1])) return none();
@@ -302,11 +299,11 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
         const int64_t rows = rows_of(given, w[0]);
         const int K = w[0].K;
         if (rows < 1) return none();
-        const bool gemm = rows > 8;
-        if (gemm && ap_gemm_kbit_group_pays(count, N, (int)rows, K, bits) != 1 &&
-            !(ap_gemm_kbit_group_taken(count, N, (int)rows, K, bits) == 1 && plain_execution() && product_is_half() && plain_half(args[1], nullptr)))
+        const bool staged = ap_linear_staged(count, N, (int)rows, K, bits) == 1, gemm = rows > 8 || staged;
+        if (rows > 8 && ap_gemm_kbit_group_pays(count, N, (int)rows, K, bits) != 1 &&
+            !((staged || ap_gemm_kbit_group_taken(count, N, (int)rows, K, bits) == 1) && plain_execution() && product_is_half() && plain_half(args[1], nullptr)))
             return none();
-        // side by side in one allocation: one row's results always are dense, and the tiled kernel writes rows that are not
+        // side by side in one allocation: one row's results always are dense, and the tiled, block-tile and staged kernels write rows that are not
         const bool joint = concat && (gemm ? K % 128 == 0 : rows == 1);
         if (concat && !joint && at::impl::torch_function_mode_enabled()) return none();  // the mode sees torch.cat
         Tensor all, outs[MOST];
@@ -330,7 +327,7 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
                     to[g] = half_out(outs[g]);
                 }
             }
-            rc = gemm ? ap_gemm_kbit_group(half_ptr(x), count, planes, luts, to, N, joint ? ldo : nullptr, (int)rows, K, bits, on.stream)
+            rc = gemm ? ap_linear_group(half_ptr(x), count, planes, luts, to, N, joint ? ldo : nullptr, (int)rows, K, bits, on.stream)
                       : ap_matmul_kbit_group(half_ptr(x), count, planes, luts, to, N, (int)rows, K, bits, on.stream);
             if (rc == AP_OK && concat && !joint) all = at::cat(std::vector<Tensor>(outs, outs + count), -1);
         }

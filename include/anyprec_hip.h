@@ -34,7 +34,7 @@
 extern "C" {
 #endif
 
-#define AP_ABI_VERSION 11
+#define AP_ABI_VERSION 12
 
 enum {
     AP_OK = 0,
@@ -98,13 +98,14 @@ int ap_matmul_kbit_swiglu(const uint16_t *x, const uint32_t *qweight_gate, const
 /* Fused dequant -> MFMA GEMM, M >= 1: out[M,N] = x[M,K] . dequant(qweight, lut)^T
  * without materialising the fp16 weight.  No single counterpart in the reference: it is the
  * M > 8 branch of AnyPrecisionLinear.forward (AnyPrecisionLinear.py:60-62: dequant_kbit,
- * main.cu:60-91, then torch.matmul) fused.  Three kernels: up to 128 activation rows a K-split
+ * main.cu:60-91, then torch.matmul) fused.  Four kernels: up to 128 activation rows a K-split
  * kernel with the weights of 16 rows in registers (more than 32 rows may run as launches of 32
  * each); from 81 rows on, and from 9..65 rows on where it measured faster, a tiled kernel whose
  * workgroups own 64 weight rows x 16..128 activation rows (the narrower the fewer tiles the grid
  * has) for the whole of K, ONE launch for any M (it needs K % 128 == 0; other row lengths go through the K-split kernel in chunks of 128 rows,
  * in order, on the same stream); from 9 rows on on wide linears, and from 65 nearly everywhere on rows of
- * 1024 elements or more, a block-tile kernel that rebuilds a weight once per tile of up to 256 activation rows, ONE launch for any M and K >= 256.  Correct for every M; faster than dequant +
+ * 1024 elements or more, a block-tile kernel that rebuilds a weight once per tile of up to 256 activation rows, ONE launch for any M and K >= 256.
+ * Correct for every M; faster than dequant +
  * a library GEMM up to 256..2048 rows (ap_gemm_kbit_taken) -- beyond that use that pair.
  * fp32 accumulation, fp16 result. */
 int ap_gemm_kbit(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut,
@@ -130,6 +131,20 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
  * it is the caller's.  Same value either way: fp16(fp16(sum) + bias). */
 int ap_linear_bias(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, const uint16_t *bias, uint16_t *out,
                    int M, int N, int K, int w_bits, void *stream, int *added);
+
+/* What AnyPrecisionLinear launches: the kernels of ap_matmul_kbit (up to 8 activation rows) and ap_gemm_kbit (beyond), or, on rows of a
+ * multiple of 128 elements and up to 32 activation rows, the staged K-split kernel wherever that is the faster one; those two keep to
+ * the kernels that they name.  `bias` may
+ * be NULL; with one, as ap_linear_bias. */
+int ap_linear(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, const uint16_t *bias, uint16_t *out,
+              int M, int N, int K, int w_bits, void *stream, int *added);
+/* The same for 1..4 linears that share x: ap_gemm_kbit_group, or one launch of the staged kernel wherever that is the faster one.
+ * Arguments, refusals and ldo as there. */
+int ap_linear_group(const uint16_t *x, int count, const uint32_t *const *qweight, const uint16_t *const *lut, uint16_t *const *out,
+                    const int *N, const long long *ldo, int M, int K, int w_bits, void *stream);
+/* 1 if ap_linear (count = 1) or ap_linear_group serves these linears by one launch of the staged kernel, else 0; argument errors as for
+ * those. */
+int ap_linear_staged(int count, const int *N, int M, int K, int w_bits);
 
 /* Where the fused GEMM is the faster way to compute x . dequant(W)^T, from this library's measurements on
  * MI355X: ap_gemm_kbit_pays returns 1 if ap_gemm_kbit beats ap_dequant_kbit + a library fp16 GEMM for M
@@ -181,7 +196,7 @@ int ap_matmul_kbit_group_route(int count, const int *N, int M, int K, int w_bits
  * beyond the 1e-2 bar of the entry points; the defaults are what measured fastest.  Names:
  * gemv_target_waves, gemv_rows, gemv_wpl, dequant_blocks_per_cu, matmul_mfma_from, gemm_split,
  * matmul_mfma4, gemv4_groups, gemm_rb2, gemv_stream, gemv_stream_waves, gemv_fine,
- * gemm_walk, gemm_walk_wgs, gemm_tiled, gemm_tile, gemm_tile_split, gemm_lookahead.  Returns AP_OK, AP_ENULL or AP_EKNOB.
+ * gemm_walk, gemm_walk_wgs, gemm_tiled, gemm_tile, gemm_tile_split, gemm_lookahead, gemm_block, gemm_block_tile, gemm_staged.  Returns AP_OK, AP_ENULL or AP_EKNOB.
  * For tests and measurements only: the knobs are plain process-wide integers, NOT thread-safe against
  * concurrent launches (a launch that races with a change sees either value); a serving process leaves
  * them alone. */
