@@ -63,6 +63,8 @@ lib.ap_strerror.argtypes = [_ci]
 lib.ap_strerror.restype = ctypes.c_char_p
 lib.ap_dequant_kbit.argtypes = [_vp, _vp, _vp, _ci, _ci, _ci, _vp]
 lib.ap_dequant_kbit.restype = _ci
+lib.ap_dequant_kbit_near.argtypes = lib.ap_dequant_kbit.argtypes
+lib.ap_dequant_kbit_near.restype = _ci
 lib.ap_matmul_kbit.argtypes = [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp]
 lib.ap_matmul_kbit.restype = _ci
 lib.ap_gemm_kbit.argtypes = [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp]
@@ -130,7 +132,7 @@ if lib.ap_abi_version() != AP_ABI_VERSION:
         f"{LIB_PATH} has ABI version {lib.ap_abi_version()}, this binding needs {AP_ABI_VERSION}: rebuild it"
     )
 
-EXPORTS = ("ap_abi_version", "ap_strerror", "ap_dequant_kbit", "ap_matmul_kbit", "ap_matmul_kbit_group",
+EXPORTS = ("ap_abi_version", "ap_strerror", "ap_dequant_kbit", "ap_dequant_kbit_near", "ap_matmul_kbit", "ap_matmul_kbit_group",
            "ap_gemm_kbit", "ap_matmul_kbit_geometry", "ap_set_tuning", "ap_get_tuning", "ap_probe_stream", "ap_probe_empty", "ap_probe_write", "ap_matmul_kbit_route", "ap_matmul_kbit_group_route",
            "ap_add_rmsnorm", "ap_silu_mul", "ap_decode_attention", "ap_matmul_kbit_swiglu", "ap_decode_advance", "ap_gemm_kbit_group", "ap_dequant_kbit_group", "ap_gemm_kbit_pays",
            "ap_gemm_kbit_group_pays", "ap_gemm_kbit_taken", "ap_gemm_kbit_group_taken", "ap_linear_bias", "ap_linear", "ap_linear_group", "ap_linear_staged", "ap_prompt_rope", "ap_prompt_attention", "ap_rope_heads")

@@ -186,7 +186,7 @@ int gemv_geometry(int M, const int *n, int count, int K, int w_bits, GemvGeometr
 
 // One launch of the dequantiser over `count` linears (arguments already checked): fills the member table and sizes the grid.
 template <int BITS>
-void launch_dequant(const DequantMembers &mem, hipStream_t stream) {
+void launch_dequant(const DequantMembers &mem, bool near, hipStream_t stream) {
     const long long items = mem.items;  // 64-word segments of all members
     long long blocks = (items + kDequantWaves - 1) / kDequantWaves;
     // One item per wave (the hardware hands out workgroups as others retire) measured best or within 1-2 % of best
@@ -200,7 +200,8 @@ void launch_dequant(const DequantMembers &mem, hipStream_t stream) {
     if (knob(kDequantBlocksPerCu) > 0) cap = cus * knob(kDequantBlocksPerCu);
     else if (blocks > 5 * cus && blocks <= 12 * cus) cap = 5 * cus;
     if (blocks > cap) blocks = cap;
-    dequant_kbit_kernel<BITS><<<dim3((unsigned)blocks), dim3(kDequantWaves * kWave), 0, stream>>>(mem);
+    if (near) dequant_kbit_kernel<BITS, true><<<dim3((unsigned)blocks), dim3(kDequantWaves * kWave), 0, stream>>>(mem);
+    else dequant_kbit_kernel<BITS, false><<<dim3((unsigned)blocks), dim3(kDequantWaves * kWave), 0, stream>>>(mem);
 }
 
 // hipGetLastError() returns AND clears the thread's sticky error, whoever left it: an entry point
@@ -466,13 +467,8 @@ int ap_prompt_attention(const uint16_t *qkv, const uint16_t *kcache, const uint1
     return launch_status();
 }
 
-int ap_dequant_kbit(const uint32_t *qweight, const uint16_t *lut, uint16_t *out, int N, int K, int w_bits,
-                    void *stream) {
-    return ap_dequant_kbit_group(1, &qweight, &lut, &out, &N, &K, w_bits, stream);
-}
-
-int ap_dequant_kbit_group(int count, const uint32_t *const *qweight, const uint16_t *const *lut, uint16_t *const *out,
-                          const int *N, const int *K, int w_bits, void *stream) {
+static int dequant_set(int count, const uint32_t *const *qweight, const uint16_t *const *lut, uint16_t *const *out, const int *N, const int *K,
+                       int w_bits, bool near, void *stream) {
     if (!qweight || !lut || !out || !N || !K) return AP_ENULL;
     if (count < 1 || count > kDequantMaxGroup) return AP_ELIMIT;
     DequantMembers mem = {};
@@ -498,14 +494,27 @@ int ap_dequant_kbit_group(int count, const uint32_t *const *qweight, const uint1
     hipStream_t st = static_cast<hipStream_t>(stream);
     drain_stale_error();
     switch (w_bits) {
-        case 3: launch_dequant<3>(mem, st); break;
-        case 4: launch_dequant<4>(mem, st); break;
-        case 5: launch_dequant<5>(mem, st); break;
-        case 6: launch_dequant<6>(mem, st); break;
-        case 7: launch_dequant<7>(mem, st); break;
-        default: launch_dequant<8>(mem, st); break;
+        case 3: launch_dequant<3>(mem, near, st); break;
+        case 4: launch_dequant<4>(mem, near, st); break;
+        case 5: launch_dequant<5>(mem, near, st); break;
+        case 6: launch_dequant<6>(mem, near, st); break;
+        case 7: launch_dequant<7>(mem, near, st); break;
+        default: launch_dequant<8>(mem, near, st); break;
     }
     return launch_status();
+}
+
+int ap_dequant_kbit(const uint32_t *qweight, const uint16_t *lut, uint16_t *out, int N, int K, int w_bits, void *stream) {
+    return dequant_set(1, &qweight, &lut, &out, &N, &K, w_bits, false, stream);
+}
+
+int ap_dequant_kbit_near(const uint32_t *qweight, const uint16_t *lut, uint16_t *out, int N, int K, int w_bits, void *stream) {
+    return dequant_set(1, &qweight, &lut, &out, &N, &K, w_bits, true, stream);
+}
+
+int ap_dequant_kbit_group(int count, const uint32_t *const *qweight, const uint16_t *const *lut, uint16_t *const *out, const int *N, const int *K,
+                          int w_bits, void *stream) {
+    return dequant_set(count, qweight, lut, out, N, K, w_bits, false, stream);
 }
 
 int ap_matmul_kbit_geometry(int M, int N, int K, int w_bits, int *wpl, int *segments, int *rows, int *grid) {

@@ -256,7 +256,11 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
             } else {
                 op = "dequant_kbit";
                 const Tensor dense = empty_half({w.N, w.K}, x.device());
-                rc = ap_dequant_kbit(w.planes, w.lut, half_out(dense), w.N, w.K, bits, on.stream);
+                // The product finds a weight of up to 192 MB (and its activations) in the last-level cache of 256: us past the caches / through
+                // them 4096 x 11008 at 512 rows 102 / 88, at 2048 196 / 181, 4096 x 4096 at 1024 rows 56 / 53, 14336 x 4096 127 / 123 (8 bits);
+                // a larger one is written out before it is read: 28672 x 8192 at 512 rows 301 / 317, 32000 x 4096 159 / 170.
+                const auto dequant = (int64_t)w.N * w.K <= 96 << 20 ? ap_dequant_kbit_near : ap_dequant_kbit;
+                rc = dequant(w.planes, w.lut, half_out(dense), w.N, w.K, bits, on.stream);
                 if (rc == AP_OK) out = at::matmul(x, dense.t());
             }
             if (rc == AP_OK && bias.defined() && !added) out.add_(bias);

@@ -53,6 +53,10 @@ enum {
 int ap_dequant_kbit(const uint32_t *qweight, const uint16_t *lut, uint16_t *out,
                     int N, int K, int w_bits, void *stream);
 
+/* The same for a weight that the next launch reads (a linear's product): it may stay in the caches. */
+int ap_dequant_kbit_near(const uint32_t *qweight, const uint16_t *lut, uint16_t *out,
+                         int N, int K, int w_bits, void *stream);
+
 /* ap_dequant_kbit for `count` (1..8) linears of any shapes at one w_bits in ONE launch:
  * out[g][N[g], K[g]] = dequant(qweight[g], lut[g]).  The arrays are host arrays of `count` device
  * pointers / sizes.  For dequantising a whole decoder layer (seven linears) or a whole checkpoint
