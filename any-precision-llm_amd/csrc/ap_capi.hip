@@ -1372,7 +1372,7 @@ bool gemms_pays(int M, const int *N, int count, int K, int b) {
         tiles += (N[g] + 63) / 64;
         largest = N[g] > largest ? N[g] : largest;
     }
-    if (M < 3) return false;
+    if (M < 3 || K < 512) return false;  // (shorter rows: one wave of four has work)
     if (M == 3) {
         if (count > 1) return b == 3 && total > 8192;
         return K > 8192 ? (b <= 4 ? total > 2048 : b <= 6 && total > 2560 && total <= 4096) : b <= 4 && total > 8192 && K > 4096;
