@@ -385,12 +385,13 @@ int ap_decode_attention(const uint16_t *qkv, const float *cos_table, const float
     half_t *kc = reinterpret_cast<half_t *>(kcache), *vc = reinterpret_cast<half_t *>(vcache), *o = reinterpret_cast<half_t *>(out);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const dim3 grid(n_heads), block(kAttnThreads);
+    const int group = n_heads / n_kv_heads;
     drain_stale_error();
     switch (head_dim) {
-        case 32: decode_attention_kernel<32><<<grid, block, 0, st>>>(q, cos_table, sin_table, kc, vc, pos, o, n_heads, n_kv_heads, max_len, scale); break;
-        case 64: decode_attention_kernel<64><<<grid, block, 0, st>>>(q, cos_table, sin_table, kc, vc, pos, o, n_heads, n_kv_heads, max_len, scale); break;
-        case 128: decode_attention_kernel<128><<<grid, block, 0, st>>>(q, cos_table, sin_table, kc, vc, pos, o, n_heads, n_kv_heads, max_len, scale); break;
-        default: decode_attention_kernel<256><<<grid, block, 0, st>>>(q, cos_table, sin_table, kc, vc, pos, o, n_heads, n_kv_heads, max_len, scale); break;
+        case 32: decode_attention_kernel<32><<<grid, block, 0, st>>>(q, cos_table, sin_table, kc, vc, pos, o, n_heads, n_kv_heads, group, max_len, scale); break;
+        case 64: decode_attention_kernel<64><<<grid, block, 0, st>>>(q, cos_table, sin_table, kc, vc, pos, o, n_heads, n_kv_heads, group, max_len, scale); break;
+        case 128: decode_attention_kernel<128><<<grid, block, 0, st>>>(q, cos_table, sin_table, kc, vc, pos, o, n_heads, n_kv_heads, group, max_len, scale); break;
+        default: decode_attention_kernel<256><<<grid, block, 0, st>>>(q, cos_table, sin_table, kc, vc, pos, o, n_heads, n_kv_heads, group, max_len, scale); break;
     }
     return launch_status();
 }

@@ -7,6 +7,8 @@
 #pragma once
 #include <math.h>
 
+#include <type_traits>
+
 #include "ap_device.hpp"
 
 namespace ap {
@@ -207,7 +209,7 @@ __global__ __launch_bounds__(kAdvanceThreads) void decode_advance_kernel(const h
     }
 }
 
-// Attention of one new token at cache row pos = *pos_p, one workgroup per query head.
+// Attention of one new token at cache row pos = *pos_p, one workgroup per query head; `group` query heads share a key head.
 //   qkv     [n_heads + 2 n_kv_heads, HD]: the token's query, key and value heads before the rotary embedding
 //   cosT, sinT [max_len, HD / 2] fp32: cos / sin of position * inverse frequency i
 //   kcache, vcache [n_kv_heads, max_len, HD]: rows 0 .. pos-1 are read; row pos is written (rotated key, value)
@@ -217,169 +219,219 @@ __global__ __launch_bounds__(kAdvanceThreads) void decode_advance_kernel(const h
 // Rotary convention of the Hugging Face Llama model: x * cos + rotate_half(x) * sin with
 // rotate_half(x) = (-x[HD/2:], x[:HD/2]).  Scores = (q . k) * scale, softmax and the weighted sum in fp32.
 // A position outside 0 .. max_len-1 makes every workgroup return without touching memory.
+//
+// A chain of latencies at a decoder's lengths: arguments, position, rows, and what stands between the barriers.  So a wave takes its keys all the way
+// -- scores, softmax with its own running maximum, weighted sum -- and the workgroup meets twice: behind the rotary embedding, with the
+// first rows on their way, and to add the waves' parts, each scaled from its maximum to the largest.  LPK lanes share a key, 8 elements each; a
+// step is the KPW keys of every wave, and up to four are requested together (no loads of keys that are not there: they cost more than a
+// later start).  us with the phases one after the other and six barriers / so: 32 heads of 128 at position 40 4.95 / 3.68, at 80 5.20 / 3.85, at 383
+// 7.2 / 5.6, at 2000 35 / 22; 8 heads of 256 at 383 13.4 / 7.8; 16 heads of 64 at 80 5.13 / 4.01.  Results further than half an ulp of
+// fp16 from the exact ones, of 69632 (heads of 128, up to 60 keys): 63 / 46.
 template <int HD>
 __global__ __launch_bounds__(kAttnThreads) void decode_attention_kernel(
     const half_t *__restrict__ qkv, const float *__restrict__ cosT, const float *__restrict__ sinT, half_t *kcache,
-    half_t *vcache, const long long *__restrict__ pos_p, half_t *__restrict__ out, int nh, int nkv, int max_len,
-    float scale) {
+    half_t *vcache, const long long *__restrict__ pos_p, half_t *__restrict__ out, int nh, int nkv, int group,
+    int max_len, float scale) {
     constexpr int HALF = HD / 2;
-    constexpr int DPL = HD / 4;    // score pass: four lanes share a key, DPL dims each
-    constexpr int NCH = DPL / 8;   // 16-byte chunks of those
     constexpr int NW = kAttnThreads / kWave;
-    constexpr int DPT = 8;                  // value pass: dims per lane (one 16-byte load)
-    constexpr int LPK = HD / DPT;           // lanes per key
+    constexpr int LPK = HD / 8;             // lanes per key
     constexpr int KPW = kWave / LPK;        // keys per wave and step
-    static_assert(HD % 32 == 0 && HD <= 256 && LPK <= kWave, "");
-    __shared__ float q_s[HD], kn_s[HD], vn_s[HD];
-    __shared__ float sc[kAttnMaxLen];
-    __shared__ float red[2][NW];
-    __shared__ float ctx_s[NW * KPW][HD];
+    constexpr int STEP = NW * KPW;
+    constexpr int MOST = 4;                 // steps requested together
+    static_assert(HD % 32 == 0 && HD <= 256 && HD <= kAttnThreads, "");
+    __shared__ __attribute__((aligned(16))) float q_s[HD], kn_s[HD], vn_s[HD];
+    __shared__ float max_s[NW], sum_s[NW];
+    __shared__ __attribute__((aligned(16))) float part_s[NW][HD];
 
-    const int head = blockIdx.x, tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-    const int group = nh / nkv, kvh = head / group;
-    const bool writer = head % group == 0;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int head = blockIdx.x, kvh = head / group;
+    const bool writer = head == kvh * group;
+    const int dl = lane % LPK, sub = lane / LPK;
+
+    // ---- waves 0, 1, 2: the query, the new key (and the new row of the cache) and the new value into LDS
+    const half_t *const mine = qkv + (size_t)(wave == 0 ? head : (wave == 1 ? nh + kvh : nh + nkv + kvh)) * HD;
+    constexpr int PER = (HALF + kWave - 1) / kWave;
+    half_t lo[PER], hi[PER];
+    if (wave < 3)
+#pragma unroll
+        for (int r = 0; r < PER; r++) {
+            const int i = min(lane + r * kWave, HALF - 1);
+            lo[r] = mine[i];
+            hi[r] = mine[i + HALF];
+        }
     const long long p64 = *pos_p;
     if (p64 < 0 || p64 >= max_len) return;  // uniform over the grid
     const int pos = (int)p64;
+    const int steps = (pos + STEP - 1) / STEP;
+    const half_t *const kbase = kcache + (size_t)kvh * max_len * HD + dl * 8, *const vbase = vcache + (size_t)kvh * max_len * HD + dl * 8;
+    const int first = wave * KPW + sub;     // this lane's key of step 0
 
-    // ---- rotary embedding of the query and the new key; the new row of the cache
-    {
-        const half_t *qr = qkv + (size_t)head * HD, *kr = qkv + (size_t)(nh + kvh) * HD;
-        const half_t *vr = qkv + (size_t)(nh + nkv + kvh) * HD;
-        half_t *kdst = kcache + ((size_t)kvh * max_len + pos) * HD, *vdst = vcache + ((size_t)kvh * max_len + pos) * HD;
-        for (int i = tid; i < HALF; i += kAttnThreads) {
-            const float c = cosT[(size_t)pos * HALF + i], s = sinT[(size_t)pos * HALF + i];
-            const float q1 = (float)qr[i], q2 = (float)qr[i + HALF], k1 = (float)kr[i], k2 = (float)kr[i + HALF];
-            q_s[i] = (q1 * c - q2 * s) * scale;
-            q_s[i + HALF] = (q2 * c + q1 * s) * scale;
-            const half_t a = (half_t)(k1 * c - k2 * s), b = (half_t)(k2 * c + k1 * s);
-            kn_s[i] = (float)a;
-            kn_s[i + HALF] = (float)b;
-            if (writer) {
-                kdst[i] = a;
-                kdst[i + HALF] = b;
-            }
-        }
-        for (int d = tid; d < HD; d += kAttnThreads) {
-            const half_t v = vr[d];
-            vn_s[d] = (float)v;
-            if (writer) vdst[d] = v;
-        }
-    }
-    __syncthreads();
-
-    // ---- the first value rows this lane will need are requested now: they do not depend on the scores, and the
-    // score pass and the softmax then hide their latency (LPK lanes per key, 8 dims = 16 bytes each)
-    constexpr int PF = 6;  // steps of NW * KPW keys held in registers (384 keys at HD = 128); later ones load in place
-    const int dl = lane % LPK, sub = lane / LPK;
-    const half_t *vbase = vcache + (size_t)kvh * max_len * HD + dl * DPT;
-    half8_t vpre[PF];
+    auto fresh_rows = [&]() {
+        if (wave >= 3) return;
+        float *const dst = wave == 0 ? q_s : (wave == 1 ? kn_s : vn_s);
 #pragma unroll
-    for (int it = 0; it < PF; it++) {
-        const int j = wave * KPW + sub + it * NW * KPW;
-        vpre[it] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-        if (j < pos) vpre[it] = *reinterpret_cast<const half8_t *>(vbase + (size_t)j * HD);
-    }
-
-    // ---- scores against the cached keys: four lanes per key
-    {
-        const int quad = tid >> 2, part = tid & 3;
-        float qreg[DPL];
-#pragma unroll
-        for (int d = 0; d < DPL; d++) qreg[d] = q_s[part * DPL + d];
-        const half_t *kbase = kcache + (size_t)kvh * max_len * HD + part * DPL;
-#pragma unroll 4
-        for (int j0 = 0; j0 < pos; j0 += kAttnThreads / 4) {
-            const int j = j0 + quad;
-            float s = 0.f;
-            if (j < pos) {
-                const u32x4 *p = reinterpret_cast<const u32x4 *>(kbase + (size_t)j * HD);
-#pragma unroll
-                for (int c = 0; c < NCH; c++) {
-                    const u32x4 v = p[c];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const uint32_t w = v[e];  // a copy: bit-casting the vector element itself reads element 0
-                        const half2_t h2 = __builtin_bit_cast(half2_t, w);
-                        s += (float)h2.x * qreg[c * 8 + 2 * e] + (float)h2.y * qreg[c * 8 + 2 * e + 1];
-                    }
+        for (int r = 0; r < PER; r++) {
+            const int i = lane + r * kWave;
+            if (i >= HALF) break;
+            float a = (float)lo[r], b = (float)hi[r];
+            if (wave < 2) {
+                const float c = cosT[(size_t)pos * HALF + i], s = sinT[(size_t)pos * HALF + i];
+                if (wave == 0) {
+                    const float x1 = a, x2 = b, base2 = scale * 1.44269504088896341f;   // scores to base 2
+                    a = (x1 * c - x2 * s) * base2;
+                    b = (x2 * c + x1 * s) * base2;
+                } else {
+                    // rounded by the instruction that adds, as the rows of a prompt are
+                    const half_t y1 = (half_t)((float)lo[r] * c - (float)hi[r] * s), y2 = (half_t)((float)hi[r] * c + (float)lo[r] * s);
+                    a = (float)y1;
+                    b = (float)y2;
                 }
             }
-            s = dpp_add<0xB1>(s);  // the four lanes of a key
-            s = dpp_add<0x4E>(s);
-            if (part == 0 && j < pos) sc[j] = s;
+            dst[i] = a;
+            dst[i + HALF] = b;
+            if (wave > 0 && writer) {
+                half_t *const row = (wave == 1 ? kcache : vcache) + ((size_t)kvh * max_len + pos) * HD;
+                row[i] = (half_t)a;
+                row[i + HALF] = (half_t)b;
+            }
         }
-        if (tid < kWave) {  // the new key, from LDS
+    };
+    auto over_key = [](float s) {           // the sum over the lanes of a key
+        s = dpp_add<0xB1>(s);
+        s = dpp_add<0x4E>(s);
+        if constexpr (LPK >= 8) s = dpp_add<0x141>(s);
+        if constexpr (LPK >= 16) s = dpp_add<0x140>(s);
+        if constexpr (LPK >= 32) s += __shfl_xor(s, 16, kWave);
+        return s;
+    };
+    float m = -INFINITY, l = 0.f, acc[8];   // of this lane's keys: maximum, sum of exp(score - m), weighted sum of 8 elements
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[e] = 0.f;
+    float q[8];
+    // The rotary embedding, and what needs no row of the cache: the new key is the first wave's first.  The rows requested before stay on their way.
+    auto meet = [&]() {
+        fresh_rows();
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+#pragma unroll
+        for (int e = 0; e < 8; e++) q[e] = q_s[dl * 8 + e];
+        if (wave == 0) {
             float s = 0.f;
-            for (int d = tid; d < HD; d += kWave) s += q_s[d] * kn_s[d];
-            s = wave_sum(s);
-            if (tid == kSumLane) sc[pos] = s;
-        }
-    }
-    __syncthreads();
-
-    // ---- softmax over rows 0 .. pos
-    const int n = pos + 1;
-    float m = -INFINITY;
-    for (int j = tid; j < n; j += kAttnThreads) m = fmaxf(m, sc[j]);
-    m = wave_max(m);
-    if (lane == 0) red[0][wave] = m;
-    __syncthreads();
-    m = red[0][0];
 #pragma unroll
-    for (int w = 1; w < NW; w++) m = fmaxf(m, red[0][w]);
-    float l = 0.f;
-    for (int j = tid; j < n; j += kAttnThreads) {
-        const float p = __expf(sc[j] - m);
-        sc[j] = p;
-        l += p;
-    }
-    l = wave_sum(l);
-    if (lane == kSumLane) red[1][wave] = l;
-    __syncthreads();  // also: every probability is in LDS
-    l = 0.f;
+            for (int e = 0; e < 8; e++) s += kn_s[dl * 8 + e] * q[e];
+            s = over_key(s);
+            if (sub == 0) {
+                m = s;
+                l = s - s + 1.f;    // NaN where the score is none, or infinite
 #pragma unroll
-    for (int w = 0; w < NW; w++) l += red[1][w];
-
-    // ---- weighted sum of the values
-    {
-        float acc[DPT];
-#pragma unroll
-        for (int e = 0; e < DPT; e++) acc[e] = 0.f;
-#pragma unroll
-        for (int it = 0; it < PF; it++) {  // the prefetched rows (zeros past pos, and a zero weight past n)
-            const int j = wave * KPW + sub + it * NW * KPW;
-            const float p = j < n ? sc[j] : 0.f;
-            if (j == pos) {
-#pragma unroll
-                for (int e = 0; e < DPT; e++) acc[e] += p * vn_s[dl * DPT + e];
-            } else {
-#pragma unroll
-                for (int e = 0; e < DPT; e++) acc[e] += p * (float)vpre[it][e];
+                for (int e = 0; e < 8; e++) acc[e] = l * vn_s[dl * 8 + e];
             }
         }
-#pragma unroll 4
-        for (int j = wave * KPW + sub + PF * NW * KPW; j < n; j += NW * KPW) {
-            const float p = sc[j];
-            if (j < pos) {
-                const half8_t v = *reinterpret_cast<const half8_t *>(vbase + (size_t)j * HD);
+    };
+    // scores of U keys and their values (score -inf: no key)
+    auto take = [&](auto u_c, const float (&s)[MOST], const half8_t (&v)[MOST]) {
+        constexpr int U = decltype(u_c)::value;
+        float top = m;
 #pragma unroll
-                for (int e = 0; e < DPT; e++) acc[e] += p * (float)v[e];
-            } else {
+        for (int u = 0; u < U; u++) top = fmaxf(top, s[u]);
+        const float base = top == -INFINITY ? 0.f : top, old = __builtin_amdgcn_exp2f(m - base);
+        l *= old;
 #pragma unroll
-                for (int e = 0; e < DPT; e++) acc[e] += p * vn_s[dl * DPT + e];
-            }
+        for (int e = 0; e < 8; e++) acc[e] *= old;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const float p = __builtin_amdgcn_exp2f(s[u] - base);
+            l += p;
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc[e] += p * (float)v[u][e];
+        }
+        m = top;
+    };
+    // U steps from step t on; FIRST: the query is not there yet; LAST: the last step may have lanes past the end
+    auto run = [&](auto u_c, auto first_c, auto last_c, int t) {
+        constexpr int U = decltype(u_c)::value;
+        constexpr bool LAST = decltype(last_c)::value;
+        half8_t k[MOST], v[MOST];
+        float s[MOST];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int j = min(first + (t + u) * STEP, pos - 1);
+            k[u] = *reinterpret_cast<const half8_t *>(kbase + (size_t)j * HD);
         }
 #pragma unroll
-        for (int e = 0; e < DPT; e++) ctx_s[wave * KPW + sub][dl * DPT + e] = acc[e];
+        for (int u = 0; u < U; u++) {
+            const int j = min(first + (t + u) * STEP, pos - 1);
+            v[u] = *reinterpret_cast<const half8_t *>(vbase + (size_t)j * HD);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (decltype(first_c)::value) meet();
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            float a = 0.f, b = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                a += (float)k[u][e] * q[e];
+                b += (float)k[u][e + 1] * q[e + 1];
+            }
+            s[u] = over_key(a + b);
+            if (LAST && u == U - 1 && first + (t + u) * STEP >= pos) {
+                s[u] = -INFINITY;
+                v[u] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+            }
+        }
+        take(u_c, s, v);
+    };
+    int t = 0;
+    if (steps == 0) meet();
+    else if (steps == 1) run(std::integral_constant<int, 1>{}, std::true_type{}, std::true_type{}, 0);
+    else if (steps == 2) run(std::integral_constant<int, 2>{}, std::true_type{}, std::true_type{}, 0);
+    else if (steps == 3) run(std::integral_constant<int, 3>{}, std::true_type{}, std::true_type{}, 0);
+    else {
+        run(std::integral_constant<int, 4>{}, std::true_type{}, std::true_type{}, 0);
+        for (t = 4; t + 4 <= steps; t += 4) run(std::integral_constant<int, 4>{}, std::false_type{}, std::true_type{}, t);
+        const int left = steps - t;
+        if (left == 1) run(std::integral_constant<int, 1>{}, std::false_type{}, std::true_type{}, t);
+        else if (left == 2) run(std::integral_constant<int, 2>{}, std::false_type{}, std::true_type{}, t);
+        else if (left == 3) run(std::integral_constant<int, 3>{}, std::false_type{}, std::true_type{}, t);
+    }
+    // ---- the wave's keys together, then the waves'
+    float top = m;
+#pragma unroll
+    for (int off = kWave / 2; off >= LPK; off /= 2) top = fmaxf(top, __shfl_xor(top, off, kWave));
+    const float f = __builtin_amdgcn_exp2f(m - (top == -INFINITY ? 0.f : top));
+    l *= f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[e] *= f;
+#pragma unroll
+    for (int off = kWave / 2; off >= LPK; off /= 2) {
+        l += __shfl_xor(l, off, kWave);
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[e] += __shfl_xor(acc[e], off, kWave);
+    }
+    if (sub == 0) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) part_s[wave][dl * 8 + e] = acc[e];
+    }
+    if (lane == 0) {
+        max_s[wave] = top;
+        sum_s[wave] = l;
     }
     __syncthreads();
-    for (int d = tid; d < HD; d += kAttnThreads) {
-        float s = 0.f;
-#pragma unroll 8
-        for (int r = 0; r < NW * KPW; r++) s += ctx_s[r][d];
-        out[(size_t)head * HD + d] = (half_t)(s / l);
+    if (tid >= HD) return;
+    float all = max_s[0], sum = 0.f, g[NW], y = 0.f;
+#pragma unroll
+    for (int w = 1; w < NW; w++) all = fmaxf(all, max_s[w]);
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        g[w] = __builtin_amdgcn_exp2f(max_s[w] - all);
+        sum += sum_s[w] * g[w];
     }
+    const float whole = 1.f / sum;
+#pragma unroll
+    for (int w = 0; w < NW; w++) y += part_s[w][tid] * g[w];
+    out[(size_t)head * HD + tid] = (half_t)(y * whole);
 }
 
 }  // namespace ap

@@ -266,3 +266,28 @@ def test_add_rmsnorm_of_more_rows_than_a_grid_has_threads_for(with_delta):
     _, got = add_rmsnorm(h, delta, w, 1e-5, h_out=h)
     assert torch.equal(torch.cat((got[:4], got[-4:])), want)
     assert bool((got[4:-4] == want[0]).all()) and bool((h[:-4] == h[0]).all())
+
+
+@pytest.mark.parametrize("hd", [32, 64, 128, 256])
+def test_decode_attention_at_the_edges_of_its_steps(hd):
+    """A step is 8192 / hd keys and four are requested together: one key more or less than 1..4, 5..8 steps.  Rows from the position on hold
+    NaN and must not be read; keys with a score of -inf (a whole wave's among them) weigh nothing."""
+    from any_precision_amd.decode_ops import decode_attention
+    nh, nkv, step = 4, 2, 8192 // hd
+    max_len = 8 * step + 8
+    cos, sin = torch.ones((max_len, hd // 2), device="cuda"), torch.zeros((max_len, hd // 2), device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(hd)
+    for pos in (0, 1, step - 1, step, step + 1, 2 * step, 3 * step - 1, 3 * step + 1, 4 * step, 4 * step + 1, 5 * step + 1, 7 * step - 1, 8 * step, max_len - 1):
+        for masked in (False, True):
+            print(f"decode_attention steps hd={hd} pos={pos} masked={masked}", flush=True)
+            kcache = torch.randn((nkv, max_len, hd), device="cuda", generator=g).half()
+            vcache = torch.randn((nkv, max_len, hd), device="cuda", generator=g).half()
+            kcache[:, pos:], vcache[:, pos:] = float("nan"), float("nan")
+            qkv = torch.rand((nh + 2 * nkv, hd), device="cuda", generator=g).half() + 0.5
+            if masked:      # positive queries: -inf scores
+                kcache[:, :min(pos, step // 2)] = float("-inf")
+                kcache[:, step + 3:pos:7] = float("-inf")
+            p = torch.tensor([pos], dtype=torch.int64, device="cuda")
+            want, _, _ = _attention_reference(qkv, cos, sin, kcache.clone(), vcache.clone(), pos, nh, 0.05)
+            got = decode_attention(qkv, cos, sin, kcache, vcache, p, nh, 0.05)
+            _close(got, want, 4e-3, f"hd={hd} pos={pos} masked={masked}")
