@@ -81,6 +81,8 @@ lib.ap_linear.argtypes = [_vp, _vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp, _pi]
 lib.ap_linear.restype = _ci
 lib.ap_gemm_kbit_taken.argtypes = [_ci, _ci, _ci, _ci]
 lib.ap_gemm_kbit_taken.restype = _ci
+lib.ap_gemm_kbit_quick.argtypes = [_ci, _ci, _ci, _ci]
+lib.ap_gemm_kbit_quick.restype = _ci
 lib.ap_gemm_kbit_group_taken.argtypes = [_ci, _pi, _ci, _ci, _ci]
 lib.ap_gemm_kbit_group_taken.restype = _ci
 lib.ap_gemm_kbit_group_pays.argtypes = [_ci, _pi, _ci, _ci, _ci]
@@ -135,7 +137,7 @@ if lib.ap_abi_version() != AP_ABI_VERSION:
 EXPORTS = ("ap_abi_version", "ap_strerror", "ap_dequant_kbit", "ap_dequant_kbit_near", "ap_matmul_kbit", "ap_matmul_kbit_group",
            "ap_gemm_kbit", "ap_matmul_kbit_geometry", "ap_set_tuning", "ap_get_tuning", "ap_probe_stream", "ap_probe_empty", "ap_probe_write", "ap_matmul_kbit_route", "ap_matmul_kbit_group_route",
            "ap_add_rmsnorm", "ap_silu_mul", "ap_decode_attention", "ap_matmul_kbit_swiglu", "ap_decode_advance", "ap_gemm_kbit_group", "ap_dequant_kbit_group", "ap_gemm_kbit_pays",
-           "ap_gemm_kbit_group_pays", "ap_gemm_kbit_taken", "ap_gemm_kbit_group_taken", "ap_linear_bias", "ap_linear", "ap_linear_group", "ap_linear_staged", "ap_prompt_rope", "ap_prompt_attention", "ap_rope_heads")
+           "ap_gemm_kbit_group_pays", "ap_gemm_kbit_taken", "ap_gemm_kbit_quick", "ap_gemm_kbit_group_taken", "ap_linear_bias", "ap_linear", "ap_linear_group", "ap_linear_staged", "ap_prompt_rope", "ap_prompt_attention", "ap_rope_heads")
 GEMM_MAX_M = 128
 GROUP_MAX = 4
 DEQUANT_GROUP_MAX = 8

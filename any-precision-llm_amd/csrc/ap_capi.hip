@@ -1670,6 +1670,25 @@ int ap_gemm_kbit_taken(int M, int N, int K, int w_bits) {
            (gemmt_pays(M, N, K, w_bits) && gemmt_geometry(M, (N + 63) / 64, K, w_bits, &tiled) && gemmt_us(tiled, K, w_bits) <= pair);
 }
 
+// A caller that issues dequant_kbit and a library GEMM one call at a time waits 26 us for the host to issue the two, whatever their size, and 5 for
+// a fused GEMM.  Where the device is faster with the pair, the fused form still is where it saves the host more than it costs the device
+// (the line lies halfway: streams that keep the device busy lose at most what the others win).  One call at a time, us pair / fused: 717 x 256 at
+// 248 rows, 3 bits 26.2 / 6.2; 1743 x 928, 178 rows, 8 bits 26.2 / 13.8; 2562 x 448, 298 rows, 8 bits 26.6 / 14.1; 1024 x 4096, 320 rows, 8
+// bits 26.2 / 20.9; beyond the line 4296 x 1024, 700 rows, 7 bits 28.3 / 22.  What the K-split kernel takes is a fit on 60 calls of up to 128
+// rows, 20 % off on average; more rows are launches of 128 each.
+int ap_gemm_kbit_quick(int M, int N, int K, int w_bits) {
+    const int rc = ap_gemm_kbit_taken(M, N, K, w_bits);
+    if (rc != 0 || N < 256 || knob(kGemmBlock) != 1 || knob(kGemmTiled) != 1) return rc;  // (narrower ones have not been timed)
+    constexpr double kPairCall = 26;
+    GemmbGeometry block;
+    GemmtGeometry tiled;
+    double us;
+    if (takes_gemmb(M, N, K, w_bits, &block)) us = block.us;
+    else if (gemmt_pays(M, N, K, w_bits) && gemmt_geometry(M, (N + 63) / 64, K, w_bits, &tiled)) us = gemmt_us(tiled, K, w_bits);
+    else us = (3 + 0.0035 * K + 0.03 * (M < kGemmMaxM ? M : kGemmMaxM)) * ((M + kGemmMaxM - 1) / kGemmMaxM) * fmax(1.0, N / 4096.0);
+    return 2 * us <= pair_us(M, N, K, w_bits) + kPairCall && us <= kPairCall ? 1 : 0;
+}
+
 int ap_gemm_kbit_group_taken(int count, const int *N, int M, int K, int w_bits) {
     const int rc = ap_gemm_kbit_group_pays(count, N, M, K, w_bits);
     if (rc != 0) return rc;

@@ -165,6 +165,9 @@ int ap_gemm_kbit_group_pays(int count, const int *N, int M, int K, int w_bits);
  * GEMM does not: ap_gemm_kbit_pays says where the host module has always taken the fused form, these where it may for a plain
  * forward.  Argument errors as above. */
 int ap_gemm_kbit_taken(int M, int N, int K, int w_bits);
+/* 1 also where the pair would only be faster to a caller that does not wait for the host to issue its two calls (a captured graph): what
+ * AnyPrecisionLinear asks outside of one. */
+int ap_gemm_kbit_quick(int M, int N, int K, int w_bits);
 int ap_gemm_kbit_group_taken(int count, const int *N, int M, int K, int w_bits);
 
 /* Human-readable text for a return code of the functions above. */

@@ -367,3 +367,47 @@ def test_which_kernels_take_the_bias_along(N, K, M, b, knobs, added):
         want = (ext.matmul_kbit if M <= 8 else ext.gemm_kbit)(x, q, t, b)
     assert rc == 0 and flag.value == added
     assert torch.equal(out, want + bias if added else want)
+
+
+@pytest.mark.parametrize("N,K,M,b", [(717, 256, 248, 3), (1024, 4096, 320, 8), (2562, 448, 298, 8), (300, 704, 82, 4)])
+def test_small_linears_take_the_fused_form_outside_a_graph(N, K, M, b):
+    """Where the host would wait for the pair's two calls: the fused kernel's bits one call at a time, the pair's in a captured graph, with
+    gradients and for a subclass, whichever replays."""
+    import any_precision_ext as ext
+    from any_precision_amd import _capi
+    from any_precision_amd.linear import AnyPrecisionLinear
+    assert _capi.lib.ap_gemm_kbit_taken(M, N, K, b) == 0 and _capi.lib.ap_gemm_kbit_quick(M, N, K, b) == 1
+    m = AnyPrecisionLinear(K, N, [b], bias=False, device="cuda", dtype=torch.float16)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    m.qweight.copy_(torch.randint(-2**31, 2**31, m.qweight.shape, dtype=torch.int32, device="cuda", generator=g))
+    table = m._buffers[f"lut{b}"]
+    table.copy_(torch.randn(table.shape, device="cuda", generator=g) * 0.02)
+    x = torch.randn((M, K), device="cuda", generator=g).half()
+    pair = torch.matmul(x, ext.dequant_kbit(m.qweight, table, b).T)
+    assert torch.equal(m(x, precision=b), ext.gemm_kbit(x, m.qweight, table, b))
+    grad = m(x.clone().requires_grad_(), precision=b)
+    assert grad.requires_grad and torch.equal(grad.detach(), pair)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = m(x, precision=b)
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, pair)
+
+
+def test_where_the_fused_form_is_quick():
+    """No GPU is asked: never beyond its range, everything that ap_gemm_kbit_taken takes, and errors as there."""
+    from any_precision_amd import _capi
+    for N in (64, 255, 256, 1024, 4096, 14336):
+        for K in (32, 256, 1024, 4096, 14336):
+            for M in (1, 33, 128, 129, 512, 2048, 16384):
+                for b in (3, 5, 8):
+                    taken, quick = _capi.lib.ap_gemm_kbit_taken(M, N, K, b), _capi.lib.ap_gemm_kbit_quick(M, N, K, b)
+                    assert quick == 1 if taken == 1 else quick in (0, 1) and (quick == 0 or (N >= 256 and M * K * N < 2**34))
+    assert _capi.lib.ap_gemm_kbit_quick(0, 256, 256, 4) < 0 and _capi.lib.ap_gemm_kbit_quick(64, 256, 250, 4) < 0
+    with _capi.tuning(gemm_block=0):
+        assert _capi.lib.ap_gemm_kbit_quick(320, 1024, 4096, 8) == _capi.lib.ap_gemm_kbit_taken(320, 1024, 4096, 8)
