@@ -324,7 +324,7 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_kernel(
             s = over_key(s);
             if (sub == 0) {
                 m = s;
-                l = s - s + 1.f;    // NaN where the score is none, or infinite
+                l = s == -INFINITY ? 0.f : s - s + 1.f;    // nothing at -inf, as any other key; NaN where the score is NaN or +inf
 #pragma unroll
                 for (int e = 0; e < 8; e++) acc[e] = l * vn_s[dl * 8 + e];
             }

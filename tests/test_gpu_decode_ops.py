@@ -291,3 +291,27 @@ def test_decode_attention_at_the_edges_of_its_steps(hd):
             want, _, _ = _attention_reference(qkv, cos, sin, kcache.clone(), vcache.clone(), pos, nh, 0.05)
             got = decode_attention(qkv, cos, sin, kcache, vcache, p, nh, 0.05)
             _close(got, want, 4e-3, f"hd={hd} pos={pos} masked={masked}")
+
+
+@pytest.mark.parametrize("hd", [32, 64, 128, 256])
+def test_decode_attention_new_key_with_a_score_of_minus_infinity(hd):
+    """The token's own key may overflow fp16 by its rotation.  At a score of -inf it weighs nothing beside the cached keys; alone it leaves NaN."""
+    from any_precision_amd.decode_ops import decode_attention
+    nh, nkv, max_len = 4, 2, 16384 // hd + 8
+    cos = torch.full((max_len, hd // 2), math.cos(math.pi / 4), device="cuda")
+    sin = torch.full((max_len, hd // 2), math.sin(math.pi / 4), device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(hd)
+    for pos in (0, 1, 7, max_len - 1):
+        print(f"decode_attention -inf hd={hd} pos={pos}", flush=True)
+        kcache = torch.randn((nkv, max_len, hd), device="cuda", generator=g).half()
+        vcache = torch.randn((nkv, max_len, hd), device="cuda", generator=g).half()
+        qkv = torch.rand((nh + 2 * nkv, hd), device="cuda", generator=g).half() + 0.5      # rotated: the second half positive
+        qkv[nh:nh + nkv, 0], qkv[nh:nh + nkv, hd // 2] = -60000, -60000                    # to about 0 and -84853
+        p = torch.tensor([pos], dtype=torch.int64, device="cuda")
+        want, k, _ = _attention_reference(qkv, cos, sin, kcache.clone(), vcache.clone(), pos, nh, 0.05)
+        assert bool((k[:, hd // 2] == float("-inf")).all())
+        got = decode_attention(qkv, cos, sin, kcache, vcache, p, nh, 0.05)
+        if pos == 0:
+            assert bool(want.isnan().all()) and bool(got.isnan().all())
+        else:
+            _close(got, want, 4e-3, f"hd={hd} pos={pos}")
