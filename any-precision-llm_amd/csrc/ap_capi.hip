@@ -630,8 +630,8 @@ constexpr int kGemmbTileCount = sizeof(kGemmbTiles) / sizeof(kGemmbTiles[0]);
 // Rounds of tiles over the CUs: workgroups go to the 8 XCDs in turn, and both tiled kernels number their tiles so that those of one block of
 // weight rows run on one XCD.  So the XCDs with one block more decide: 20 blocks are 3 on four XCDs and 2 on the others (2560 x 2560 at
 // 1395 rows, 128 x 128 tiles: 220 tiles are 33 for 32 CUs, two rounds, 43 us at 3 bits; one round of 180 tiles, 1026 rows, is 22).
-inline long long tile_rounds(long long tiles_n, long long tiles_m) {
-    const long long cus = cu_count() < 8 ? 1 : cu_count() / 8;  // of an XCD
+inline long long tile_rounds(long long tiles_n, long long tiles_m, int device_cus) {
+    const long long cus = device_cus < 8 ? 1 : device_cus / 8;  // of an XCD
     return ((tiles_n + 7) / 8 * tiles_m + cus - 1) / cus;
 }
 
@@ -673,7 +673,7 @@ bool gemmb_geometry(int M, const int *N, int count, int K, int w_bits, GemmbGeom
         odd = odd || (N[g] & 7) != 0;
     }
     const int forced = knob(kGemmBlockTile);
-    const double cus = cu_count();
+    const int cus = cu_count();  // asked once: the runtime's answer takes longer than the estimate of a tile
     geo->mb = 0;
     for (int t = 0; t < kGemmbTileCount; t++) {
         const auto &tile = kGemmbTiles[t];
@@ -685,7 +685,7 @@ bool gemmb_geometry(int M, const int *N, int count, int K, int w_bits, GemmbGeom
         if ((n + 7) / 8 * 8 * m > 0x7fffffffLL) continue;
         const int h = (K / 256 + tile.wk - 1) / tile.wk;
         const double fill = fmin(1.0, (double)(n * m) / cus);
-        const double us = c[0] + tile_rounds(n, m) * (c[1] + h * (c[2] + c[3] * fill) + ((K & 255) ? c[4] : 0.f) + (odd ? c[5] : 0.f));
+        const double us = c[0] + tile_rounds(n, m, cus) * (c[1] + h * (c[2] + c[3] * fill) + ((K & 255) ? c[4] : 0.f) + (odd ? c[5] : 0.f));
         if (geo->mb == 0 || us < geo->us) *geo = {tile.mb, tile.wn, tile.wk, (int)n, (int)m, us};
     }
     return geo->mb != 0;
@@ -704,7 +704,7 @@ constexpr float kGemmtCost[6][5][3] = {
 double gemmt_us(const GemmtGeometry &geo, int K, int w_bits) {
     const int form = geo.mbw == 1 ? 0 : (geo.mbw == 2 ? 1 : (geo.mbw == 8 ? 4 : (geo.kh == 2 ? 2 : 3)));
     const float *c = kGemmtCost[w_bits - 3][form];
-    return c[0] + tile_rounds(geo.grid_n, geo.grid_m) * (c[1] + (K + 511) / 512 * c[2]);
+    return c[0] + tile_rounds(geo.grid_n, geo.grid_m, cu_count()) * (c[1] + (K + 511) / 512 * c[2]);
 }
 
 // And for dequant_kbit + a library GEMM: the two launches, the weight written and read, the product, what the library takes per 1000
@@ -1678,7 +1678,8 @@ int ap_gemm_kbit_taken(int M, int N, int K, int w_bits) {
 // rows, 20 % off on average; more rows are launches of 128 each.
 int ap_gemm_kbit_quick(int M, int N, int K, int w_bits) {
     const int rc = ap_gemm_kbit_taken(M, N, K, w_bits);
-    if (rc != 0 || N < 256 || knob(kGemmBlock) != 1 || knob(kGemmTiled) != 1) return rc;  // (narrower ones have not been timed)
+    // (from 1.4e10 products on no fused form is through within the host's time: 1.01 PFLOP/s is the most that one reaches)
+    if (rc != 0 || N < 256 || (double)M * N * K >= 1.4e10 || knob(kGemmBlock) != 1 || knob(kGemmTiled) != 1) return rc;  // (narrower ones have not been timed)
     constexpr double kPairCall = 26;
     GemmbGeometry block;
     GemmtGeometry tiled;
