@@ -786,7 +786,6 @@ bool gemms_fits(int M, const int *N, int count, int K) {
     return blocks <= 0x7fffffffLL;
 }
 
-
 // What a launch of the staged kernel takes at 9..16 and at 17..32 activation rows, in us: a + h s + g (p + h q) + w c, where h = the steps of 512
 // elements of the busiest wave, g = workgroups of a CU (at least 1) and w = steps x workgroups a wave slot of all CUs has.  {a, s, p, q, c} per
 // bit-width, non-negative least squares over 4200 calls: linears and sets of 256..30000 rows of 512..16384 elements; 6 % off on average.

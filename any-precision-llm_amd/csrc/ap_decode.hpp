@@ -16,13 +16,7 @@ namespace ap {
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 
 constexpr int kAttnThreads = 1024;  // sixteen waves: the kernel is a chain of load latencies, more waves = more loads in flight
-constexpr int kAttnMaxLen = 8192;  // cache rows one launch can attend over (scores live in LDS)
-
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, kWave));
-    return v;
-}
+constexpr int kAttnMaxLen = 8192;  // cache rows one launch attends over: the limit of the entry point (the kernel itself keeps nothing per row)
 
 // One workgroup per row of H elements (H % 8 == 0):
 //     s = h + delta (rounded to fp16, as an fp16 add; delta only with DELTA), written to h_out;

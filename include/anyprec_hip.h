@@ -102,7 +102,7 @@ int ap_matmul_kbit_swiglu(const uint16_t *x, const uint32_t *qweight_gate, const
 /* Fused dequant -> MFMA GEMM, M >= 1: out[M,N] = x[M,K] . dequant(qweight, lut)^T
  * without materialising the fp16 weight.  No single counterpart in the reference: it is the
  * M > 8 branch of AnyPrecisionLinear.forward (AnyPrecisionLinear.py:60-62: dequant_kbit,
- * main.cu:60-91, then torch.matmul) fused.  Four kernels: up to 128 activation rows a K-split
+ * main.cu:60-91, then torch.matmul) fused.  Three kernels: up to 128 activation rows a K-split
  * kernel with the weights of 16 rows in registers (more than 32 rows may run as launches of 32
  * each); from 81 rows on, and from 9..65 rows on where it measured faster, a tiled kernel whose
  * workgroups own 64 weight rows x 16..128 activation rows (the narrower the fewer tiles the grid
