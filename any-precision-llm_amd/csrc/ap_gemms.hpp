@@ -47,6 +47,30 @@ struct GemmsLds {
     static constexpr int kCopies = kSlots / 16;
 };
 
+// What a wave has requested behind a stage when the first read of that stage is due, in the order in which run_step requests: the stages of the
+// ring (DMA loads each) lie ahead of the step; with NEXT its first loads are the BITS planes of the next one; a stage's buffer is refilled
+// behind its last products -- in a ring of four after the first reads of the stage behind it, in a ring of two before them.  Loads
+// complete in order: when no more than behind(j) are outstanding, stage j has landed.
+template <int BITS, int RING, int DMA, bool NEXT>
+struct GemmsOrder {
+    static constexpr int behind(int j) {
+        int requested = RING * DMA, landed[4] = {};  // landed[k]: requests up to the last of stage k
+        for (int k = 0; k < RING; k++) landed[k] = (k + 1) * DMA;
+        if (NEXT) requested += BITS;
+        for (int k = 0; k < j; k++) {  // the end of stage k, up to the reads of stage k + 1
+            if (RING == 4 && k + 1 == j) break;
+            if (RING == 4 ? NEXT : (k < 2 || NEXT)) requested += DMA;
+            if (RING == 2 && k < 2) landed[k + 2] = requested;
+        }
+        return requested - landed[j];
+    }
+    static_assert(RING == 2 || RING == 4, "");
+    static_assert(behind(0) == (RING - 1) * DMA + (NEXT ? BITS : 0), "");
+    static_assert(RING == 4 || (behind(1) == behind(0) && behind(2) == DMA && behind(3) == (NEXT ? DMA : 0)), "");
+    static_assert(RING == 2 || !NEXT || (behind(1) == 2 * DMA + BITS && behind(2) == behind(1) && behind(3) == behind(1)), "");
+    static_assert(RING == 2 || NEXT || (behind(1) == 2 * DMA && behind(2) == DMA && behind(3) == 0), "");
+};
+
 // Grid: a workgroup of (64, 4) threads per block of 16 weight rows of all members.  ROWS: activation rows staged (M <= ROWS).
 template <int BITS, int ROWS>
 __global__ __launch_bounds__(kGemmsWaves *kWave, ROWS <= 8 ? 3 : 2) void gemms_kbit_kernel(const half_t *__restrict__ x, const GemmsMembers mem,
@@ -252,17 +276,13 @@ __global__ __launch_bounds__(kGemmsWaves *kWave, ROWS <= 8 ? 3 : 2) void gemms_k
     // One step.  NEXT: the wave has another, step + WAVES.
     auto run_step = [&](auto next_c, auto check_c, int step) {
         constexpr bool NEXT = decltype(next_c)::value;
-        constexpr int AHEAD = NEXT ? BITS : 0;  // loads that go out ahead of the stages
+        using Order = GemmsOrder<BITS, RING, DMA, NEXT>;
         const bool live = 16 * step + 4 * quad < W;
         convert();
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (NEXT) fetch(step + WAVES);
         __builtin_amdgcn_sched_barrier(0);
-        auto ready = [&](auto j_c) {  // loads requested after those of stage j when it is needed
-            constexpr int j = decltype(j_c)::value;
-            constexpr int n = RING == 4 ? (NEXT ? 3 * DMA + AHEAD : (3 - j) * DMA) : (j < 2 ? DMA + AHEAD : (j == 2 || NEXT ? DMA : 0));
-            wait(std::integral_constant<int, n>{});
-        };
+        auto ready = [&](auto j_c) { wait(std::integral_constant<int, Order::behind(decltype(j_c)::value)>{}); };
         ready(std::integral_constant<int, 0>{});
         request(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
         // units of two octets, the operands of the next requested before the products of the current
