@@ -62,6 +62,32 @@ def test_one_hot_rows_give_the_weights_exactly(ext, oracle):
 
 
 @gpu
+@pytest.mark.parametrize("N,K", ((4096, 11008), (14336, 4096), (11008, 4224)))
+def test_rings_refilled_on_a_full_chip(ext, N, K):
+    """Two or three workgroups a CU that go around their rings, planes from memory: against the product of the dequantised weight, and one-hot
+    rows exactly over all weight rows.  A result is fp16 of an fp32 sum: 2**-11 of its value, and 2**-13 of the norm of its K terms for the sums of
+    both sides (K roundings of 2**-24 as a random walk are 2**-17 of it at most, 2**-15 the largest of half a million)."""
+    from any_precision_amd import _capi
+    gen = torch.Generator(device="cuda").manual_seed(N + K)
+    q = torch.randint(-2**31, 2**31, (8, N, K // 32), dtype=torch.int32, device="cuda", generator=gen)
+    for b in (3, 4, 5, 8):
+        table = (torch.randn((N, 1 << b), device="cuda", generator=gen) * 0.02).half()
+        w = ext.dequant_kbit(q, table, b)
+        for M in (4, 8, 16, 32):
+            print(f"staged full chip N={N} K={K} b={b} M={M}", flush=True)
+            x = torch.randn((M, K), device="cuda", generator=gen).half()
+            ks = torch.randint(0, K, (M,), device="cuda", generator=gen)
+            hot = torch.zeros((M, K), dtype=torch.float16, device="cuda")
+            hot[torch.arange(M, device="cuda"), ks] = 1.0
+            want = x.float() @ w.float().t()
+            with _capi.tuning(gemm_staged=2):
+                first, exact = ext.gemm_kbit(x, q, table, b), ext.gemm_kbit(hot, q, table, b)
+                again = ext.gemm_kbit(x, q, table, b)
+            assert ((first.float() - want).abs() <= want.abs() * 2**-11 + 2**-13 * 0.02 * K ** 0.5).all(), (b, M)
+            assert torch.equal(first, again) and torch.equal(exact, w[:, ks].t()), (b, M)
+
+
+@gpu
 @pytest.mark.parametrize("K", (1024, 1152))
 def test_what_is_not_a_number_stays_in_its_row(ext, K):
     """NaN and infinities in one activation row, infinite table entries that no weight of the row uses."""
