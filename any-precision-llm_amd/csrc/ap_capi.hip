@@ -1669,24 +1669,25 @@ int ap_gemm_kbit_taken(int M, int N, int K, int w_bits) {
            (gemmt_pays(M, N, K, w_bits) && gemmt_geometry(M, (N + 63) / 64, K, w_bits, &tiled) && gemmt_us(tiled, K, w_bits) <= pair);
 }
 
-// A caller that issues dequant_kbit and a library GEMM one call at a time waits 26 us for the host to issue the two, whatever their size, and 5 for
-// a fused GEMM.  Where the device is faster with the pair, the fused form still is where it saves the host more than it costs the device
-// (the line lies halfway: streams that keep the device busy lose at most what the others win).  One call at a time, us pair / fused: 717 x 256 at
-// 248 rows, 3 bits 26.2 / 6.2; 1743 x 928, 178 rows, 8 bits 26.2 / 13.8; 2562 x 448, 298 rows, 8 bits 26.6 / 14.1; 1024 x 4096, 320 rows, 8
-// bits 26.2 / 20.9; beyond the line 4296 x 1024, 700 rows, 7 bits 28.3 / 22.  What the K-split kernel takes is a fit on 60 calls of up to 128
-// rows, 20 % off on average; more rows are launches of 128 each.
+// Small linears, beside what ap_gemm_kbit_taken says: a caller that issues dequant_kbit and a library GEMM one call at a time waits 23 us for the
+// host to issue the two, whatever their size, and 5 for a fused GEMM.  The line is drawn where the fused form is the faster one on the device
+// as well, so that a stream that is busy, a captured graph and the call that warmed it up all take the same form.  Device time of the pair and of the
+// fused form, of 21700 drawn linears of 256..14336 rows at 33..1024 activation rows (and fewer than 1.4e10 products):
+//  - one launch of the K-split kernel on short rows: 0.70 of the pair's time on average, by more than 3 % slower in 1 of 100 (66 x 3719 x 416, 4 bits
+//    12.1 / 5.9; 93 x 262 x 416, 8 bits 10.0 / 6.3; 106 x 1072 x 1504, 4 bits 15.7 / 10.0).  Longer rows and several launches lose up to 1.9 times
+//    (126 x 343 x 4448, 8 bits 16.9 / 29.5; 240 x 749 x 448, 6 bits 9.4 / 16.0);
+//  - the tiled kernel up to 6 bits where its estimate is below 0.65 of pair_us, which is high by a third here: 0.77 on average, 1 of 200 slower (373 x 756 x
+//    512, 3 bits 10.0 / 6.2); at 7 and 8 bits half of them are (904 x 965 x 640, 7 bits 11.1 / 21.1).
+// (Sizes as rows x N x K.)
 int ap_gemm_kbit_quick(int M, int N, int K, int w_bits) {
     const int rc = ap_gemm_kbit_taken(M, N, K, w_bits);
-    // (from 1.4e10 products on no fused form is through within the host's time: 1.01 PFLOP/s is the most that one reaches)
-    if (rc != 0 || N < 256 || (double)M * N * K >= 1.4e10 || knob(kGemmBlock) != 1 || knob(kGemmTiled) != 1) return rc;  // (narrower ones have not been timed)
-    constexpr double kPairCall = 26;
+    if (rc != 0 || N < 256 || N > 14336 || (double)M * N * K >= 1.4e10 || knob(kGemmBlock) != 1 || knob(kGemmTiled) != 1) return rc;
     GemmbGeometry block;
     GemmtGeometry tiled;
-    double us;
-    if (takes_gemmb(M, N, K, w_bits, &block)) us = block.us;
-    else if (gemmt_pays(M, N, K, w_bits) && gemmt_geometry(M, (N + 63) / 64, K, w_bits, &tiled)) us = gemmt_us(tiled, K, w_bits);
-    else us = (3 + 0.0035 * K + 0.03 * (M < kGemmMaxM ? M : kGemmMaxM)) * ((M + kGemmMaxM - 1) / kGemmMaxM) * fmax(1.0, N / 4096.0);
-    return 2 * us <= pair_us(M, N, K, w_bits) + kPairCall && us <= kPairCall ? 1 : 0;
+    if (takes_gemmb(M, N, K, w_bits, &block)) return 0;
+    if (gemmt_pays(M, N, K, w_bits) && gemmt_geometry(M, (N + 63) / 64, K, w_bits, &tiled))
+        return w_bits <= 6 && gemmt_us(tiled, K, w_bits) <= 0.65 * pair_us(M, N, K, w_bits) ? 1 : 0;
+    return (K & 127) != 0 && M <= kGemmMaxM && K <= (M <= 96 ? 2048 : 1024) ? 1 : 0;
 }
 
 int ap_gemm_kbit_group_taken(int count, const int *N, int M, int K, int w_bits) {

@@ -98,12 +98,6 @@ Tensor result_for(const Tensor &x, int64_t N) {
     return empty_half(shape, x.device());
 }
 
-// Whether the device's current stream records a graph.
-bool capturing(c10::DeviceIndex d) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(d).stream(), &status) != hipSuccess || status != hipStreamCaptureStatusNone;
-}
-
 // Makes the tensors' device the current one for a call (a no-op where it is) and gives its current stream.
 struct OnDevice {
     explicit OnDevice(c10::DeviceIndex d) {
@@ -224,7 +218,7 @@ bool tensors_of(PyObject *module_dict, int bits, ModuleTensors *m) {
 }
 
 // linear(module.__dict__, x, w_bits): AnyPrecisionLinear.forward.  ap_linear up to 8 rows, and beyond
-// where ap_gemm_kbit_pays, or ap_gemm_kbit_taken and nothing but plain execution follows the call; else the weight in fp16 and
+// where ap_gemm_kbit_pays, or ap_gemm_kbit_quick and nothing but plain execution follows the call; else the weight in fp16 and
 // torch's own product (which takes part in autograd and autocast).
 PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (n != 3 || !is_tensor(args[1])) return none();
@@ -240,8 +234,7 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
         const int64_t rows = rows_of(x, w);
         if (rows < 1) return none();
         const bool pays = rows <= 8 || ap_gemm_kbit_pays((int)rows, w.N, w.K, bits) == 1 ||
-                          ((ap_gemm_kbit_taken((int)rows, w.N, w.K, bits) == 1 || (ap_gemm_kbit_quick((int)rows, w.N, w.K, bits) == 1 && !capturing(w.device))) &&
-                           plain_execution() && product_is_half() && plain_half(args[1], nullptr));
+                          (ap_gemm_kbit_quick((int)rows, w.N, w.K, bits) == 1 && plain_execution() && product_is_half() && plain_half(args[1], nullptr));
         // torch's product and sum as Python calls them, where a subclass or a mode wants to see them
         const bool torch_op = !pays || bias.defined();
         if (torch_op && (at::impl::torch_function_mode_enabled() || !exact_tensor(args[1]) || (m.bias != nullptr && !exact_tensor(m.bias))))

@@ -165,8 +165,8 @@ int ap_gemm_kbit_group_pays(int count, const int *N, int M, int K, int w_bits);
  * GEMM does not: ap_gemm_kbit_pays says where the host module has always taken the fused form, these where it may for a plain
  * forward.  Argument errors as above. */
 int ap_gemm_kbit_taken(int M, int N, int K, int w_bits);
-/* 1 also where the pair would only be faster to a caller that does not wait for the host to issue its two calls (a captured graph): what
- * AnyPrecisionLinear asks outside of one. */
+/* 1 also for small linears (256..14336 weight rows, more than 32 activation rows) where the host would be waited for to issue the pair's two calls
+ * and the fused form takes no longer on the device either: what AnyPrecisionLinear asks, captured into a graph or not. */
 int ap_gemm_kbit_quick(int M, int N, int K, int w_bits);
 int ap_gemm_kbit_group_taken(int count, const int *N, int M, int K, int w_bits);
 

@@ -1,4 +1,6 @@
 """AnyPrecisionLinear on the GPU: state-dict format, precision switching, both batch branches."""
+import os
+
 import numpy as np
 import pytest
 import torch
@@ -369,22 +371,32 @@ def test_which_kernels_take_the_bias_along(N, K, M, b, knobs, added):
     assert torch.equal(out, want + bias if added else want)
 
 
-@pytest.mark.parametrize("N,K,M,b", [(717, 256, 248, 3), (1024, 4096, 320, 8), (2562, 448, 298, 8), (300, 704, 82, 4)])
-def test_small_linears_take_the_fused_form_outside_a_graph(N, K, M, b):
-    """Where the host would wait for the pair's two calls: the fused kernel's bits one call at a time, the pair's in a captured graph, with
-    gradients and for a subclass, whichever replays."""
-    import any_precision_ext as ext
-    from any_precision_amd import _capi
+SMALL = [(3719, 416, 66, 4), (611, 992, 120, 6), (756, 512, 373, 3), (300, 704, 82, 4)]      # N, K, rows, bits
+
+
+def _small(N, K, M, b):
     from any_precision_amd.linear import AnyPrecisionLinear
-    assert _capi.lib.ap_gemm_kbit_taken(M, N, K, b) == 0 and _capi.lib.ap_gemm_kbit_quick(M, N, K, b) == 1
     m = AnyPrecisionLinear(K, N, [b], bias=False, device="cuda", dtype=torch.float16)
     g = torch.Generator(device="cuda").manual_seed(N)
     m.qweight.copy_(torch.randint(-2**31, 2**31, m.qweight.shape, dtype=torch.int32, device="cuda", generator=g))
     table = m._buffers[f"lut{b}"]
     table.copy_(torch.randn(table.shape, device="cuda", generator=g) * 0.02)
-    x = torch.randn((M, K), device="cuda", generator=g).half()
+    return m, table, torch.randn((M, K), device="cuda", generator=g).half()
+
+
+# the last three: beyond the line, the pair's calls in both
+@pytest.mark.parametrize("N,K,M,b", SMALL + [(717, 256, 248, 7), (2562, 448, 298, 8), (1024, 4096, 320, 8)])
+def test_small_linears_take_one_form_in_a_graph_and_outside(N, K, M, b):
+    """The fused kernel's bits within the line of ap_gemm_kbit_quick, the pair's beyond, with gradients and for a subclass; a captured call is the
+    one that warmed it up, whichever replays."""
+    import any_precision_ext as ext
+    from any_precision_amd import _capi
+    quick = (N, K, M, b) in SMALL
+    assert _capi.lib.ap_gemm_kbit_taken(M, N, K, b) == 0 and _capi.lib.ap_gemm_kbit_quick(M, N, K, b) == quick
+    m, table, x = _small(N, K, M, b)
     pair = torch.matmul(x, ext.dequant_kbit(m.qweight, table, b).T)
-    assert torch.equal(m(x, precision=b), ext.gemm_kbit(x, m.qweight, table, b))
+    want = ext.gemm_kbit(x, m.qweight, table, b) if quick else pair
+    assert torch.equal(m(x, precision=b), want)
     grad = m(x.clone().requires_grad_(), precision=b)
     assert grad.requires_grad and torch.equal(grad.detach(), pair)
     torch.cuda.synchronize()
@@ -396,7 +408,38 @@ def test_small_linears_take_the_fused_form_outside_a_graph(N, K, M, b):
         torch.cuda.synchronize()
         graph.replay()
         torch.cuda.synchronize()
-        assert torch.equal(y, pair)
+        assert torch.equal(y, want)
+
+
+def test_a_module_s_own_call_is_all_the_warm_up_that_its_capture_needs():
+    """In a fresh process: nothing but the module has run before it is captured, on either side of the line."""
+    import subprocess
+    import sys
+    code = f"""
+import sys
+sys.path[:0] = {sys.path!r}
+import torch
+from test_gpu_linear import SMALL, _small
+for case in (SMALL[0], (2562, 448, 298, 8)):
+    m, _, x = _small(*case)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        want = m(x, precision=case[3])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = m(x, precision=case[3])
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), case
+print("captured")
+"""
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100, cwd=os.path.dirname(os.path.abspath(__file__)))
+    assert res.returncode == 0 and "captured" in res.stdout, res.stdout + res.stderr
 
 
 def test_where_the_fused_form_is_quick():
@@ -410,4 +453,4 @@ def test_where_the_fused_form_is_quick():
                     assert quick == 1 if taken == 1 else quick in (0, 1) and (quick == 0 or (N >= 256 and M * K * N < 2**34))
     assert _capi.lib.ap_gemm_kbit_quick(0, 256, 256, 4) < 0 and _capi.lib.ap_gemm_kbit_quick(64, 256, 250, 4) < 0
     with _capi.tuning(gemm_block=0):
-        assert _capi.lib.ap_gemm_kbit_quick(320, 1024, 4096, 8) == _capi.lib.ap_gemm_kbit_taken(320, 1024, 4096, 8)
+        assert all(_capi.lib.ap_gemm_kbit_quick(M, N, K, b) == _capi.lib.ap_gemm_kbit_taken(M, N, K, b) for N, K, M, b in SMALL)
