@@ -271,7 +271,7 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
 }
 
 // linear_group(__dict__ of 2..4 modules, x, w_bits, concat as a bool): forward_group for bias-free linears of one input length.  A list of
-// results, or with concat one tensor of them side by side.  ap_linear_group where ap_linear_staged or, beyond 8 rows, where
+// results, or with concat one tensor of them side by side (a list yet where a torch-function mode is to see torch.cat).  ap_linear_group where ap_linear_staged or, beyond 8 rows, where
 // ap_gemm_kbit_group_pays or _taken; up to 8 rows ap_matmul_kbit_group else; None where the modules are better called one by one.
 PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
     constexpr int MOST = 4;
@@ -307,9 +307,11 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (rows > 8 && ap_gemm_kbit_group_pays(count, N, (int)rows, K, bits) != 1 &&
             !((staged || ap_gemm_kbit_group_taken(count, N, (int)rows, K, bits) == 1) && plain_execution() && product_is_half() && plain_half(args[1], nullptr)))
             return none();
-        // side by side in one allocation: one row's results always are dense, and the tiled, block-tile and staged kernels write rows that are not
-        const bool joint = concat && (gemm ? K % 128 == 0 : rows == 1);
-        if (concat && !joint && at::impl::torch_function_mode_enabled()) return none();  // the mode sees torch.cat
+        // side by side in one allocation: one row's results always are dense, and the tiled, block-tile and staged kernels write rows that are
+        // not.  At 2..8 rows torch joins them wherever something else than plain execution may look at that; for a torch-function mode the
+        // caller does.
+        const bool joint = concat && (rows > 8 ? K % 128 == 0 : rows == 1 || (staged && plain_execution()));
+        const bool join = concat && !joint && !at::impl::torch_function_mode_enabled();
         Tensor all, outs[MOST];
         int rc;
         {
@@ -333,11 +335,11 @@ PyObject *linear_group(PyObject *, PyObject *const *args, Py_ssize_t n) {
             }
             rc = gemm ? ap_linear_group(half_ptr(x), count, planes, luts, to, N, joint ? ldo : nullptr, (int)rows, K, bits, on.stream)
                       : ap_matmul_kbit_group(half_ptr(x), count, planes, luts, to, N, (int)rows, K, bits, on.stream);
-            if (rc == AP_OK && concat && !joint) all = at::cat(std::vector<Tensor>(outs, outs + count), -1);
+            if (rc == AP_OK && join) all = at::cat(std::vector<Tensor>(outs, outs + count), -1);
         }
         if (rc == AP_ELIMIT) return none();  // beyond the tiled kernel's offsets
         if (rc != AP_OK) return library_error(rc, gemm ? "gemm_kbit_group" : "matmul_kbit_group");
-        if (concat) return wrap(std::move(all));
+        if (joint || join) return wrap(std::move(all));
         PyObject *list = PyList_New(count);
         if (list == nullptr) return nullptr;
         for (int g = 0; g < count; g++) {

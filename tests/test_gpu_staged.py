@@ -174,6 +174,43 @@ def test_modules_of_three_to_thirty_two_rows_are_served_by_it():
         assert all(torch.equal(s.view(rows, -1), w) for s, w in zip(split, wants)), (rows, b)
 
 
+@gpu
+@pytest.mark.parametrize("rows", (2, 4, 8, 16))
+def test_modes_see_a_small_set_joined(rows):
+    """At 2..8 rows torch joins a set's results wherever a mode could see it, also where the staged kernel serves the set; the same results."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from any_precision_amd import AnyPrecisionLinear
+    from any_precision_amd.linear import forward_group
+    K, Ns = 4096, (4096, 4096, 4096)
+    assert _staged(Ns, rows, K, 3) == (rows > 2)
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    members = []
+    for N in Ns:
+        m = AnyPrecisionLinear(K, N, [3], bias=False, device="cuda", dtype=torch.float16)
+        m.qweight.copy_(torch.randint(-2**31, 2**31, m.qweight.shape, dtype=torch.int32, device="cuda", generator=gen))
+        m._buffers["lut3"].copy_(torch.randn((N, 8), device="cuda", generator=gen) * 0.02)
+        members.append(m)
+    x = torch.randn((rows, K), device="cuda", generator=gen).half()
+    want, seen = forward_group(members, x, 3, concat=True), []
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func._schema.name.split("::")[-1])
+            return func(*args, **(kwargs or {}))
+
+    for mode in (Functions, Dispatch):
+        seen.clear()
+        with mode():
+            got = forward_group(members, x, 3, concat=True)
+        assert torch.equal(got, want) and ("cat" in seen) == (rows <= 8), (mode, seen)
+
+
 def test_which_calls_the_rule_takes():
     """Only calls that the kernel serves, none that another knob forces or forbids, and one row and two never; errors as ap_gemm_kbit has them."""
     from any_precision_amd import _capi
