@@ -4,6 +4,8 @@
 #include <math.h>
 #include <string.h>
 
+#include <mutex>
+
 #include "anyprec_hip.h"
 #include "ap_decode.hpp"
 #include "ap_dequant.hpp"
@@ -28,7 +30,10 @@ using namespace ap;
 // at every call: a caller that changes a knob while another thread launches gets either value.
 struct Knob {
     const char *name;
+    int initial;
+    bool form;  // chooses a kernel or its form (the others only size grids): off its default it also means that the staged kernel is not to come first
     int value;
+    constexpr Knob(const char *n, int v, bool f) : name(n), initial(v), form(f), value(v) {}
 };
 enum {
     kGemvTargetWaves,   // waves the dot-product GEMV grid aims for (rows per workgroup follows)
@@ -55,14 +60,15 @@ enum {
     kKnobCount
 };
 Knob g_knobs[kKnobCount] = {
-    {"gemv_target_waves", 16384}, {"gemv_rows", 0},      {"gemv_wpl", 0},     {"dequant_blocks_per_cu", 0},
-    {"matmul_mfma_from", 5},      {"gemm_split", 0},     {"matmul_mfma4", 1}, {"gemv4_groups", 0},
-    {"gemm_rb2", 1},              {"gemv_stream", 1},    {"gemv_stream_waves", 24},
-    {"gemv_fine", 1},
-    {"gemm_walk", 1},             {"gemm_walk_wgs", 1},  {"gemm_tiled", 1},   {"gemm_tile", 0},
-    {"gemm_tile_split", 0},       {"gemm_lookahead", 1},
-    {"gemm_block", 1},            {"gemm_block_tile", 0}, {"gemm_staged", 1},
+    {"gemv_target_waves", 16384, true}, {"gemv_rows", 0, true},    {"gemv_wpl", 0, true},      {"dequant_blocks_per_cu", 0, false},
+    {"matmul_mfma_from", 5, true},      {"gemm_split", 0, true},   {"matmul_mfma4", 1, true},  {"gemv4_groups", 0, true},
+    {"gemm_rb2", 1, true},              {"gemv_stream", 1, true},  {"gemv_stream_waves", 24, false},
+    {"gemv_fine", 1, true},
+    {"gemm_walk", 1, true},             {"gemm_walk_wgs", 1, false}, {"gemm_tiled", 1, true},  {"gemm_tile", 0, true},
+    {"gemm_tile_split", 0, true},       {"gemm_lookahead", 1, true},
+    {"gemm_block", 1, true},            {"gemm_block_tile", 0, true}, {"gemm_staged", 1, false},
 };
+int g_forms_set;  // how many knobs that choose a form are off their default: kept by ap_set_tuning, so that a call reads one int for all of them
 inline int knob(int k) { return __atomic_load_n(&g_knobs[k].value, __ATOMIC_RELAXED); }
 
 // Compute units of the current device (256 on MI355X), looked up once per device.
@@ -263,7 +269,12 @@ int ap_set_tuning(const char *name, int value) {
     if (!name) return AP_ENULL;
     for (int k = 0; k < kKnobCount; k++)
         if (strcmp(name, g_knobs[k].name) == 0) {
+            static std::mutex one;  // or, of two threads that set knobs, the one that counted first could store last
+            const std::lock_guard<std::mutex> hold(one);
             __atomic_store_n(&g_knobs[k].value, value, __ATOMIC_RELAXED);
+            int set = 0;
+            for (int i = 0; i < kKnobCount; i++) set += g_knobs[i].form && knob(i) != g_knobs[i].initial;
+            __atomic_store_n(&g_forms_set, set, __ATOMIC_RELAXED);
             return AP_OK;
         }
     return AP_EKNOB;
@@ -1404,16 +1415,11 @@ bool gemms_pays(int M, const int *N, int count, int K, int b) {
 // ap_matmul_kbit keep to the kernels that they have always named, whose sums a caller may hold to each other bit for bit.  A caller that forces or
 // forbids another kernel means this one too.
 bool takes_gemms(int M, const int *N, int count, int K, int w_bits, bool linear) {
+    if (M > kGemmsMaxM) return false;
     const int mode = knob(kGemmStaged);
-    if (mode <= 0 || !gemms_fits(M, N, count, K)) return false;
-    if (mode >= 2) return true;
-    if (!linear) return false;
-    static const int others[] = {kGemmSplit, kGemmRb2, kGemmWalk, kGemmTiled, kGemmTile, kGemmTileSplit, kGemmLookahead, kGemmBlock, kGemmBlockTile,
-                                 kMatmulMfmaFrom, kMatmulMfma4, kGemvStream, kGemvFine, kGemvRows, kGemvWpl, kGemvTargetWaves, kGemv4Groups};
-    static const int defaults[] = {0, 1, 1, 1, 0, 0, 1, 1, 0, 5, 1, 1, 1, 0, 0, 16384, 0};
-    for (int i = 0; i < (int)(sizeof others / sizeof others[0]); i++)
-        if (knob(others[i]) != defaults[i]) return false;
-    return gemms_pays(M, N, count, K, w_bits);
+    if (mode >= 2) return gemms_fits(M, N, count, K);
+    if (mode <= 0 || !linear || M < 3 || __atomic_load_n(&g_forms_set, __ATOMIC_RELAXED) != 0) return false;  // (M < 3: as gemms_pays; the calls that the host bounds leave here)
+    return gemms_fits(M, N, count, K) && gemms_pays(M, N, count, K, w_bits);
 }
 
 // One launch of the block-tile kernel over `count` linears (arguments already checked; geo from gemmb_geometry over all of them).
@@ -1442,15 +1448,16 @@ int run_gemmb(const GemmbGeometry &geo, const uint16_t *x, int count, const uint
     return ok ? launch_status() : AP_ELIMIT;
 }
 
+// staged: what takes_gemms has said of the call.
 static int gemm_one(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, const uint16_t *bias, uint16_t *out, int M, int N, int K,
-                    int w_bits, void *stream, bool *added, bool linear = false) {
+                    int w_bits, void *stream, bool *added, bool staged) {
     if (!x || !qweight || !lut || !out) return AP_ENULL;
     const int rc = check_common(N, K, w_bits);
     if (rc != AP_OK) return rc;
     if (M < 1) return AP_EBATCH;
     if (!aligned16(x) || !aligned16(qweight) || !aligned16(lut)) return AP_EALIGN;
     drain_stale_error();
-    if (takes_gemms(M, &N, 1, K, w_bits, linear)) {
+    if (staged) {
         *added = bias != nullptr;
         return run_gemms(x, 1, &qweight, &lut, bias, &out, &N, nullptr, M, K, w_bits, static_cast<hipStream_t>(stream));
     }
@@ -1479,7 +1486,7 @@ static int gemm_one(const uint16_t *x, const uint32_t *qweight, const uint16_t *
 int ap_gemm_kbit(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, uint16_t *out, int M, int N, int K,
                  int w_bits, void *stream) {
     bool added = false;
-    return gemm_one(x, qweight, lut, nullptr, out, M, N, K, w_bits, stream, &added);
+    return gemm_one(x, qweight, lut, nullptr, out, M, N, K, w_bits, stream, &added, takes_gemms(M, &N, 1, K, w_bits, false));
 }
 
 int ap_linear_bias(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, const uint16_t *bias, uint16_t *out, int M, int N, int K,
@@ -1487,7 +1494,7 @@ int ap_linear_bias(const uint16_t *x, const uint32_t *qweight, const uint16_t *l
     if (!bias || !added) return AP_ENULL;
     bool with = false;
     const int rc = M <= 8 ? matmul_set(x, 1, &qweight, &lut, bias, &out, &N, M, K, w_bits, stream, &with)
-                          : gemm_one(x, qweight, lut, bias, out, M, N, K, w_bits, stream, &with);
+                          : gemm_one(x, qweight, lut, bias, out, M, N, K, w_bits, stream, &with, takes_gemms(M, &N, 1, K, w_bits, false));
     *added = with ? 1 : 0;
     return rc;
 }
@@ -1496,9 +1503,9 @@ int ap_linear(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, c
               void *stream, int *added) {
     if (!added) return AP_ENULL;
     bool with = false;
-    const int rc = M <= 8 && !(check_common(N, K, w_bits) == AP_OK && takes_gemms(M, &N, 1, K, w_bits, true))
-                       ? matmul_set(x, 1, &qweight, &lut, bias, &out, &N, M, K, w_bits, stream, &with)
-                       : gemm_one(x, qweight, lut, bias, out, M, N, K, w_bits, stream, &with, true);
+    const bool staged = check_common(N, K, w_bits) == AP_OK && takes_gemms(M, &N, 1, K, w_bits, true);
+    const int rc = M <= 8 && !staged ? matmul_set(x, 1, &qweight, &lut, bias, &out, &N, M, K, w_bits, stream, &with)
+                                     : gemm_one(x, qweight, lut, bias, out, M, N, K, w_bits, stream, &with, staged);
     *added = with ? 1 : 0;
     return rc;
 }
@@ -1547,7 +1554,7 @@ static int gemm_set(const uint16_t *x, int count, const uint32_t *const *qweight
     if (strided) return (K & 127) != 0 ? AP_ESHAPE : AP_ELIMIT;
     for (int g = 0; g < count; g++) {
         bool added = false;
-        const int r = gemm_one(x, qweight[g], lut[g], nullptr, out[g], M, N[g], K, w_bits, stream, &added, linear);
+        const int r = gemm_one(x, qweight[g], lut[g], nullptr, out[g], M, N[g], K, w_bits, stream, &added, takes_gemms(M, N + g, 1, K, w_bits, linear));
         if (r != AP_OK) return r;
     }
     return AP_OK;

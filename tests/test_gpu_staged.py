@@ -211,6 +211,11 @@ def test_modes_see_a_small_set_joined(rows):
         assert torch.equal(got, want) and ("cat" in seen) == (rows <= 8), (mode, seen)
 
 
+_KNOBS = ("gemv_target_waves", "gemv_rows", "gemv_wpl", "dequant_blocks_per_cu", "matmul_mfma_from", "gemm_split", "matmul_mfma4", "gemv4_groups", "gemm_rb2",
+          "gemv_stream", "gemv_stream_waves", "gemv_fine", "gemm_walk", "gemm_walk_wgs", "gemm_tiled", "gemm_tile", "gemm_tile_split", "gemm_lookahead",
+          "gemm_block", "gemm_block_tile", "gemm_staged")
+
+
 def test_which_calls_the_rule_takes():
     """Only calls that the kernel serves, none that another knob forces or forbids, and one row and two never; errors as ap_gemm_kbit has them."""
     from any_precision_amd import _capi
@@ -228,5 +233,14 @@ def test_which_calls_the_rule_takes():
     for knobs in ({"gemm_tiled": 2}, {"gemm_block": 0}, {"gemm_rb2": 2}, {"matmul_mfma_from": 9}, {"gemv_rows": 2}):
         with _capi.tuning(**knobs):
             assert _staged([4096], 16, 4096, 4) == 0, knobs
+    # every knob that chooses a form, and two at once; those that size a grid leave the choice alone
+    value = ctypes.c_int()
+    for name in _KNOBS:
+        assert _capi.lib.ap_get_tuning(name.encode(), ctypes.byref(value)) == 0
+        with _capi.tuning(**{name: value.value + 1}):
+            assert _staged([4096], 16, 4096, 4) == (name in ("dequant_blocks_per_cu", "gemv_stream_waves", "gemm_walk_wgs", "gemm_staged")), name
+            with _capi.tuning(gemm_split=2):
+                assert _staged([4096], 16, 4096, 4) == (name == "gemm_staged")
+        assert _staged([4096], 16, 4096, 4) == 1
     assert _staged([4096], 16, 4096, 9) < 0 and _staged([4096], 0, 4096, 4) < 0 and _staged([64] * 5, 16, 4096, 4) < 0
     assert _staged([1 << 25], 16, 1 << 14, 3) == 0           # planes of 4 GiB and more: beyond 32-bit offsets
