@@ -1368,12 +1368,19 @@ bool takes_gemmb_set(int M, const int *N, int count, int K, int w_bits, GemmbGeo
 //    but short rows, where the tables are not paid back, and beyond 8192 rows, where the kernels that share a tile of activations between 64 weight
 //    rows or more may be faster: there the estimates decide (14336 x 4096 at 3 bits: 12.9 / 14.4 at 16 rows; 14.7 / 18.8 at 32), and rows that
 //    only the K-split kernel serves otherwise are the staged kernel's from 1280 elements on (17408 x 1152, 28 rows, 6 bits 21.4 / 17.9; 16752 x 1536,
-//    4 bits 23.0 / 15.1).  Sets of up to 8192 rows always: the others take their members one by one (3 x 4096 x 4096 at 16 rows, 3 bits 15.5 / 10.4);
+//    4 bits 23.0 / 15.1; up to 16 rows at 5 bits and more from 1664).  Sets of up to 8192 rows always: the others take their members one by one (3 x 4096 x 4096 at 16 rows, 3 bits 15.5 / 10.4);
 //  - at 5..8 rows beyond 2048 rows (4096 x 4096 at 8 rows 6.5 / 5.4 at 3 bits, 10.3 / 9.2 at 8; 4096 x 14336, 5 bits 22.5 / 14.5; 11008 x 4096,
 //    3 bits 13.1 / 9.4), fewer only where the rows are long (1600 x 11392, 7 rows, 3 bits 12.1 / 9.9): on few workgroups the dot-product kernel's short
-//    waves win (1024 x 4096 at 8 rows, 5 bits 5.7 / 6.3);
-//  - at 3 and 4 rows on long rows, at few bits (4096 x 14336 at 4 rows, 4 bits 15.6 / 11.3; 8 bits 22 / 19.5 but 16432 x 6784, 6 bits 32 / 35), sets at
-//    few bits (2 x 11008 x 4096, 4 rows, 3 bits 18 / 14); not at 2 (0.9-1.4 times as long).
+//    waves win (1024 x 4096 at 8 rows, 5 bits 5.7 / 6.3; sets of up to 4096 rows of up to 2560
+//    elements 1.06 of the time at 6 rows, 7 bits, 1.10 and 1.04 at 6 and 7 rows, 8 bits);
+//  - at 3 and 4 rows on long rows, at few bits (4096 x 14336 at 4 rows, 4 bits: 15.6 / 11.3; 5 bits on rows of 4224..8192 elements beyond 8192 rows 0.7-0.95
+//    of the time, 6 bits 0.93-1.17), sets at few bits (2 x 11008 x 4096, 4 rows, 3 bits 18 / 14; at 3 rows of more than 2048 elements, on shorter ones 1.02);
+//    not at 2 (0.9-1.4 times as long);
+//  - at more bits there, on rows of more than 8192 elements, where the CUs are used evenly: the kernel has one block a CU in about the time that the
+//    others have most of one, and a few blocks more are a round of their own (its time over theirs at 9216..14336 elements, 4 rows 8 bits / 3 rows 6 bits, at
+//    2048 rows 1.23 / 1.21, 3072 0.96 / 0.97, 4096 0.83 / 0.83, 4608 1.07 / 1.07, 5120 1.03 / 1.03, 6144 0.89 / 0.93, 8192 0.77 / 0.82).
+// Drawn anew, the 35500 of 79000 linears that the rule takes run in 0.76 of their time, 23900 sets in 0.56; 8 in 1000 of either are slower by more
+// than 3 %.
 bool gemms_pays(int M, const int *N, int count, int K, int b) {
     long long total = 0, blocks = 0, tiles = 0;
     int largest = 0;
@@ -1384,18 +1391,20 @@ bool gemms_pays(int M, const int *N, int count, int K, int b) {
         largest = N[g] > largest ? N[g] : largest;
     }
     if (M < 3 || K < 512) return false;  // (shorter rows: one wave of four has work)
-    if (M == 3) {
-        if (count > 1) return b == 3 && total > 8192;
-        return K > 8192 ? (b <= 4 ? total > 2048 : b <= 6 && total > 2560 && total <= 4096) : b <= 4 && total > 8192 && K > 4096;
-    }
-    if (M == 4) {
+    if (M <= 4) {
+        const long long cus = cu_count();
+        const bool even = blocks > 2 * cus || 4 * blocks >= 3 * ((blocks + cus - 1) / cus) * cus;  // the last block of a CU: three quarters of them have it
+        if (M == 3) {
+            if (count > 1) return b == 3 && total > 8192 && K > 2048;
+            return K > 8192 ? (b <= 4 ? total > 2048 : b <= 6 && even) : b <= 4 && total > 8192 && K > 4096;
+        }
         if (total <= 2048 || K < 4096) return false;
         if (count > 1) return total > 8192 ? b <= 5 || (b == 6 && total > 12288) : b == 3;
-        if (K > 8192) return b <= 6 || (total > 3072 && total <= 4096);
-        return K > 4096 ? total > 4096 && (b <= 4 || (b <= 6 && total > 8192 && total <= 16384)) : b <= 4 && total > 8192;
+        if (K > 8192) return b <= 6 || even;
+        return K > 4096 ? total > 4096 && (b <= 4 || (b == 5 && total > 8192)) : b <= 4 && total > 8192;
     }
     if (M <= 8) {
-        if (count > 1 && M == 5 && b >= 5) return false;
+        if (count > 1 && b >= 5 && (M == 5 || (b >= 7 && M <= b - 1 && total <= 4096 && K <= 2560))) return false;
         if (total > 2048) return K > 1024 || (b <= 4 && total <= 4096);
         return count == 1 && total > 1024 && M >= 7 && ((K > 8192 && b <= 6) || (K > 4096 && b <= 4));
     }
@@ -1408,7 +1417,9 @@ bool gemms_pays(int M, const int *N, int count, int K, int b) {
         return gemms_us(M, blocks, K, b) <= block.us;
     if ((count > 1 ? gemmt_set_pays(M, largest, K) : gemmt_pays(M, N[0], K, b)) && gemmt_geometry(M, tiles, K, b, &tiled))
         return gemms_us(M, blocks, K, b) <= gemmt_us(tiled, K, b);
-    return b >= 5 || (K > 1152 && (total <= 12288 || K > 1536));
+    // (a single linear of up to 16 rows at 5 bits and more, 1152..1536 elements: the K-split kernel's 1.10, 1.05, 1.01, 1.00 at 5, 6, 7, 8 bits)
+    if (b >= 5) return M > 16 || K > 1536 || count > 1;
+    return K > 1152 && (total <= 12288 || K > 1536);
 }
 
 // Whether the staged kernel takes a linear or a set in one launch: by its rule in ap_linear and ap_linear_group (`linear`).  ap_gemm_kbit and

@@ -244,3 +244,15 @@ def test_which_calls_the_rule_takes():
         assert _staged([4096], 16, 4096, 4) == 1
     assert _staged([4096], 16, 4096, 9) < 0 and _staged([4096], 0, 4096, 4) < 0 and _staged([64] * 5, 16, 4096, 4) < 0
     assert _staged([1 << 25], 16, 1 << 14, 3) == 0           # planes of 4 GiB and more: beyond 32-bit offsets
+
+
+def test_the_rule_at_a_few_rows_is_one_of_rounds():
+    """Many bits on long rows at 3 and 4 rows: where the CUs are used evenly, one block of 16 rows each or two; and what the kernel is slower at."""
+    for M, b in ((3, 5), (3, 6), (4, 7), (4, 8)):
+        for K in (8320, 11008, 14336):
+            for rows, taken in ((2048, 0), (2944, 0), (3072, 1), (4096, 1), (4112, 0), (5120, 0), (6144, 1), (8192, 1), (8208, 1), (14336, 1)):
+                assert _staged([rows], M, K, b) == taken, (rows, M, K, b)
+    assert [_staged([16384], 4, 5120, b) for b in (4, 5, 6)] == [1, 1, 0]
+    assert [_staged([12288], 12, K, 5) for K in (1152, 1536, 1664)] == [0, 0, 1]
+    assert [_staged([4096] * 3, 3, K, 3) for K in (1024, 2048, 4096)] == [0, 0, 1]
+    assert [_staged([1024] * 3, 6, K, 8) for K in (1280, 2560, 4096)] == [0, 0, 1] and [_staged([1024] * 3, M, 2048, 7) for M in (6, 7, 8)] == [0, 1, 1]
