@@ -303,7 +303,9 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_kernel(
 #pragma unroll
     for (int e = 0; e < 8; e++) acc[e] = 0.f;
     float q[8];
-    // The rotary embedding, and what needs no row of the cache: the new key is the first wave's first.  The rows requested before stay on their way.
+    // The rotary embedding, and what needs no row of the cache: the new key is the first wave's first.  The rows requested before stay on their way
+    // in the waves that only wait here; waves 0 to 2 have theirs when they come to the barrier: loads complete in order, cosines and sines
+    // come behind them, and wave 2 shares the wait.
     auto meet = [&]() {
         fresh_rows();
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -343,10 +345,9 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_kernel(
         }
         m = top;
     };
-    // U steps from step t on; FIRST: the query is not there yet; LAST: the last step may have lanes past the end
-    auto run = [&](auto u_c, auto first_c, auto last_c, int t) {
+    // U steps from step t on, the last of which may have lanes past the end; FIRST: the query is not there yet
+    auto run = [&](auto u_c, auto first_c, int t) {
         constexpr int U = decltype(u_c)::value;
-        constexpr bool LAST = decltype(last_c)::value;
         half8_t k[MOST], v[MOST];
         float s[MOST];
 #pragma unroll
@@ -370,7 +371,7 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_kernel(
                 b += (float)k[u][e + 1] * q[e + 1];
             }
             s[u] = over_key(a + b);
-            if (LAST && u == U - 1 && first + (t + u) * STEP >= pos) {
+            if (u == U - 1 && first + (t + u) * STEP >= pos) {
                 s[u] = -INFINITY;
                 v[u] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
             }
@@ -379,16 +380,16 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_kernel(
     };
     int t = 0;
     if (steps == 0) meet();
-    else if (steps == 1) run(std::integral_constant<int, 1>{}, std::true_type{}, std::true_type{}, 0);
-    else if (steps == 2) run(std::integral_constant<int, 2>{}, std::true_type{}, std::true_type{}, 0);
-    else if (steps == 3) run(std::integral_constant<int, 3>{}, std::true_type{}, std::true_type{}, 0);
+    else if (steps == 1) run(std::integral_constant<int, 1>{}, std::true_type{}, 0);
+    else if (steps == 2) run(std::integral_constant<int, 2>{}, std::true_type{}, 0);
+    else if (steps == 3) run(std::integral_constant<int, 3>{}, std::true_type{}, 0);
     else {
-        run(std::integral_constant<int, 4>{}, std::true_type{}, std::true_type{}, 0);
-        for (t = 4; t + 4 <= steps; t += 4) run(std::integral_constant<int, 4>{}, std::false_type{}, std::true_type{}, t);
+        run(std::integral_constant<int, 4>{}, std::true_type{}, 0);
+        for (t = 4; t + 4 <= steps; t += 4) run(std::integral_constant<int, 4>{}, std::false_type{}, t);
         const int left = steps - t;
-        if (left == 1) run(std::integral_constant<int, 1>{}, std::false_type{}, std::true_type{}, t);
-        else if (left == 2) run(std::integral_constant<int, 2>{}, std::false_type{}, std::true_type{}, t);
-        else if (left == 3) run(std::integral_constant<int, 3>{}, std::false_type{}, std::true_type{}, t);
+        if (left == 1) run(std::integral_constant<int, 1>{}, std::false_type{}, t);
+        else if (left == 2) run(std::integral_constant<int, 2>{}, std::false_type{}, t);
+        else if (left == 3) run(std::integral_constant<int, 3>{}, std::false_type{}, t);
     }
     // ---- the wave's keys together, then the waves'
     float top = m;
