@@ -857,7 +857,7 @@ int run_gemm(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, co
         // one-shot kernel is up to 20 % faster).
         // (By default the block-tile kernel comes first beyond 16 rows except on rows of less than 4096 elements of linears below 20000 rows,
         // and at 9..16 rows of 8192 elements or more: what reaches this rule there is short rows, 4 bits on 20000 rows or more, and calls
-        // with that kernel off.)
+        // with that kernel off.  All of it from the operators: what a module calls is the staged kernel's by then.)
         const bool pays = gemmw_geometry(M, N, K, w_bits, &wgeo) && N >= 40 * wgeo.spw * cu_count() &&
                           (wgeo.spw == 1 ? (M > 16 || w_bits == 8) : (M > 8 || (M >= 5 && w_bits <= 4)));
         if (mode > 0 && (mode >= 2 ? gemmw_geometry(M, N, K, w_bits, &wgeo) : pays)) {
@@ -1061,6 +1061,9 @@ int forced_route(const RouteQuery &q) {
     return -1;
 }
 
+// The routes of ap_matmul_kbit and ap_matmul_kbit_group, ranked among themselves.  A module's call of 3 to 8 rows (ap_linear, ap_linear_group) comes
+// here only where gemms_pays leaves it: of the linears named below the staged kernel has those of more than 2048 rows from 5 activation rows on, most
+// rows of more than 8192 elements at 3 and 4, and at 4 up to 4 bits the wide ones of 4096 elements.
 // M = 1..4.  One route for the whole set.
 int few_rows_route(const RouteQuery &q) {
     const int M = q.M, K = q.K, b = q.w_bits;
@@ -1209,8 +1212,8 @@ int plan_matmul(int M, const int *N, int count, int K, int w_bits, uint16_t *con
 //    to 5 bits -- except, on rows of more than 4096 elements, from 6 bits on linears of 5120 rows or more and from 5
 //    bits on linears of at most 2048 rows; up to 128 on linears of 4096..8191 rows of at most 4096 elements.
 // Beyond, one table lookup per weight and tile of these kernels' activation rows costs more than materialising the weight once.
-// The figures are those of the K-split and tiled kernels.  The rule stays as it is drawn on them, also where the block-tile kernel serves the
-// call by now (14336 x 4096, 256 rows, 8 bits: fused 53, pair 84): it says where calls that autograd or autocast follows are fused.
+// The figures are those of the K-split and tiled kernels.  The rule stays as it is drawn on them, also where the block-tile kernel, or up to 32 rows
+// the staged one, serves the call by now (14336 x 4096, 256 rows, 8 bits: fused 53, pair 84): it says where calls that autograd or autocast follows are fused.
 bool fused_gemm_pays(int M, int N, int K, int b) {
     if (M <= 32) return true;
     if ((K & 127) == 0 && M <= 512) {
@@ -1546,11 +1549,10 @@ static int gemm_set(const uint16_t *x, int count, const uint32_t *const *qweight
     // Tiles of different members run side by side, and the launch costs about what its largest member alone would,
     // while the K-split kernel's launches add up: measured on the q/k/v and gate/up sets of the 7B / 8B / 13B layers at
     // 48..256 rows the one launch is 1.1-3x faster than the members one by one (q/k/v of the 7B layer at 128 rows,
-    // 3 bits: 39 us against 69; of the 13B layer at 64 rows: 31 against 94) wherever there are more than 32 rows.  Sets
-    // whose members all have fewer than 8192 rows (q/k/v) take it from 9 rows on, in tiles of 16 or 32 activation
+    // 3 bits: 39 us against 69; of the 13B layer at 64 rows: 31 against 94) wherever there are more than 32 rows.
     // At 9..32 rows, sets whose members have at most 8192 rows (q/k/v) take it too, in tiles of 16 or 32 activation rows
     // (7B q/k/v at 16 rows: 16-24 us against 23-26 at 3-5 bits; 13B: 20-40 against 36-68; 70B: 21-48 against 39-64); wide
-    // members (gate/up) are within 10 % either way one by one.
+    // members (gate/up) are within 10 % either way one by one.  (In a module's call the staged kernel has most sets of up to 32 rows, gemms_pays.)
     const bool pays = gemmt_set_pays(M, rows, K);
     // (Rows of no multiple of 128 elements are served dense only.)
     if ((count > 1 || strided) && takes_gemms(M, N, count, K, w_bits, linear))

@@ -310,8 +310,8 @@ __global__ __launch_bounds__(WN *WK *kWave) void gemmb_kbit_kernel(const half_t 
 
     // The planes were requested first: their index arithmetic while the tables and the activations, every load behind them, are on
     // their way.  (Fenced on both sides, or the scheduler takes the arithmetic ahead of the wait; and an instruction between, or the
-    // compiler joins the wait with its own at the first use, which is for every load: it does not count across direct loads.  us so, and
-    // with all loads waited for: 1024 x 512 at 512 rows, 4 bits 6.68 / 6.92; 4096 x 768 at 128 rows, 3 bits 5.79 / 5.97; 4096 x 11008 at
+    // compiler joins the wait with its own at the first use.  That one was for every load while the direct loads were global_load_lds,
+    // which are of the FLAT family; then, us so, and with all loads waited for: 1024 x 512 at 512 rows, 4 bits 6.68 / 6.92; 4096 x 768 at 128 rows, 3 bits 5.79 / 5.97; 4096 x 11008 at
     // 128 rows, 4 bits 29.9 / 30.2; of rows of 4096 elements 1 % at most.)
     __builtin_amdgcn_sched_barrier(0);
     {

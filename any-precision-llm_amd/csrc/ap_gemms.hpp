@@ -4,8 +4,9 @@
 // What bounds such a call is the time a wave spends waiting, not the rate of any unit: a linear of a decoder layer has 5..60 MB of planes, a few us
 // at the rate of memory, on workgroups that live for a few steps each.  So a workgroup is small -- 16 weight rows, 4 waves that share the words
 // of K, two or three workgroups a CU -- and every wave keeps its whole next step in flight: the planes in registers, the activations in a ring in
-// LDS that is the wave's own, so that no barrier stands between the tables' and the last one.  The waits count (load_to_lds): a stage is
-// waited for when its products start, while the loads behind it stay out.
+// LDS that is the wave's own, so that no barrier stands between the tables' and the last one.  The waits count (load_to_lds, GemmsOrder): a
+// stage is waited for ahead of its first read, while the loads behind it stay out.  The loads of a wave's first step are the exception: the release
+// ahead of the tables' barrier is for LDS, which direct loads write, and waits for all that is outstanding.
 //  - Activations come by direct loads of rows of 256 bytes, a byte group of a step each; read from global memory by every wave's lanes in
 //    pieces of 16 or 64 bytes, as the other K-split kernel does, they cost more than the weights from 9 rows on.  A row's 16-byte units are
 //    permuted by its number, and the reads of an octet are free of conflicts.
@@ -321,12 +322,12 @@ __global__ __launch_bounds__(kGemmsWaves *kWave, ROWS <= 8 ? 3 : 2) void gemms_k
     __builtin_amdgcn_sched_barrier(0);
     static_for<RING>([&](auto j_c) { stage(step0, j_c); });
     __builtin_amdgcn_sched_barrier(0);
-    wait(std::integral_constant<int, BITS + RING * DMA>{});
+    wait(std::integral_constant<int, BITS + RING * DMA>{});  // the tables, ahead of planes and stages
     put_tables();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    wait(std::integral_constant<int, RING * DMA>{});
+    wait(std::integral_constant<int, RING * DMA>{});  // the planes: holds by the release already, which compiles to a wait for every load
 #pragma unroll
     for (int mb = 0; mb < MB; mb++) acc[mb] = float4_t{0.f, 0.f, 0.f, 0.f};
     int step = step0;

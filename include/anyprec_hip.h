@@ -132,7 +132,8 @@ int ap_gemm_kbit_group(const uint16_t *x, int count, const uint32_t *const *qwei
 
 /* A linear with a bias (fp16 [N]): ap_matmul_kbit up to 8 activation rows, ap_gemm_kbit beyond, the bias added to the fp16 results in
  * the same launch where the kernel that serves the call can (*added = 1); else the results are left without it (*added = 0) and adding
- * it is the caller's.  Same value either way: fp16(fp16(sum) + bias). */
+ * it is the caller's.  Same value either way: fp16(fp16(sum) + bias).
+ * (AnyPrecisionLinear calls ap_linear, which also has the staged kernel.) */
 int ap_linear_bias(const uint16_t *x, const uint32_t *qweight, const uint16_t *lut, const uint16_t *bias, uint16_t *out,
                    int M, int N, int K, int w_bits, void *stream, int *added);
 
