@@ -1691,23 +1691,27 @@ int ap_gemm_kbit_taken(int M, int N, int K, int w_bits) {
 
 // Small linears, beside what ap_gemm_kbit_taken says: a caller that issues dequant_kbit and a library GEMM one call at a time waits 23 us for the
 // host to issue the two, whatever their size, and 5 for a fused GEMM.  The line is drawn where the fused form is the faster one on the device
-// as well, so that a stream that is busy, a captured graph and the call that warmed it up all take the same form.  Device time of the pair and of the
-// fused form, of 21700 drawn linears of 256..14336 rows at 33..1024 activation rows (and fewer than 1.4e10 products):
-//  - one launch of the K-split kernel on short rows: 0.70 of the pair's time on average, by more than 3 % slower in 1 of 100 (66 x 3719 x 416, 4 bits
-//    12.1 / 5.9; 93 x 262 x 416, 8 bits 10.0 / 6.3; 106 x 1072 x 1504, 4 bits 15.7 / 10.0).  Longer rows and several launches lose up to 1.9 times
-//    (126 x 343 x 4448, 8 bits 16.9 / 29.5; 240 x 749 x 448, 6 bits 9.4 / 16.0);
-//  - the tiled kernel up to 6 bits where its estimate is below 0.65 of pair_us, which is high by a third here: 0.77 on average, 1 of 200 slower (373 x 756 x
-//    512, 3 bits 10.0 / 6.2); at 7 and 8 bits half of them are (904 x 965 x 640, 7 bits 11.1 / 21.1).
-// (Sizes as rows x N x K.)
+// as well, so that a stream that is busy, a captured graph and the call that warmed it up all take the same form.  Drawn on the device times of both for
+// 21700 linears of 256..14336 rows at 33..1024 activation rows.  The pair at these sizes (pair_us, fitted on larger ones, is 12 % high here) and one
+// launch of the K-split kernel on rows of no multiple of 128 elements -- blocks of 16 activation rows, steps of 4 words of the average and of the busiest
+// of 8 waves, workgroups a CU -- are estimated to 7 and 9 % on average; the tiled kernel's estimate has to be 10 % below the pair's.  The 3377 that it takes run
+// in 0.75 of the pair's time (66 x 3719 x 416, rows x N x K, 4 bits 12.1 / 5.9 us; 106 x 1072 x 1504, 4 bits 15.7 / 10.0; 373 x 756 x 512, 3 bits 10.0 / 6.2),
+// 1.6 % of them are more than 3 % slower, at most by 19 % (of 1993 drawn anew: 0.75, 2.4 %, 25 %).  Beyond, the fused forms lose: several launches of the K-split kernel up to 1.9 times
+// (240 x 749 x 448, 6 bits 9.4 / 16.0), the tiled kernel at many bits (904 x 965 x 640, 7 bits 11.1 / 21.1), the block-tile kernel in half of the calls.
 int ap_gemm_kbit_quick(int M, int N, int K, int w_bits) {
     const int rc = ap_gemm_kbit_taken(M, N, K, w_bits);
-    if (rc != 0 || N < 256 || N > 14336 || (double)M * N * K >= 1.4e10 || knob(kGemmBlock) != 1 || knob(kGemmTiled) != 1) return rc;
+    if (rc != 0 || M > 1024 || N < 256 || N > 14336 || knob(kGemmBlock) != 1 || knob(kGemmTiled) != 1) return rc;
+    const double pair = 8.82 + 9.87e-7 * N * K + 3.158e-9 * M * N * K + 1.129e-3 * K + 4.35e-4 * N;
+    if (pair > 26) return 0;  // (longer ones do not wait for the host)
     GemmbGeometry block;
     GemmtGeometry tiled;
     if (takes_gemmb(M, N, K, w_bits, &block)) return 0;
-    if (gemmt_pays(M, N, K, w_bits) && gemmt_geometry(M, (N + 63) / 64, K, w_bits, &tiled))
-        return w_bits <= 6 && gemmt_us(tiled, K, w_bits) <= 0.65 * pair_us(M, N, K, w_bits) ? 1 : 0;
-    return (K & 127) != 0 && M <= kGemmMaxM && K <= (M <= 96 ? 2048 : 1024) ? 1 : 0;
+    if (gemmt_pays(M, N, K, w_bits) && gemmt_geometry(M, (N + 63) / 64, K, w_bits, &tiled)) return gemmt_us(tiled, K, w_bits) <= 0.9 * pair ? 1 : 0;
+    if ((K & 127) == 0 || M > kGemmMaxM) return 0;
+    const int steps = ((K >> 5) + 3) / 4, mb = (M + 15) / 16;
+    const double load = (N + 15) / 16 / (double)cu_count(), wgs = fmax(1.0, load);
+    const double us = 2.504 + 0.31 * mb + (K / 1024.0) * mb * (0.117 * fmin(1.0, load) + 0.559 * wgs) + 0.153 * ((steps + 7) / 8) * wgs * w_bits;
+    return us <= pair ? 1 : 0;
 }
 
 int ap_gemm_kbit_group_taken(int count, const int *N, int M, int K, int w_bits) {
